@@ -100,10 +100,13 @@ struct fl_terrain {
   uint32_t jump_rounds = 4;  // pointer-jumping rounds of the previous iteration
   uint32_t last_rounds = 0;  // sweep rounds of the previous iteration
   std::vector<uint32_t> last_boff;  // its bucket offsets (boff[nb+1], bnoff[nb+1]): launch-size estimates
-  uint32_t tail_split = 0;          // first round of the pipelined iterations' tail launches
-  uint32_t tail_units = FL_TAIL_WAVES;  // rounds of at most this many fold units go to the tail launches
+  uint32_t tail_units = FL_TAIL_WAVES;  // synchronous iterations: rounds of at most this many units go to the tail launches
+  // a sweep's wait ended without its value (FL_FLAG_STALL): the hand-over
+  // words are reset, and the terrain's later iterations run every round
+  // behind barriers
+  bool stalled = false, reset_words = false;
   // captured pipelined iterations, one per elevation-buffer parity, for the
-  // (jump rounds, sweep rounds) they were captured with
+  // jump rounds they were captured with
   // elevation buffers: an iteration reads hb[i] and writes hb[(i+1) % 3], so
   // an iteration in flight never overwrites the input of the one before it
   double* hb[3] = {nullptr, nullptr, nullptr};
@@ -123,7 +126,7 @@ struct fl_terrain {
   // synchronously and takes subtree sizes as its heavy-child hint
   bool hint_stale = false;
   hipGraphExec_t gexec[3] = {nullptr, nullptr, nullptr};
-  uint32_t gJ[3] = {0, 0, 0}, gR[3] = {0, 0, 0}, gS[3] = {0, 0, 0};
+  uint32_t gJ[3] = {0, 0, 0}, gW[3] = {0, 0, 0};
   int gF[3] = {0, 0, 0};
   // launch tuning a graph was captured with (workgroup size, long-chain
   // cutoff): another tuning captures afresh, so that it is the one timed
@@ -421,7 +424,7 @@ fl_tuning effective_tuning(const fl_ctx* c, uint64_t sites, uint32_t terrains) {
       t.compact_min_idle = r.compact_min_idle;
       break;
     }
-  if (!t.site_block) t = fl_tuning{256, 6, FL_TAIL_WAVES, 1, 1u << 16, {0, 0, 0}};
+  if (!t.site_block) t = fl_tuning{256, 16, FL_TAIL_WAVES, 1, 1u << 16, {0, 0, 0}};
   if (c->tune_set & 2) t.pipelining = c->tune.pipelining;
   if (c->tune_set & 4) t.compact_min_idle = c->tune.compact_min_idle;
   return t;
@@ -446,7 +449,7 @@ struct TuneScope {
     c->graphs = t.pipelining == 3 && !c->forbid_graphs;
     c->compact_min_idle = t.compact_min_idle;
     if (T) {
-      T->w.long_min = t.long_chain;
+      T->w.long_min = std::min<uint32_t>(t.long_chain, FL_LONG_MAX);
       T->tail_units = t.tail_units;
     }
   }
@@ -665,10 +668,10 @@ int32_t decompose(fl_ctx* c, fl_terrain* T, bool full, bool joined) {
   T->jump_rounds = quiet + 1;
   w.guard = w.ctrl + FL_CTRL_JUMPS + (round - 1);  // a round at or after the quiet one: zero
   fl_launch_chain_count(s, T->t, w);
-  fl_launch_chain_layout(s, T->t, w, 0);
+  fl_launch_chain_layout(s, T->t, w);
   FLCHK(read_ctrl(c, T));
   uint32_t nb = 2 * (host_counter(c, FL_CNT_MAXLD) + 1);  // short and long bucket per light depth
-  if (nb > 2 * n + 2) return set_err(FL_ERR_HIP, "light depth out of range");
+  if (nb > n + 2) return set_err(FL_ERR_HIP, "light depth out of range");
   T->prev_nb = nb;
   c->host_boff.resize(2 * (nb + 1));
   if (nb <= FL_CTRL_HEAD) {
@@ -687,25 +690,32 @@ int32_t decompose(fl_ctx* c, fl_terrain* T, bool full, bool joined) {
   return FL_OK;
 }
 
-// Launch shape of round l from bucket offsets (boff[nb+1] then bnoff[nb+1]).
-fl_round_grid exact_grid(const std::vector<uint32_t>& off, uint32_t l) {
-  uint32_t nb = (uint32_t)off.size() / 2 - 1;
+// Sweep units of round l from bucket offsets (boff[nb+1] then bnoff[nb+1]):
+// its long chains and the tiles of its short chains' positions; positions:
+// all of its positions.
+struct RoundSize {
+  uint32_t units = 0;
+  uint64_t positions = 0;
+};
+RoundSize round_size(const std::vector<uint32_t>& off, uint32_t l, uint32_t long_min) {
+  const uint32_t nb = (uint32_t)off.size() / 2 - 1;
   const uint32_t* bo = off.data();
   const uint32_t* bn = bo + nb + 1;
-  fl_round_grid g{};
-  if (2 * l + 2 > nb) return g;
-  g.positions = bn[2 * l + 2] - bn[2 * l];
-  g.fold_blocks = (bo[2 * l + 2] - bo[2 * l + 1]) + (bo[2 * l + 1] - bo[2 * l] + 63) / 64;
-  return g;
+  RoundSize r;
+  if (2 * l + 2 > nb) return r;
+  const uint32_t stride = 65 - long_min;
+  r.positions = bn[2 * l + 2] - bn[2 * l];
+  r.units = (bo[2 * l + 2] - bo[2 * l + 1]) + (bn[2 * l + 1] - bn[2 * l] + stride - 1) / stride;
+  return r;
 }
 
 // First round of the tail launches: the rounds from it on each hold at most
-// `units` fold units (tuned; the tail's FL_TAIL_WAVES wavefronts loop over
+// `units` sweep units (tuned; the tail's FL_TAIL_WAVES wavefronts loop over
 // more); `rounds` (no tail) when fewer than two rounds qualify, as one round
 // gains nothing.
-uint32_t tail_start(const std::vector<uint32_t>& off, uint32_t rounds, uint32_t units) {
+uint32_t tail_start(const std::vector<uint32_t>& off, uint32_t rounds, uint32_t long_min, uint32_t units) {
   uint32_t l = rounds;
-  while (l > 0 && exact_grid(off, l - 1).fold_blocks <= units) l--;
+  while (l > 0 && round_size(off, l - 1, long_min).units <= units) l--;
   return rounds - l >= 2 ? l : rounds;
 }
 
@@ -716,10 +726,14 @@ uint64_t all_positions(const std::vector<uint32_t>& off) {
   return off.back();
 }
 
-uint64_t tail_positions(const std::vector<uint32_t>& off, uint32_t from, uint32_t rounds) {
-  uint64_t units = 0;
-  for (uint32_t l = from; l < rounds; l++) units += exact_grid(off, l).positions;
-  return units;
+RoundSize rounds_size(const std::vector<uint32_t>& off, uint32_t from, uint32_t to, uint32_t long_min) {
+  RoundSize sum;
+  for (uint32_t l = from; l < to; l++) {
+    const RoundSize r = round_size(off, l, long_min);
+    sum.units += r.units;
+    sum.positions += r.positions;
+  }
+  return sum;
 }
 
 // A decomposition far deeper than subtree-size heavy children allow (light
@@ -744,7 +758,12 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
   hipStream_t s = c->stream;
   fl_dev_work& w = T->w;
   uint32_t n = T->t.n;
-  fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, 2 * n + 2));
+  const bool hint_stale = T->hint_stale;
+  if (T->reset_words) {
+    fl_launch_reset_words(s, T->t, w);
+    T->reset_words = false;
+  }
+  fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, n + 2));
   fl_launch_receivers(s, T->t, w, keep, !full);
   if (T->hint_stale) {
     // the heavy children follow subtree sizes of the final tree: with the
@@ -754,7 +773,7 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
     *had_lake = host_flag(c, FL_FLAG_LAKE) != 0;
     if (*had_lake) {
       FLCHK(join_lakes(c, T));
-      fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, 2 * n + 2));
+      fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, n + 2));
     }
     // sizes of the whole forest: sites of basins kept from the previous tree
     // get them too (their drainage areas are read by no recomputed basin)
@@ -768,13 +787,13 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
     *had_lake = host_flag(c, FL_FLAG_LAKE) != 0;
     if (*had_lake) {
       FLCHK(join_lakes(c, T));
-      fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, 2 * n + 2));
+      fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, n + 2));
       FLCHK(decompose(c, T, full, true));
     }
     if (deep_rounds(c, T->last_rounds, n)) {
       // decompose again with subtree sizes as the hint
       std::string err;
-      fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, 2 * n + 2));
+      fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, n + 2));
       if (fl_device_subtree_sizes(s, n, w.next, T->d_tid, T->d_active, w.A, &err, &T->arena) != FL_OK)
         return set_err(FL_ERR_HIP, "%s", err.c_str());
       T->stat_rehinted++;
@@ -785,82 +804,68 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
   const std::vector<uint32_t>& off = c->host_boff;
   bool clamp = T->t.any_max_slope;
   uint32_t rounds = nb / 2;
-  // the deep rounds, which hold few chains, go to one launch per sweep
-  uint32_t split = tail_start(off, rounds, T->tail_units);
-  uint64_t tail_units = tail_positions(off, split, rounds);
-  if (split < rounds) fl_launch_da_tail(s, T->t, w, split, rounds - 1, tail_units, clamp);
-  for (uint32_t l = split; l-- > 0;) fl_launch_da_round(s, T->t, w, l, exact_grid(off, l), clamp);
-  for (uint32_t l = 0; l < split; l++) fl_launch_tau_round(s, T->t, w, l, exact_grid(off, l), clamp);
-  if (split < rounds) fl_launch_tau_tail(s, T->t, w, split, rounds - 1, tail_units, clamp);
+  // the deep rounds, which hold few units, behind barriers in one workgroup
+  // (every round of a terrain whose waits have ended without their values),
+  // the others in one launch
+  const uint32_t lm = w.long_min;
+  const uint32_t split = T->stalled ? 0 : tail_start(off, rounds, lm, T->tail_units);
+  const RoundSize flow = rounds_size(off, 0, split, lm), tail = rounds_size(off, split, rounds, lm);
+  if (split < rounds) fl_launch_da_tail(s, T->t, w, split, tail.positions, clamp);
+  if (split > 0) fl_launch_da_fold(s, T->t, w, split, flow.units, flow.positions, clamp);
+  if (split > 0) fl_launch_tau_fold(s, w, split, flow.units, flow.positions, clamp);
+  if (split < rounds) fl_launch_tau_tail(s, w, split, tail.positions, clamp);
   if (T->d_tchanged) fl_launch_fill_u32(s, T->d_tchanged, T->nterr, 0);
   fl_launch_tau_scatter(s, T->t, w, clamp, T->d_tid, T->d_active, T->d_tchanged);
   if (T->d_tchanged)
     HIPCHK(hipMemcpyAsync(T->h_tchanged, T->d_tchanged, T->nterr * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   FLCHK(read_ctrl(c, T));
+  if (host_flag(c, FL_FLAG_STALL)) {
+    // its input is untouched: once more, without waits
+    if (T->stalled) return set_err(FL_ERR_HIP, "a sweep did not finish");
+    T->stalled = T->reset_words = true;
+    T->hint_stale = hint_stale;
+    return one_iteration(c, T, full, keep, changed, had_lake);
+  }
   *changed = host_flag(c, FL_FLAG_CHANGED) != 0;
   std::swap(w.h, w.h2);
   if (*had_lake) T->hint_stale = true;
   return FL_OK;
 }
 
-// The kernels of one pipelined iteration (J jump rounds, R sweep rounds,
-// rounds S..R-1 in the tail launches), enqueued on the context's stream or
-// recorded by a capture.  rec_* receive the profiler records of the launches
-// (when profiling).
-void enqueue_fast_body(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t R, uint32_t S, bool full, bool keep,
-                       std::vector<size_t>* rec_da, std::vector<size_t>* rec_tau, size_t* rec_tail,
-                       size_t* rec_scatter) {
+// The kernels of one pipelined iteration (J jump rounds, sweeps of W
+// wavefronts), enqueued on the context's stream or recorded by a capture.
+// rec_* receive the profiler records of the launches (when profiling).
+void enqueue_fast_body(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool full, bool keep, size_t* rec_da,
+                       size_t* rec_tau) {
   hipStream_t s = c->stream;
   fl_dev_work& w = T->w;
   uint32_t n = T->t.n;
   bool clamp = T->t.any_max_slope;
-  // the previous iteration used 2 * (R - 1) bucket entries at most
-  fl_launch_clear_iter(s, w, std::min<uint32_t>(2 * R + 1, 2 * n + 2));
+  // the bucket entries that the previous iteration used
+  fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, n + 2));
   fl_launch_receivers(s, T->t, w, keep, !full);
   fl_launch_children(s, T->t, w, full, T->d_tid, T->d_active);
   for (uint32_t r = 0; r < J; r++) fl_launch_chain_jump(s, T->t, w, r);
   w.guard = w.ctrl + FL_CTRL_JUMPS + (J - 1);
   fl_launch_chain_count(s, T->t, w);
-  fl_launch_chain_layout(s, T->t, w, R);
-  // launch sizes from the previous iteration's rounds (grid-stride kernels:
-  // any size is correct), profiler units filled in once the bounds are known
-  uint32_t fold_default = std::max<uint32_t>(1, std::min<uint32_t>((n + 127) / 128, 8192));
-  auto guess = [&](uint32_t l) {
-    fl_round_grid g = T->last_boff.empty() ? fl_round_grid{} : exact_grid(T->last_boff, l);
-    g.fold_blocks = g.fold_blocks ? std::min<uint32_t>(g.fold_blocks + g.fold_blocks / 4 + 8, fold_default) : 8;
-    if (T->last_boff.empty()) g.fold_blocks = fold_default;
-    g.positions = 0;
-    return g;
-  };
-  if (S < R) {
-    if (c->prof && rec_tail) rec_tail[0] = c->prof->pending.size();
-    fl_launch_da_tail(s, T->t, w, S, R - 1, 0, clamp);
-  }
-  for (uint32_t l = S; l-- > 0;) {
-    if (c->prof && rec_da) (*rec_da)[l] = c->prof->pending.size();
-    fl_launch_da_round(s, T->t, w, l, guess(l), clamp);
-  }
-  for (uint32_t l = 0; l < S; l++) {
-    if (c->prof && rec_tau) (*rec_tau)[l] = c->prof->pending.size();
-    fl_launch_tau_round(s, T->t, w, l, guess(l), clamp);
-  }
-  if (S < R) {
-    if (c->prof && rec_tail) rec_tail[1] = c->prof->pending.size();
-    fl_launch_tau_tail(s, T->t, w, S, R - 1, 0, clamp);
-  }
+  fl_launch_chain_layout(s, T->t, w);
+  if (c->prof && rec_da) *rec_da = c->prof->pending.size();
+  fl_launch_da_fold(s, T->t, w, FL_NONE_ROUND, W, 0, clamp);
+  if (c->prof && rec_tau) *rec_tau = c->prof->pending.size();
+  fl_launch_tau_fold(s, w, FL_NONE_ROUND, W, 0, clamp);
   if (T->d_tchanged) fl_launch_fill_u32(s, T->d_tchanged, T->nterr, 0);
-  if (c->prof && rec_scatter) *rec_scatter = c->prof->pending.size();
   fl_launch_tau_scatter(s, T->t, w, clamp, T->d_tid, T->d_active, T->d_tchanged);
 }
 
-// The pipelined iteration for (J, R) and the current buffer parity as a
+// The pipelined iteration for J and the current buffer parity as a
 // graph, captured on first use.  False when capture is not possible (the
 // caller launches directly).
-bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t R, uint32_t S, bool full, bool keep) {
+bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool full, bool keep) {
   if (T->graphs_failed) return false;
   int p = T->w.h == T->hb[0] ? 0 : (T->w.h == T->hb[1] ? 1 : 2);
   const int mode = (full ? 1 : 0) | (keep ? 2 : 0);
-  if (!T->gexec[p] || T->gJ[p] != J || T->gR[p] != R || T->gS[p] != S || T->gF[p] != mode ||
+  // (a captured launch size serves until the units differ by more than half)
+  if (!T->gexec[p] || T->gJ[p] != J || W > T->gW[p] + T->gW[p] / 2 || T->gW[p] > W + W / 2 || T->gF[p] != mode ||
       T->gB[p] != fl_site_block || T->gL[p] != T->w.long_min) {
     if (T->gexec[p]) {
       hipGraphExecDestroy(T->gexec[p]);
@@ -871,7 +876,7 @@ bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t R, uint32_
       T->graphs_failed = true;
       return false;
     }
-    enqueue_fast_body(c, T, J, R, S, full, keep, nullptr, nullptr, nullptr, nullptr);
+    enqueue_fast_body(c, T, J, W, full, keep, nullptr, nullptr);
     hipError_t e = hipStreamEndCapture(c->stream, &graph);
     if (e == hipSuccess) e = hipGraphInstantiate(&T->gexec[p], graph, nullptr, nullptr, 0);
     if (graph) hipGraphDestroy(graph);
@@ -882,8 +887,7 @@ bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t R, uint32_
       return false;
     }
     T->gJ[p] = J;
-    T->gR[p] = R;
-    T->gS[p] = S;
+    T->gW[p] = W;
     T->gF[p] = mode;
     T->gB[p] = fl_site_block;
     T->gL[p] = T->w.long_min;
@@ -897,44 +901,34 @@ struct Flight {
   int slot = 0;
   bool full = false;  // every basin recomputed (no previous tree)
   bool keep = false;  // receivers kept where the neighbourhood did not change
-  uint32_t J = 0, R = 0, S = 0;
+  uint32_t J = 0;
   std::vector<uint8_t> mask;  // terrains iterating in it
-  std::vector<size_t> rec_da, rec_tau;
-  size_t rec_tail[2] = {SIZE_MAX, SIZE_MAX};
-  size_t rec_scatter = SIZE_MAX;
+  size_t rec_da = SIZE_MAX, rec_tau = SIZE_MAX;
 };
 
 // One outer iteration enqueued whole, without waiting for the previous one.
-// Three things are taken from the last confirmed iteration instead of being
+// Two things are taken from the last confirmed iteration instead of being
 // read back in between: the number of pointer-jumping rounds (one more is
-// launched; a round after a quiet one returns at once), the number of sweep
-// rounds (one more; rounds past the deepest light depth are empty, their
-// bounds read on the device) and the absence of lakes.  Its control block
-// and changed flags are copied to the host slot f.slot and an event marks
-// its end.
+// launched; a round after a quiet one returns at once) and the absence of
+// lakes.  The sweeps' launch size follows its sweep units (any size is
+// correct).  Its control block and changed flags are copied to the host slot
+// f.slot and an event marks its end.
+constexpr uint32_t FL_SWEEP_WAVES = 8192;  // more wavefronts than run at once gain nothing
 int32_t enqueue_fast(fl_ctx* c, fl_terrain* T, Flight& f) {
   hipStream_t s = c->stream;
   fl_dev_work& w = T->w;
   f.J = std::min<uint32_t>(T->jump_rounds + 1, FL_MAX_JUMP_ROUNDS);
-  f.R = std::max<uint32_t>(T->last_rounds, 1) + 1;
-  if (c->pipelined == 2) f.J = f.R = 1;
-  // tail launches for the rounds that were small in the last confirmed
-  // iteration; a split within one round of the previous one is kept (the
-  // captured graphs stay valid)
-  f.S = f.R;
+  if (c->pipelined == 2) f.J = 1;
+  uint32_t W = (T->t.n + 63) / 64;
   if (!T->last_boff.empty()) {
-    uint32_t want = tail_start(T->last_boff, f.R, T->tail_units);
-    uint32_t keep = T->tail_split;
-    f.S = (want < f.R && keep < f.R && want + 1 >= keep && want <= keep + 1) ? keep : want;
+    const uint32_t u = rounds_size(T->last_boff, 0, T->last_rounds, T->w.long_min).units;
+    W = std::min<uint32_t>(u + u / 4 + FL_FOLD_WAVES, T->t.n);
   }
-  T->tail_split = f.S;
+  W = std::min<uint32_t>(W, FL_SWEEP_WAVES);
   set_slots(T, f.in);
-  f.rec_da.assign(f.R, SIZE_MAX);
-  f.rec_tau.assign(f.R, SIZE_MAX);
-  f.rec_tail[0] = f.rec_tail[1] = SIZE_MAX;
-  bool graphed = !c->prof && c->graphs && launch_fast_graph(c, T, f.J, f.R, f.S, f.full, f.keep);
-  if (!graphed)
-    enqueue_fast_body(c, T, f.J, f.R, f.S, f.full, f.keep, &f.rec_da, &f.rec_tau, f.rec_tail, &f.rec_scatter);
+  f.rec_da = f.rec_tau = SIZE_MAX;
+  bool graphed = !c->prof && c->graphs && launch_fast_graph(c, T, f.J, W, f.full, f.keep);
+  if (!graphed) enqueue_fast_body(c, T, f.J, W, f.full, f.keep, &f.rec_da, &f.rec_tau);
   if (T->d_tchanged)
     HIPCHK(hipMemcpyAsync(T->h_tslot[f.slot], T->d_tchanged, T->nterr * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   HIPCHK(hipMemcpyAsync(c->host_slot[f.slot], w.ctrl, FL_CTRL_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
@@ -944,8 +938,8 @@ int32_t enqueue_fast(fl_ctx* c, fl_terrain* T, Flight& f) {
 
 // Wait for flight f and check what it assumed.  *valid is false when any
 // assumption failed: the decomposition had not converged (the kernels after
-// it then did nothing), a lake was found, or the tree was deeper.  Its input
-// hb[f.in] is untouched either way.  *changed: the changed flag; per-terrain
+// it then did nothing), a lake was found, or a sweep's wait ended without its
+// value.  Its input hb[f.in] is untouched either way.  *changed: the changed flag; per-terrain
 // flags are in T->h_tslot[f.slot].
 int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool* changed) {
   HIPCHK(hipEventSynchronize(c->slot_ev[f.slot]));
@@ -961,13 +955,17 @@ int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool
     T->jump_rounds = std::max(T->jump_rounds, f.J + 1);
     return FL_OK;
   }
-  if (nb > 2 * n + 2) return set_err(FL_ERR_HIP, "light depth out of range");
+  if (nb > n + 2) return set_err(FL_ERR_HIP, "light depth out of range");
   for (uint32_t r = 0; r < f.J; r++)
     if (hc[FL_CTRL_JUMPS + r] == 0) {
       T->jump_rounds = r + 1;
       break;
     }
-  if (lake || nb / 2 > f.R) return FL_OK;
+  if (hc[FL_FLAG_STALL]) {
+    T->stalled = T->reset_words = true;
+    return FL_OK;
+  }
+  if (lake) return FL_OK;
   *valid = true;
   T->prev_nb = nb;
   T->last_rounds = nb / 2;
@@ -982,14 +980,8 @@ int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool
     T->last_boff.assign(head, head + nb + 1);
     T->last_boff.insert(T->last_boff.end(), head + FL_CTRL_HEAD + 1, head + FL_CTRL_HEAD + 1 + nb + 1);
     if (c->prof) {
-      for (uint32_t l = 0; l < f.R; l++) {
-        uint64_t units = exact_grid(T->last_boff, l).positions;
-        for (size_t q : {f.rec_da[l], f.rec_tau[l]})
-          if (q < c->prof->pending.size()) c->prof->pending[q].units = units;
-      }
-      uint64_t tail_units = tail_positions(T->last_boff, f.S, f.R);
-      for (size_t q : f.rec_tail)
-        if (q < c->prof->pending.size()) c->prof->pending[q].units = tail_units;
+      for (size_t q : {f.rec_da, f.rec_tau})
+        if (q < c->prof->pending.size()) c->prof->pending[q].units = all_positions(T->last_boff);
     }
   } else {
     T->last_boff.clear();
@@ -1211,21 +1203,23 @@ int32_t layout_device(fl_terrain* P, uint32_t n, uint32_t nnz, uint32_t count, b
   }
   FLCHK(dev_alloc(P, &w.dirty, n));
   FLCHK(dev_alloc(P, &w.act, n));
-  FLCHK(dev_alloc(P, &w.cval, 4 * (uint64_t)n));
+  FLCHK(dev_alloc(P, &w.cval, (uint64_t)FL_LIST * n));
   FLCHK(dev_alloc(P, &P->hb[2], n));
   P->hb[0] = w.h;
   P->hb[1] = w.h2;
   set_slots(P, 0);
   if (clamp)
-    for (double** p : {&w.hnp, &w.up, &w.tanp, &w.dp, &w.hop}) FLCHK(dev_alloc(P, p, n));
-  for (uint32_t** p : {&w.sub, &w.sub2, &w.hc, &w.pcnt, &w.pdest, &w.head_chain, &w.head_base, &w.perm})
+    for (double** p : {&w.hnp, &w.up, &w.tanp, &w.hop}) FLCHK(dev_alloc(P, p, n));
+  if (clamp) FLCHK(dev_alloc(P, &w.pro, n));
+  for (uint32_t** p : {&w.sub, &w.sub2, &w.hc, &w.pcnt, &w.pdest, &w.ppos, &w.head_base, &w.perm})
     FLCHK(dev_alloc(P, p, n));
+  FLCHK(dev_alloc(P, &w.cover, n));
   FLCHK(dev_alloc(P, &w.cmeta, n));
   FLCHK(dev_alloc(P, &w.cp, n));
   FLCHK(dev_alloc(P, &w.rt, n));
   FLCHK(dev_alloc(P, &w.cmask, n));
-  for (uint32_t** p : {&w.bcnt, &w.bnodes, &w.boff, &w.bnoff, &w.bcur, &w.bncur})
-    FLCHK(dev_alloc(P, p, 2 * (uint64_t)n + 4));
+  for (uint32_t** p : {&w.bcnt, &w.bnodes, &w.boff, &w.bnoff, &w.bcur, &w.bncur, &w.ucum})
+    FLCHK(dev_alloc(P, p, (uint64_t)n + FL_BUCKET_PAD));
   FLCHK(dev_alloc(P, &w.lake_key, n));
   FLCHK(dev_alloc(P, &w.ctrl, FL_CTRL_WORDS));
   w.flags = (int*)w.ctrl;
@@ -1291,10 +1285,11 @@ int32_t alloc_device(fl_ctx* c, fl_terrain* P, uint32_t n, uint32_t nnz, uint32_
   // basin roots are site indices at all times (dirty-basin marks index by them)
   for (int k = 0; k < 3; k++) fl_launch_fill_u32(s, P->rtb[k], n, 0);
   P->prev_valid = false;
-  fl_launch_fill_u32(s, w.bcnt, 2 * (uint64_t)n + 4, 0);
-  fl_launch_fill_u32(s, w.bnodes, 2 * (uint64_t)n + 4, 0);
-  fl_launch_fill_u32(s, w.bcur, 2 * (uint64_t)n + 4, 0);
-  fl_launch_fill_u32(s, w.bncur, 2 * (uint64_t)n + 4, 0);
+  fl_launch_fill_u32(s, w.bcnt, (uint64_t)n + FL_BUCKET_PAD, 0);
+  fl_launch_fill_u32(s, w.bnodes, (uint64_t)n + FL_BUCKET_PAD, 0);
+  fl_launch_fill_u32(s, w.bcur, (uint64_t)n + FL_BUCKET_PAD, 0);
+  fl_launch_fill_u32(s, w.bncur, (uint64_t)n + FL_BUCKET_PAD, 0);
+  fl_launch_reset_words(s, P->t, w);
   P->prev_nb = 0;
   return FL_OK;
 }
@@ -1838,7 +1833,7 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
     // the first iteration, those whose heavy-child hint is stale (after lake
     // joins: a deep decomposition there would also make a poor speculation
     // for the iterations after it) and the unpipelined form
-    if (it == 0 || (cur->hint_stale && q.empty()) || !c->pipelined) {
+    if (it == 0 || ((cur->hint_stale || cur->stalled) && q.empty()) || !c->pipelined) {
       bool changed = false, lake = false;
       std::vector<uint8_t> mask(cur->t_active);
       FLCHK(upload_mask(mask));
@@ -1858,7 +1853,7 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
     } else {
       // keep two iterations in flight: the host enqueues the next one while
       // the device runs the current one
-      while (!drain && !cur->hint_stale && q.size() < 2) {
+      while (!drain && !cur->hint_stale && !cur->stalled && q.size() < 2) {
         std::vector<uint8_t> mask(cur->nterr);
         bool any = false;
         for (uint32_t g = 0; g < cur->nterr; g++) {
@@ -2203,7 +2198,7 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
     }
   };
   const double* result = nullptr;  // the buffer holding the confirmed iteration's elevations
-  if (L->sync_next || (cur->hint_stale && L->q.empty()) || !c->pipelined) {
+  if (L->sync_next || ((cur->hint_stale || cur->stalled) && L->q.empty()) || !c->pipelined) {
     std::vector<uint8_t> mask(cur->t_active);
     FLCHK(lane_upload_mask(L, mask));
     set_slots(cur, L->hin);
@@ -2221,7 +2216,7 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
   } else {
     // a drain for a join whose terrains went to another lane: go on
     if (L->drain && L->q.empty() && !L->compact_wanted) L->drain = false;
-    while (!L->drain && !cur->hint_stale && L->q.size() < 2) {
+    while (!L->drain && !cur->hint_stale && !cur->stalled && L->q.size() < 2) {
       std::vector<uint8_t> mask(cur->nterr);
       bool any = false;
       for (uint32_t g = 0; g < cur->nterr; g++) {
@@ -2463,7 +2458,7 @@ extern "C" int32_t fl_stage_receivers(fl_ctx* c, fl_terrain* T, const double* el
   if (T->t.n == 0) return FL_OK;
   HIPCHK(hipSetDevice(c->device));
   FLCHK(upload_h(c, T, elev));
-  fl_launch_clear_iter(c->stream, T->w, std::min<uint32_t>(T->prev_nb + 1, 2 * T->t.n + 2));
+  fl_launch_clear_iter(c->stream, T->w, std::min<uint32_t>(T->prev_nb + 1, T->t.n + 2));
   fl_launch_receivers(c->stream, T->t, T->w, false, false);
   return download_idx_old(c, T, next_out, T->w.next);
 }
@@ -2476,7 +2471,7 @@ extern "C" int32_t fl_stage_stream_tree(fl_ctx* c, fl_terrain* T, const double* 
   if (T->t.n == 0) return FL_OK;
   HIPCHK(hipSetDevice(c->device));
   FLCHK(upload_h(c, T, elev));
-  fl_launch_clear_iter(c->stream, T->w, std::min<uint32_t>(T->prev_nb + 1, 2 * T->t.n + 2));
+  fl_launch_clear_iter(c->stream, T->w, std::min<uint32_t>(T->prev_nb + 1, T->t.n + 2));
   fl_launch_receivers(c->stream, T->t, T->w, false, false);
   FLCHK(read_ctrl(c, T));
   bool lake = host_flag(c, FL_FLAG_LAKE) != 0;
@@ -2595,7 +2590,7 @@ extern "C" int32_t fl_autotune(fl_ctx* c, fl_terrain* T, uint32_t repeats, fl_tu
   const double table_time = cur_ms;
   // coordinate descent, two passes; a candidate replaces the current one
   // only when it is faster by more than 1% (timing noise)
-  const std::vector<uint32_t> chains = {3, 4, 6, 8, 12, 16, 24}, tails = {0, 8, 16, 32, 64},
+  const std::vector<uint32_t> chains = {6, 8, 12, 16, 24, 33}, tails = {0, 8, 16, 32, 64},
                               blocks = {128, 256, 512, 1024}, pipes = {1, 3},
                               compacts = {16384, 65536, 262144, 0xffffffffu};
   for (int pass = 0; pass < 2 && rc == FL_OK; pass++) {
@@ -2737,7 +2732,7 @@ extern "C" int32_t fl_stage_basin_order(fl_ctx* c, fl_terrain* T, const double* 
   uint32_t n = T->t.n;
   FLCHK(upload_h(c, T, elev));
   hipStream_t s = c->stream;
-  fl_launch_clear_iter(s, T->w, std::min<uint32_t>(T->prev_nb + 1, 2 * n + 2));
+  fl_launch_clear_iter(s, T->w, std::min<uint32_t>(T->prev_nb + 1, n + 2));
   fl_launch_receivers(s, T->t, T->w, false, false);
   FLCHK(read_ctrl(c, T));
   if (host_flag(c, FL_FLAG_LAKE)) FLCHK(join_lakes(c, T));

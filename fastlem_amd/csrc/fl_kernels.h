@@ -33,8 +33,28 @@ struct fl_profiler {
 extern thread_local fl_profiler* fl_current_profiler;
 
 // Control block read back once per phase: [flags | counters | boff head | bnoff head].
-enum { FL_FLAG_LAKE = 0, FL_FLAG_JUMP = 1 /* and 2: alternating */, FL_FLAG_CHANGED = 3, FL_NUM_FLAGS = 4 };
-enum { FL_CNT_MAXLD = 0, FL_CNT_CHAINS = 1, FL_CNT_POSITIONS = 2, FL_NUM_COUNTERS = 4 };
+// FL_FLAG_STALL: a sweep's wait ended without its value
+enum { FL_FLAG_LAKE = 0, FL_FLAG_JUMP = 1, FL_FLAG_STALL = 2, FL_FLAG_CHANGED = 3, FL_NUM_FLAGS = 4 };
+enum {
+  FL_CNT_MAXLD = 0,
+  FL_CNT_CHAINS = 1,
+  FL_CNT_POSITIONS = 2,
+  FL_CNT_TICKET_DA = 3,  // units taken from the sweeps
+  FL_CNT_TICKET_TAU = 4,
+  FL_NUM_COUNTERS = 6
+};
+// Entries of a bucket array past its n: a light edge has a heavy sibling, so
+// a path with d of them needs 2d + 1 sites, the rounds of n sites are at most
+// (n + 1) / 2 and their buckets (two a round) at most n + 1.
+enum { FL_BUCKET_PAD = 8 };
+// Light children listed per chain position.  A position with more walks its
+// row, which takes as long as ten light edges (13 us), so the list holds what
+// a planar triangulation has (four were too few at one position in about a
+// thousand, and every path to an outlet met one).
+enum { FL_LIST = 6 };
+// Chains are short below at most this length (a sweep's short-chain tile of
+// 64 positions advances by 65 - long_min).
+enum { FL_LONG_MAX = 33 };
 enum { FL_CTRL_HEAD = 512 };  // bucket offsets mirrored into the control block
 enum { FL_MAX_JUMP_ROUNDS = 96 };  // one "pointers moved" word per doubling round
 enum { FL_CTRL_JUMPS = FL_NUM_FLAGS + FL_NUM_COUNTERS + 2 * (FL_CTRL_HEAD + 1) };
@@ -72,7 +92,7 @@ struct fl_dev_work {
   double* hnp = nullptr;    // [n] new elevation, chain-major (max-slope form)
   double* up = nullptr;     // [n] uplift, chain-major (max-slope form)
   double* tanp = nullptr;   // [n] tan(max slope), chain-major (max-slope form)
-  double* dp = nullptr;     // [n] receiver distance, chain-major (max-slope form)
+  uint32_t* pro = nullptr;  // [n] the basin outlet's position, chain-major (max-slope form)
   double* hop = nullptr;    // [n] old elevation, chain-major (max-slope form)
   double* A = nullptr;      // [n] drainage area (kept: heavy-child hint)
   double* tau = nullptr;    // [n] response time
@@ -89,13 +109,15 @@ struct fl_dev_work {
   // list counts, own area, erodibility, receiver distance; the listed light
   // children's drainage areas (FL_LIST slots per position, fold order,
   // filled by the children's rounds: pdest at a chain's base position names
-  // the slot of its head)
-  uint32_t* pcnt = nullptr;   // [n] npre | npost << 8, or the overflow flag
+  // the slot of its head, ppos there the position of its receiver)
+  uint32_t* pcnt = nullptr;   // [n] npre | npost << 8, or the overflow flag; tail and head flags
   double* parea = nullptr;    // [n]
   double* pK = nullptr;       // [n]
   double* pdn = nullptr;      // [n]
-  double* cval = nullptr;     // [FL_LIST n]
+  double* cval = nullptr;     // [FL_LIST n] hand-over words
+  double* cover = nullptr;    // [n] hand-over words past the lists, at the children's bases
   uint32_t* pdest = nullptr;  // [n]
+  uint32_t* ppos = nullptr;   // [n]
 
   // pointer jumping, two (pointer, count) pairs per site, pointer in the low
   // word: cp = (chain ancestor, distance to it), rt = (tree ancestor, light
@@ -103,11 +125,9 @@ struct fl_dev_work {
   uint64_t* cp = nullptr;
   uint64_t* rt = nullptr;
   uint32_t *bcnt = nullptr, *bnodes = nullptr, *boff = nullptr, *bnoff = nullptr, *bcur = nullptr,
-           *bncur = nullptr;                                  // [n+2] light-depth buckets
-  // chains by bucket: (base position, length, position of the head's
-  // receiver or FL_NONE, position of the basin outlet)
-  uint4* cmeta = nullptr;                                    // [n]
-  uint32_t* head_chain = nullptr;                            // [n] at a chain head: its chain
+           *bncur = nullptr;                                  // [n + FL_BUCKET_PAD] light-depth buckets
+  uint32_t* ucum = nullptr;                                  // [n + FL_BUCKET_PAD] sweep units before each round
+  uint2* cmeta = nullptr;                                    // [n] long chains: (base position, length)
   uint32_t* head_base = nullptr;                             // [n] at a chain head: its base position
   uint32_t* perm = nullptr;                                  // [n] chain-major site order
   uint32_t* ctrl = nullptr;                                  // [FL_CTRL_WORDS]
@@ -116,9 +136,9 @@ struct fl_dev_work {
   const uint32_t* guard = nullptr;
   int* flags = nullptr;                                      // = ctrl
   uint32_t* counters = nullptr;                              // = ctrl + FL_NUM_FLAGS
-  // chains of at least long_min sites fold in a wavefront, shorter ones in
-  // one lane (a tuning: results do not depend on it)
-  uint32_t long_min = 6;
+  // chains of at least long_min sites (at most FL_LONG_MAX) take a wavefront
+  // each, shorter ones share one (a tuning: results do not depend on it)
+  uint32_t long_min = 16;
   // Basins recomputed in an iteration.  A new elevation is a function of the
   // drainage tree alone (and the static parameters), so a basin of the
   // previous iteration's tree in which no site's receiver changed -- nor any
@@ -162,34 +182,27 @@ void fl_launch_children(hipStream_t s, const fl_dev_terrain& t, const fl_dev_wor
                         const uint8_t* t_active);
 void fl_launch_chain_jump(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t round);
 void fl_launch_chain_count(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w);
-// Bucket offsets (scan), chain placement and the chain-major permutation;
-// offsets are written up to round `rounds` (rounds past the deepest light
-// depth are empty).
-void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t rounds);
-// Launch shape of one sweep round; the round's chain and position bounds are
-// read by the kernels from the bucket offsets (boff/bnoff at 2l..2l+2), so a
-// round can be enqueued before its bounds are known on the host.  Kernels
-// loop over their range, so any non-zero grid is correct.
-struct fl_round_grid {
-  uint32_t fold_blocks;  // k_da_fold / k_tau_fold, 64 threads each
-  uint64_t positions;    // profiler units (0 when not known at launch)
-};
-// Round l of the drainage-area sweep; also writes the response-time inputs
-// of its positions (and, with clamp, the max-slope recurrence's inputs).
-void fl_launch_da_round(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t l,
-                        const fl_round_grid& g, bool clamp);
-// Rounds lsplit..min(deepest light depth, cap) of the drainage-area sweep
-// (deepest first), then of the response-time sweep (shallowest first), in
-// one launch of one workgroup of FL_TAIL_WAVES wavefronts each: for the
-// deep rounds, which hold few chains.
+// Bucket offsets (scan), chain placement and the chain-major permutation.
+void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w);
+// The sweeps.  Rounds 0..min(deepest, cap - 1) in one launch of about `waves`
+// wavefronts (any number is correct; the sweep units of the rounds are best);
+// the drainage-area sweep also writes the response-time inputs.  positions:
+// profiler units (0 when not known at launch).
+enum { FL_FOLD_WAVES = 8 };
+void fl_launch_da_fold(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t cap, uint32_t waves,
+                       uint64_t positions, bool clamp);
+void fl_launch_tau_fold(hipStream_t s, const fl_dev_work& w, uint32_t cap, uint32_t waves, uint64_t positions,
+                        bool clamp);
+// Rounds lsplit..deepest (deepest first, then shallowest first) in one
+// workgroup of FL_TAIL_WAVES wavefronts, a barrier between rounds.
 enum { FL_TAIL_WAVES = 16 };
-void fl_launch_da_tail(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t lsplit, uint32_t cap,
-                       uint64_t units, bool clamp);
-void fl_launch_tau_tail(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t lsplit, uint32_t cap,
-                        uint64_t units, bool clamp);
+void fl_launch_da_tail(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t lsplit,
+                       uint64_t positions, bool clamp);
+void fl_launch_tau_tail(hipStream_t s, const fl_dev_work& w, uint32_t lsplit, uint64_t positions, bool clamp);
+// The drainage-area sweep's hand-over words before a first sweep, or after
+// one whose waits ended without their values.
+void fl_launch_reset_words(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w);
 void fl_launch_clear_iter(hipStream_t s, const fl_dev_work& w, uint32_t nb);
-void fl_launch_tau_round(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t l,
-                         const fl_round_grid& g, bool clamp);
 // Back to site order, one thread per site.
 void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool clamp,
                            const uint32_t* tid, const uint8_t* active, uint32_t* tchanged);

@@ -16,14 +16,15 @@
 //     k_bucket_*        chains bucketed by light depth, laid out contiguously
 //     k_chain_perm      sites scattered to chain-major positions, with
 //                                             each site's light children
-//   sweeps, one round per light depth (deepest first for drainage area)
+//   sweeps, every round (light depth) in one launch, deepest first for
+//   drainage area
 //     k_da_fold         generator.rs:154-159  drainage area along the chains,
 //                       generator.rs:172      exact fold order; then each
 //                                             site's 1/(K*A^0.5) * distance
 //     k_tau_fold        generator.rs:162-203  response time (+ clamped
 //                                             elevation), head to tail
-//     k_da_tail, k_tau_tail                   the deep rounds (few chains
-//                                             each) in one launch per sweep
+//     k_da_tail, k_tau_tail                   rounds behind barriers in one
+//                                             workgroup
 //     k_tau_scatter     generator.rs:177-202  elevation, changed flag
 //
 // Per-site kernels take their site ranges XCD by XCD (xcd_block): each of
@@ -32,7 +33,7 @@
 // Exactness.  Every floating-point expression is evaluated in the order the
 // reference writes it; the library is built with -ffp-contract=off so no
 // multiply-add is fused.  No floating-point atomics are used: the drainage
-// area of site u is folded by one lane as
+// area of site u is folded as
 //     A_u = ((a_u + A_{c_m}) + A_{c_{m-1}}) + ... + A_{c_1}
 // (children c_1..c_m in row order), which is the association the reference's
 // reverse-BFS accumulation produces; response time is a sequential
@@ -45,9 +46,12 @@
 #include "fl_kernels.h"
 
 #define FL_NONE 0xffffffffu
-#define FL_LIST 4                   // light children listed per chain position
+#define FL_POSTS 4                  // most of them after the heavy child
 #define FL_LIST_OVERFLOW 0x10000u   // pcnt flag: more light children than listed
 #define FL_ROW 8                    // graph row entries loaded together
+#define FL_TAIL 0x20000u            // pcnt flag: the position is its chain's tail
+#define FL_HEAD 0x40000u            // ... its chain's head
+#define FL_DEST_OVER 0xfffffffeu    // pdest: the receiver reads the chain's word in cover
 
 namespace {
 
@@ -527,43 +531,54 @@ k_bucket_count(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* _
 
 // Exclusive scans of the bucket histograms over the light depths actually
 // present (2 * (counters[FL_CNT_MAXLD] + 1) buckets), one workgroup.  The first
-// FL_CTRL_HEAD + 1 offsets are mirrored into the control block; offsets up to
-// `fill` are written.
+// FL_CTRL_HEAD + 1 offsets are mirrored into the control block.  ucum[l]: the
+// sweep units (see the sweeps) of the rounds before round l.
 #define FL_SCAN_BLOCK 1024  // k_bucket_scan: one workgroup of this size
 __global__ void __launch_bounds__(FL_SCAN_BLOCK)
-k_bucket_scan(uint32_t n, uint32_t fill, uint32_t* __restrict__ ctrl,
+k_bucket_scan(uint32_t n, uint32_t long_min, uint32_t* __restrict__ ctrl,
                               const uint32_t* __restrict__ bcnt, const uint32_t* __restrict__ bnodes,
-                              uint32_t* __restrict__ boff, uint32_t* __restrict__ bnoff) {
+                              uint32_t* __restrict__ boff, uint32_t* __restrict__ bnoff,
+                              uint32_t* __restrict__ ucum) {
   __shared__ uint32_t s_a[FL_SCAN_BLOCK], s_b[FL_SCAN_BLOCK];
-  __shared__ uint32_t carry_a, carry_b;
+  __shared__ uint32_t s_u[FL_SCAN_BLOCK];
+  __shared__ uint32_t carry_a, carry_b, carry_u;
+  const uint32_t stride = 65u - long_min;
   uint32_t* counters = ctrl + FL_NUM_FLAGS;
   uint32_t nb = 2 * (counters[FL_CNT_MAXLD] + 1);
-  if (nb > 2 * n + 2) nb = 2 * n + 2;
+  if (nb > n + 2) nb = n + 2;
   uint32_t* head_c = counters + FL_NUM_COUNTERS;
   uint32_t* head_n = head_c + FL_CTRL_HEAD + 1;
   if (threadIdx.x == 0) {
     carry_a = 0;
     carry_b = 0;
+    carry_u = 0;
   }
   __syncthreads();
   for (uint32_t base = 0; base < nb; base += FL_SCAN_BLOCK) {
     uint32_t i = base + threadIdx.x;
     uint32_t a = i < nb ? bcnt[i] : 0, b = i < nb ? bnodes[i] : 0;
+    // a round's units in its second bucket's place: its long chains and the
+    // tiles of its short chains' positions
+    uint32_t q = (i & 1u) && i < nb ? a + (bnodes[i - 1] + stride - 1) / stride : 0u;
     s_a[threadIdx.x] = a;
     s_b[threadIdx.x] = b;
+    s_u[threadIdx.x] = q;
     __syncthreads();
     for (uint32_t off = 1; off < FL_SCAN_BLOCK; off <<= 1) {
       uint32_t ta = threadIdx.x >= off ? s_a[threadIdx.x - off] : 0;
       uint32_t tb = threadIdx.x >= off ? s_b[threadIdx.x - off] : 0;
+      uint32_t tu = threadIdx.x >= off ? s_u[threadIdx.x - off] : 0;
       __syncthreads();
       s_a[threadIdx.x] += ta;
       s_b[threadIdx.x] += tb;
+      s_u[threadIdx.x] += tu;
       __syncthreads();
     }
     if (i < nb) {
       uint32_t oa = carry_a + s_a[threadIdx.x] - a, ob = carry_b + s_b[threadIdx.x] - b;
       boff[i] = oa;
       bnoff[i] = ob;
+      if ((i & 1u) == 0) ucum[i >> 1] = carry_u + s_u[threadIdx.x];  // (its own round's sit at i + 1)
       if (i <= FL_CTRL_HEAD) {
         head_c[i] = oa;
         head_n[i] = ob;
@@ -573,12 +588,14 @@ k_bucket_scan(uint32_t n, uint32_t fill, uint32_t* __restrict__ ctrl,
     if (threadIdx.x == FL_SCAN_BLOCK - 1) {
       carry_a += s_a[threadIdx.x];
       carry_b += s_b[threadIdx.x];
+      carry_u += s_u[threadIdx.x];
     }
     __syncthreads();
   }
   if (threadIdx.x == 0) {
     boff[nb] = carry_a;
     bnoff[nb] = carry_b;
+    ucum[nb >> 1] = carry_u;
     if (nb <= FL_CTRL_HEAD) {
       head_c[nb] = carry_a;
       head_n[nb] = carry_b;
@@ -586,25 +603,18 @@ k_bucket_scan(uint32_t n, uint32_t fill, uint32_t* __restrict__ ctrl,
     counters[FL_CNT_CHAINS] = carry_a;
     counters[FL_CNT_POSITIONS] = carry_b;
   }
-  // offsets nb+1..fill repeat the totals: rounds launched beyond the deepest
-  // light depth find empty ranges
-  for (uint32_t i = nb + 1 + threadIdx.x; i <= fill; i += FL_SCAN_BLOCK) {
-    boff[i] = carry_a;
-    bnoff[i] = carry_b;
-  }
 }
 
 // Give every chain (through its tail) a slot in its light-depth bucket and a
 // contiguous range of positions: LDS atomics rank the chains of a workgroup,
 // one global atomic per (workgroup, bucket) reserves the ranges.  Order
-// inside a bucket is immaterial to the results.  Chain q's record starts
-// (base, len) (k_chain_perm adds the receiver's and the outlet's positions),
-// its head knows q and its base, and the base's receiver slot starts empty.
-__device__ __forceinline__ void place_chain(uint32_t q, uint32_t pos, uint32_t len, uint32_t hd,
-                                            uint4* __restrict__ cmeta, uint32_t* __restrict__ head_chain,
-                                            uint32_t* __restrict__ head_base, uint32_t* __restrict__ pdest) {
-  reinterpret_cast<uint2*>(cmeta)[2ull * q] = make_uint2(pos, len);
-  head_chain[hd] = q;
+// inside a bucket is immaterial to the results.  A long chain's record is
+// (base, len), a chain's head knows its base, and the base's receiver slot
+// starts empty.
+__device__ __forceinline__ void place_chain(uint32_t q, uint32_t pos, uint32_t len, uint32_t hd, uint32_t long_min,
+                                            uint2* __restrict__ cmeta, uint32_t* __restrict__ head_base,
+                                            uint32_t* __restrict__ pdest) {
+  if (len >= long_min) cmeta[q] = make_uint2(pos, len);
   head_base[hd] = pos;
   pdest[pos] = FL_NONE;
 }
@@ -614,7 +624,7 @@ k_bucket_place(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* _
                const unsigned long long* __restrict__ rt, const uint8_t* __restrict__ is_outlet,
                const uint32_t* __restrict__ boff,
                const uint32_t* __restrict__ bnoff, uint32_t* __restrict__ bcur, uint32_t* __restrict__ bncur,
-               uint4* __restrict__ cmeta, uint32_t* __restrict__ head_chain, uint32_t* __restrict__ pdest,
+               uint2* __restrict__ cmeta, uint32_t* __restrict__ pdest,
                uint32_t* __restrict__ head_base, uint32_t long_min, const uint8_t* __restrict__ act) {
   const uint32_t base = xcd_block() * (FL_BUCKET_BLOCK * FL_BUCKET_PER_THREAD);
   fl_tail tl[FL_BUCKET_PER_THREAD];
@@ -639,7 +649,7 @@ k_bucket_place(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* _
       } else {
         uint32_t q = boff[l] + atomicAdd(bcur + l, 1u);
         uint32_t pos = bnoff[l] + atomicAdd(bncur + l, len);
-        place_chain(q, pos, len, pair_ptr(c), cmeta, head_chain, head_base, pdest);
+        place_chain(q, pos, len, pair_ptr(c), long_min, cmeta, head_base, pdest);
       }
     }
   }
@@ -658,19 +668,19 @@ k_bucket_place(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* _
     uint32_t l = 2u * pair_cnt(tl[j].r) + (len >= long_min ? 1u : 0u);
     uint32_t q = boff[l] + s_bc[l] + lc[j];
     uint32_t pos = bnoff[l] + s_bn[l] + ln[j];
-    place_chain(q, pos, len, pair_ptr(c), cmeta, head_chain, head_base, pdest);
+    place_chain(q, pos, len, pair_ptr(c), long_min, cmeta, head_base, pdest);
   }
 }
 
 // Scatter sites to their chain-major positions with the inputs the sweeps
 // read there: the drainage-area fold's list counts, area, erodibility and
-// receiver distance (with max slopes also uplift, tan(max slope), distance
-// and old elevation), and for each listed light child the slot its chain's
-// head fills with its drainage area (pdest at the child chain's base).  A
-// chain's record gets the positions of the head's receiver (FL_NONE for an
-// outlet) and of the basin's outlet.  Sites outside every basin keep their
-// elevation, drainage area = own area and response time 0 (generator.rs:
-// 144-145), as the reference leaves them.
+// receiver distance (with max slopes also uplift, tan(max slope), old
+// elevation and the basin outlet's position), and for each listed light child
+// the slot its chain's head fills with its drainage area (pdest at the child
+// chain's base).  A chain's base gets the position of the head's receiver
+// (FL_NONE for an outlet).  Sites outside every basin keep their elevation,
+// drainage area = own area and response time 0 (generator.rs:144-145), as the
+// reference leaves them.
 struct fl_perm_out {
   uint32_t* perm;
   uint32_t* pcnt;
@@ -680,15 +690,15 @@ struct fl_perm_out {
   double* pdn;
   double* up;
   double* tanp;
-  double* dp;
   double* hop;
-  uint4* cmeta;
+  uint32_t* ppos;
+  uint32_t* pro;
 };
 
 __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, uint32_t n, const unsigned long long* __restrict__ cp,
                              const unsigned long long* __restrict__ rt, const uint32_t* __restrict__ next,
                              const uint8_t* __restrict__ is_outlet, const uint32_t* __restrict__ head_base,
-                             const uint32_t* __restrict__ head_chain, fl_perm_out o,
+                             fl_perm_out o,
                              const double* __restrict__ area, const double* __restrict__ K,
                              const double* __restrict__ dnext, const double* __restrict__ U,
                              const double* __restrict__ tan_ms, int clamp, double* __restrict__ A,
@@ -705,12 +715,11 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
   const uint32_t mld = *maxld;
   const bool on = v < n && act[v];
   unsigned long long rv = 0ull, cv = 0ull, m = 0ull;
-  uint32_t hq = 0u, b = 0u, e = 0u, hk = 0u, p = 0u;
+  uint32_t b = 0u, e = 0u, hk = 0u, p = 0u;
   double Kv = 0.0, dv = 0.0, av = 0.0;
   if (on) {
     rv = rt[v];
     cv = cp[v];
-    hq = head_chain[v];  // meaningful at a chain head only
     b = rp[v];
     e = rp[v + 1];
     hk = hc[v];
@@ -724,7 +733,7 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
   // the bucket histograms are used up (count, scan, place): clear the
   // entries this decomposition touched for the next one
   const uint32_t nb = 2u * (mld + 1u);
-  for (uint32_t i = v; i <= nb && i < 2u * n + 4u; i += gridDim.x * bs) {
+  for (uint32_t i = v; i <= nb && i < n + FL_BUCKET_PAD; i += gridDim.x * bs) {
     bcnt[i] = 0;
     bnodes[i] = 0;
     bcur[i] = 0;
@@ -734,13 +743,13 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
   const uint32_t r = pair_ptr(rv), hd = pair_ptr(cv), deg = e - b;
   root[v] = r;
   // the second level of loads, issued together: the root's outlet flag, the
-  // chain's base, the row (up to FL_ROW entries) and, at a chain head, the
-  // receiver's pair and the outlet's base
+  // chain's base, the row (up to FL_ROW entries), at a chain head the
+  // receiver's pair and with max slopes the outlet's base
   const uint8_t outlet = is_outlet[r];
   const uint32_t base = head_base[hd];
   const bool head = hd == v;
   const unsigned long long cpp = head ? cp[p] : 0ull;
-  const uint32_t hbr = head ? head_base[r] : 0u;
+  const uint32_t hbr = clamp ? head_base[r] : 0u;
   uint32_t cc[FL_ROW];
   const bool short_row = deg <= FL_ROW;
   if (short_row && deg > 0) {
@@ -760,13 +769,13 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
   if (clamp) {
     o.up[P] = U[v];
     o.tanp[P] = tan_ms[v];
-    o.dp[P] = dv;
     o.hop[P] = h[v];
+    o.pro[P] = hbr;
   }
   // the light children in fold order (descending slot), those before the
   // heavy child first: the first FL_LIST get slots FL_LIST * P + i for
-  // their chains' heads to fill; more set the overflow bit and the fold
-  // reads the graph instead
+  // their chains' heads to fill; with more, the overflow bit is set (the fold
+  // walks the row) and the others' heads hand over at their own bases
   {
     uint32_t npre = 0, npost = 0;
     bool after = false;
@@ -787,7 +796,7 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
           continue;
         }
         uint32_t idx = npre + npost;
-        if (idx < FL_LIST) o.pdest[hb[j]] = FL_LIST * P + idx;
+        o.pdest[hb[j]] = idx < FL_LIST ? FL_LIST * P + idx : FL_DEST_OVER;
         if (after) ++npost;
         else ++npre;
       }
@@ -800,197 +809,122 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
           continue;
         }
         uint32_t idx = npre + npost;
-        if (idx < FL_LIST) o.pdest[head_base[ch]] = FL_LIST * P + idx;
+        o.pdest[head_base[ch]] = idx < FL_LIST ? FL_LIST * P + idx : FL_DEST_OVER;
         if (after) ++npost;
         else ++npre;
       }
     }
-    bool over = npre + npost > FL_LIST;
-    o.pcnt[P] = over ? FL_LIST_OVERFLOW : (npre | (npost << 8));
+    bool over = npre + npost > FL_LIST || npost > FL_POSTS;
+    o.pcnt[P] = (over ? FL_LIST_OVERFLOW : (npre | (npost << 8))) | (hk == FL_NONE ? FL_TAIL : 0u) |
+                (head ? FL_HEAD : 0u);
     o.parea[P] = av;
   }
-  if (head) {
-    const uint32_t pp = (p == v) ? FL_NONE : head_base[pair_ptr(cpp)] + pair_cnt(cpp);
-    reinterpret_cast<uint2*>(o.cmeta)[2ull * hq + 1] = make_uint2(pp, hbr);
-  }
+  if (head) o.ppos[P] = (p == v) ? FL_NONE : head_base[pair_ptr(cpp)] + pair_cnt(cpp);
 }
 
 // --------------------------------------------------------------- sweeps ---
-
-#define FL_BATCH 8
-
-// Drainage area of the site at chain position P, folded in the reference's
-// order (generator.rs:154-159 accumulates children in reverse BFS order, so
-// A_k = ((a_k + A_{c_m}) + A_{c_{m-1}}) + ... + A_{c_1} over the children in
-// row order).  The heavy child's value is not known here: the fold is split
-// into `pre` (the part before it) and the light children after it, posts
-// p0..p3 in fold order (more than four are re-read by da_post_rest).  Light
-// children head chains of a deeper round, already finished.
 //
-// Absent posts are -0.0, and the chain fold starts from r = -0.0 at the
-// tail: x + (-0.0) == x exactly for every x (signed zeros included), so
-//     A = ((pre + r) + p0) + p1
-// is the reference's value at every position without a branch; positions
-// with three or more posts (about 1% of sites) add p2, p3, ... after it.
+// Both sweeps run every round (light depth) in one launch.  A round's work
+// is cut into units of one wavefront each: a long chain, or a tile of 64
+// consecutive chain positions of its short chains.  Wavefronts take the units
+// in round order (drainage area deepest round first, response time shallowest
+// first) and a unit waits for just the values it reads, not for the round
+// before it: a chain's head hands its drainage area to its receiver's list
+// slot, a position its response time (and, with max slopes, its elevation) to
+// the heads below it, and the word itself says whether it is there yet.
+//
+// What bounds it: the longest path of the forest, one dependent chain of
+// FP64 adds, plus a hand-over per light edge on it.  One launch per round made
+// every round as long as its longest chain and paid 4.5 us a launch; a
+// hand-over between two wavefronts of different XCDs takes 0.57 us.
+//
+// A hand-over word holds FL_SENT, a signalling NaN that no arithmetic
+// produces, until its value is stored (publish() quiets a value that equals
+// it).  Words are stored and read with relaxed device-scope atomics: the value
+// is the flag, no fence is needed.  Drainage-area words are set back to
+// FL_SENT by the one unit that reads them, response times and elevations by
+// the drainage-area sweep before.
+//
+// Waits end.  A workgroup takes FL_FOLD_WAVES units at a time from one
+// counter, so every unit a wavefront waits for was taken by a wavefront that
+// runs: the lowest unit not finished waits for nothing.  Should a wait still
+// last FL_SPIN_MAX polls, the wavefront raises FL_FLAG_STALL and goes on, every
+// other wait sees the flag and ends, and the host redoes the iteration in one
+// workgroup with barriers between the rounds (k_da_tail, k_tau_tail).
+#define FL_SENT 0x7ff45eed0badf00dull
+#define FL_SPIN_MAX (1u << 20)
 #define FL_NEG0 (-0.0)
-#define FL_POSTS 4
 
-__device__ __forceinline__ void da_partial(uint32_t k, const uint32_t* __restrict__ rp,
-                                           const uint32_t* __restrict__ col, const uint32_t* __restrict__ next,
-                                           const unsigned long long* __restrict__ cmask,
-                                           const uint32_t* __restrict__ hc, const double* __restrict__ area,
-                                           const double* __restrict__ A, double& pre, double& p0, double& p1,
-                                           double& p2, double& p3, uint32_t& np) {
-  uint32_t b = rp[k], deg = rp[k + 1] - b, hk = hc[k];
-  unsigned long long m = cmask[k];
-  double acc = area[k];
-  p0 = p1 = p2 = p3 = FL_NEG0;
-  np = 0;
-  bool after = false;
-  for (uint32_t s = deg; s-- > 0;) {
-    if (!is_child(m, deg, s, b, col, next, k)) continue;
-    uint32_t c = col[b + s];
-    if (c == hk) {
-      after = true;
-      continue;
-    }
-    double v = A[c];
-    if (!after) {
-      acc = acc + v;
-    } else {
-      // selects, not an indexed store: keeps the posts in registers
-      p3 = (np == 3) ? v : p3;
-      p2 = (np == 2) ? v : p2;
-      p1 = (np == 1) ? v : p1;
-      p0 = (np == 0) ? v : p0;
-      ++np;
-    }
+#if defined(__has_builtin)
+#if __has_builtin(__hip_atomic_load) && __has_builtin(__hip_atomic_store)
+#define FL_DEVICE_ATOMICS 1
+#endif
+#if __has_builtin(__builtin_amdgcn_update_dpp)
+#define FL_WAVE_SHIFT 1
+#endif
+#endif
+
+// The rounds of a decomposition and the counters its units are taken from.
+struct fl_flow {
+  const uint32_t* maxld;  // the deepest round
+  const uint32_t* ucum;   // units before each round
+  const uint32_t* boff;   // chains before each bucket (short, long of each round)
+  const uint32_t* bnoff;  // positions before each bucket
+  uint32_t* ticket_da;
+  uint32_t* ticket_tau;
+  uint32_t long_min;
+};
+
+namespace {
+
+__device__ __forceinline__ double bits_double(unsigned long long u) {
+  return __hiloint2double((int)(uint32_t)(u >> 32), (int)(uint32_t)u);
+}
+
+// A hand-over word, read and written at device scope.
+__device__ __forceinline__ unsigned long long peek(const double* p) {
+  const unsigned long long* w = reinterpret_cast<const unsigned long long*>(p);
+#ifdef FL_DEVICE_ATOMICS
+  return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#else
+  return __atomic_load_n(w, __ATOMIC_RELAXED);
+#endif
+}
+__device__ __forceinline__ void poke(double* p, unsigned long long u) {
+  unsigned long long* w = reinterpret_cast<unsigned long long*>(p);
+#ifdef FL_DEVICE_ATOMICS
+  __hip_atomic_store(w, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#else
+  __atomic_store_n(w, u, __ATOMIC_RELAXED);
+#endif
+}
+__device__ __forceinline__ void publish(double* p, double v) {
+  unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  if (u == FL_SENT) u |= 1ull << 51;
+  poke(p, u);
+}
+
+// One more poll of a wait: false when the wait is to end without its value.
+__device__ __forceinline__ bool wait_more(uint32_t& spins, int* stall) {
+  ++spins;
+#ifdef FL_WAVE_SHIFT
+  __builtin_amdgcn_s_sleep(1);
+#endif
+  if ((spins & 255u) != 0) return true;
+  if (spins >= FL_SPIN_MAX) __atomic_store_n(stall, 1, __ATOMIC_RELAXED);
+  return __atomic_load_n(stall, __ATOMIC_RELAXED) == 0;
+}
+
+// The word at p where `need`, waited for by the whole wavefront.
+__device__ __forceinline__ double await(const double* p, bool need, double otherwise, int* stall) {
+  unsigned long long u = need ? peek(p) : 0ull;
+  uint32_t spins = 0;
+  while (__any(need && u == FL_SENT)) {
+    if (!wait_more(spins, stall)) break;
+    if (need && u == FL_SENT) u = peek(p);
   }
-  pre = acc;
+  return need ? bits_double(u) : otherwise;
 }
-
-// The light children after the heavy one beyond the first FL_POSTS.
-__device__ __forceinline__ double da_post_rest(double r, uint32_t k, const uint32_t* __restrict__ rp,
-                                               const uint32_t* __restrict__ col, const uint32_t* __restrict__ next,
-                                               const unsigned long long* __restrict__ cmask,
-                                               const uint32_t* __restrict__ hc, const double* __restrict__ A) {
-  uint32_t b = rp[k], deg = rp[k + 1] - b, hk = hc[k];
-  unsigned long long m = cmask[k];
-  bool after = false;
-  uint32_t seen = 0;
-  for (uint32_t s = deg; s-- > 0;) {
-    if (!is_child(m, deg, s, b, col, next, k)) continue;
-    uint32_t c = col[b + s];
-    if (c == hk) {
-      after = true;
-      continue;
-    }
-    if (after) {
-      if (seen >= FL_POSTS) r = r + A[c];
-      ++seen;
-    }
-  }
-  return r;
-}
-
-// The terms after ((pre + r) + p0) + p1 of a position with np >= 3 posts.
-__device__ __forceinline__ double da_tail_terms(double r, uint32_t np, double c, double d, uint32_t k,
-                                                const uint32_t* __restrict__ rp, const uint32_t* __restrict__ col,
-                                                const uint32_t* __restrict__ next,
-                                                const unsigned long long* __restrict__ cmask,
-                                                const uint32_t* __restrict__ hc, const double* __restrict__ A) {
-  r = r + c;
-  if (np >= 4) r = r + d;
-  if (np > FL_POSTS) r = da_post_rest(r, k, rp, col, next, cmask, hc, A);
-  return r;
-}
-
-// The partial folds of a listed position from the values of its listed light
-// children (v_i = the i-th listed child's A, or anything when the list has
-// fewer entries: such slots are replaced by -0.0 before any arithmetic).
-__device__ __forceinline__ void da_combine(uint32_t cn, double area_k, double v0, double v1, double v2, double v3,
-                                           double& pre, double& p0, double& p1, double& p2, double& p3,
-                                           uint32_t& np) {
-  const uint32_t npre = cn & 0xffu, nl = npre + ((cn >> 8) & 0xffu);
-  v0 = nl > 0 ? v0 : FL_NEG0;
-  v1 = nl > 1 ? v1 : FL_NEG0;
-  v2 = nl > 2 ? v2 : FL_NEG0;
-  v3 = nl > 3 ? v3 : FL_NEG0;
-  // pre: x + (-0.0) == x, so the terms past npre are added as -0.0
-  pre = (((area_k + (npre > 0 ? v0 : FL_NEG0)) + (npre > 1 ? v1 : FL_NEG0)) + (npre > 2 ? v2 : FL_NEG0)) +
-        (npre > 3 ? v3 : FL_NEG0);
-  // posts: list entries npre, npre+1, ... (entries past nl read as -0.0)
-  p0 = npre == 0 ? v0 : npre == 1 ? v1 : npre == 2 ? v2 : npre == 3 ? v3 : FL_NEG0;
-  p1 = npre == 0 ? v1 : npre == 1 ? v2 : npre == 2 ? v3 : FL_NEG0;
-  p2 = npre == 0 ? v2 : npre == 1 ? v3 : FL_NEG0;
-  p3 = npre == 0 ? v3 : FL_NEG0;
-  np = nl - npre;
-}
-
-#define FL_DA_BLOCK 4
-
-// Everything the drainage-area fold reads at chain position P, in
-// chain-major order (written by k_chain_perm, the children's values by the
-// deeper rounds): one level of loads, no gathers.
-//   k: the site; cn: npre | npost << 8, or the overflow flag;
-//   v0..v3: the listed light children's A (cval[FL_LIST * P + i]);
-//   area, K, d: the site's area, erodibility and receiver distance.
-struct fl_da_pos {
-  uint32_t k, cn;
-  double v0, v1, v2, v3, area, K, d;
-};
-
-// The arrays of a drainage-area round.
-struct fl_da_args {
-  const uint32_t* perm;
-  const uint32_t* pcnt;
-  const double* cval;   // [FL_LIST n] light children's A by (position, list slot)
-  const double* parea;
-  const double* pK;
-  const double* pdn;
-  const uint32_t* pdest;  // at a chain's base position: its head's slot in cval, or FL_NONE
-  double* cval_out;
-  double* xp;
-  // the graph, for positions with more light children than listed
-  const uint32_t* rp;
-  const uint32_t* col;
-  const uint32_t* next;
-  const unsigned long long* cmask;
-  const uint32_t* hc;
-  const double* area;
-  double* A;
-};
-
-__device__ __forceinline__ fl_da_pos da_load(const fl_da_args& g, uint32_t P) {
-  const double2* __restrict__ cv = reinterpret_cast<const double2*>(g.cval);
-  const double2 a = cv[2ull * P], b = cv[2ull * P + 1];
-  return fl_da_pos{g.perm[P], g.pcnt[P], a.x, a.y, b.x, b.y, g.parea[P], g.pK[P], g.pdn[P]};
-}
-
-// A site's drainage area is final: store it and the response-time input of
-// its position, x = 1.0 / (K * a^0.5) * d (generator.rs:172-173, the
-// reference's association).
-__device__ __forceinline__ void da_store(const fl_da_args& g, uint32_t P, uint32_t k, double a, double K, double d) {
-  g.A[k] = a;
-  double celerity = K * rust_pow_half(a);
-  g.xp[P] = 1.0 / celerity * d;
-}
-
-// Drainage area of one light depth: the sequential fold along each chain,
-// tail to head, A = ((pre + A_heavy) + p0) + p1 (+ p2 + p3 ...), with the
-// partial folds of each position made from its listed children's values.
-// Long chains [c1, c2) take one 64-lane wavefront each: tiles of 64
-// positions are prepared by the whole wavefront and staged in LDS, lane 0
-// folds them eight at a time (reads first, then the dependent adds;
-// positions with three or more posts marked by a ballot), the wavefront
-// stores the results.  Short chains [c0, c1) take one lane each,
-// FL_DA_BLOCK positions at a time.  A chain's head hands its A to its
-// receiver's list slot (pdest).  Bounds from the bucket offsets of round l.
-// One wavefront's LDS tile of a drainage-area round.
-struct fl_da_lds {
-  double p[64], a[64], b[64], c[64], d[64], r[64];
-  uint32_t n[64], k[64];
-};
 
 // Synchronisation of one wavefront's lanes around its own LDS tile: a
 // wavefront-scope fence (orders the LDS accesses; the wavefront's LDS
@@ -1001,529 +935,787 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Wavefront `wave` of `nwaves` in drainage-area round l (short chains
-// [c0, c1), long chains [c1, c2)); cmeta: (base, len, ...) per chain.  A
-// long chain's tiles are loaded D - 1 ahead of the fold (D = 2 or 3: the
-// registers a workgroup of 1024 lanes has allow two).
-template <int D>
-__device__ __forceinline__ void da_round(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t wave, uint32_t nwaves,
-                                         uint32_t lane, fl_da_lds& L, const uint4* __restrict__ cmeta,
-                                         const fl_da_args& g) {
-  const uint2* __restrict__ cm2 = reinterpret_cast<const uint2*>(cmeta);
-  // long chains: one per block (uniform per block).  Tiles of 64 positions
-  // from the tail, software-pipelined D deep: a tile's loads are issued
-  // D - 1 tiles before its fold, unconditionally and at positions clamped
-  // into the chain, into registers of their own (the loop is unrolled D
-  // times: moving a register a load is still writing would wait for it), so
-  // waiting for one tile never waits for the tiles loaded after it.  No tile
-  // input depends on this round's results (light children head chains of
-  // deeper rounds).
-  for (uint32_t c = c1 + wave; c < c2; c += nwaves) {
-    const uint2 m = cm2[2ull * c];
-    const uint32_t base = m.x, len = m.y;
-    const uint32_t pd = g.pdest[base];
-    // position of this lane in the tile ending at `e` (e > 0; lanes past
-    // the tile read its first position)
-    auto pos_of = [&](uint32_t e) {
-      const uint32_t cs = e > 64 ? e - 64 : 0;
-      return base + (lane < e - cs ? cs + lane : cs);
-    };
-    // the tile ending `ahead` tiles below `e`, or the tail tile past the head
-    auto ahead_of = [&](uint32_t e, uint32_t ahead) { return e > 64 * ahead ? e - 64 * ahead : len; };
-    uint32_t end = len;
-    double r = FL_NEG0;  // lane 0's running value
-    // fold the tile ending at `end` from cur, then load into cur the tile D
-    // tiles further towards the head
-    auto step = [&](fl_da_pos& cur) {
-      const uint32_t cs = end > 64 ? end - 64 : 0, cnt = end - cs;
-      const bool mine = lane < cnt;
-      double p = 0.0, a = 0.0, b = 0.0, x = 0.0, y = 0.0;
-      uint32_t np = 0;
-      if (__any(mine && (cur.cn & FL_LIST_OVERFLOW))) {
-        // a position with more light children than listed (rare) reads the
-        // graph; kept apart so that the usual tiles issue no load here
-        if (mine) {
-          if (cur.cn & FL_LIST_OVERFLOW)
-            da_partial(cur.k, g.rp, g.col, g.next, g.cmask, g.hc, g.area, g.A, p, a, b, x, y, np);
-          else
-            da_combine(cur.cn, cur.area, cur.v0, cur.v1, cur.v2, cur.v3, p, a, b, x, y, np);
-        }
-      } else {
-        da_combine(cur.cn, cur.area, cur.v0, cur.v1, cur.v2, cur.v3, p, a, b, x, y, np);
-        if (!mine) {
-          p = a = b = x = y = 0.0;
-          np = 0;
-        }
-      }
-      L.p[lane] = p;
-      L.a[lane] = a;
-      L.b[lane] = b;
-      L.c[lane] = x;
-      L.d[lane] = y;
-      L.n[lane] = np;
-      L.k[lane] = mine ? cur.k : FL_NONE;
-      // positions with a second post, and with three or more (those add p2,
-      // p3 and, past FL_POSTS posts, read the graph: rare, and such "deep"
-      // tiles take a fold of their own, so that no other fold holds a load)
-      const unsigned long long post2 = __ballot(np >= 2), rare = __ballot(np >= 3), post4 = __ballot(np >= 4);
-      const bool deep = __any(np > FL_POSTS);
-      const uint32_t kk = cur.k;
-      const double Kk = cur.K, dk = cur.d;
-      wave_sync();
-      if (lane == 0 && !deep) {
-        // x + (-0.0) == x: positions add the -0.0 pads of the posts they do
-        // not have, so a batch of eight folds without branches, with as
-        // many dependent adds a position as the most posts in the batch
-        // require (two for none or one post, up to five for four).  Every
-        // operand of a batch is read from the tile before its adds: no wait
-        // inside them, and no load from global memory in this loop (waiting
-        // for one would wait for the tiles in flight too)
-        int e = (int)cnt - 1;
-        for (; e >= 7; e -= 8) {
-          double tp[8], ta[8], tb[8];
+// v of the next lane (up) or of the previous one (down); the lane at the
+// wavefront's edge gets its `edge`.
+#ifndef FL_WAVE_SHIFT
+__device__ __forceinline__ double shift_lanes(double edge, double v, int from) {
+  __shared__ double fl_shift_tile[16][64];
+  const int lane = (int)(threadIdx.x & 63u);
+  double* t = fl_shift_tile[threadIdx.x >> 6];
+  t[lane] = v;
+  wave_sync();
+  const int src = lane + from;
+  const double r = src >= 0 && src < 64 ? t[src] : edge;
+  wave_sync();
+  return r;
+}
+__device__ __forceinline__ double from_next(double edge, double v) { return shift_lanes(edge, v, 1); }
+__device__ __forceinline__ double from_prev(double edge, double v) { return shift_lanes(edge, v, -1); }
+#else
+__device__ __forceinline__ double from_next(double edge, double v) {  // DPP wave_shl:1
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x130, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x130, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double from_prev(double edge, double v) {  // DPP wave_shr:1
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x138, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x138, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+#endif
+__device__ __forceinline__ double of_lane(double v, uint32_t lane) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), (int)lane);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), (int)lane);
+  return __hiloint2double(hi, lo);
+}
+
+// A value that every lane of the wavefront holds, for scalar registers.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 0); }
+
+// Length of the longest run of set bits, plus one: the positions of the
+// longest chain of a tile whose non-first positions are marked.
+__device__ __forceinline__ uint32_t run_steps(unsigned long long m) {
+  uint32_t steps = 1;
+  for (; m; m &= m << 1) ++steps;
+  return steps;
+}
+
+// The rounds of a decomposition, lane i holding round `first` + i.
+struct fl_rounds {
+  uint32_t first, u0, u1, c1, c2, n0, n1;
+};
+__device__ __forceinline__ fl_rounds load_rounds(const fl_flow& f, uint32_t first, uint32_t rounds, uint32_t lane) {
+  fl_rounds r{first, 0u, 0u, 0u, 0u, 0u, 0u};
+  const uint32_t l = first + lane;
+  if (l < rounds) {
+    r.u0 = f.ucum[l];
+    r.u1 = f.ucum[l + 1];
+    r.c1 = f.boff[2ull * l + 1];
+    r.c2 = f.boff[2ull * l + 2];
+    r.n0 = f.bnoff[2ull * l];
+    r.n1 = f.bnoff[2ull * l + 1];
+  } else {
+    r.u0 = r.u1 = 0xffffffffu;
+  }
+  return r;
+}
+
+// A unit of round l: long chain `chain` (FL_NONE: none), or the short-chain
+// positions [n0, n1) from tile start T on.
+struct fl_unit {
+  uint32_t l, chain, T, n1;
+};
+__device__ __forceinline__ fl_unit unit_of(uint32_t l, uint32_t off, uint32_t c1, uint32_t c2, uint32_t n0,
+                                           uint32_t n1, uint32_t stride) {
+  fl_unit u{l, FL_NONE, 0u, n1};
+  if (off < c2 - c1) u.chain = c1 + off;
+  else u.T = n0 + (off - (c2 - c1)) * stride;
+  return u;
+}
+// Unit v of the units of rounds 0, 1, ... (`back`: its place in the round
+// counted from the round's end, so that long chains still come first).
+__device__ __forceinline__ fl_unit find_unit(const fl_flow& f, fl_rounds& R, uint32_t rounds, uint32_t v, bool back,
+                                             uint32_t lane) {
+  uint32_t j;
+  for (;;) {
+    // (wavefront-uniform: every lane asks for the same unit)
+    const uint32_t below = (uint32_t)__builtin_popcountll(__ballot(R.u1 <= v));
+    const bool before = R.first > 0 && v < (uint32_t)__builtin_amdgcn_readlane((int)R.u0, 0);
+    if (!before && below < 64) {
+      j = below;
+      break;
+    }
+    R = load_rounds(f, before ? 0 : R.first + 64, rounds, lane);
+  }
+  const uint32_t u0 = (uint32_t)__builtin_amdgcn_readlane((int)R.u0, (int)j);
+  const uint32_t u1 = (uint32_t)__builtin_amdgcn_readlane((int)R.u1, (int)j);
+  const uint32_t c1 = (uint32_t)__builtin_amdgcn_readlane((int)R.c1, (int)j);
+  const uint32_t c2 = (uint32_t)__builtin_amdgcn_readlane((int)R.c2, (int)j);
+  const uint32_t n0 = (uint32_t)__builtin_amdgcn_readlane((int)R.n0, (int)j);
+  const uint32_t n1 = (uint32_t)__builtin_amdgcn_readlane((int)R.n1, (int)j);
+  return unit_of(R.first + j, back ? u1 - 1 - v : v - u0, c1, c2, n0, n1, 65u - f.long_min);
+}
+
+// A short-chain tile: lane i holds position T + i.  The tile owns the chains
+// whose heads lie in its first `stride` positions: with at most
+// long_min - 1 = 64 - stride positions they end within the tile, so every
+// chain lies whole in the tile that owns it (the tiles overlap).
+struct fl_short_tile {
+  uint32_t P;  // this lane's position, clamped into the round's
+  bool own;
+};
+__device__ __forceinline__ fl_short_tile short_tile(const uint32_t* __restrict__ pcnt, uint32_t T, uint32_t n1,
+                                                    uint32_t stride, uint32_t lane, uint32_t& cn) {
+  const bool in = T + lane < n1;
+  fl_short_tile t{in ? T + lane : n1 - 1, false};
+  cn = pcnt[t.P];
+  const unsigned long long heads = __ballot(in && (cn & FL_HEAD) && lane < stride);
+  // the last head at or before this lane, of any chain: owned when it is one
+  // of `heads`
+  const unsigned long long all = __ballot(in && (cn & FL_HEAD));
+  const unsigned long long upto = all & (~0ull >> (63u - lane));
+  t.own = in && upto != 0 && ((heads >> (63 - __builtin_clzll(upto | 1ull))) & 1ull) != 0;
+  return t;
+}
+
+}  // namespace
+
+// Drainage area of the site at chain position P, folded in the reference's
+// order (generator.rs:154-159 accumulates children in reverse BFS order, so
+// A_k = ((a_k + A_{c_m}) + A_{c_{m-1}}) + ... + A_{c_1} over the children in
+// row order).  The heavy child's value comes from the position after it: the
+// fold is split into `pre` (the part before it) and the light children after
+// it, posts p0..p3 in fold order.
+//
+// Absent posts are -0.0, and the chain fold starts from r = -0.0 at the
+// tail: x + (-0.0) == x exactly for every x (signed zeros included), so
+//     A = ((pre + r) + p0) + p1 ...
+// is the reference's value at every position without a branch.
+//
+// The partial folds of a listed position from the values of its listed light
+// children (v_i = the i-th listed child's A, -0.0 past the list).
+struct fl_da_part {
+  double pre, p0, p1, p2, p3;
+  uint32_t np;
+};
+struct fl_da_words {
+  unsigned long long u[FL_LIST];
+};
+__device__ __forceinline__ fl_da_part da_combine(uint32_t cn, double area_k, const fl_da_words& w, bool mine) {
+  if (!mine) return fl_da_part{FL_NEG0, FL_NEG0, FL_NEG0, FL_NEG0, FL_NEG0, 0u};
+  fl_da_part q;
+  const uint32_t npre = cn & 0xffu;
+  double v[FL_LIST];
 #pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            tp[u] = L.p[e - u];
-            ta[u] = L.a[e - u];
-            tb[u] = L.b[e - u];
-          }
-          const uint32_t sh = (uint32_t)(e - 7);
-          const uint32_t m2 = (uint32_t)(post2 >> sh) & 0xffu, m3 = (uint32_t)(rare >> sh) & 0xffu;
-          if (m3 == 0) {
-            if (m2 == 0) {
+  for (uint32_t i = 0; i < FL_LIST; ++i) v[i] = bits_double(w.u[i]);
+  // pre: x + (-0.0) == x, so the terms past npre are added as -0.0
+  q.pre = area_k;
 #pragma unroll
-              for (int u = 0; u < 8; ++u) {
-                r = (tp[u] + r) + ta[u];
-                L.r[e - u] = r;
-              }
-            } else {
+  for (uint32_t i = 0; i < FL_LIST; ++i) q.pre = q.pre + (i < npre ? v[i] : FL_NEG0);
+  // posts: list entries npre, npre + 1, ... (entries past the list are -0.0)
+  double p[FL_POSTS];
 #pragma unroll
-              for (int u = 0; u < 8; ++u) {
-                r = ((tp[u] + r) + ta[u]) + tb[u];
-                L.r[e - u] = r;
-              }
-            }
-          } else {
-            // (the third and fourth posts in two halves of four positions:
-            // registers)
-            const bool four = ((uint32_t)(post4 >> sh) & 0xffu) != 0;
+  for (uint32_t j = 0; j < FL_POSTS; ++j) {
+    p[j] = FL_NEG0;
 #pragma unroll
-            for (int h = 0; h < 8; h += 4) {
-              double tc[4], td[4];
+    for (uint32_t i = 0; i + j < FL_LIST; ++i) p[j] = npre == i ? v[i + j] : p[j];
+  }
+  q.p0 = p[0];
+  q.p1 = p[1];
+  q.p2 = p[2];
+  q.p3 = p[3];
+  q.np = (cn >> 8) & 0xffu;
+  return q;
+}
+
+// What the drainage-area fold reads at chain position P besides its counts and
+// listed children, in chain-major order (written by k_chain_perm): the site,
+// its area, erodibility and receiver distance.
+struct fl_da_pos {
+  uint32_t k;
+  double area, K, d;
+};
+
+// The arrays of the drainage-area sweep.
+struct fl_da_args {
+  const uint32_t* perm;
+  const uint32_t* pcnt;
+  double* cval;   // [FL_LIST n] light children's A by (position, list slot): hand-over words
+  double* cover;  // [n] at a chain's base: its head's A for a receiver with more light children than listed
+  const double* parea;
+  const double* pK;
+  const double* pdn;
+  const uint32_t* pdest;  // at a chain's base position: its head's slot in cval, FL_DEST_OVER or FL_NONE
+  const uint2* cmeta;     // long chains: (base, length)
+  double* xp;
+  double* taup;  // set to FL_SENT
+  double* hnp;   // with max slopes, too (else null)
+  // the graph, for positions with more light children than listed
+  const uint32_t* rp;
+  const uint32_t* col;
+  const uint32_t* next;
+  const unsigned long long* cmask;
+  const uint32_t* hc;
+  const uint32_t* head_base;
+  const double* area;
+  double* A;
+  int* stall;
+};
+
+__device__ __forceinline__ fl_da_pos da_load(const fl_da_args& g, uint32_t P) {
+  return fl_da_pos{g.perm[P], g.parea[P], g.pK[P], g.pdn[P]};
+}
+
+// The words of position P's listed children (-0.0 past the list).
+__device__ __forceinline__ uint32_t da_listed(uint32_t cn, bool mine) {
+  return mine ? (cn & 0xffu) + ((cn >> 8) & 0xffu) : 0u;
+}
+__device__ __forceinline__ fl_da_words da_words(const fl_da_args& g, uint32_t P, uint32_t cn, bool mine) {
+  const uint32_t nl = da_listed(cn, mine);
+  const double* w = g.cval + (uint64_t)FL_LIST * P;
+  fl_da_words q;
 #pragma unroll
-              for (int q = 0; q < 4; ++q) {
-                tc[q] = L.c[e - h - q];
-                td[q] = L.d[e - h - q];
-              }
-              if (!four) {
+  for (uint32_t i = 0; i < FL_LIST; ++i) q.u[i] = i < nl ? peek(w + i) : 1ull << 63;
+  return q;
+}
+__device__ __forceinline__ bool da_missing(const fl_da_words& q) {
+  bool m = false;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                  r = (((tp[h + q] + r) + ta[h + q]) + tb[h + q]) + tc[q];
-                  L.r[e - h - q] = r;
-                }
-              } else {
+  for (uint32_t i = 0; i < FL_LIST; ++i) m = m || q.u[i] == FL_SENT;
+  return m;
+}
+__device__ __forceinline__ void da_again(const fl_da_args& g, uint32_t P, fl_da_words& q) {
+  const double* w = g.cval + (uint64_t)FL_LIST * P;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                  r = ((((tp[h + q] + r) + ta[h + q]) + tb[h + q]) + tc[q]) + td[q];
-                  L.r[e - h - q] = r;
-                }
-              }
-            }
-          }
-        }
-        for (; e >= 0; --e) {
-          r = ((((L.p[e] + r) + L.a[e]) + L.b[e]) + L.c[e]) + L.d[e];
-          L.r[e] = r;
-        }
-      }
-      if (lane == 0 && deep) {
-        // a tile with a position of more posts than staged: those read the
-        // graph (da_tail_terms)
-        for (int e = (int)cnt - 1; e >= 0; --e) {
-          r = ((L.p[e] + r) + L.a[e]) + L.b[e];
-          if ((rare >> e) & 1ull)
-            r = da_tail_terms(r, L.n[e], L.c[e], L.d[e], L.k[e], g.rp, g.col, g.next, g.cmask, g.hc, g.A);
-          L.r[e] = r;
-        }
-      }
-      wave_sync();
-      // the tile D tiles further, loaded after the fold: a fold that waits
-      // for a load of its own (a deep tile) then waits for no tile's loads
-      cur = da_load(g, pos_of(ahead_of(end, D)));
-      if (mine) da_store(g, base + cs + lane, kk, L.r[lane], Kk, dk);
-      wave_sync();  // the tile arrays are rewritten next
-      end = cs;
-    };
-    fl_da_pos q0 = da_load(g, pos_of(end));
-    fl_da_pos q1 = da_load(g, pos_of(ahead_of(end, 1)));
-    if (D >= 3) {
-      fl_da_pos q2 = da_load(g, pos_of(ahead_of(end, 2)));
-      for (;;) {
-        step(q0);
-        if (end == 0) break;
-        step(q1);
-        if (end == 0) break;
-        step(q2);
-        if (end == 0) break;
-      }
+  for (uint32_t i = 0; i < FL_LIST; ++i)
+    if (q.u[i] == FL_SENT) q.u[i] = peek(w + i);
+}
+// Words that were read are given back.
+__device__ __forceinline__ void da_give_back(const fl_da_args& g, uint32_t P, uint32_t cn, bool mine) {
+  const uint32_t nl = da_listed(cn, mine);
+  unsigned long long* w = reinterpret_cast<unsigned long long*>(g.cval) + (uint64_t)FL_LIST * P;
+#pragma unroll
+  for (uint32_t i = 0; i < FL_LIST; ++i)
+    if (i < nl) w[i] = FL_SENT;
+}
+
+// A position with more light children than listed (rare) walks its row: the
+// first FL_LIST of them in fold order have list slots, the others their
+// chain's word in cover.
+__device__ __forceinline__ double* da_over_word(const fl_da_args& g, uint32_t P, uint32_t idx, uint32_t c) {
+  return idx < FL_LIST ? g.cval + (uint64_t)FL_LIST * P + idx : g.cover + g.head_base[c];
+}
+__device__ __forceinline__ bool da_over_ready(const fl_da_args& g, uint32_t k, uint32_t P) {
+  const uint32_t b = g.rp[k], deg = g.rp[k + 1] - b, hk = g.hc[k];
+  const unsigned long long m = g.cmask[k];
+  uint32_t idx = 0;
+  for (uint32_t s = deg; s-- > 0;) {
+    if (!is_child(m, deg, s, b, g.col, g.next, k)) continue;
+    const uint32_t c = g.col[b + s];
+    if (c != hk && peek(da_over_word(g, P, idx++, c)) == FL_SENT) return false;
+  }
+  return true;
+}
+__device__ __forceinline__ double da_over_fold(const fl_da_args& g, uint32_t k, uint32_t P, double r) {
+  const uint32_t b = g.rp[k], deg = g.rp[k + 1] - b, hk = g.hc[k];
+  const unsigned long long m = g.cmask[k];
+  double acc = g.area[k];
+  uint32_t idx = 0;
+  for (uint32_t s = deg; s-- > 0;) {
+    if (!is_child(m, deg, s, b, g.col, g.next, k)) continue;
+    const uint32_t c = g.col[b + s];
+    if (c == hk) {
+      acc = acc + r;
+      continue;
+    }
+    double* w = da_over_word(g, P, idx++, c);
+    acc = acc + bits_double(peek(w));
+    *reinterpret_cast<unsigned long long*>(w) = FL_SENT;
+  }
+  return acc;
+}
+
+template <int posts>
+__device__ __forceinline__ double da_step(const fl_da_part& q, double r) {
+  r = (q.pre + r) + q.p0;
+  if (posts > 1) r = r + q.p1;
+  if (posts > 2) r = (r + q.p2) + q.p3;
+  return r;
+}
+
+// The drainage areas of a tile of B consecutive positions a lane (r[0] the
+// one nearest the head), each from the position after it:
+//   r_i = ((pre_i + r_{i+1}) + p0_i) + p1_i ...
+// Every lane takes every step: once lane i + 1 holds its final values, lane i
+// gets its own in the next step and keeps them, so `steps` steps settle chains
+// over that many lanes without a lane ever being singled out.  Two DPP moves
+// and B times the adds a step: 14 ns a position with one a lane and two adds
+// (37 ns when one lane read the operands of eight positions at a time from
+// LDS).  As many posts are added as the tile's largest position has; the
+// others add -0.0.  Lanes past the tile pass `carry` on (pre and posts -0.0);
+// at a chain's tail (`tail`) the fold starts from -0.0.
+template <int B, int posts, bool tails>
+__device__ __forceinline__ void da_tile_steps(const fl_da_part (&q)[B], bool tail, double carry, uint32_t steps,
+                                              double (&r)[B]) {
+  double s = carry;
+#pragma unroll
+  for (int b = 0; b < B; ++b) r[b] = carry;
+#pragma unroll 4
+  for (uint32_t i = 0; i < steps; ++i) {
+    s = from_next(s, r[0]);
+    double v = tails && tail ? FL_NEG0 : s;
+#pragma unroll
+    for (int b = B - 1; b >= 0; --b) r[b] = v = da_step<posts>(q[b], v);
+  }
+}
+template <int B, bool tails>
+__device__ __forceinline__ void da_tile_fold(const fl_da_part (&q)[B], bool tail, double carry, uint32_t steps,
+                                             double (&r)[B]) {
+  uint32_t np = q[0].np;
+#pragma unroll
+  for (int b = 1; b < B; ++b) np = max(np, q[b].np);
+  if (!__any(np >= 2)) da_tile_steps<B, 1, tails>(q, tail, carry, steps, r);
+  else if (!__any(np >= 3)) da_tile_steps<B, 2, tails>(q, tail, carry, steps, r);
+  else da_tile_steps<B, 4, tails>(q, tail, carry, steps, r);
+}
+
+// The same for a tile with positions of more light children than listed: one
+// lane after the other.
+template <int B>
+__device__ __forceinline__ void da_tile_walk(const fl_da_args& g, const fl_da_pos (&t)[B], const uint32_t (&cn)[B],
+                                             const uint32_t (&P)[B], const bool (&mine)[B], const fl_da_part (&q)[B],
+                                             bool tail, double carry, uint32_t lane, double (&r)[B]) {
+  uint32_t spins = 0;
+  for (;;) {
+    bool wait = false;
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+      wait = wait || (mine[b] && (cn[b] & FL_LIST_OVERFLOW) && !da_over_ready(g, t[b].k, P[b]));
+    if (!__any(wait) || !wait_more(spins, g.stall)) break;
+  }
+  double v = carry;
+  for (uint32_t e = 64; e-- > 0;) {
+    if (lane == e) {
+      double x = tail ? FL_NEG0 : v;
+#pragma unroll
+      for (int b = B - 1; b >= 0; --b)
+        r[b] = x = mine[b] && (cn[b] & FL_LIST_OVERFLOW) ? da_over_fold(g, t[b].k, P[b], x) : da_step<4>(q[b], x);
+      v = x;
+    }
+    v = of_lane(v, e);
+  }
+}
+
+// A position's drainage area is final: store it and the response-time input
+// x = 1.0 / (K * a^0.5) * d (generator.rs:172-173, the reference's
+// association); the response-time words are to be waited for from here on.
+__device__ __forceinline__ void da_store(const fl_da_args& g, uint32_t P, const fl_da_pos& q, double a) {
+  g.A[q.k] = a;
+  const double celerity = q.K * rust_pow_half(a);
+  g.xp[P] = 1.0 / celerity * q.d;
+  reinterpret_cast<unsigned long long*>(g.taup)[P] = FL_SENT;
+  if (g.hnp) reinterpret_cast<unsigned long long*>(g.hnp)[P] = FL_SENT;
+}
+__device__ __forceinline__ void da_hand_over(const fl_da_args& g, uint32_t base, uint32_t pd, double a) {
+  if (pd == FL_NONE) return;
+  publish(pd == FL_DEST_OVER ? g.cover + base : g.cval + pd, a);
+}
+
+// One unit of the drainage-area sweep, tail to head along its chains.  A long
+// chain goes through tiles of 128 positions, two a lane (a step of two
+// positions costs 1.5 of one); a tile's words and inputs are loaded before the
+// fold of the tile before it, its counts one tile earlier.
+__device__ __forceinline__ void da_unit(const fl_da_args& g, const fl_unit& un, uint32_t stride, uint32_t lane) {
+  if (un.chain == FL_NONE) {
+    uint32_t cn[1];
+    const fl_short_tile t = short_tile(g.pcnt, un.T, un.n1, stride, lane, cn[0]);
+    const fl_da_pos at[1] = {da_load(g, t.P)};
+    const bool head = t.own && (cn[0] & FL_HEAD) != 0, tail = (cn[0] & FL_TAIL) != 0;
+    const uint32_t pd = head ? g.pdest[t.P] : FL_NONE;
+    fl_da_words w = da_words(g, t.P, cn[0], t.own);
+    uint32_t spins = 0;
+    while (__any(da_missing(w))) {
+      if (!wait_more(spins, g.stall)) break;
+      da_again(g, t.P, w);
+    }
+    const fl_da_part q[1] = {da_combine(cn[0], at[0].area, w, t.own)};
+    double r[1];
+    if (__any(t.own && (cn[0] & FL_LIST_OVERFLOW))) {
+      const uint32_t P[1] = {t.P};
+      const bool mine[1] = {t.own};
+      da_tile_walk<1>(g, at, cn, P, mine, q, tail, FL_NEG0, lane, r);
     } else {
-      for (;;) {
-        step(q0);
-        if (end == 0) break;
-        step(q1);
-        if (end == 0) break;
-      }
+      da_tile_fold<1, true>(q, tail, FL_NEG0, run_steps(__ballot(t.own && !tail)), r);
     }
-    // lane 0's value is the head's A
-    if (lane == 0 && pd != FL_NONE) g.cval_out[pd] = r;
+    if (head) da_hand_over(g, t.P, pd, r[0]);
+    da_give_back(g, t.P, cn[0], t.own);
+    if (t.own) da_store(g, t.P, at[0], r[0]);
+    return;
   }
-  // short chains: one lane each, the last blocks first (they hold no long
-  // chain).  When one pass covers them, the 64-chain groups of the wavefronts
-  // that share an XCD (workgroup index mod 8) are contiguous: chains placed
-  // together hold nearby sites, whose site-ordered stores then share an L2.
-  const uint32_t groups = (c1 - c0 + 63u) >> 6;
-  uint32_t sw = nwaves - 1 - wave;
-  if (groups <= nwaves && sw < groups) {
-    const uint32_t q = groups >> 3, rq = groups & 7u, x = sw & 7u;
-    sw = x * q + (x < rq ? x : rq) + (sw >> 3);
+  const uint2 m = g.cmeta[un.chain];
+  const uint32_t base = uniform(m.x), len = uniform(m.y);
+  const uint32_t pd = g.pdest[base];
+  // the lane's position b of the tile ending at `e` (past the tile: its first
+  // position); the tile after that one, or the tail's again past the head
+  auto pos_of = [&](uint32_t e, uint32_t b) {
+    const uint32_t cs = e > 128 ? e - 128 : 0, i = 2 * lane + b;
+    return base + (i < e - cs ? cs + i : cs);
+  };
+  auto in_tile = [&](uint32_t e, uint32_t b) { return 2 * lane + b < (e > 128 ? 128 : e); };
+  auto after = [&](uint32_t e) { return e > 128 ? e - 128 : len; };
+  double carry = FL_NEG0;
+  uint32_t cn[2], cn1[2];
+  fl_da_pos at[2];
+  fl_da_words w[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) cn[b] = g.pcnt[pos_of(len, b)];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    at[b] = da_load(g, pos_of(len, b));
+    cn1[b] = g.pcnt[pos_of(after(len), b)];
   }
-  for (uint32_t c = c0 + sw * 64u + lane; c < c1; c += nwaves * 64u) {
-    const uint2 m = cm2[2ull * c];
-    const uint32_t base = m.x, len = m.y;
-    const uint32_t pd = g.pdest[base];
-    double r = FL_NEG0;
-    uint32_t end = len;
-    while (end > 0) {
-      const uint32_t cs = end > FL_DA_BLOCK ? end - FL_DA_BLOCK : 0, cnt = end - cs;
-      fl_da_pos q[FL_DA_BLOCK];
 #pragma unroll
-      for (uint32_t u = 0; u < FL_DA_BLOCK; ++u)
-        if (u < cnt) q[u] = da_load(g, base + end - 1 - u);
-#pragma unroll
-      for (uint32_t u = 0; u < FL_DA_BLOCK; ++u) {
-        if (u < cnt) {
-          double pre, p0, p1, p2, p3;
-          uint32_t np;
-          if (q[u].cn & FL_LIST_OVERFLOW)
-            da_partial(q[u].k, g.rp, g.col, g.next, g.cmask, g.hc, g.area, g.A, pre, p0, p1, p2, p3, np);
-          else
-            da_combine(q[u].cn, q[u].area, q[u].v0, q[u].v1, q[u].v2, q[u].v3, pre, p0, p1, p2, p3, np);
-          r = ((pre + r) + p0) + p1;
-          if (np >= 3) r = da_tail_terms(r, np, p2, p3, q[u].k, g.rp, g.col, g.next, g.cmask, g.hc, g.A);
-          da_store(g, base + end - 1 - u, q[u].k, r, q[u].K, q[u].d);
-        }
-      }
-      end = cs;
+  for (int b = 0; b < 2; ++b) w[b] = da_words(g, pos_of(len, b), cn[b], in_tile(len, b));
+  for (uint32_t end = len;;) {
+    const uint32_t nxt = after(end), cnt = end > 128 ? 128 : end;
+    const uint32_t P[2] = {pos_of(end, 0), pos_of(end, 1)};
+    const bool mine[2] = {in_tile(end, 0), in_tile(end, 1)};
+    uint32_t spins = 0;
+    while (__any(da_missing(w[0]) || da_missing(w[1]))) {
+      if (!wait_more(spins, g.stall)) break;
+      da_again(g, P[0], w[0]);
+      da_again(g, P[1], w[1]);
     }
-    if (pd != FL_NONE) g.cval_out[pd] = r;
+    fl_da_part q[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) q[b] = da_combine(cn[b], at[b].area, w[b], mine[b]);
+    // (past the head these load what nothing reads: no word is listed)
+    fl_da_pos at1[2];
+    uint32_t cn2[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      w[b] = da_words(g, pos_of(nxt, b), cn1[b], end > 128 && in_tile(nxt, b));
+      at1[b] = da_load(g, pos_of(nxt, b));
+      cn2[b] = g.pcnt[pos_of(after(nxt), b)];
+    }
+    double r[2];
+    if (__any((mine[0] && (cn[0] & FL_LIST_OVERFLOW)) || (mine[1] && (cn[1] & FL_LIST_OVERFLOW))))
+      da_tile_walk<2>(g, at, cn, P, mine, q, false, carry, lane, r);
+    else
+      da_tile_fold<2, false>(q, false, carry, (cnt + 1) / 2, r);
+    carry = of_lane(r[0], 0);
+    if (end <= 128 && lane == 0) da_hand_over(g, base, pd, r[0]);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      da_give_back(g, P[b], cn[b], mine[b]);
+      if (mine[b]) da_store(g, P[b], at[b], r[b]);
+    }
+    if (end <= 128) break;
+    end = nxt;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      cn[b] = cn1[b];
+      cn1[b] = cn2[b];
+      at[b] = at1[b];
+    }
   }
 }
 
-__global__ void __launch_bounds__(64)
-k_da_fold(const uint32_t* __restrict__ guard, uint32_t l, const uint32_t* __restrict__ boff,
-          const uint4* __restrict__ cmeta, fl_da_args g) {
-  // the round's bounds are read together with the guard (one load latency;
-  // the bounds enter the test so that their loads stay above it: offsets are
-  // ascending, c2 < c0 never holds once the guard is clear)
-  const uint32_t c0 = boff[2 * l], c1 = boff[2 * l + 1], c2 = boff[2 * l + 2];
-  if (*guard != 0 || c2 < c0) return;  // pointer jumping has not converged: the iteration is redone
-  __shared__ fl_da_lds L;
-  da_round<3>(c0, c1, c2, blockIdx.x, gridDim.x, threadIdx.x, L, cmeta, g);
+// Rounds 0..min(deepest, cap - 1) of the drainage-area sweep, deepest first.
+__global__ void __launch_bounds__(64 * FL_FOLD_WAVES)
+k_da_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_da_args g) {
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t deepest = *f.maxld;
+  if (*guard != 0) return;  // pointer jumping has not converged: the iteration is redone
+  const uint32_t rounds = deepest < cap ? deepest + 1 : cap;
+  const uint32_t total = f.ucum[rounds];
+  fl_rounds R = load_rounds(f, 0, rounds, lane);
+  __shared__ uint32_t s_ticket;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) s_ticket = atomicAdd(f.ticket_da, (uint32_t)FL_FOLD_WAVES);
+    __syncthreads();
+    const uint32_t t = s_ticket;
+    if (t >= total) return;
+    if (t + wave < total) {
+      const fl_unit un = find_unit(f, R, rounds, total - 1 - (t + wave), true, lane);
+      da_unit(g, un, 65u - f.long_min, lane);
+    }
+    if ((uint64_t)gridDim.x * FL_FOLD_WAVES >= total) return;  // one turn covers the units
+  }
 }
 
-// Drainage-area rounds maxld, maxld - 1, ..., lsplit (the small deep ones) in
-// one workgroup of FL_TAIL_WAVES wavefronts, a workgroup barrier between rounds (a
-// round's results are read by the next one, within the workgroup): one
-// launch instead of one per round.  Rounds above `cap` are left out.
+// Rounds lsplit..deepest, deepest first, in one workgroup with a barrier
+// between rounds: the small deep rounds of an iteration whose sizes the host
+// knows, and every round of one whose waits ended without their values.
 __global__ void __launch_bounds__(64 * FL_TAIL_WAVES)
-k_da_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, uint32_t cap, const uint32_t* __restrict__ maxld,
-          const uint32_t* __restrict__ boff, const uint4* __restrict__ cmeta, fl_da_args g) {
-  uint32_t top = *maxld;
+k_da_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, fl_flow f, fl_da_args g) {
+  const uint32_t top = *f.maxld;
   if (*guard != 0 || top > 0xfffffffeu) return;  // pointer jumping has not converged: the iteration is redone
-  top = top < cap ? top : cap;
-  __shared__ fl_da_lds L[FL_TAIL_WAVES];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u, nwaves = FL_TAIL_WAVES;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
   for (uint32_t l = top + 1; l-- > lsplit;) {
-    const uint32_t c0 = boff[2 * l], c1 = boff[2 * l + 1], c2 = boff[2 * l + 2];
-    da_round<2>(c0, c1, c2, wave, nwaves, lane, L[wave], cmeta, g);
+    const uint32_t n = f.ucum[l + 1] - f.ucum[l];
+    for (uint32_t i = wave; i < n; i += FL_TAIL_WAVES)
+      da_unit(g, unit_of(l, i, f.boff[2ull * l + 1], f.boff[2ull * l + 2], f.bnoff[2ull * l], f.bnoff[2ull * l + 1],
+                         65u - f.long_min),
+              65u - f.long_min, lane);
     __syncthreads();
   }
 }
 
-// Response time along the chains of one light depth, head to tail:
-// rt_i = 0.0 + (rt_next + x_i) (generator.rs:173 with rt_i initially 0),
-// the basin outlet first (its receiver is itself).  A head's receiver lies
-// on a chain finished in an earlier round.  With clamp, also the elevation
-// recurrence of generator.rs:177-202, whose max-slope limit depends on the
-// receiver's new elevation.  Long chains [c1, c2) take one wavefront each
-// (blocks [0, c2 - c1)): tiles of 64 positions are staged in LDS, lane 0
-// runs the recurrence, the wavefront stores; short chains [c0, c1) one lane
-// each (the remaining blocks).
-// One wavefront's LDS tile of a response-time round.
-struct fl_tau_lds {
-  double x[64], u[64], t[64], d[64], tau[64], h[64];
+// The arrays of the response-time sweep.
+struct fl_tau_args {
+  const uint32_t* pcnt;
+  const uint32_t* ppos;  // at a chain's base: the position of its head's receiver, FL_NONE at a basin outlet
+  const uint2* cmeta;
+  const double* xp;
+  double* taup;
+  // with max slopes: by position the basin outlet's position, uplift,
+  // tan(max slope), receiver distance and old elevation; new elevations
+  const uint32_t* pro;
+  const double* up;
+  const double* tanp;
+  const double* dp;
+  const double* hop;
+  double* hnp;
+  int* stall;
 };
 
-// Wavefront `wave` of `nwaves` in response-time round l (short chains
-// [c0, c1), long chains [c1, c2)).
+// Response times of a tile of B consecutive positions a lane, each from the
+// position before it (first: a chain's head, from its receiver's value `tp`).
 //
 // The reference's step rt = 0.0 + (rt_next + x) adds 0.0, which changes
 // nothing unless y = rt_next + x is -0.0 (0.0 + -0.0 = +0.0; a NaN y is
 // already quiet and passes unchanged).  A sum is -0.0 only when both terms
 // are, and no running value is: a basin's outlet starts at 0.0 + (...),
 // never -0.0, and every other chain starts from its receiver's value.  So
-// the chains take the single add (one dependent operation per position
-// instead of two, bit for bit the same).
-template <bool clamp>
-__device__ __forceinline__ void
-tau_round(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t wave, uint32_t nwaves, uint32_t lane, fl_tau_lds& L,
-          const uint4* __restrict__ cmeta, const double* __restrict__ xp,
-          double* __restrict__ taup, const double* __restrict__ up, const double* __restrict__ tanp,
-          const double* __restrict__ dp, const double* __restrict__ hop, double* __restrict__ hnp) {
-  // long chains: one per block (uniform per block).  Tiles of 64 positions
-  // from the head, loaded three tiles ahead of their fold, unconditionally
-  // at positions clamped into the chain and into registers of their own
-  // (the loop is unrolled three times), so waiting for one tile never waits
-  // for the tiles loaded after it.
-  for (uint32_t c = c1 + wave; c < c2; c += nwaves) {
-    // base, length, position of the head's receiver (FL_NONE at the basin
-    // outlet) and of the basin outlet
-    const uint4 m = cmeta[c];
-    const uint32_t base = m.x, len = m.y;
-    // lane 0's recurrence state (at a basin outlet 0.0 + x_o, the
-    // reference's 0.0 + (0.0 + x_o): the same value, see above)
-    double tau = 0.0, tau_o = 0.0, h_p = 0.0, h_o = 0.0;
-    const uint32_t pp = m.z;
-    if (lane == 0 && pp != FL_NONE) {
-      tau = taup[pp];
-      if (clamp) {
-        uint32_t ro = m.w;
-        tau_o = taup[ro];
-        h_o = hnp[ro];
-        h_p = hnp[pp];
-      }
-    }
-    struct TauIn {
-      double x, u, t, d;
-    };
-    auto tile_in = [&](uint32_t t0) {
-      const uint32_t P = base + (t0 + lane < len ? t0 + lane : len - 1);
-      TauIn q{xp[P], 0.0, 0.0, 0.0};
-      if (clamp) {
-        q.u = up[P];
-        q.t = tanp[P];
-        q.d = dp[P];
-      }
-      return q;
-    };
-    uint32_t t = 0;
-    // fold the tile starting at t from q, then load into q the tile three
-    // tiles further
-    auto step = [&](TauIn& q) {
-      const uint32_t cnt = (len - t) < 64 ? (len - t) : 64;
-      const bool in = lane < cnt;
-      L.x[lane] = in ? q.x : 0.0;
-      if (clamp) {
-        L.u[lane] = in ? q.u : 0.0;
-        L.t[lane] = in ? q.t : 0.0;
-        L.d[lane] = in ? q.d : 0.0;
-      }
-      wave_sync();
-      q = tile_in(t + 192);
-      if (lane == 0) {
-        if (!clamp) {
-          // batches of eight, all within the tile (positions past the chain
-          // fold zeros into values nothing reads)
-          for (uint32_t j = 0; j < cnt; j += 8) {
-            double tx[8];
+// the chains take the single add, bit for bit the same.
+template <int B, bool heads>
+__device__ __forceinline__ void tau_tile_fold(const double (&x)[B], bool first, double tp, uint32_t steps,
+                                              double (&r)[B]) {
+  double s = tp;
 #pragma unroll
-            for (uint32_t u = 0; u < 8; ++u) tx[u] = L.x[j + u];
+  for (int b = 0; b < B; ++b) r[b] = tp;
+#pragma unroll 4
+  for (uint32_t i = 0; i < steps; ++i) {
+    s = from_prev(s, r[B - 1]);
+    double v = heads && first ? tp : s;
 #pragma unroll
-            for (uint32_t u = 0; u < 8; ++u) {
-              tau = tau + tx[u];  // 0.0 + y == y here (see above)
-              L.tau[j + u] = tau;
-            }
-          }
-        } else {
-          uint32_t j = 0;
-          if (t == 0 && pp == FL_NONE) {
-            // the outlet: rt_o = 0.0 + (0.0 + x_o); h_o' = h_o + U_o * max(0, 0)
-            tau = 0.0 + (0.0 + L.x[0]);
-            L.tau[0] = tau;
-            double ho = hop[base];
-            double nh = ho + L.u[0] * rust_max(tau - tau, 0.0);
-            double slope = (nh - ho) / L.d[0];
-            if (slope > L.t[0]) nh = ho + L.t[0] * L.d[0];
-            L.h[0] = nh;
-            h_p = nh;
-            h_o = nh;
-            tau_o = tau;
-            j = 1;
-          }
-          while (j < cnt) {
-            const uint32_t mm = (cnt - j) < 8 ? (cnt - j) : 8;
-            double tx[8], tu[8], tt[8], td[8];
-#pragma unroll
-            for (uint32_t u = 0; u < 8; ++u) {
-              if (u < mm) {
-                tx[u] = L.x[j + u];
-                tu[u] = L.u[j + u];
-                tt[u] = L.t[j + u];
-                td[u] = L.d[j + u];
-              }
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < 8; ++u) {
-              if (u < mm) {
-                tau = tau + tx[u];  // 0.0 + y == y here (see above)
-                double nh = h_o + tu[u] * rust_max(tau - tau_o, 0.0);
-                double slope = (nh - h_p) / td[u];
-                if (slope > tt[u]) nh = h_p + tt[u] * td[u];
-                L.tau[j + u] = tau;
-                L.h[j + u] = nh;
-                h_p = nh;
-              }
-            }
-            j += mm;
-          }
-        }
-      }
-      wave_sync();
-      if (in) {
-        taup[base + t + lane] = L.tau[lane];
-        if (clamp) hnp[base + t + lane] = L.h[lane];
-      }
-      wave_sync();  // the tile arrays are rewritten next
-      t += 64;
-    };
-    TauIn q0 = tile_in(0), q1 = tile_in(64), q2 = tile_in(128);
-    for (;;) {
-      step(q0);
-      if (t >= len) break;
-      step(q1);
-      if (t >= len) break;
-      step(q2);
-      if (t >= len) break;
-    }
-  }
-  // short chains: one lane each, the last blocks first (they hold no long
-  // chain); the groups of the wavefronts that share an XCD are contiguous
-  // when one pass covers them
-  const uint32_t groups = (c1 - c0 + 63u) >> 6;
-  uint32_t sw = nwaves - 1 - wave;
-  if (groups <= nwaves && sw < groups) {
-    const uint32_t q = groups >> 3, rq = groups & 7u, x = sw & 7u;
-    sw = x * q + (x < rq ? x : rq) + (sw >> 3);
-  }
-  for (uint32_t c = c0 + sw * 64u + lane; c < c1; c += nwaves * 64u) {
-    const uint4 m = cmeta[c];
-    const uint32_t base = m.x, len = m.y, pp = m.z;
-    double tau, tau_o = 0.0, h_p = 0.0, h_o = 0.0;
-    uint32_t t = 0;
-    if (pp == FL_NONE) {
-      tau = 0.0 + (0.0 + xp[base]);
-      taup[base] = tau;
-      if (clamp) {
-        double ho = hop[base];
-        double nh = ho + up[base] * rust_max(tau - tau, 0.0);
-        double tm = tanp[base], d = dp[base];
-        double slope = (nh - ho) / d;  // the receiver is the outlet itself, not yet updated
-        if (slope > tm) nh = ho + tm * d;
-        hnp[base] = nh;
-        h_p = nh;
-        h_o = nh;
-        tau_o = tau;
-      }
-      t = 1;
-    } else {
-      tau = taup[pp];
-      if (clamp) {
-        uint32_t ro = m.w;
-        tau_o = taup[ro];
-        h_o = hnp[ro];
-        h_p = hnp[pp];
-      }
-    }
-    if (!clamp) {
-      while (t < len) {
-        uint32_t cnt = (len - t) < FL_BATCH ? (len - t) : FL_BATCH;
-        // every slot loads (slots past the chain read its last position): no
-        // branch per load, so the batch's loads are in flight together
-        double vx[FL_BATCH];
-#pragma unroll
-        for (uint32_t q = 0; q < FL_BATCH; ++q) vx[q] = xp[base + t + (q < cnt ? q : cnt - 1)];
-#pragma unroll
-        for (uint32_t q = 0; q < FL_BATCH; ++q) {
-          if (q < cnt) {
-            tau = tau + vx[q];  // 0.0 + y == y here (see tau_round)
-            taup[base + t + q] = tau;
-          }
-        }
-        t += cnt;
-      }
-    } else {
-      while (t < len) {
-        uint32_t cnt = (len - t) < FL_BATCH ? (len - t) : FL_BATCH;
-        double vx[FL_BATCH], vu[FL_BATCH], vt[FL_BATCH], vd[FL_BATCH];
-#pragma unroll
-        for (uint32_t q = 0; q < FL_BATCH; ++q) {
-          const uint32_t P = base + t + (q < cnt ? q : cnt - 1);  // every slot loads (see above)
-          vx[q] = xp[P];
-          vu[q] = up[P];
-          vt[q] = tanp[P];
-          vd[q] = dp[P];
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < FL_BATCH; ++q) {
-          if (q < cnt) {
-            tau = tau + vx[q];  // 0.0 + y == y here (see tau_round)
-            double nh = h_o + vu[q] * rust_max(tau - tau_o, 0.0);
-            double slope = (nh - h_p) / vd[q];
-            if (slope > vt[q]) nh = h_p + vt[q] * vd[q];
-            taup[base + t + q] = tau;
-            hnp[base + t + q] = nh;
-            h_p = nh;
-          }
-        }
-        t += cnt;
-      }
-    }
+    for (int b = 0; b < B; ++b) r[b] = v = v + x[b];
   }
 }
 
-template <bool clamp>
-__global__ void __launch_bounds__(64)
-k_tau_fold(const uint32_t* __restrict__ guard, uint32_t l, const uint32_t* __restrict__ boff,
-           const uint4* __restrict__ cmeta, const double* __restrict__ xp, double* __restrict__ taup,
-           const double* __restrict__ up, const double* __restrict__ tanp, const double* __restrict__ dp,
-           const double* __restrict__ hop, double* __restrict__ hnp) {
-  // the round's bounds are read together with the guard (one load latency;
-  // the bounds enter the test so that their loads stay above it: offsets are
-  // ascending, c2 < c0 never holds once the guard is clear)
-  const uint32_t c0 = boff[2 * l], c1 = boff[2 * l + 1], c2 = boff[2 * l + 2];
-  if (*guard != 0 || c2 < c0) return;  // pointer jumping has not converged: the iteration is redone
-  __shared__ fl_tau_lds L;
-  tau_round<clamp>(c0, c1, c2, blockIdx.x, gridDim.x, threadIdx.x, L, cmeta, xp, taup, up, tanp, dp, hop, hnp);
+// Elevations of a tile with max slopes (generator.rs:177-202): z the value
+// without the limit, hp the receiver's new elevation at a chain's head
+// (`first`) and before the tile, t and d tan(max slope) and the receiver's
+// distance.  A site is limited when RN((z - hp) / d) > t; then its elevation
+// is hp + t * d.  `fixed` lanes keep z.
+//
+// The division stays off the serial chain: with d > 0 and t finite,
+//   z - hp > t * d * (1 + 2^-50)  implies  (z - hp) / d >= the double after t,
+//   z - hp < t * d * (1 - 2^-50)  implies  (z - hp) / d < t,
+// and rounding is monotonic, so either comparison decides it; only a
+// difference between the two bounds divides.  A tile in which no site is
+// limited needs one step.
+struct fl_clamp_pos {
+  double z, t, d;
+  bool fixed;
+};
+template <int B, bool heads>
+__device__ __forceinline__ void clamp_tile_fold(const fl_clamp_pos (&q)[B], bool first, double hp, uint32_t steps,
+                                                double (&h)[B]) {
+  double lo[B], hi[B];
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const double td = q[b].t * q[b].d, mag = __builtin_fabs(td), at = __builtin_fabs(q[b].t);
+    if (q[b].fixed || q[b].t != q[b].t) {
+      lo[b] = hi[b] = __builtin_inf();  // below both: not limited
+    } else if (q[b].d > 0.0 && mag >= 0x1p-900 && mag <= 0x1p900 && at >= 0x1p-900 && at <= 0x1p900) {
+      lo[b] = td - mag * 0x1p-50;
+      hi[b] = td + mag * 0x1p-50;
+    } else {
+      lo[b] = -__builtin_inf();  // between both: divides
+      hi[b] = __builtin_inf();
+    }
+    h[b] = q[b].z;
+  }
+  double s = hp;
+  for (uint32_t i = 0; i < steps; ++i) {
+    s = from_prev(s, h[B - 1]);
+    double v = heads && first ? hp : s;
+    bool some = false;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const double diff = q[b].z - v;
+      bool c = diff > hi[b];
+      const bool near = !c && !(diff < lo[b]) && !q[b].fixed;
+      if (__any(near)) c = near ? diff / q[b].d > q[b].t : c;
+      c = c && !q[b].fixed;
+      h[b] = v = c ? v + q[b].t * q[b].d : q[b].z;
+      some = some || c;
+    }
+    // no site limited: every lane started from its receiver's unlimited value
+    // and the values before it, and kept its own
+    if (i == 0 && !__any(some)) break;
+  }
 }
 
-// Response-time rounds lsplit, lsplit + 1, ..., maxld (the small deep ones)
-// in one workgroup of FL_TAIL_WAVES wavefronts, a workgroup barrier between rounds (a
-// round reads the response times and elevations of the previous ones): one
-// launch instead of one per round.  Rounds above `cap` are left out.
+// One unit of the response-time sweep, head to tail along its chains:
+// rt_i = rt_next + x_i, the basin outlet first (its receiver is itself).  With
+// clamp, also the elevation recurrence, whose max-slope limit depends on the
+// receiver's new elevation.
+template <bool clamp>
+__device__ __forceinline__ void tau_unit(const fl_tau_args& g, const fl_unit& un, uint32_t stride, uint32_t lane) {
+  if (un.chain == FL_NONE) {
+    uint32_t cn;
+    const fl_short_tile t = short_tile(g.pcnt, un.T, un.n1, stride, lane, cn);
+    const uint32_t P = t.P;
+    const double x = g.xp[P];
+    const bool head = t.own && (cn & FL_HEAD) != 0;
+    const uint32_t pp = head ? g.ppos[P] : FL_NONE;
+    const bool outlet = head && pp == FL_NONE;
+    double u = 0.0, tm = 0.0, d = 1.0, ho = 0.0;
+    uint32_t ro = 0;
+    if (clamp) {
+      u = g.up[P];
+      tm = g.tanp[P];
+      d = g.dp[P];
+      ho = g.hop[P];
+      ro = g.pro[P];
+    }
+    const double tp = await(g.taup + pp, head && !outlet, 0.0, g.stall);
+    const uint32_t steps = run_steps(__ballot(t.own && !head));
+    const double xs[1] = {x};
+    double tau[1];
+    tau_tile_fold<1, true>(xs, head, tp, steps, tau);
+    if (t.own) publish(g.taup + P, tau[0]);
+    if (clamp) {
+      const bool deep = un.l > 0;
+      double to = await(g.taup + ro, deep && t.own, 0.0, g.stall);
+      double h0 = await(g.hnp + ro, deep && t.own, 0.0, g.stall);
+      if (!deep) {
+        // the chains of the outlets: an outlet's elevation is
+        // h_o + U_o * max(0, 0), limited against its own old elevation
+        to = tau[0];
+        h0 = ho + u * rust_max(tau[0] - tau[0], 0.0);
+        if ((h0 - ho) / d > tm) h0 = ho + tm * d;
+        double st = to, sh = h0;
+        for (uint32_t i = 1; i < steps; ++i) {
+          st = from_prev(st, to);
+          sh = from_prev(sh, h0);
+          if (!head) {
+            to = st;
+            h0 = sh;
+          }
+        }
+      }
+      const double z = outlet ? h0 : h0 + u * rust_max(tau[0] - to, 0.0);
+      const double hp = await(g.hnp + pp, head && !outlet, 0.0, g.stall);
+      const fl_clamp_pos q[1] = {{z, tm, d, outlet || !t.own}};
+      double h[1];
+      clamp_tile_fold<1, true>(q, head, hp, steps, h);
+      if (t.own) publish(g.hnp + P, h[0]);
+    }
+    return;
+  }
+  // a long chain: tiles of B positions a lane, loaded two tiles ahead
+  constexpr int B = clamp ? 2 : 4;
+  constexpr uint32_t tile = 64 * B;
+  const uint2 m = g.cmeta[un.chain];
+  const uint32_t base = uniform(m.x), len = uniform(m.y);
+  const uint32_t pp = uniform(g.ppos[base]);
+  const bool outlet = pp == FL_NONE;  // the chain of a basin outlet
+  struct In {
+    double x[B], u[B], t[B], d[B];
+  };
+  auto load = [&](uint32_t t0, In& q) {
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const uint32_t i = t0 + B * lane + b, P = base + (i < len ? i : len - 1);
+      q.x[b] = g.xp[P];
+      if (clamp) {
+        q.u[b] = g.up[P];
+        q.t[b] = g.tanp[P];
+        q.d[b] = g.dp[P];
+      }
+    }
+  };
+  double tau_c = 0.0, h_c = 0.0, to = 0.0, h0 = 0.0;
+  auto fold = [&](uint32_t t0, const In& q) {
+    const uint32_t cnt = len - t0 < tile ? len - t0 : tile;
+    const uint32_t P = base + t0 + B * lane;
+    const uint32_t last = (cnt - 1) / B;  // the lane of the tile's last position
+    double tau[B];
+    tau_tile_fold<B, false>(q.x, false, tau_c, last + 1, tau);
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+      if (B * lane + b < cnt) publish(g.taup + P + b, tau[b]);
+    tau_c = of_lane(tau[B - 1], last);  // (read past the chain's end only when nothing follows)
+    if (clamp) {
+      const bool first = t0 == 0 && outlet;
+      if (first) {
+        // (see the short chains) lane 0's first position is the outlet
+        const double ho = g.hop[base];
+        double nh = ho + q.u[0] * rust_max(tau[0] - tau[0], 0.0);
+        if ((nh - ho) / q.d[0] > q.t[0]) nh = ho + q.t[0] * q.d[0];
+        to = of_lane(tau[0], 0);
+        h0 = of_lane(nh, 0);
+      }
+      fl_clamp_pos c[B];
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        const bool fixed = first && lane == 0 && b == 0;
+        c[b] = fl_clamp_pos{fixed ? h0 : h0 + q.u[b] * rust_max(tau[b] - to, 0.0), q.t[b], q.d[b],
+                            fixed || B * lane + b >= cnt};
+      }
+      double h[B];
+      clamp_tile_fold<B, false>(c, false, h_c, last + 1, h);
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+        if (B * lane + b < cnt) publish(g.hnp + P + b, h[b]);
+      h_c = of_lane(h[B - 1], last);
+    }
+  };
+  In q0, q1;
+  load(0, q0);
+  load(tile, q1);
+  uint32_t ro = 0;
+  if (clamp) ro = g.pro[base];
+  tau_c = await(g.taup + pp, !outlet, 0.0, g.stall);
+  if (clamp) {
+    to = await(g.taup + ro, !outlet, 0.0, g.stall);
+    h0 = await(g.hnp + ro, !outlet, 0.0, g.stall);
+    h_c = await(g.hnp + pp, !outlet, 0.0, g.stall);
+  }
+  for (uint32_t t0 = 0;;) {
+    fold(t0, q0);
+    if ((t0 += tile) >= len) break;
+    load(t0 + tile, q0);
+    fold(t0, q1);
+    if ((t0 += tile) >= len) break;
+    load(t0 + tile, q1);
+  }
+}
+
+// Rounds 0..min(deepest, cap - 1) of the response-time sweep, shallowest
+// first.
+template <bool clamp>
+__global__ void __launch_bounds__(64 * FL_FOLD_WAVES)
+k_tau_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_tau_args g) {
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t deepest = *f.maxld;
+  if (*guard != 0) return;  // pointer jumping has not converged: the iteration is redone
+  const uint32_t rounds = deepest < cap ? deepest + 1 : cap;
+  const uint32_t total = f.ucum[rounds];
+  fl_rounds R = load_rounds(f, 0, rounds, lane);
+  __shared__ uint32_t s_ticket;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) s_ticket = atomicAdd(f.ticket_tau, (uint32_t)FL_FOLD_WAVES);
+    __syncthreads();
+    const uint32_t t = s_ticket;
+    if (t >= total) return;
+    if (t + wave < total) {
+      const fl_unit un = find_unit(f, R, rounds, t + wave, false, lane);
+      tau_unit<clamp>(g, un, 65u - f.long_min, lane);
+    }
+    if ((uint64_t)gridDim.x * FL_FOLD_WAVES >= total) return;  // one turn covers the units
+  }
+}
+
+// Rounds lsplit..deepest, shallowest first, in one workgroup (see k_da_tail).
 template <bool clamp>
 __global__ void __launch_bounds__(64 * FL_TAIL_WAVES)
-k_tau_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, uint32_t cap, const uint32_t* __restrict__ maxld,
-           const uint32_t* __restrict__ boff, const uint4* __restrict__ cmeta, const double* __restrict__ xp,
-          double* __restrict__ taup, const double* __restrict__ up, const double* __restrict__ tanp,
-          const double* __restrict__ dp, const double* __restrict__ hop, double* __restrict__ hnp) {
-  uint32_t top = *maxld;
+k_tau_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, fl_flow f, fl_tau_args g) {
+  const uint32_t top = *f.maxld;
   if (*guard != 0 || top > 0xfffffffeu) return;  // pointer jumping has not converged: the iteration is redone
-  top = top < cap ? top : cap;
-  __shared__ fl_tau_lds L[FL_TAIL_WAVES];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u, nwaves = FL_TAIL_WAVES;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
   for (uint32_t l = lsplit; l <= top; ++l) {
-    const uint32_t c0 = boff[2 * l], c1 = boff[2 * l + 1], c2 = boff[2 * l + 2];
-    tau_round<clamp>(c0, c1, c2, wave, nwaves, lane, L[wave], cmeta, xp, taup, up, tanp, dp, hop, hnp);
+    const uint32_t n = f.ucum[l + 1] - f.ucum[l];
+    for (uint32_t i = wave; i < n; i += FL_TAIL_WAVES)
+      tau_unit<clamp>(g, unit_of(l, i, f.boff[2ull * l + 1], f.boff[2ull * l + 2], f.bnoff[2ull * l],
+                                 f.bnoff[2ull * l + 1], 65u - f.long_min),
+                      65u - f.long_min, lane);
     __syncthreads();
   }
 }
@@ -1867,64 +2059,66 @@ void fl_launch_chain_count(hipStream_t s, const fl_dev_terrain& t, const fl_dev_
                  w.long_min, w.act);
 }
 
-void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t rounds) {
-  uint64_t fill = std::min<uint64_t>(2ull * rounds, 2ull * t.n + 2);
-  FL_LAUNCH_GRID(k_bucket_scan, dim3(1), dim3(FL_SCAN_BLOCK), 0, s, t.n, (uint32_t)fill, w.ctrl, w.bcnt, w.bnodes, w.boff,
-                 w.bnoff);
+void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w) {
+  FL_LAUNCH_GRID(k_bucket_scan, dim3(1), dim3(FL_SCAN_BLOCK), 0, s, t.n, w.long_min, w.ctrl, w.bcnt, w.bnodes, w.boff,
+                 w.bnoff, w.ucum);
   uint32_t per = FL_BUCKET_BLOCK * FL_BUCKET_PER_THREAD;
   FL_LAUNCH_GRID(k_bucket_place, dim3((t.n + per - 1) / per), dim3(FL_BUCKET_BLOCK), t.n, s, w.guard, t.n, w.hc,
                  (const unsigned long long*)w.cp, (const unsigned long long*)w.rt, t.is_outlet, w.boff, w.bnoff,
-                 w.bcur, w.bncur, w.cmeta, w.head_chain, w.pdest, w.head_base, w.long_min, w.act);
-  fl_perm_out o{w.perm, w.pcnt, w.pdest, w.parea, w.pK, w.pdn, w.up, w.tanp, w.dp, w.hop, w.cmeta};
+                 w.bcur, w.bncur, w.cmeta, w.pdest, w.head_base, w.long_min, w.act);
+  fl_perm_out o{w.perm, w.pcnt, w.pdest, w.parea, w.pK, w.pdn, w.up, w.tanp, w.hop, w.ppos, w.pro};
   FL_LAUNCH(k_chain_perm, t.n, s, w.guard, t.n, (const unsigned long long*)w.cp, (const unsigned long long*)w.rt,
-            w.next, t.is_outlet, w.head_base, w.head_chain, o, t.area, t.erod, w.dnext, t.uplift, t.tan_ms,
+            w.next, t.is_outlet, w.head_base, o, t.area, t.erod, w.dnext, t.uplift, t.tan_ms,
             t.any_max_slope ? 1 : 0, w.A, w.tau, w.h, w.h2, w.counters + FL_CNT_MAXLD, w.bcnt, w.bnodes, w.bcur,
             w.bncur, t.row_ptr, t.col, (const unsigned long long*)w.cmask, w.hc, w.act, w.root);
 }
 
 namespace {
-fl_da_args da_args(const fl_dev_terrain& t, const fl_dev_work& w) {
-  return fl_da_args{w.perm, w.pcnt,   w.cval, w.parea, w.pK, w.pdn, w.pdest, w.cval, w.xp,
-                    t.row_ptr, t.col, w.next, (const unsigned long long*)w.cmask, w.hc, t.area, w.A};
+fl_flow flow(const fl_dev_work& w) {
+  return fl_flow{w.counters + FL_CNT_MAXLD,       w.ucum, w.boff, w.bnoff, w.counters + FL_CNT_TICKET_DA,
+                 w.counters + FL_CNT_TICKET_TAU, w.long_min};
 }
+fl_da_args da_args(const fl_dev_terrain& t, const fl_dev_work& w, bool clamp) {
+  return fl_da_args{w.perm, w.pcnt,  w.cval, w.cover, w.parea, w.pK, w.pdn, w.pdest, w.cmeta, w.xp, w.taup,
+                    clamp ? w.hnp : nullptr, t.row_ptr, t.col, w.next, (const unsigned long long*)w.cmask, w.hc,
+                    w.head_base, t.area, w.A, w.flags + FL_FLAG_STALL};
+}
+fl_tau_args tau_args(const fl_dev_work& w) {
+  return fl_tau_args{w.pcnt, w.ppos, w.cmeta, w.xp, w.taup, w.pro, w.up, w.tanp, w.pdn, w.hop, w.hnp,
+                     w.flags + FL_FLAG_STALL};
+}
+dim3 fold_grid(uint32_t waves) { return dim3((std::max<uint32_t>(waves, 1) + FL_FOLD_WAVES - 1) / FL_FOLD_WAVES); }
 }  // namespace
 
-void fl_launch_da_round(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t l,
-                        const fl_round_grid& g, bool clamp) {
-  (void)clamp;  // the max-slope inputs are laid out by k_chain_perm
-  if (g.fold_blocks)
-    FL_LAUNCH_GRID(k_da_fold, dim3(g.fold_blocks), dim3(64), g.positions, s, w.guard, l, w.boff, w.cmeta,
-                   da_args(t, w));
+void fl_launch_da_fold(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t cap, uint32_t waves,
+                       uint64_t positions, bool clamp) {
+  FL_LAUNCH_GRID(k_da_fold, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w),
+                 da_args(t, w, clamp));
 }
 
-void fl_launch_da_tail(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t lsplit, uint32_t cap,
-                       uint64_t units, bool clamp) {
-  (void)clamp;
-  FL_LAUNCH_GRID(k_da_tail, dim3(1), dim3(64 * FL_TAIL_WAVES), units, s, w.guard, lsplit, cap,
-                 w.counters + FL_CNT_MAXLD, w.boff, w.cmeta, da_args(t, w));
+void fl_launch_da_tail(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t lsplit,
+                       uint64_t positions, bool clamp) {
+  FL_LAUNCH_GRID(k_da_tail, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w),
+                 da_args(t, w, clamp));
 }
 
-void fl_launch_tau_tail(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t lsplit, uint32_t cap,
-                        uint64_t units, bool clamp) {
-  (void)t;
+void fl_launch_tau_fold(hipStream_t s, const fl_dev_work& w, uint32_t cap, uint32_t waves, uint64_t positions,
+                        bool clamp) {
   if (clamp)
-    FL_LAUNCH_GRID(k_tau_tail<true>, dim3(1), dim3(64 * FL_TAIL_WAVES), units, s, w.guard, lsplit, cap,
-                   w.counters + FL_CNT_MAXLD, w.boff, w.cmeta, w.xp, w.taup, w.up, w.tanp, w.dp, w.hop, w.hnp);
+    FL_LAUNCH_GRID(k_tau_fold<true>, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w),
+                   tau_args(w));
   else
-    FL_LAUNCH_GRID(k_tau_tail<false>, dim3(1), dim3(64 * FL_TAIL_WAVES), units, s, w.guard, lsplit, cap,
-                   w.counters + FL_CNT_MAXLD, w.boff, w.cmeta, w.xp, w.taup, w.up, w.tanp, w.dp, w.hop, w.hnp);
+    FL_LAUNCH_GRID(k_tau_fold<false>, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w),
+                   tau_args(w));
 }
 
-void fl_launch_tau_round(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t l,
-                         const fl_round_grid& g, bool clamp) {
-  (void)t;
-  if (!g.fold_blocks) return;
+void fl_launch_tau_tail(hipStream_t s, const fl_dev_work& w, uint32_t lsplit, uint64_t positions, bool clamp) {
   if (clamp)
-    FL_LAUNCH_GRID(k_tau_fold<true>, dim3(g.fold_blocks), dim3(64), g.positions, s, w.guard, l, w.boff, w.cmeta,
-                   w.xp, w.taup, w.up, w.tanp, w.dp, w.hop, w.hnp);
+    FL_LAUNCH_GRID(k_tau_tail<true>, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w),
+                   tau_args(w));
   else
-    FL_LAUNCH_GRID(k_tau_fold<false>, dim3(g.fold_blocks), dim3(64), g.positions, s, w.guard, l, w.boff, w.cmeta,
-                   w.xp, w.taup, w.up, w.tanp, w.dp, w.hop, w.hnp);
+    FL_LAUNCH_GRID(k_tau_tail<false>, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w),
+                   tau_args(w));
 }
 
 void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool clamp,
@@ -1937,6 +2131,13 @@ void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_
 void fl_launch_clear_iter(hipStream_t s, const fl_dev_work& w, uint32_t nb) {
   uint32_t cnt = nb > FL_CTRL_WORDS ? nb : FL_CTRL_WORDS;
   FL_LAUNCH(k_clear_iter, cnt, s, nb, w.ctrl, w.bcnt, w.bnodes, w.bcur, w.bncur);
+}
+
+// (launched in parts: the kernel counts items in 32 bits)
+void fl_launch_reset_words(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w) {
+  for (uint32_t i = 0; i < FL_LIST; i++)
+    FL_LAUNCH(k_fill_u64, t.n, s, t.n, (uint64_t*)w.cval + (uint64_t)i * t.n, FL_SENT);
+  FL_LAUNCH(k_fill_u64, t.n, s, t.n, (uint64_t*)w.cover, FL_SENT);
 }
 
 void fl_launch_fill_u32(hipStream_t s, uint32_t* p, uint64_t count, uint32_t v) {

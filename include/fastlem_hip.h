@@ -155,12 +155,13 @@ int32_t fl_ctx_set_rehint_rounds(fl_ctx *ctx, uint32_t rounds);
  * same bits); they shape the work:
  *   site_block        workgroup size of the per-site kernels (64..1024, a
  *                     multiple of 64);
- *   long_chain        chains of at least this many sites fold in a wavefront
- *                     with LDS-staged tiles, shorter ones in one lane (the
- *                     switch between the two forms of a sweep round, >= 1);
- *   tail_units        sweep rounds of at most this many fold units run
- *                     together, one launch per sweep (levels per launch; 0:
- *                     one launch per round);
+ *   long_chain        chains of at least this many sites take a wavefront
+ *                     each in the sweeps, shorter ones share tiles of 64
+ *                     positions (>= 1; more than 33 acts as 33);
+ *   tail_units        iterations whose sizes the host reads first (a
+ *                     solve's first ones): deep sweep rounds of at most
+ *                     this many wavefronts each run in one workgroup, a
+ *                     barrier between rounds;
  *   pipelining        0, 1 or 3 as fl_ctx_set_pipelining (3: HIP graphs);
  *   compact_min_idle  batches: as fl_ctx_set_batch_compaction.
  * Without fl_ctx_set_tuning a solve takes the library's table, chosen by
