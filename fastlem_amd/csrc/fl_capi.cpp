@@ -691,7 +691,7 @@ int32_t decompose(fl_ctx* c, fl_terrain* T, bool full, bool joined) {
 }
 
 // Sweep units of round l from bucket offsets (boff[nb+1] then bnoff[nb+1]):
-// its long chains and the tiles of its short chains' positions; positions:
+// its long chains' tiles and those of its short chains' positions; positions:
 // all of its positions.
 struct RoundSize {
   uint32_t units = 0;

@@ -48,10 +48,10 @@ enum {
 // (n + 1) / 2 and their buckets (two a round) at most n + 1.
 enum { FL_BUCKET_PAD = 8 };
 // Light children listed per chain position.  A position with more walks its
-// row, which takes as long as ten light edges (13 us), so the list holds what
-// a planar triangulation has (four were too few at one position in about a
-// thousand, and every path to an outlet met one).
-enum { FL_LIST = 6 };
+// row: 15 us on a wavefront that every path below it waits for, where a light
+// edge takes 2.  A random triangulation has one with seven or more in ten thousand
+// sites, one with nine or more in millions.
+enum { FL_LIST = 8 };
 // Chains are short below at most this length (a sweep's short-chain tile of
 // 64 positions advances by 65 - long_min).
 enum { FL_LONG_MAX = 33 };
@@ -107,15 +107,15 @@ struct fl_dev_work {
   uint32_t* hc = nullptr;     // [n] heavy child
   // drainage-area inputs in chain-major order (written by k_chain_perm):
   // list counts, own area, erodibility, receiver distance; the listed light
-  // children's drainage areas (FL_LIST slots per position, fold order,
-  // filled by the children's rounds: pdest at a chain's base position names
-  // the slot of its head, ppos there the position of its receiver)
+  // children's drainage areas (FL_LIST slots per position, filled by the
+  // children's rounds: pdest at a chain's base position names the slot of its
+  // head, ppos there the position of its receiver)
   uint32_t* pcnt = nullptr;   // [n] npre | npost << 8, or the overflow flag; tail and head flags
   double* parea = nullptr;    // [n]
   double* pK = nullptr;       // [n]
   double* pdn = nullptr;      // [n]
   double* cval = nullptr;     // [FL_LIST n] hand-over words
-  double* cover = nullptr;    // [n] hand-over words past the lists, at the children's bases
+  double* cover = nullptr;    // [n] hand-over words past the lists, at the children's bases, and between a chain's tiles
   uint32_t* pdest = nullptr;  // [n]
   uint32_t* ppos = nullptr;   // [n]
 
@@ -127,7 +127,7 @@ struct fl_dev_work {
   uint32_t *bcnt = nullptr, *bnodes = nullptr, *boff = nullptr, *bnoff = nullptr, *bcur = nullptr,
            *bncur = nullptr;                                  // [n + FL_BUCKET_PAD] light-depth buckets
   uint32_t* ucum = nullptr;                                  // [n + FL_BUCKET_PAD] sweep units before each round
-  uint2* cmeta = nullptr;                                    // [n] long chains: (base position, length)
+  uint2* cmeta = nullptr;                                    // [n] long chains' tiles: (base position, length or end)
   uint32_t* head_base = nullptr;                             // [n] at a chain head: its base position
   uint32_t* perm = nullptr;                                  // [n] chain-major site order
   uint32_t* ctrl = nullptr;                                  // [FL_CTRL_WORDS]
@@ -136,8 +136,8 @@ struct fl_dev_work {
   const uint32_t* guard = nullptr;
   int* flags = nullptr;                                      // = ctrl
   uint32_t* counters = nullptr;                              // = ctrl + FL_NUM_FLAGS
-  // chains of at least long_min sites (at most FL_LONG_MAX) take a wavefront
-  // each, shorter ones share one (a tuning: results do not depend on it)
+  // chains of at least long_min sites (at most FL_LONG_MAX) take wavefronts of
+  // their own, shorter ones share one (a tuning: results do not depend on it)
   uint32_t long_min = 16;
   // Basins recomputed in an iteration.  A new elevation is a function of the
   // drainage tree alone (and the static parameters), so a basin of the

@@ -46,12 +46,12 @@
 #include "fl_kernels.h"
 
 #define FL_NONE 0xffffffffu
-#define FL_POSTS 4                  // most of them after the heavy child
 #define FL_LIST_OVERFLOW 0x10000u   // pcnt flag: more light children than listed
 #define FL_ROW 8                    // graph row entries loaded together
+static_assert(FL_ROW <= FL_LIST, "a row loaded at once fits its position's list");
 #define FL_TAIL 0x20000u            // pcnt flag: the position is its chain's tail
 #define FL_HEAD 0x40000u            // ... its chain's head
-#define FL_DEST_OVER 0xfffffffeu    // pdest: the receiver reads the chain's word in cover
+#define FL_DEST_OVER 0xfffffffeu    // pdest: the receiver reads the chain's word in cover, not a slot
 
 namespace {
 
@@ -445,9 +445,16 @@ __global__ void k_chain_jump(uint32_t bs, uint32_t n, unsigned long long* cp, un
 }
 
 // Buckets: 2 * light depth + (chain length >= long_min), so every round
-// has a range of short chains (one lane each) followed by long ones (one
-// wavefront each); long_min is a launch parameter (tuned; any value >= 1
-// gives the same results).
+// has a range of short chains followed by long ones; long_min is a launch
+// parameter (tuned; any value >= 1 gives the same results).  A short bucket
+// counts its chains, a long one the tiles of its chains: FL_TILE positions
+// each, counted from the chain's head (its tail's tile may hold fewer).
+#define FL_TILE 128
+#define FL_CHAIN_PART 0x80000000u  // cmeta.y: not the tile of the chain's head (the tile's end, else the length)
+#define FL_CHAIN_TAIL 0x80000000u  // cmeta.x: the tile of the chain's tail
+__device__ __forceinline__ uint32_t bucket_weight(uint32_t len, uint32_t long_min) {
+  return len >= long_min ? (len + FL_TILE - 1) / FL_TILE : 1u;
+}
 #define FL_LDS_BUCKETS 128
 #define FL_BUCKET_BLOCK 1024
 #define FL_BUCKET_PER_THREAD 2
@@ -485,7 +492,7 @@ __device__ __forceinline__ void load_tails(uint32_t base, uint32_t n, const uint
     if (q[j].t) q[j].t = is_outlet[pair_ptr(q[j].r)] != 0;
 }
 
-// Light-depth histogram of the chains (count and total length), aggregated
+// Light-depth histogram of the chains (buckets' counts and total length), aggregated
 // per workgroup in LDS before one global atomic per (workgroup, bucket).
 // Each chain is counted by its tail (the member without a heavy child),
 // which knows the chain's length (its position + 1) and light depth.
@@ -509,11 +516,12 @@ k_bucket_count(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* _
   for (uint32_t j = 0; j < FL_BUCKET_PER_THREAD; ++j) {
     if (q[j].t) {
       uint32_t lw = pair_cnt(q[j].r), len = pair_cnt(q[j].c) + 1, l = 2u * lw + (len >= long_min ? 1u : 0u);
+      const uint32_t wt = bucket_weight(len, long_min);
       if (l < FL_LDS_BUCKETS) {
-        atomicAdd(s_c + l, 1u);
+        atomicAdd(s_c + l, wt);
         atomicAdd(s_n + l, len);
       } else {
-        atomicAdd(bcnt + l, 1u);
+        atomicAdd(bcnt + l, wt);
         atomicAdd(bnodes + l, len);
       }
       atomicMax(&s_max, lw);
@@ -557,8 +565,8 @@ k_bucket_scan(uint32_t n, uint32_t long_min, uint32_t* __restrict__ ctrl,
   for (uint32_t base = 0; base < nb; base += FL_SCAN_BLOCK) {
     uint32_t i = base + threadIdx.x;
     uint32_t a = i < nb ? bcnt[i] : 0, b = i < nb ? bnodes[i] : 0;
-    // a round's units in its second bucket's place: its long chains and the
-    // tiles of its short chains' positions
+    // a round's units in its second bucket's place: its long chains' tiles
+    // and the tiles of its short chains' positions
     uint32_t q = (i & 1u) && i < nb ? a + (bnodes[i - 1] + stride - 1) / stride : 0u;
     s_a[threadIdx.x] = a;
     s_b[threadIdx.x] = b;
@@ -608,13 +616,18 @@ k_bucket_scan(uint32_t n, uint32_t long_min, uint32_t* __restrict__ ctrl,
 // Give every chain (through its tail) a slot in its light-depth bucket and a
 // contiguous range of positions: LDS atomics rank the chains of a workgroup,
 // one global atomic per (workgroup, bucket) reserves the ranges.  Order
-// inside a bucket is immaterial to the results.  A long chain's record is
-// (base, len), a chain's head knows its base, and the base's receiver slot
-// starts empty.
+// inside a bucket is immaterial to the results.  A long chain has a record
+// per tile, the tail's first, (base, end of the tile), the head's (base, len);
+// a chain's head knows its base, and the base's receiver slot starts empty.
 __device__ __forceinline__ void place_chain(uint32_t q, uint32_t pos, uint32_t len, uint32_t hd, uint32_t long_min,
                                             uint2* __restrict__ cmeta, uint32_t* __restrict__ head_base,
                                             uint32_t* __restrict__ pdest) {
-  if (len >= long_min) cmeta[q] = make_uint2(pos, len);
+  if (len >= long_min) {
+    uint32_t end = len;
+    for (; end > FL_TILE; end = (end - 1) & ~(FL_TILE - 1u))
+      cmeta[q++] = make_uint2(pos | (end == len ? FL_CHAIN_TAIL : 0u), end | FL_CHAIN_PART);
+    cmeta[q] = make_uint2(pos | (end == len ? FL_CHAIN_TAIL : 0u), len);
+  }
   head_base[hd] = pos;
   pdest[pos] = FL_NONE;
 }
@@ -644,10 +657,10 @@ k_bucket_place(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* _
       const unsigned long long c = tl[j].c;
       uint32_t len = pair_cnt(c) + 1, l = 2u * pair_cnt(tl[j].r) + (len >= long_min ? 1u : 0u);
       if (l < FL_LDS_BUCKETS) {
-        lc[j] = atomicAdd(s_c + l, 1u);
+        lc[j] = atomicAdd(s_c + l, bucket_weight(len, long_min));
         ln[j] = atomicAdd(s_n + l, len);
       } else {
-        uint32_t q = boff[l] + atomicAdd(bcur + l, 1u);
+        uint32_t q = boff[l] + atomicAdd(bcur + l, bucket_weight(len, long_min));
         uint32_t pos = bnoff[l] + atomicAdd(bncur + l, len);
         place_chain(q, pos, len, pair_ptr(c), long_min, cmeta, head_base, pdest);
       }
@@ -772,16 +785,17 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
     o.hop[P] = h[v];
     o.pro[P] = hbr;
   }
-  // the light children in fold order (descending slot), those before the
-  // heavy child first: the first FL_LIST get slots FL_LIST * P + i for
-  // their chains' heads to fill; with more, the overflow bit is set (the fold
-  // walks the row) and the others' heads hand over at their own bases
+  // the light children in fold order (descending slot): those before the
+  // heavy child get their receiver's slots 0, 1, ..., those after it the slots
+  // FL_LIST - 1, FL_LIST - 2, ... for their chains' heads to fill; with more
+  // than FL_LIST the overflow bit is set (the fold walks the row) and all of
+  // their heads hand over at their own bases
   {
     uint32_t npre = 0, npost = 0;
     bool after = false;
     if (short_row) {
       // the children's bases loaded together (a row of at most FL_ROW
-      // entries: the child mask covers it)
+      // entries, no more than a list holds: the child mask covers it)
       uint32_t hb[FL_ROW];
 #pragma unroll
       for (int j = 0; j < FL_ROW; ++j) {
@@ -795,12 +809,13 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
           after = true;
           continue;
         }
-        uint32_t idx = npre + npost;
-        o.pdest[hb[j]] = idx < FL_LIST ? FL_LIST * P + idx : FL_DEST_OVER;
-        if (after) ++npost;
-        else ++npre;
+        o.pdest[hb[j]] = after ? FL_LIST - 1 - npost++ : npre++;
       }
+      o.pcnt[P] = npre | (npost << 8) | (hk == FL_NONE ? FL_TAIL : 0u) | (head ? FL_HEAD : 0u);
     } else {
+      uint32_t light = 0;
+      for (uint32_t s = deg; s-- > 0;) light += is_child(m, deg, s, b, col, next, v) && col[b + s] != hk ? 1u : 0u;
+      const bool over = light > FL_LIST;
       for (uint32_t s = deg; s-- > 0;) {
         if (!is_child(m, deg, s, b, col, next, v)) continue;
         uint32_t ch = col[b + s];
@@ -808,15 +823,14 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
           after = true;
           continue;
         }
-        uint32_t idx = npre + npost;
-        o.pdest[head_base[ch]] = idx < FL_LIST ? FL_LIST * P + idx : FL_DEST_OVER;
+        const uint32_t slot = over ? FL_DEST_OVER : (after ? FL_LIST - 1 - npost : npre);
+        o.pdest[head_base[ch]] = slot;
         if (after) ++npost;
         else ++npre;
       }
+      o.pcnt[P] = (over ? FL_LIST_OVERFLOW : (npre | (npost << 8))) | (hk == FL_NONE ? FL_TAIL : 0u) |
+                  (head ? FL_HEAD : 0u);
     }
-    bool over = npre + npost > FL_LIST || npost > FL_POSTS;
-    o.pcnt[P] = (over ? FL_LIST_OVERFLOW : (npre | (npost << 8))) | (hk == FL_NONE ? FL_TAIL : 0u) |
-                (head ? FL_HEAD : 0u);
     o.parea[P] = av;
   }
   if (head) o.ppos[P] = (p == v) ? FL_NONE : head_base[pair_ptr(cpp)] + pair_cnt(cpp);
@@ -825,13 +839,15 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
 // --------------------------------------------------------------- sweeps ---
 //
 // Both sweeps run every round (light depth) in one launch.  A round's work
-// is cut into units of one wavefront each: a long chain, or a tile of 64
-// consecutive chain positions of its short chains.  Wavefronts take the units
+// is cut into units of one wavefront each: a tile of a long chain (response
+// time: the whole chain, at its head's tile), or a tile of 64 consecutive chain
+// positions of its short chains.  Wavefronts take the units
 // in round order (drainage area deepest round first, response time shallowest
 // first) and a unit waits for just the values it reads, not for the round
 // before it: a chain's head hands its drainage area to its receiver's list
-// slot, a position its response time (and, with max slopes, its elevation) to
-// the heads below it, and the word itself says whether it is there yet.
+// slot, a tile of a long chain its last one to the tile after it, a position its
+// response time (and, with max slopes, its elevation) to the heads below it,
+// and the word itself says whether it is there yet.
 //
 // What bounds it: the longest path of the forest, one dependent chain of
 // FP64 adds, plus a hand-over per light edge on it.  One launch per round made
@@ -868,7 +884,7 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
 struct fl_flow {
   const uint32_t* maxld;  // the deepest round
   const uint32_t* ucum;   // units before each round
-  const uint32_t* boff;   // chains before each bucket (short, long of each round)
+  const uint32_t* boff;   // counts before each bucket (short: chains, long: tiles of each round)
   const uint32_t* bnoff;  // positions before each bucket
   uint32_t* ticket_da;
   uint32_t* ticket_tau;
@@ -926,6 +942,24 @@ __device__ __forceinline__ double await(const double* p, bool need, double other
   return need ? bits_double(u) : otherwise;
 }
 
+// A hand-over word in LDS, between wavefronts of a workgroup (read by every
+// lane, stored by one).
+__device__ __forceinline__ void publish_lds(double* p, double v) {
+  unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  if (u == FL_SENT) u |= 1ull << 51;
+  *reinterpret_cast<volatile unsigned long long*>(p) = u;
+}
+__device__ __forceinline__ double await_lds(const double* p, int* stall) {
+  const volatile unsigned long long* w = reinterpret_cast<const volatile unsigned long long*>(p);
+  unsigned long long u = *w;
+  uint32_t spins = 0;
+  while (__any(u == FL_SENT)) {
+    if (!wait_more(spins, stall)) break;
+    u = *w;
+  }
+  return bits_double(u);
+}
+
 // Synchronisation of one wavefront's lanes around its own LDS tile: a
 // wavefront-scope fence (orders the LDS accesses; the wavefront's LDS
 // operations execute in order) and a wave barrier.
@@ -969,6 +1003,33 @@ __device__ __forceinline__ double of_lane(double v, uint32_t lane) {
   return __hiloint2double(hi, lo);
 }
 
+// Sums over lanes 0..lane.
+#ifndef FL_WAVE_SHIFT
+__device__ __forceinline__ double prefix_lanes(double v) {
+  for (int off = 1; off < 64; off <<= 1) v = v + shift_lanes(0.0, v, -off);
+  return v;
+}
+#else
+template <int ctrl, int rows>
+__device__ __forceinline__ double plus_dpp(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, rows, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, rows, 0xf, false);
+  return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double prefix_lanes(double v) {
+  v = plus_dpp<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8 within rows of 16 lanes
+  v = plus_dpp<0x112, 0xf>(v);
+  v = plus_dpp<0x114, 0xf>(v);
+  v = plus_dpp<0x118, 0xf>(v);
+  v = plus_dpp<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = plus_dpp<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+#endif
+__device__ __forceinline__ bool same_bits(double a, double b) {
+  return __double_as_longlong(a) == __double_as_longlong(b);
+}
+
 // A value that every lane of the wavefront holds, for scalar registers.
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 0); }
 
@@ -978,6 +1039,72 @@ __device__ __forceinline__ uint32_t run_steps(unsigned long long m) {
   uint32_t steps = 1;
   for (; m; m &= m << 1) ++steps;
   return steps;
+}
+
+// A long chain's tile: every lane's running value from the lane before it,
+// out = step(in), lane 0 from `carry` -- bit for bit what one lane after the
+// other gives, without waiting for 64 of them.
+//
+// A sum of positive terms stays in one binade (a power of two c to 2 c) for
+// most of a long chain.  There the running values are multiples of one unit u,
+// and a term adds the same multiple of u to all of them unless it lies halfway
+// between two: then it rounds to the even one, and what a lane adds depends on
+// whether its value is an even or an odd multiple (its lowest bit) -- but after
+// it the value is even either way.  So each lane's steps from c (even) and from
+// c + u (odd) tell what it adds to either; its value's lowest bit follows from
+// the last lane before it with a halfway term and the odd sums since, which
+// three ballots hold; and the prefix sum of what the lanes add, exact, is every
+// lane's value at once.  All of that is a guess, and it is checked: each lane
+// takes its real steps from its guess, and the guess of the lane after it has
+// to be the result.  Up to the first lane where it is not, everything is the
+// serial fold's value, and from there on it is guessed again (a new binade).
+//
+// 64 serial steps take 1.3 to 2.5 us, a guess and its check 0.3 us.  A tile
+// that begins at a chain's tail, where the binade changes with every few
+// positions, one of fewer than FL_GUESS_LANES lanes and one still wrong after
+// FL_GUESSES guesses take the serial steps.  `last`: the last lane whose value
+// counts.
+#define FL_GUESSES 4
+#define FL_GUESS_LANES 24
+template <class Step>
+__device__ __forceinline__ void tile_fold(double carry, uint32_t lane, uint32_t last, Step step) {
+  auto bits = [](double v) { return (unsigned long long)__double_as_longlong(v); };
+  auto grows = [](double v) { return v > 0.0 && v < __builtin_inf(); };
+  const unsigned long long below = (1ull << lane) - 1ull;
+  uint32_t at = 0;  // the lanes before it are final, and its `in`
+  double in = carry, real = carry, out;
+  bool guessed = last >= FL_GUESS_LANES && grows(carry);
+#pragma unroll 1
+  for (uint32_t k = 0; guessed && k < FL_GUESSES; ++k) {
+    const double c0 = bits_double(bits(real) & 0x7ff0000000000000ull), c1 = bits_double(bits(c0) + 1ull);
+    const double w0 = step(c0), w1 = step(c1);
+    const bool half = bits(w1) != bits(w0) + 1ull, odd = (bits(w0) & 1ull) != 0, here = lane >= at;
+    const unsigned long long halves = __ballot(here && half), odds = __ballot(here && odd);
+    const unsigned long long hb = halves & below;
+    const uint32_t t = 63u - (uint32_t)__builtin_clzll(hb | 1ull);
+    // the bit after lane t, then the odd sums of the lanes after it
+    const unsigned long long from = hb ? ~0ull << t : ~0ull;
+    const uint32_t bit = (hb ? 0u : (uint32_t)(bits(real) & 1ull)) +
+                         (uint32_t)__builtin_popcountll(odds & below & from);
+    const double add = !here ? 0.0 : ((bit & 1u) ? w1 - c1 : w0 - c0);
+    const double before = prefix_lanes(add) - add;
+    if (lane >= at) in = real + before;
+    if (lane == at) in = real;
+    out = step(in);
+    const double s = from_prev(carry, out);
+    const unsigned long long bad = __ballot(lane <= last && !same_bits(s, in));
+    if (bad == 0) return;
+    at = (uint32_t)__builtin_ctzll(bad);
+    real = of_lane(s, at);
+    guessed = grows(real);
+  }
+  if (lane == at) in = real;
+  out = step(in);
+#pragma unroll 2
+  for (uint32_t i = at; i < last; ++i) {
+    in = from_prev(carry, out);
+    out = step(in);
+  }
 }
 
 // The rounds of a decomposition, lane i holding round `first` + i.
@@ -1000,7 +1127,7 @@ __device__ __forceinline__ fl_rounds load_rounds(const fl_flow& f, uint32_t firs
   return r;
 }
 
-// A unit of round l: long chain `chain` (FL_NONE: none), or the short-chain
+// A unit of round l: long tile `chain` (FL_NONE: none), or the short-chain
 // positions [n0, n1) from tile start T on.
 struct fl_unit {
   uint32_t l, chain, T, n1;
@@ -1065,47 +1192,42 @@ __device__ __forceinline__ fl_short_tile short_tile(const uint32_t* __restrict__
 // A_k = ((a_k + A_{c_m}) + A_{c_{m-1}}) + ... + A_{c_1} over the children in
 // row order).  The heavy child's value comes from the position after it: the
 // fold is split into `pre` (the part before it) and the light children after
-// it, posts p0..p3 in fold order.
+// it, posts p0, p1, ... in fold order.
 //
 // Absent posts are -0.0, and the chain fold starts from r = -0.0 at the
 // tail: x + (-0.0) == x exactly for every x (signed zeros included), so
 //     A = ((pre + r) + p0) + p1 ...
 // is the reference's value at every position without a branch.
 //
-// The partial folds of a listed position from the values of its listed light
-// children (v_i = the i-th listed child's A, -0.0 past the list).
-struct fl_da_part {
-  double pre, p0, p1, p2, p3;
-  uint32_t np;
-};
+// The partial folds of a listed position from the values of its light
+// children: those before the heavy child in fold order from its first slot on,
+// those after it from its last slot backwards, -0.0 in the others.
 struct fl_da_words {
   unsigned long long u[FL_LIST];
 };
-__device__ __forceinline__ fl_da_part da_combine(uint32_t cn, double area_k, const fl_da_words& w, bool mine) {
-  if (!mine) return fl_da_part{FL_NEG0, FL_NEG0, FL_NEG0, FL_NEG0, FL_NEG0, 0u};
-  fl_da_part q;
-  const uint32_t npre = cn & 0xffu;
-  double v[FL_LIST];
+__device__ __forceinline__ uint32_t da_posts(uint32_t cn, bool mine) { return mine ? (cn >> 8) & 0xffu : 0u; }
+// The part before the heavy child; the words it takes become -0.0 (x + (-0.0)
+// == x), so that the last ones are the posts p0, p1, ...
+__device__ __forceinline__ double da_pre(uint32_t cn, double area_k, fl_da_words& w, bool mine) {
+  const uint32_t npre = mine ? cn & 0xffu : 0u;
+  double pre = mine ? area_k : FL_NEG0;
 #pragma unroll
-  for (uint32_t i = 0; i < FL_LIST; ++i) v[i] = bits_double(w.u[i]);
-  // pre: x + (-0.0) == x, so the terms past npre are added as -0.0
-  q.pre = area_k;
-#pragma unroll
-  for (uint32_t i = 0; i < FL_LIST; ++i) q.pre = q.pre + (i < npre ? v[i] : FL_NEG0);
-  // posts: list entries npre, npre + 1, ... (entries past the list are -0.0)
-  double p[FL_POSTS];
-#pragma unroll
-  for (uint32_t j = 0; j < FL_POSTS; ++j) {
-    p[j] = FL_NEG0;
-#pragma unroll
-    for (uint32_t i = 0; i + j < FL_LIST; ++i) p[j] = npre == i ? v[i + j] : p[j];
+  for (uint32_t i = 0; i < FL_LIST; ++i) {
+    if (!__any(i < npre)) break;
+    const bool take = i < npre;
+    pre = pre + (take ? bits_double(w.u[i]) : FL_NEG0);
+    if (take) w.u[i] = 1ull << 63;
   }
-  q.p0 = p[0];
-  q.p1 = p[1];
-  q.p2 = p[2];
-  q.p3 = p[3];
-  q.np = (cn >> 8) & 0xffu;
-  return q;
+  return pre;
+}
+// As many posts are added as the tile's largest position has (`posts`: 1, 2, 4
+// or all of the list); the others are -0.0.
+template <int posts>
+__device__ __forceinline__ double da_step(double pre, const fl_da_words& w, double r) {
+  r = pre + r;
+#pragma unroll
+  for (int j = 0; j < posts; ++j) r = r + bits_double(w.u[FL_LIST - 1 - j]);
+  return r;
 }
 
 // What the drainage-area fold reads at chain position P besides its counts and
@@ -1120,13 +1242,19 @@ struct fl_da_pos {
 struct fl_da_args {
   const uint32_t* perm;
   const uint32_t* pcnt;
-  double* cval;   // [FL_LIST n] light children's A by (position, list slot): hand-over words
-  double* cover;  // [n] at a chain's base: its head's A for a receiver with more light children than listed
+  double* cval;   // [FL_LIST n] light children's A by (position, slot): hand-over words
+  // [n] at a chain's base: its head's A for a receiver with more light
+  // children than listed; at the last position of a long chain's tile: the A
+  // that enters it
+  double* cover;
   const double* parea;
   const double* pK;
   const double* pdn;
-  const uint32_t* pdest;  // at a chain's base position: its head's slot in cval, FL_DEST_OVER or FL_NONE
-  const uint2* cmeta;     // long chains: (base, length)
+  // at a chain's base position: its head's slot with its receiver, FL_DEST_OVER
+  // or FL_NONE, and the receiver's position
+  const uint32_t* pdest;
+  const uint32_t* ppos;
+  const uint2* cmeta;     // long chains' tiles: (base, length or end)
   double* xp;
   double* taup;  // set to FL_SENT
   double* hnp;   // with max slopes, too (else null)
@@ -1146,16 +1274,15 @@ __device__ __forceinline__ fl_da_pos da_load(const fl_da_args& g, uint32_t P) {
   return fl_da_pos{g.perm[P], g.parea[P], g.pK[P], g.pdn[P]};
 }
 
-// The words of position P's listed children (-0.0 past the list).
-__device__ __forceinline__ uint32_t da_listed(uint32_t cn, bool mine) {
-  return mine ? (cn & 0xffu) + ((cn >> 8) & 0xffu) : 0u;
+// The words of position P's listed children (-0.0 in the other slots).
+__device__ __forceinline__ bool da_slot(uint32_t cn, uint32_t i) {
+  return i < (cn & 0xffu) || i + ((cn >> 8) & 0xffu) >= FL_LIST;
 }
 __device__ __forceinline__ fl_da_words da_words(const fl_da_args& g, uint32_t P, uint32_t cn, bool mine) {
-  const uint32_t nl = da_listed(cn, mine);
   const double* w = g.cval + (uint64_t)FL_LIST * P;
   fl_da_words q;
 #pragma unroll
-  for (uint32_t i = 0; i < FL_LIST; ++i) q.u[i] = i < nl ? peek(w + i) : 1ull << 63;
+  for (uint32_t i = 0; i < FL_LIST; ++i) q.u[i] = mine && da_slot(cn, i) ? peek(w + i) : 1ull << 63;
   return q;
 }
 __device__ __forceinline__ bool da_missing(const fl_da_words& q) {
@@ -1172,35 +1299,28 @@ __device__ __forceinline__ void da_again(const fl_da_args& g, uint32_t P, fl_da_
 }
 // Words that were read are given back.
 __device__ __forceinline__ void da_give_back(const fl_da_args& g, uint32_t P, uint32_t cn, bool mine) {
-  const uint32_t nl = da_listed(cn, mine);
   unsigned long long* w = reinterpret_cast<unsigned long long*>(g.cval) + (uint64_t)FL_LIST * P;
 #pragma unroll
   for (uint32_t i = 0; i < FL_LIST; ++i)
-    if (i < nl) w[i] = FL_SENT;
+    if (mine && da_slot(cn, i)) w[i] = FL_SENT;
 }
 
-// A position with more light children than listed (rare) walks its row: the
-// first FL_LIST of them in fold order have list slots, the others their
-// chain's word in cover.
-__device__ __forceinline__ double* da_over_word(const fl_da_args& g, uint32_t P, uint32_t idx, uint32_t c) {
-  return idx < FL_LIST ? g.cval + (uint64_t)FL_LIST * P + idx : g.cover + g.head_base[c];
-}
-__device__ __forceinline__ bool da_over_ready(const fl_da_args& g, uint32_t k, uint32_t P) {
+// A position with more light children than listed (rare) walks its row; their
+// chains' words are in cover.
+__device__ __forceinline__ bool da_over_ready(const fl_da_args& g, uint32_t k) {
   const uint32_t b = g.rp[k], deg = g.rp[k + 1] - b, hk = g.hc[k];
   const unsigned long long m = g.cmask[k];
-  uint32_t idx = 0;
   for (uint32_t s = deg; s-- > 0;) {
     if (!is_child(m, deg, s, b, g.col, g.next, k)) continue;
     const uint32_t c = g.col[b + s];
-    if (c != hk && peek(da_over_word(g, P, idx++, c)) == FL_SENT) return false;
+    if (c != hk && peek(g.cover + g.head_base[c]) == FL_SENT) return false;
   }
   return true;
 }
-__device__ __forceinline__ double da_over_fold(const fl_da_args& g, uint32_t k, uint32_t P, double r) {
+__device__ __forceinline__ double da_over_fold(const fl_da_args& g, uint32_t k, double r) {
   const uint32_t b = g.rp[k], deg = g.rp[k + 1] - b, hk = g.hc[k];
   const unsigned long long m = g.cmask[k];
   double acc = g.area[k];
-  uint32_t idx = 0;
   for (uint32_t s = deg; s-- > 0;) {
     if (!is_child(m, deg, s, b, g.col, g.next, k)) continue;
     const uint32_t c = g.col[b + s];
@@ -1208,78 +1328,80 @@ __device__ __forceinline__ double da_over_fold(const fl_da_args& g, uint32_t k, 
       acc = acc + r;
       continue;
     }
-    double* w = da_over_word(g, P, idx++, c);
+    double* w = g.cover + g.head_base[c];
     acc = acc + bits_double(peek(w));
     *reinterpret_cast<unsigned long long*>(w) = FL_SENT;
   }
   return acc;
 }
 
+// The drainage areas of a short-chain tile, one position a lane, each from the
+// position after it:
+//   r_i = ((pre_i + r_{i+1}) + p0_i) + p1_i ...
+// Every lane takes every step: once lane i + 1 holds its final value, lane i
+// gets its own in the next step and keeps it, so `steps` steps settle chains
+// of that many positions without a lane ever being singled out (two DPP moves
+// and the adds a step, 14 ns).  At a chain's tail the fold starts from -0.0.
 template <int posts>
-__device__ __forceinline__ double da_step(const fl_da_part& q, double r) {
-  r = (q.pre + r) + q.p0;
-  if (posts > 1) r = r + q.p1;
-  if (posts > 2) r = (r + q.p2) + q.p3;
+__device__ __forceinline__ double da_short_steps(double pre, const fl_da_words& w, bool tail, uint32_t steps) {
+  double s = FL_NEG0, r = FL_NEG0;
+#pragma unroll 2
+  for (uint32_t i = 0; i < steps; ++i) {
+    s = from_next(s, r);
+    r = da_step<posts>(pre, w, tail ? FL_NEG0 : s);
+  }
   return r;
 }
-
-// The drainage areas of a tile of B consecutive positions a lane (r[0] the
-// one nearest the head), each from the position after it:
-//   r_i = ((pre_i + r_{i+1}) + p0_i) + p1_i ...
-// Every lane takes every step: once lane i + 1 holds its final values, lane i
-// gets its own in the next step and keeps them, so `steps` steps settle chains
-// over that many lanes without a lane ever being singled out.  Two DPP moves
-// and B times the adds a step: 14 ns a position with one a lane and two adds
-// (37 ns when one lane read the operands of eight positions at a time from
-// LDS).  As many posts are added as the tile's largest position has; the
-// others add -0.0.  Lanes past the tile pass `carry` on (pre and posts -0.0);
-// at a chain's tail (`tail`) the fold starts from -0.0.
-template <int B, int posts, bool tails>
-__device__ __forceinline__ void da_tile_steps(const fl_da_part (&q)[B], bool tail, double carry, uint32_t steps,
-                                              double (&r)[B]) {
-  double s = carry;
-#pragma unroll
-  for (int b = 0; b < B; ++b) r[b] = carry;
-#pragma unroll 4
-  for (uint32_t i = 0; i < steps; ++i) {
-    s = from_next(s, r[0]);
-    double v = tails && tail ? FL_NEG0 : s;
-#pragma unroll
-    for (int b = B - 1; b >= 0; --b) r[b] = v = da_step<posts>(q[b], v);
-  }
+__device__ __forceinline__ double da_short_fold(uint32_t np, double pre, const fl_da_words& w, bool tail,
+                                                uint32_t steps) {
+  if (!__any(np >= 2)) return da_short_steps<1>(pre, w, tail, steps);
+  if (!__any(np >= 3)) return da_short_steps<2>(pre, w, tail, steps);
+  if (!__any(np >= 5)) return da_short_steps<4>(pre, w, tail, steps);
+  return da_short_steps<FL_LIST>(pre, w, tail, steps);
 }
-template <int B, bool tails>
-__device__ __forceinline__ void da_tile_fold(const fl_da_part (&q)[B], bool tail, double carry, uint32_t steps,
-                                             double (&r)[B]) {
-  uint32_t np = q[0].np;
-#pragma unroll
-  for (int b = 1; b < B; ++b) np = max(np, q[b].np);
-  if (!__any(np >= 2)) da_tile_steps<B, 1, tails>(q, tail, carry, steps, r);
-  else if (!__any(np >= 3)) da_tile_steps<B, 2, tails>(q, tail, carry, steps, r);
-  else da_tile_steps<B, 4, tails>(q, tail, carry, steps, r);
+
+// The drainage areas of a long chain's tile, two positions a lane, the chain's
+// tail side first (r[0], then r[1], then the next lane's).  Positions past the
+// tile pass the value on (pre and posts -0.0).
+template <int posts>
+__device__ __forceinline__ void da_long_steps(const double (&pre)[2], const fl_da_words (&w)[2], double carry,
+                                              uint32_t lane, uint32_t last, double (&r)[2]) {
+  tile_fold(carry, lane, last, [&](double v) {
+    r[0] = da_step<posts>(pre[0], w[0], v);
+    return r[1] = da_step<posts>(pre[1], w[1], r[0]);
+  });
+}
+__device__ __forceinline__ void da_long_fold(uint32_t np, const double (&pre)[2], const fl_da_words (&w)[2],
+                                             double carry, uint32_t lane, uint32_t last, double (&r)[2]) {
+  if (!__any(np >= 2)) da_long_steps<1>(pre, w, carry, lane, last, r);
+  else if (!__any(np >= 3)) da_long_steps<2>(pre, w, carry, lane, last, r);
+  else if (!__any(np >= 5)) da_long_steps<4>(pre, w, carry, lane, last, r);
+  else da_long_steps<FL_LIST>(pre, w, carry, lane, last, r);
 }
 
 // The same for a tile with positions of more light children than listed: one
-// lane after the other.
-template <int B>
+// lane after the other, from lane 0 on (`up`) or from lane 63 down.
+template <int B, bool up>
 __device__ __forceinline__ void da_tile_walk(const fl_da_args& g, const fl_da_pos (&t)[B], const uint32_t (&cn)[B],
-                                             const uint32_t (&P)[B], const bool (&mine)[B], const fl_da_part (&q)[B],
-                                             bool tail, double carry, uint32_t lane, double (&r)[B]) {
+                                             const bool (&mine)[B], const double (&pre)[B],
+                                             const fl_da_words (&w)[B], bool tail, double carry, uint32_t lane, double (&r)[B]) {
   uint32_t spins = 0;
   for (;;) {
     bool wait = false;
 #pragma unroll
     for (int b = 0; b < B; ++b)
-      wait = wait || (mine[b] && (cn[b] & FL_LIST_OVERFLOW) && !da_over_ready(g, t[b].k, P[b]));
+      wait = wait || (mine[b] && (cn[b] & FL_LIST_OVERFLOW) && !da_over_ready(g, t[b].k));
     if (!__any(wait) || !wait_more(spins, g.stall)) break;
   }
   double v = carry;
-  for (uint32_t e = 64; e-- > 0;) {
+  for (uint32_t i = 0; i < 64; ++i) {
+    const uint32_t e = up ? i : 63 - i;
     if (lane == e) {
       double x = tail ? FL_NEG0 : v;
 #pragma unroll
-      for (int b = B - 1; b >= 0; --b)
-        r[b] = x = mine[b] && (cn[b] & FL_LIST_OVERFLOW) ? da_over_fold(g, t[b].k, P[b], x) : da_step<4>(q[b], x);
+      for (int b = 0; b < B; ++b)
+        r[b] = x = mine[b] && (cn[b] & FL_LIST_OVERFLOW) ? da_over_fold(g, t[b].k, x)
+                   : da_step<FL_LIST>(pre[b], w[b], x);
       v = x;
     }
     v = of_lane(v, e);
@@ -1296,108 +1418,101 @@ __device__ __forceinline__ void da_store(const fl_da_args& g, uint32_t P, const 
   reinterpret_cast<unsigned long long*>(g.taup)[P] = FL_SENT;
   if (g.hnp) reinterpret_cast<unsigned long long*>(g.hnp)[P] = FL_SENT;
 }
-__device__ __forceinline__ void da_hand_over(const fl_da_args& g, uint32_t base, uint32_t pd, double a) {
+// (pd, pp: the words at its base)
+__device__ __forceinline__ void da_hand_over(const fl_da_args& g, uint32_t base, uint32_t pd, uint32_t pp, double a) {
   if (pd == FL_NONE) return;
-  publish(pd == FL_DEST_OVER ? g.cover + base : g.cval + pd, a);
+  publish(pd == FL_DEST_OVER ? g.cover + base : g.cval + (uint64_t)FL_LIST * pp + pd, a);
 }
 
-// One unit of the drainage-area sweep, tail to head along its chains.  A long
-// chain goes through tiles of 128 positions, two a lane (a step of two
-// positions costs 1.5 of one); a tile's words and inputs are loaded before the
-// fold of the tile before it, its counts one tile earlier.
-__device__ __forceinline__ void da_unit(const fl_da_args& g, const fl_unit& un, uint32_t stride, uint32_t lane) {
+// One unit of the drainage-area sweep, tail to head along its chains.
+//
+// A long chain's tile is 128 positions, two a lane, lane 0 nearest the tail.
+// The tiles of a chain are units of their own: all their loads, list waits,
+// divisions and stores overlap, and one after the other is only the value that
+// a tile hands to the next, through LDS where the next wavefront of the workgroup
+// has it (s_carry), else through cover.  A chain of 8192 positions takes 57 us
+// (224 with the tiles one after the other on one wavefront, 64 serial steps each).
+__device__ __forceinline__ void da_unit(const fl_da_args& g, const fl_unit& un, uint32_t stride, uint32_t lane,
+                                        double* s_carry, uint32_t wave) {
   if (un.chain == FL_NONE) {
     uint32_t cn[1];
     const fl_short_tile t = short_tile(g.pcnt, un.T, un.n1, stride, lane, cn[0]);
     const fl_da_pos at[1] = {da_load(g, t.P)};
     const bool head = t.own && (cn[0] & FL_HEAD) != 0, tail = (cn[0] & FL_TAIL) != 0;
-    const uint32_t pd = head ? g.pdest[t.P] : FL_NONE;
+    const uint32_t pd = head ? g.pdest[t.P] : FL_NONE, pp = head ? g.ppos[t.P] : FL_NONE;
     fl_da_words w = da_words(g, t.P, cn[0], t.own);
     uint32_t spins = 0;
     while (__any(da_missing(w))) {
       if (!wait_more(spins, g.stall)) break;
       da_again(g, t.P, w);
     }
-    const fl_da_part q[1] = {da_combine(cn[0], at[0].area, w, t.own)};
+    const double pre[1] = {da_pre(cn[0], at[0].area, w, t.own)};
     double r[1];
     if (__any(t.own && (cn[0] & FL_LIST_OVERFLOW))) {
-      const uint32_t P[1] = {t.P};
       const bool mine[1] = {t.own};
-      da_tile_walk<1>(g, at, cn, P, mine, q, tail, FL_NEG0, lane, r);
+      const fl_da_words ws[1] = {w};
+      da_tile_walk<1, false>(g, at, cn, mine, pre, ws, tail, FL_NEG0, lane, r);
     } else {
-      da_tile_fold<1, true>(q, tail, FL_NEG0, run_steps(__ballot(t.own && !tail)), r);
+      r[0] = da_short_fold(da_posts(cn[0], t.own), pre[0], w, tail, run_steps(__ballot(t.own && !tail)));
     }
-    if (head) da_hand_over(g, t.P, pd, r[0]);
+    if (head) da_hand_over(g, t.P, pd, pp, r[0]);
     da_give_back(g, t.P, cn[0], t.own);
     if (t.own) da_store(g, t.P, at[0], r[0]);
     return;
   }
   const uint2 m = g.cmeta[un.chain];
-  const uint32_t base = uniform(m.x), len = uniform(m.y);
-  const uint32_t pd = g.pdest[base];
-  // the lane's position b of the tile ending at `e` (past the tile: its first
-  // position); the tile after that one, or the tail's again past the head
-  auto pos_of = [&](uint32_t e, uint32_t b) {
-    const uint32_t cs = e > 128 ? e - 128 : 0, i = 2 * lane + b;
-    return base + (i < e - cs ? cs + i : cs);
-  };
-  auto in_tile = [&](uint32_t e, uint32_t b) { return 2 * lane + b < (e > 128 ? 128 : e); };
-  auto after = [&](uint32_t e) { return e > 128 ? e - 128 : len; };
-  double carry = FL_NEG0;
-  uint32_t cn[2], cn1[2];
+  const uint32_t base = uniform(m.x) & ~FL_CHAIN_TAIL, my = uniform(m.y);
+  const bool first = (uniform(m.x) & FL_CHAIN_TAIL) != 0, head = !(my & FL_CHAIN_PART);
+  const uint32_t end = head ? min(my, (uint32_t)FL_TILE) : my & ~FL_CHAIN_PART;
+  const uint32_t start = (end - 1) & ~(FL_TILE - 1u), cnt = end - start, last = (cnt - 1) / 2;
+  const uint32_t pd = head ? g.pdest[base] : FL_NONE, pp = head ? g.ppos[base] : FL_NONE;
+  uint32_t P[2], cn[2];
+  bool mine[2];
   fl_da_pos at[2];
   fl_da_words w[2];
 #pragma unroll
-  for (int b = 0; b < 2; ++b) cn[b] = g.pcnt[pos_of(len, b)];
-#pragma unroll
   for (int b = 0; b < 2; ++b) {
-    at[b] = da_load(g, pos_of(len, b));
-    cn1[b] = g.pcnt[pos_of(after(len), b)];
+    const uint32_t i = 2 * lane + b;
+    mine[b] = i < cnt;
+    P[b] = base + (mine[b] ? end - 1 - i : start);
+    cn[b] = g.pcnt[P[b]];
+    at[b] = da_load(g, P[b]);
   }
 #pragma unroll
-  for (int b = 0; b < 2; ++b) w[b] = da_words(g, pos_of(len, b), cn[b], in_tile(len, b));
-  for (uint32_t end = len;;) {
-    const uint32_t nxt = after(end), cnt = end > 128 ? 128 : end;
-    const uint32_t P[2] = {pos_of(end, 0), pos_of(end, 1)};
-    const bool mine[2] = {in_tile(end, 0), in_tile(end, 1)};
-    uint32_t spins = 0;
-    while (__any(da_missing(w[0]) || da_missing(w[1]))) {
-      if (!wait_more(spins, g.stall)) break;
-      da_again(g, P[0], w[0]);
-      da_again(g, P[1], w[1]);
+  for (int b = 0; b < 2; ++b) w[b] = da_words(g, P[b], cn[b], mine[b]);
+  uint32_t spins = 0;
+  while (__any(da_missing(w[0]) || da_missing(w[1]))) {
+    if (!wait_more(spins, g.stall)) break;
+    da_again(g, P[0], w[0]);
+    da_again(g, P[1], w[1]);
+  }
+  const double pre[2] = {da_pre(cn[0], at[0].area, w[0], mine[0]), da_pre(cn[1], at[1].area, w[1], mine[1])};
+  // the value before the tile
+  double carry = FL_NEG0;
+  if (!first) {
+    if (s_carry && wave > 0) {
+      carry = await_lds(s_carry + wave - 1, g.stall);
+    } else {
+      double* word = g.cover + base + end - 1;
+      carry = await(word, true, 0.0, g.stall);
+      if (lane == 0) *reinterpret_cast<unsigned long long*>(word) = FL_SENT;
     }
-    fl_da_part q[2];
+  }
+  double r[2];
+  if (__any((mine[0] && (cn[0] & FL_LIST_OVERFLOW)) || (mine[1] && (cn[1] & FL_LIST_OVERFLOW))))
+    da_tile_walk<2, true>(g, at, cn, mine, pre, w, false, carry, lane, r);
+  else
+    da_long_fold(max(da_posts(cn[0], mine[0]), da_posts(cn[1], mine[1])), pre, w, carry, lane, last, r);
+  const double out = of_lane(r[1], last);  // (a position past the tile passed it on)
+  if (lane == 0) {
+    if (head) da_hand_over(g, base, pd, pp, out);
+    else if (s_carry && wave + 1 < FL_FOLD_WAVES) publish_lds(s_carry + wave, out);
+    else publish(g.cover + base + start - 1, out);
+  }
 #pragma unroll
-    for (int b = 0; b < 2; ++b) q[b] = da_combine(cn[b], at[b].area, w[b], mine[b]);
-    // (past the head these load what nothing reads: no word is listed)
-    fl_da_pos at1[2];
-    uint32_t cn2[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      w[b] = da_words(g, pos_of(nxt, b), cn1[b], end > 128 && in_tile(nxt, b));
-      at1[b] = da_load(g, pos_of(nxt, b));
-      cn2[b] = g.pcnt[pos_of(after(nxt), b)];
-    }
-    double r[2];
-    if (__any((mine[0] && (cn[0] & FL_LIST_OVERFLOW)) || (mine[1] && (cn[1] & FL_LIST_OVERFLOW))))
-      da_tile_walk<2>(g, at, cn, P, mine, q, false, carry, lane, r);
-    else
-      da_tile_fold<2, false>(q, false, carry, (cnt + 1) / 2, r);
-    carry = of_lane(r[0], 0);
-    if (end <= 128 && lane == 0) da_hand_over(g, base, pd, r[0]);
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      da_give_back(g, P[b], cn[b], mine[b]);
-      if (mine[b]) da_store(g, P[b], at[b], r[b]);
-    }
-    if (end <= 128) break;
-    end = nxt;
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      cn[b] = cn1[b];
-      cn1[b] = cn2[b];
-      at[b] = at1[b];
-    }
+  for (int b = 0; b < 2; ++b) {
+    da_give_back(g, P[b], cn[b], mine[b]);
+    if (mine[b]) da_store(g, P[b], at[b], r[b]);
   }
 }
 
@@ -1411,15 +1526,17 @@ k_da_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_da_arg
   const uint32_t total = f.ucum[rounds];
   fl_rounds R = load_rounds(f, 0, rounds, lane);
   __shared__ uint32_t s_ticket;
+  __shared__ double s_carry[FL_FOLD_WAVES];  // from each wavefront's tile to the next one's
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) s_ticket = atomicAdd(f.ticket_da, (uint32_t)FL_FOLD_WAVES);
+    if (threadIdx.x < FL_FOLD_WAVES) s_carry[threadIdx.x] = bits_double(FL_SENT);
     __syncthreads();
     const uint32_t t = s_ticket;
     if (t >= total) return;
     if (t + wave < total) {
       const fl_unit un = find_unit(f, R, rounds, total - 1 - (t + wave), true, lane);
-      da_unit(g, un, 65u - f.long_min, lane);
+      da_unit(g, un, 65u - f.long_min, lane, s_carry, wave);
     }
     if ((uint64_t)gridDim.x * FL_FOLD_WAVES >= total) return;  // one turn covers the units
   }
@@ -1427,7 +1544,9 @@ k_da_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_da_arg
 
 // Rounds lsplit..deepest, deepest first, in one workgroup with a barrier
 // between rounds: the small deep rounds of an iteration whose sizes the host
-// knows, and every round of one whose waits ended without their values.
+// knows, and every round of one whose waits ended without their values.  (A
+// chain's tiles still wait for each other: each wavefront takes its units in
+// order, so the first one not finished waits for nothing.)
 __global__ void __launch_bounds__(64 * FL_TAIL_WAVES)
 k_da_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, fl_flow f, fl_da_args g) {
   const uint32_t top = *f.maxld;
@@ -1438,7 +1557,7 @@ k_da_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, fl_flow f, fl_da_
     for (uint32_t i = wave; i < n; i += FL_TAIL_WAVES)
       da_unit(g, unit_of(l, i, f.boff[2ull * l + 1], f.boff[2ull * l + 2], f.bnoff[2ull * l], f.bnoff[2ull * l + 1],
                          65u - f.long_min),
-              65u - f.long_min, lane);
+              65u - f.long_min, lane, nullptr, wave);
     __syncthreads();
   }
 }
@@ -1447,7 +1566,7 @@ k_da_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, fl_flow f, fl_da_
 struct fl_tau_args {
   const uint32_t* pcnt;
   const uint32_t* ppos;  // at a chain's base: the position of its head's receiver, FL_NONE at a basin outlet
-  const uint2* cmeta;
+  const uint2* cmeta;     // long chains' tiles: (base, length) at the head's
   const double* xp;
   double* taup;
   // with max slopes: by position the basin outlet's position, uplift,
@@ -1461,8 +1580,8 @@ struct fl_tau_args {
   int* stall;
 };
 
-// Response times of a tile of B consecutive positions a lane, each from the
-// position before it (first: a chain's head, from its receiver's value `tp`).
+// Response times of a tile, each from the position before it (a chain's head
+// from its receiver's value `tp`).
 //
 // The reference's step rt = 0.0 + (rt_next + x) adds 0.0, which changes
 // nothing unless y = rt_next + x is -0.0 (0.0 + -0.0 = +0.0; a NaN y is
@@ -1470,19 +1589,29 @@ struct fl_tau_args {
 // are, and no running value is: a basin's outlet starts at 0.0 + (...),
 // never -0.0, and every other chain starts from its receiver's value.  So
 // the chains take the single add, bit for bit the same.
-template <int B, bool heads>
-__device__ __forceinline__ void tau_tile_fold(const double (&x)[B], bool first, double tp, uint32_t steps,
-                                              double (&r)[B]) {
-  double s = tp;
-#pragma unroll
-  for (int b = 0; b < B; ++b) r[b] = tp;
+//
+// A short-chain tile, one position a lane, by `steps` serial steps:
+__device__ __forceinline__ double tau_short_fold(double x, bool head, double tp, uint32_t steps) {
+  double s = tp, r = tp;
 #pragma unroll 4
   for (uint32_t i = 0; i < steps; ++i) {
-    s = from_prev(s, r[B - 1]);
-    double v = heads && first ? tp : s;
-#pragma unroll
-    for (int b = 0; b < B; ++b) r[b] = v = v + x[b];
+    s = from_prev(s, r);
+    r = (head ? tp : s) + x;
   }
+  return r;
+}
+// A long chain's tile, B positions a lane, from the value before it (positions
+// past the tile hold -0.0).
+template <int B>
+__device__ __forceinline__ void tau_long_fold(const double (&x)[B], double tp, uint32_t lane, uint32_t last,
+                                              double (&r)[B]) {
+  tile_fold(
+      tp, lane, last,
+      [&](double v) {
+#pragma unroll
+        for (int b = 0; b < B; ++b) r[b] = v = v + x[b];
+        return v;
+      });
 }
 
 // Elevations of a tile with max slopes (generator.rs:177-202): z the value
@@ -1495,8 +1624,9 @@ __device__ __forceinline__ void tau_tile_fold(const double (&x)[B], bool first, 
 //   z - hp > t * d * (1 + 2^-50)  implies  (z - hp) / d >= the double after t,
 //   z - hp < t * d * (1 - 2^-50)  implies  (z - hp) / d < t,
 // and rounding is monotonic, so either comparison decides it; only a
-// difference between the two bounds divides.  A tile in which no site is
-// limited needs one step.
+// difference between the two bounds divides.  A site that is not limited
+// ends what its receiver's elevation changes, so the lanes settle after as many
+// steps as the tile's longest run of limited sites takes.
 struct fl_clamp_pos {
   double z, t, d;
   bool fixed;
@@ -1521,9 +1651,11 @@ __device__ __forceinline__ void clamp_tile_fold(const fl_clamp_pos (&q)[B], bool
   }
   double s = hp;
   for (uint32_t i = 0; i < steps; ++i) {
+    const double was = s;
     s = from_prev(s, h[B - 1]);
+    // every lane's value is what its last step started from: settled
+    if (i > 0 && !__any(!same_bits(s, was))) break;
     double v = heads && first ? hp : s;
-    bool some = false;
 #pragma unroll
     for (int b = 0; b < B; ++b) {
       const double diff = q[b].z - v;
@@ -1532,11 +1664,7 @@ __device__ __forceinline__ void clamp_tile_fold(const fl_clamp_pos (&q)[B], bool
       if (__any(near)) c = near ? diff / q[b].d > q[b].t : c;
       c = c && !q[b].fixed;
       h[b] = v = c ? v + q[b].t * q[b].d : q[b].z;
-      some = some || c;
     }
-    // no site limited: every lane started from its receiver's unlimited value
-    // and the values before it, and kept its own
-    if (i == 0 && !__any(some)) break;
   }
 }
 
@@ -1565,9 +1693,7 @@ __device__ __forceinline__ void tau_unit(const fl_tau_args& g, const fl_unit& un
     }
     const double tp = await(g.taup + pp, head && !outlet, 0.0, g.stall);
     const uint32_t steps = run_steps(__ballot(t.own && !head));
-    const double xs[1] = {x};
-    double tau[1];
-    tau_tile_fold<1, true>(xs, head, tp, steps, tau);
+    const double tau[1] = {tau_short_fold(x, head, tp, steps)};
     if (t.own) publish(g.taup + P, tau[0]);
     if (clamp) {
       const bool deep = un.l > 0;
@@ -1602,7 +1728,8 @@ __device__ __forceinline__ void tau_unit(const fl_tau_args& g, const fl_unit& un
   constexpr int B = clamp ? 2 : 4;
   constexpr uint32_t tile = 64 * B;
   const uint2 m = g.cmeta[un.chain];
-  const uint32_t base = uniform(m.x), len = uniform(m.y);
+  const uint32_t base = uniform(m.x) & ~FL_CHAIN_TAIL, len = uniform(m.y);
+  if (len & FL_CHAIN_PART) return;  // its chain is taken at the head's tile
   const uint32_t pp = uniform(g.ppos[base]);
   const bool outlet = pp == FL_NONE;  // the chain of a basin outlet
   struct In {
@@ -1625,12 +1752,14 @@ __device__ __forceinline__ void tau_unit(const fl_tau_args& g, const fl_unit& un
     const uint32_t cnt = len - t0 < tile ? len - t0 : tile;
     const uint32_t P = base + t0 + B * lane;
     const uint32_t last = (cnt - 1) / B;  // the lane of the tile's last position
-    double tau[B];
-    tau_tile_fold<B, false>(q.x, false, tau_c, last + 1, tau);
+    double x[B], tau[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) x[b] = B * lane + b < cnt ? q.x[b] : FL_NEG0;
+    tau_long_fold<B>(x, tau_c, lane, last, tau);
 #pragma unroll
     for (int b = 0; b < B; ++b)
       if (B * lane + b < cnt) publish(g.taup + P + b, tau[b]);
-    tau_c = of_lane(tau[B - 1], last);  // (read past the chain's end only when nothing follows)
+    tau_c = of_lane(tau[B - 1], last);  // (positions past the tile pass it on)
     if (clamp) {
       const bool first = t0 == 0 && outlet;
       if (first) {
@@ -2079,7 +2208,7 @@ fl_flow flow(const fl_dev_work& w) {
                  w.counters + FL_CNT_TICKET_TAU, w.long_min};
 }
 fl_da_args da_args(const fl_dev_terrain& t, const fl_dev_work& w, bool clamp) {
-  return fl_da_args{w.perm, w.pcnt,  w.cval, w.cover, w.parea, w.pK, w.pdn, w.pdest, w.cmeta, w.xp, w.taup,
+  return fl_da_args{w.perm, w.pcnt,  w.cval, w.cover, w.parea, w.pK, w.pdn, w.pdest, w.ppos, w.cmeta, w.xp, w.taup,
                     clamp ? w.hnp : nullptr, t.row_ptr, t.col, w.next, (const unsigned long long*)w.cmask, w.hc,
                     w.head_base, t.area, w.A, w.flags + FL_FLAG_STALL};
 }
