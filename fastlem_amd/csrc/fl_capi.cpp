@@ -913,7 +913,6 @@ struct Flight {
 // lakes.  The sweeps' launch size follows its sweep units (any size is
 // correct).  Its control block and changed flags are copied to the host slot
 // f.slot and an event marks its end.
-constexpr uint32_t FL_SWEEP_WAVES = 8192;  // more wavefronts than run at once gain nothing
 int32_t enqueue_fast(fl_ctx* c, fl_terrain* T, Flight& f) {
   hipStream_t s = c->stream;
   fl_dev_work& w = T->w;
@@ -924,7 +923,6 @@ int32_t enqueue_fast(fl_ctx* c, fl_terrain* T, Flight& f) {
     const uint32_t u = rounds_size(T->last_boff, 0, T->last_rounds, T->w.long_min).units;
     W = std::min<uint32_t>(u + u / 4 + FL_FOLD_WAVES, T->t.n);
   }
-  W = std::min<uint32_t>(W, FL_SWEEP_WAVES);
   set_slots(T, f.in);
   f.rec_da = f.rec_tau = SIZE_MAX;
   bool graphed = !c->prof && c->graphs && launch_fast_graph(c, T, f.J, W, f.full, f.keep);

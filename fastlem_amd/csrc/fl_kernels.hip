@@ -861,9 +861,15 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
 // FL_SENT by the one unit that reads them, response times and elevations by
 // the drainage-area sweep before.
 //
-// Waits end.  A workgroup takes FL_FOLD_WAVES units at a time from one
-// counter, so every unit a wavefront waits for was taken by a wavefront that
-// runs: the lowest unit not finished waits for nothing.  Should a wait still
+// A workgroup takes FL_FOLD_WAVES units at a time: those of its own number when
+// the launch has a wavefront for every unit, else from one counter (17 ns a
+// workgroup one after the other on one word: 22 us for the 10 500 units of a
+// million sites).
+//
+// Waits end.  Units are in the order of the counter, and workgroups start in
+// the order of their numbers on each XCD, so every unit a wavefront waits for was
+// taken by a wavefront that runs or runs next: the lowest unit not finished waits
+// for nothing.  Should a wait still
 // last FL_SPIN_MAX polls, the wavefront raises FL_FLAG_STALL and goes on, every
 // other wait sees the flag and ends, and the host redoes the iteration in one
 // workgroup with barriers between the rounds (k_da_tail, k_tau_tail).
@@ -1525,11 +1531,12 @@ k_da_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_da_arg
   const uint32_t rounds = deepest < cap ? deepest + 1 : cap;
   const uint32_t total = f.ucum[rounds];
   fl_rounds R = load_rounds(f, 0, rounds, lane);
+  const bool own = (uint64_t)gridDim.x * FL_FOLD_WAVES >= total;
   __shared__ uint32_t s_ticket;
   __shared__ double s_carry[FL_FOLD_WAVES];  // from each wavefront's tile to the next one's
   for (;;) {
     __syncthreads();
-    if (threadIdx.x == 0) s_ticket = atomicAdd(f.ticket_da, (uint32_t)FL_FOLD_WAVES);
+    if (threadIdx.x == 0) s_ticket = own ? blockIdx.x * FL_FOLD_WAVES : atomicAdd(f.ticket_da, (uint32_t)FL_FOLD_WAVES);
     if (threadIdx.x < FL_FOLD_WAVES) s_carry[threadIdx.x] = bits_double(FL_SENT);
     __syncthreads();
     const uint32_t t = s_ticket;
@@ -1538,7 +1545,7 @@ k_da_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_da_arg
       const fl_unit un = find_unit(f, R, rounds, total - 1 - (t + wave), true, lane);
       da_unit(g, un, 65u - f.long_min, lane, s_carry, wave);
     }
-    if ((uint64_t)gridDim.x * FL_FOLD_WAVES >= total) return;  // one turn covers the units
+    if (own) return;
   }
 }
 
@@ -1817,10 +1824,11 @@ k_tau_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_tau_a
   const uint32_t rounds = deepest < cap ? deepest + 1 : cap;
   const uint32_t total = f.ucum[rounds];
   fl_rounds R = load_rounds(f, 0, rounds, lane);
+  const bool own = (uint64_t)gridDim.x * FL_FOLD_WAVES >= total;
   __shared__ uint32_t s_ticket;
   for (;;) {
     __syncthreads();
-    if (threadIdx.x == 0) s_ticket = atomicAdd(f.ticket_tau, (uint32_t)FL_FOLD_WAVES);
+    if (threadIdx.x == 0) s_ticket = own ? blockIdx.x * FL_FOLD_WAVES : atomicAdd(f.ticket_tau, (uint32_t)FL_FOLD_WAVES);
     __syncthreads();
     const uint32_t t = s_ticket;
     if (t >= total) return;
@@ -1828,7 +1836,7 @@ k_tau_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_tau_a
       const fl_unit un = find_unit(f, R, rounds, t + wave, false, lane);
       tau_unit<clamp>(g, un, 65u - f.long_min, lane);
     }
-    if ((uint64_t)gridDim.x * FL_FOLD_WAVES >= total) return;  // one turn covers the units
+    if (own) return;
   }
 }
 
