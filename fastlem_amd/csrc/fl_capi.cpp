@@ -105,6 +105,9 @@ struct fl_terrain {
   // words are reset, and the terrain's later iterations run every round
   // behind barriers
   bool stalled = false, reset_words = false;
+  // the device's control block, bucket entries and changed flags are zero (the
+  // last thing enqueued that used them was a pipelined iteration)
+  bool ctrl_clean = false;
   // captured pipelined iterations, one per elevation-buffer parity, for the
   // jump rounds they were captured with
   // elevation buffers: an iteration reads hb[i] and writes hb[(i+1) % 3], so
@@ -462,6 +465,7 @@ struct TuneScope {
 };
 
 int32_t read_ctrl(fl_ctx* c, fl_terrain* T) {
+  T->ctrl_clean = false;
   HIPCHK(hipMemcpyAsync(c->host_ctrl, T->w.ctrl, FL_CTRL_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   T->stat_syncs++;
@@ -667,8 +671,8 @@ int32_t decompose(fl_ctx* c, fl_terrain* T, bool full, bool joined) {
   // quiet + 1 rounds suffice (the quiet round completes convergence)
   T->jump_rounds = quiet + 1;
   w.guard = w.ctrl + FL_CTRL_JUMPS + (round - 1);  // a round at or after the quiet one: zero
-  fl_launch_chain_count(s, T->t, w);
-  fl_launch_chain_layout(s, T->t, w);
+  fl_launch_chain_count(s, T->t, w, true);
+  fl_launch_chain_layout(s, T->t, w, true, false);
   FLCHK(read_ctrl(c, T));
   uint32_t nb = 2 * (host_counter(c, FL_CNT_MAXLD) + 1);  // short and long bucket per light depth
   if (nb > n + 2) return set_err(FL_ERR_HIP, "light depth out of range");
@@ -815,7 +819,7 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
   if (split > 0) fl_launch_tau_fold(s, w, split, flow.units, flow.positions, clamp);
   if (split < rounds) fl_launch_tau_tail(s, w, split, tail.positions, clamp);
   if (T->d_tchanged) fl_launch_fill_u32(s, T->d_tchanged, T->nterr, 0);
-  fl_launch_tau_scatter(s, T->t, w, clamp, T->d_tid, T->d_active, T->d_tchanged);
+  fl_launch_tau_scatter(s, T->t, w, clamp, true, T->d_tid, T->d_active, T->d_tchanged);
   if (T->d_tchanged)
     HIPCHK(hipMemcpyAsync(T->h_tchanged, T->d_tchanged, T->nterr * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   FLCHK(read_ctrl(c, T));
@@ -835,35 +839,31 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
 // The kernels of one pipelined iteration (J jump rounds, sweeps of W
 // wavefronts), enqueued on the context's stream or recorded by a capture.
 // rec_* receive the profiler records of the launches (when profiling).
-void enqueue_fast_body(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool full, bool keep, size_t* rec_da,
-                       size_t* rec_tau) {
+void enqueue_fast_body(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool full, bool keep, bool scan,
+                       size_t* rec_da, size_t* rec_tau) {
   hipStream_t s = c->stream;
   fl_dev_work& w = T->w;
-  uint32_t n = T->t.n;
   bool clamp = T->t.any_max_slope;
-  // the bucket entries that the previous iteration used
-  fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, n + 2));
   fl_launch_receivers(s, T->t, w, keep, !full);
   fl_launch_children(s, T->t, w, full, T->d_tid, T->d_active);
   for (uint32_t r = 0; r < J; r++) fl_launch_chain_jump(s, T->t, w, r);
-  w.guard = w.ctrl + FL_CTRL_JUMPS + (J - 1);
-  fl_launch_chain_count(s, T->t, w);
-  fl_launch_chain_layout(s, T->t, w);
+  w.guard = (uint32_t*)w.flags + FL_FLAG_JUMP;
+  fl_launch_chain_count(s, T->t, w, false);
+  fl_launch_chain_layout(s, T->t, w, false, scan);
   if (c->prof && rec_da) *rec_da = c->prof->pending.size();
   fl_launch_da_fold(s, T->t, w, FL_NONE_ROUND, W, 0, clamp);
   if (c->prof && rec_tau) *rec_tau = c->prof->pending.size();
   fl_launch_tau_fold(s, w, FL_NONE_ROUND, W, 0, clamp);
-  if (T->d_tchanged) fl_launch_fill_u32(s, T->d_tchanged, T->nterr, 0);
-  fl_launch_tau_scatter(s, T->t, w, clamp, T->d_tid, T->d_active, T->d_tchanged);
+  fl_launch_tau_scatter(s, T->t, w, clamp, false, T->d_tid, T->d_active, T->d_tchanged);
 }
 
 // The pipelined iteration for J and the current buffer parity as a
 // graph, captured on first use.  False when capture is not possible (the
 // caller launches directly).
-bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool full, bool keep) {
+bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool full, bool keep, bool scan) {
   if (T->graphs_failed) return false;
   int p = T->w.h == T->hb[0] ? 0 : (T->w.h == T->hb[1] ? 1 : 2);
-  const int mode = (full ? 1 : 0) | (keep ? 2 : 0);
+  const int mode = (full ? 1 : 0) | (keep ? 2 : 0) | (scan ? 4 : 0);
   // (a captured launch size serves until the units differ by more than half)
   if (!T->gexec[p] || T->gJ[p] != J || W > T->gW[p] + T->gW[p] / 2 || T->gW[p] > W + W / 2 || T->gF[p] != mode ||
       T->gB[p] != fl_site_block || T->gL[p] != T->w.long_min) {
@@ -876,7 +876,7 @@ bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool fu
       T->graphs_failed = true;
       return false;
     }
-    enqueue_fast_body(c, T, J, W, full, keep, nullptr, nullptr);
+    enqueue_fast_body(c, T, J, W, full, keep, scan, nullptr, nullptr);
     hipError_t e = hipStreamEndCapture(c->stream, &graph);
     if (e == hipSuccess) e = hipGraphInstantiate(&T->gexec[p], graph, nullptr, nullptr, 0);
     if (graph) hipGraphDestroy(graph);
@@ -907,17 +907,19 @@ struct Flight {
 };
 
 // One outer iteration enqueued whole, without waiting for the previous one.
-// Two things are taken from the last confirmed iteration instead of being
-// read back in between: the number of pointer-jumping rounds (one more is
-// launched; a round after a quiet one returns at once) and the absence of
-// lakes.  The sweeps' launch size follows its sweep units (any size is
-// correct).  Its control block and changed flags are copied to the host slot
-// f.slot and an event marks its end.
+// Three things are taken from the last confirmed iteration instead of being
+// read back in between: the number of pointer-jumping rounds (pairs that need
+// more hop on where they are read; a round after a quiet one returns at once),
+// a decomposition of few enough rounds, and the absence of lakes.  The sweeps' launch size follows its sweep units (any size is
+// correct).  Its control block and changed flags go to the host slot f.slot
+// and an event marks its end.
 int32_t enqueue_fast(fl_ctx* c, fl_terrain* T, Flight& f) {
   hipStream_t s = c->stream;
   fl_dev_work& w = T->w;
-  f.J = std::min<uint32_t>(T->jump_rounds + 1, FL_MAX_JUMP_ROUNDS);
+  f.J = std::min<uint32_t>(T->jump_rounds, FL_MAX_JUMP_ROUNDS);
   if (c->pipelined == 2) f.J = 1;
+  // (a depth that comes near the limit goes the other way in time)
+  const bool scan = T->last_rounds <= FL_SCAN_ROUNDS - FL_SCAN_ROUNDS / 4;
   uint32_t W = (T->t.n + 63) / 64;
   if (!T->last_boff.empty()) {
     const uint32_t u = rounds_size(T->last_boff, 0, T->last_rounds, T->w.long_min).units;
@@ -925,19 +927,23 @@ int32_t enqueue_fast(fl_ctx* c, fl_terrain* T, Flight& f) {
   }
   set_slots(T, f.in);
   f.rec_da = f.rec_tau = SIZE_MAX;
-  bool graphed = !c->prof && c->graphs && launch_fast_graph(c, T, f.J, W, f.full, f.keep);
-  if (!graphed) enqueue_fast_body(c, T, f.J, W, f.full, f.keep, &f.rec_da, &f.rec_tau);
-  if (T->d_tchanged)
-    HIPCHK(hipMemcpyAsync(T->h_tslot[f.slot], T->d_tchanged, T->nterr * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  HIPCHK(hipMemcpyAsync(c->host_slot[f.slot], w.ctrl, FL_CTRL_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  if (!T->ctrl_clean) {
+    fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, T->t.n + 2));
+    if (T->d_tchanged) fl_launch_fill_u32(s, T->d_tchanged, T->nterr, 0);
+  }
+  bool graphed = !c->prof && c->graphs && launch_fast_graph(c, T, f.J, W, f.full, f.keep, scan);
+  if (!graphed) enqueue_fast_body(c, T, f.J, W, f.full, f.keep, scan, &f.rec_da, &f.rec_tau);
+  fl_launch_report(s, w, c->host_slot[f.slot], T->nterr, T->d_tchanged, T->h_tslot[f.slot]);
+  T->ctrl_clean = true;
   HIPCHK(hipEventRecord(c->slot_ev[f.slot], s));
   return FL_OK;
 }
 
 // Wait for flight f and check what it assumed.  *valid is false when any
-// assumption failed: the decomposition had not converged (the kernels after
-// it then did nothing), a lake was found, or a sweep's wait ended without its
-// value.  Its input hb[f.in] is untouched either way.  *changed: the changed flag; per-terrain
+// assumption failed: the decomposition was too deep (the kernels after it then
+// did nothing), a lake was found, or a sweep's wait ended without its value.
+// (The form of minimal speculation takes a decomposition that one jump round
+// did not settle for a failed one, too.)  Its input hb[f.in] is untouched either way.  *changed: the changed flag; per-terrain
 // flags are in T->h_tslot[f.slot].
 int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool* changed) {
   HIPCHK(hipEventSynchronize(c->slot_ev[f.slot]));
@@ -946,13 +952,12 @@ int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool
   uint32_t n = T->t.n;
   bool lake = hc[FL_FLAG_LAKE] != 0;
   bool converged = hc[FL_CTRL_JUMPS + f.J - 1] == 0;
+  bool deep = hc[FL_FLAG_JUMP] != 0;
   uint32_t nb = 2 * (hc[FL_NUM_FLAGS + FL_CNT_MAXLD] + 1);
   *valid = false;
   *changed = false;
-  if (!converged) {
-    T->jump_rounds = std::max(T->jump_rounds, f.J + 1);
-    return FL_OK;
-  }
+  if (!converged) T->jump_rounds = std::max(T->jump_rounds, f.J + 1);
+  if (deep || (!converged && c->pipelined == 2)) return FL_OK;
   if (nb > n + 2) return set_err(FL_ERR_HIP, "light depth out of range");
   for (uint32_t r = 0; r < f.J; r++)
     if (hc[FL_CTRL_JUMPS + r] == 0) {

@@ -33,6 +33,8 @@ struct fl_profiler {
 extern thread_local fl_profiler* fl_current_profiler;
 
 // Control block read back once per phase: [flags | counters | boff head | bnoff head].
+// FL_FLAG_JUMP: chain-end labels moved; in a pipelined iteration: its
+// decomposition is deeper than its placement takes (fl_dev_work::guard)
 // FL_FLAG_STALL: a sweep's wait ended without its value
 enum { FL_FLAG_LAKE = 0, FL_FLAG_JUMP = 1, FL_FLAG_STALL = 2, FL_FLAG_CHANGED = 3, FL_NUM_FLAGS = 4 };
 enum {
@@ -131,9 +133,8 @@ struct fl_dev_work {
   uint32_t* head_base = nullptr;                             // [n] at a chain head: its base position
   uint32_t* perm = nullptr;                                  // [n] chain-major site order
   uint32_t* ctrl = nullptr;                                  // [FL_CTRL_WORDS]
-  // movement flag of the last pointer-jumping round launched: the kernels
-  // after the decomposition do nothing unless it is zero (converged)
-  const uint32_t* guard = nullptr;
+  // the kernels after the decomposition do nothing unless it is zero
+  uint32_t* guard = nullptr;
   int* flags = nullptr;                                      // = ctrl
   uint32_t* counters = nullptr;                              // = ctrl + FL_NUM_FLAGS
   // chains of at least long_min sites (at most FL_LONG_MAX) take wavefronts of
@@ -181,9 +182,14 @@ void fl_launch_dirty(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& 
 void fl_launch_children(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool full, const uint32_t* tid,
                         const uint8_t* t_active);
 void fl_launch_chain_jump(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t round);
-void fl_launch_chain_count(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w);
+// lakes: some root may be no outlet (a lake that no outlet reaches): its
+// basin's sites are left out.
+void fl_launch_chain_count(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool lakes);
 // Bucket offsets (scan), chain placement and the chain-major permutation.
-void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w);
+// scan: the placement makes the offsets itself; a decomposition of more than
+// FL_SCAN_ROUNDS rounds raises the guard instead.
+enum { FL_SCAN_ROUNDS = 64 };
+void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool lakes, bool scan);
 // The sweeps.  Rounds 0..min(deepest, cap - 1) in one launch of about `waves`
 // wavefronts (any number is correct; the sweep units of the rounds are best);
 // the drainage-area sweep also writes the response-time inputs.  positions:
@@ -203,8 +209,12 @@ void fl_launch_tau_tail(hipStream_t s, const fl_dev_work& w, uint32_t lsplit, ui
 // one whose waits ended without their values.
 void fl_launch_reset_words(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w);
 void fl_launch_clear_iter(hipStream_t s, const fl_dev_work& w, uint32_t nb);
+// The control block to host_ctrl and, with tchanged, its G words to
+// host_tchanged (pinned host memory); both zeroed on the device.
+void fl_launch_report(hipStream_t s, const fl_dev_work& w, uint32_t* host_ctrl, uint32_t G, uint32_t* tchanged,
+                      uint32_t* host_tchanged);
 // Back to site order, one thread per site.
-void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool clamp,
+void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool clamp, bool lakes,
                            const uint32_t* tid, const uint8_t* active, uint32_t* tchanged);
 void fl_launch_fill_u32(hipStream_t s, uint32_t* p, uint64_t count, uint32_t v);
 

@@ -53,6 +53,15 @@ static_assert(FL_ROW <= FL_LIST, "a row loaded at once fits its position's list"
 #define FL_HEAD 0x40000u            // ... its chain's head
 #define FL_DEST_OVER 0xfffffffeu    // pdest: the receiver reads the chain's word in cover, not a slot
 
+#if defined(__has_builtin)
+#if __has_builtin(__hip_atomic_load) && __has_builtin(__hip_atomic_store)
+#define FL_DEVICE_ATOMICS 1
+#endif
+#if __has_builtin(__builtin_amdgcn_update_dpp)
+#define FL_WAVE_SHIFT 1
+#endif
+#endif
+
 namespace {
 
 // Workgroups are dealt to the GPU's 8 XCDs in turn (workgroup b to XCD
@@ -106,6 +115,80 @@ __device__ __forceinline__ double first_len(const uint32_t* __restrict__ rp, con
   for (uint32_t k = rp[a]; k < e1; ++k)
     if (col[k] == b) return len[k];
   return 1.0;
+}
+
+__device__ __forceinline__ double bits_double(unsigned long long u) {
+  return __hiloint2double((int)(uint32_t)(u >> 32), (int)(uint32_t)u);
+}
+
+// Synchronisation of one wavefront's lanes around its own LDS tile: a
+// wavefront-scope fence (orders the LDS accesses; the wavefront's LDS
+// operations execute in order) and a wave barrier.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// v of the next lane (up) or of the previous one (down); the lane at the
+// wavefront's edge gets its `edge`.
+#ifndef FL_WAVE_SHIFT
+__device__ __forceinline__ double shift_lanes(double edge, double v, int from) {
+  __shared__ double fl_shift_tile[16][64];
+  const int lane = (int)(threadIdx.x & 63u);
+  double* t = fl_shift_tile[threadIdx.x >> 6];
+  t[lane] = v;
+  wave_sync();
+  const int src = lane + from;
+  const double r = src >= 0 && src < 64 ? t[src] : edge;
+  wave_sync();
+  return r;
+}
+__device__ __forceinline__ double from_next(double edge, double v) { return shift_lanes(edge, v, 1); }
+__device__ __forceinline__ double from_prev(double edge, double v) { return shift_lanes(edge, v, -1); }
+#else
+__device__ __forceinline__ double from_next(double edge, double v) {  // DPP wave_shl:1
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x130, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x130, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double from_prev(double edge, double v) {  // DPP wave_shr:1
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x138, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x138, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+#endif
+__device__ __forceinline__ double of_lane(double v, uint32_t lane) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), (int)lane);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), (int)lane);
+  return __hiloint2double(hi, lo);
+}
+
+// Sums over lanes 0..lane.
+#ifndef FL_WAVE_SHIFT
+__device__ __forceinline__ double prefix_lanes(double v) {
+  for (int off = 1; off < 64; off <<= 1) v = v + shift_lanes(0.0, v, -off);
+  return v;
+}
+#else
+template <int ctrl, int rows>
+__device__ __forceinline__ double plus_dpp(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, rows, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, rows, 0xf, false);
+  return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double prefix_lanes(double v) {
+  v = plus_dpp<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8 within rows of 16 lanes
+  v = plus_dpp<0x112, 0xf>(v);
+  v = plus_dpp<0x114, 0xf>(v);
+  v = plus_dpp<0x118, 0xf>(v);
+  v = plus_dpp<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = plus_dpp<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+#endif
+__device__ __forceinline__ bool same_bits(double a, double b) {
+  return __double_as_longlong(a) == __double_as_longlong(b);
 }
 
 }  // namespace
@@ -444,6 +527,19 @@ __global__ void k_chain_jump(uint32_t bs, uint32_t n, unsigned long long* cp, un
   if (__any(open) && (threadIdx.x & 63u) == 0) *flag_set = 1;
 }
 
+// v's pair p at its fixed point.  Most are after as many rounds as the
+// previous iteration's tree took; the others of a tree that needs more hop on
+// here (bounded by the path), so that no round is launched only to prove that
+// all are.
+__device__ __forceinline__ unsigned long long settle(unsigned long long p, const unsigned long long* pairs) {
+  while (!pair_fin(p)) {
+    const unsigned long long q = __atomic_load_n(pairs + pair_ptr(p), __ATOMIC_RELAXED);
+    if (pair_ptr(q) == pair_ptr(p)) break;
+    p = pair(pair_ptr(q), (pair_cnt(p) + pair_cnt(q)) | (pair_fin(q) ? FL_FIN : 0u));
+  }
+  return p;
+}
+
 // Buckets: 2 * light depth + (chain length >= long_min), so every round
 // has a range of short chains followed by long ones; long_min is a launch
 // parameter (tuned; any value >= 1 gives the same results).  A short bucket
@@ -462,7 +558,9 @@ __device__ __forceinline__ uint32_t bucket_weight(uint32_t len, uint32_t long_mi
 // The chain tails among a thread's FL_BUCKET_PER_THREAD sites of the
 // workgroup's range starting at `base`, with their pairs: activity and heavy
 // child of every site loaded first (clamped in range, all together), the
-// pairs of the tails second, the outlet flag of their roots third.
+// pairs of the tails second, the outlet flag of their roots third (without
+// lakes every root is an outlet: is_outlet is null and this load, 0.7 us in
+// each kernel of the decomposition, is left out).
 struct fl_tail {
   unsigned long long r, c;
   bool t;
@@ -489,7 +587,11 @@ __device__ __forceinline__ void load_tails(uint32_t base, uint32_t n, const uint
   }
 #pragma unroll
   for (uint32_t j = 0; j < FL_BUCKET_PER_THREAD; ++j)
-    if (q[j].t) q[j].t = is_outlet[pair_ptr(q[j].r)] != 0;
+    if (q[j].t) {
+      q[j].r = settle(q[j].r, rt);
+      q[j].c = settle(q[j].c, cp);
+      if (is_outlet) q[j].t = is_outlet[pair_ptr(q[j].r)] != 0;
+    }
 }
 
 // Light-depth histogram of the chains (buckets' counts and total length), aggregated
@@ -632,18 +734,64 @@ __device__ __forceinline__ void place_chain(uint32_t q, uint32_t pos, uint32_t l
   pdest[pos] = FL_NONE;
 }
 
+// `scan`: the bucket offsets are not there yet (no k_bucket_scan before it).
+// Every workgroup makes them for itself, one wavefront over the at most 64
+// rounds, and the first stores them: a launch of 4.5 us and its gap less.  A
+// decomposition with more rounds raises the guard (the iteration is redone).
+struct fl_bucket_out {
+  uint32_t *boff, *bnoff, *ucum, *ctrl;
+};
+template <bool scan>
 __global__ void __launch_bounds__(FL_BUCKET_BLOCK)
-k_bucket_place(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* __restrict__ hc, const unsigned long long* __restrict__ cp,
+k_bucket_place(uint32_t* __restrict__ guard, uint32_t n, const uint32_t* __restrict__ hc, const unsigned long long* __restrict__ cp,
                const unsigned long long* __restrict__ rt, const uint8_t* __restrict__ is_outlet,
-               const uint32_t* __restrict__ boff,
-               const uint32_t* __restrict__ bnoff, uint32_t* __restrict__ bcur, uint32_t* __restrict__ bncur,
+               const uint32_t* __restrict__ bcnt, const uint32_t* __restrict__ bnodes,
+               fl_bucket_out o, uint32_t* __restrict__ bcur, uint32_t* __restrict__ bncur,
                uint2* __restrict__ cmeta, uint32_t* __restrict__ pdest,
                uint32_t* __restrict__ head_base, uint32_t long_min, const uint8_t* __restrict__ act) {
   const uint32_t base = xcd_block() * (FL_BUCKET_BLOCK * FL_BUCKET_PER_THREAD);
   fl_tail tl[FL_BUCKET_PER_THREAD];
-  load_tails(base, n, hc, cp, rt, is_outlet, act, tl);  // in flight while the guard is read
-  if (*guard) return;  // pointer jumping has not converged: the iteration is redone
   __shared__ uint32_t s_c[FL_LDS_BUCKETS], s_n[FL_LDS_BUCKETS], s_bc[FL_LDS_BUCKETS], s_bn[FL_LDS_BUCKETS];
+  __shared__ uint32_t s_boff[FL_LDS_BUCKETS], s_bnoff[FL_LDS_BUCKETS];
+  static_assert(FL_LDS_BUCKETS == 128 && FL_LDS_BUCKETS == 2 * FL_SCAN_ROUNDS, "one wavefront scans the rounds");
+  const uint32_t maxld = o.ctrl[FL_NUM_FLAGS + FL_CNT_MAXLD];
+  load_tails(base, n, hc, cp, rt, is_outlet, act, tl);  // in flight while the guard is read
+  if (*guard) return;  // the iteration is redone
+  if (scan && maxld >= FL_LDS_BUCKETS / 2) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *guard = 1;
+    return;
+  }
+  if (scan && threadIdx.x < 64) {
+    const uint32_t l = threadIdx.x;  // its round
+    const bool in = l <= maxld;
+    const uint32_t c0 = in ? bcnt[2 * l] : 0u, c1 = in ? bcnt[2 * l + 1] : 0u;
+    const uint32_t n0 = in ? bnodes[2 * l] : 0u, n1 = in ? bnodes[2 * l + 1] : 0u;
+    const uint32_t stride = 65u - long_min, u = c1 + (n0 + stride - 1) / stride;
+    // (sums below 2^53: exact)
+    const uint32_t c = (uint32_t)prefix_lanes((double)(c0 + c1)), m = (uint32_t)prefix_lanes((double)(n0 + n1));
+    const uint32_t us = (uint32_t)prefix_lanes((double)u);
+    s_boff[2 * l] = c - c1 - c0;
+    s_boff[2 * l + 1] = c - c1;
+    s_bnoff[2 * l] = m - n1 - n0;
+    s_bnoff[2 * l + 1] = m - n1;
+    if (blockIdx.x == 0 && in) {
+      uint32_t* counters = o.ctrl + FL_NUM_FLAGS;
+      uint32_t* head_c = counters + FL_NUM_COUNTERS;
+      uint32_t* head_n = head_c + FL_CTRL_HEAD + 1;
+      o.ucum[l] = us - u;
+      o.boff[2 * l] = head_c[2 * l] = c - c1 - c0;
+      o.boff[2 * l + 1] = head_c[2 * l + 1] = c - c1;
+      o.bnoff[2 * l] = head_n[2 * l] = m - n1 - n0;
+      o.bnoff[2 * l + 1] = head_n[2 * l + 1] = m - n1;
+      if (l == maxld) {
+        o.ucum[l + 1] = us;
+        o.boff[2 * l + 2] = head_c[2 * l + 2] = counters[FL_CNT_CHAINS] = c;
+        o.bnoff[2 * l + 2] = head_n[2 * l + 2] = counters[FL_CNT_POSITIONS] = m;
+      }
+    }
+  }
+  auto c_off = [&](uint32_t l) { return scan ? s_boff[l] : o.boff[l]; };
+  auto n_off = [&](uint32_t l) { return scan ? s_bnoff[l] : o.bnoff[l]; };
   for (uint32_t t = threadIdx.x; t < FL_LDS_BUCKETS; t += FL_BUCKET_BLOCK) {
     s_c[t] = 0;
     s_n[t] = 0;
@@ -660,8 +808,8 @@ k_bucket_place(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* _
         lc[j] = atomicAdd(s_c + l, bucket_weight(len, long_min));
         ln[j] = atomicAdd(s_n + l, len);
       } else {
-        uint32_t q = boff[l] + atomicAdd(bcur + l, bucket_weight(len, long_min));
-        uint32_t pos = bnoff[l] + atomicAdd(bncur + l, len);
+        uint32_t q = o.boff[l] + atomicAdd(bcur + l, bucket_weight(len, long_min));
+        uint32_t pos = o.bnoff[l] + atomicAdd(bncur + l, len);
         place_chain(q, pos, len, pair_ptr(c), long_min, cmeta, head_base, pdest);
       }
     }
@@ -679,8 +827,8 @@ k_bucket_place(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* _
     const unsigned long long c = tl[j].c;
     uint32_t len = pair_cnt(c) + 1;
     uint32_t l = 2u * pair_cnt(tl[j].r) + (len >= long_min ? 1u : 0u);
-    uint32_t q = boff[l] + s_bc[l] + lc[j];
-    uint32_t pos = bnoff[l] + s_bn[l] + ln[j];
+    uint32_t q = c_off(l) + s_bc[l] + lc[j];
+    uint32_t pos = n_off(l) + s_bn[l] + ln[j];
     place_chain(q, pos, len, pair_ptr(c), long_min, cmeta, head_base, pdest);
   }
 }
@@ -708,8 +856,8 @@ struct fl_perm_out {
   uint32_t* pro;
 };
 
-__global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, uint32_t n, const unsigned long long* __restrict__ cp,
-                             const unsigned long long* __restrict__ rt, const uint32_t* __restrict__ next,
+__global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, uint32_t n, unsigned long long* cp,
+                             unsigned long long* rt, const uint32_t* __restrict__ next,
                              const uint8_t* __restrict__ is_outlet, const uint32_t* __restrict__ head_base,
                              fl_perm_out o,
                              const double* __restrict__ area, const double* __restrict__ K,
@@ -725,24 +873,13 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
   uint32_t v = gid(bs);
   // the site's own words are read together with the guard (one load
   // latency; a site of a lake basin reads some it does not use)
-  const uint32_t mld = *maxld;
-  const bool on = v < n && act[v];
-  unsigned long long rv = 0ull, cv = 0ull, m = 0ull;
-  uint32_t b = 0u, e = 0u, hk = 0u, p = 0u;
-  double Kv = 0.0, dv = 0.0, av = 0.0;
-  if (on) {
-    rv = rt[v];
-    cv = cp[v];
-    b = rp[v];
-    e = rp[v + 1];
-    hk = hc[v];
-    m = cmask[v];
-    p = next[v];
-    Kv = K[v];
-    dv = dnext[v];
-    av = area[v];
-  }
-  if (*guard) return;  // pointer jumping has not converged: the iteration is redone
+  // (an inactive site's too: one load latency less for the active ones)
+  const uint32_t mld = *maxld, redo = *guard, vv = v < n ? v : n - 1;
+  const bool on = act[vv] != 0 && v < n;
+  unsigned long long rv = rt[vv], cv = cp[vv];
+  const unsigned long long m = cmask[vv];
+  const uint32_t b = rp[vv], e = rp[vv + 1], hk = hc[vv], p = next[vv];
+  const double Kv = K[vv], dv = dnext[vv], av = area[vv];
   // the bucket histograms are used up (count, scan, place): clear the
   // entries this decomposition touched for the next one
   const uint32_t nb = 2u * (mld + 1u);
@@ -752,16 +889,24 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
     bcur[i] = 0;
     bncur[i] = 0;
   }
-  if (!on) return;
+  if (redo || !on) return;
+  if (!pair_fin(rv) || !pair_fin(cv)) {
+    rv = settle(rv, rt);
+    cv = settle(cv, cp);
+    // for the heads below it, k_tau_scatter (nothing else reads v's pair from
+    // here on but as one to hop over, which either value serves)
+    __atomic_store_n(rt + v, rv | (1ull << 63), __ATOMIC_RELAXED);
+    __atomic_store_n(cp + v, cv | (1ull << 63), __ATOMIC_RELAXED);
+  }
   const uint32_t r = pair_ptr(rv), hd = pair_ptr(cv), deg = e - b;
   root[v] = r;
   // the second level of loads, issued together: the root's outlet flag, the
   // chain's base, the row (up to FL_ROW entries), at a chain head the
   // receiver's pair and with max slopes the outlet's base
-  const uint8_t outlet = is_outlet[r];
+  const uint8_t outlet = is_outlet ? is_outlet[r] : 1;
   const uint32_t base = head_base[hd];
   const bool head = hd == v;
-  const unsigned long long cpp = head ? cp[p] : 0ull;
+  const unsigned long long cpp = head ? settle(cp[p], cp) : 0ull;
   const uint32_t hbr = clamp ? head_base[r] : 0u;
   uint32_t cc[FL_ROW];
   const bool short_row = deg <= FL_ROW;
@@ -877,15 +1022,6 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
 #define FL_SPIN_MAX (1u << 20)
 #define FL_NEG0 (-0.0)
 
-#if defined(__has_builtin)
-#if __has_builtin(__hip_atomic_load) && __has_builtin(__hip_atomic_store)
-#define FL_DEVICE_ATOMICS 1
-#endif
-#if __has_builtin(__builtin_amdgcn_update_dpp)
-#define FL_WAVE_SHIFT 1
-#endif
-#endif
-
 // The rounds of a decomposition and the counters its units are taken from.
 struct fl_flow {
   const uint32_t* maxld;  // the deepest round
@@ -898,10 +1034,6 @@ struct fl_flow {
 };
 
 namespace {
-
-__device__ __forceinline__ double bits_double(unsigned long long u) {
-  return __hiloint2double((int)(uint32_t)(u >> 32), (int)(uint32_t)u);
-}
 
 // A hand-over word, read and written at device scope.
 __device__ __forceinline__ unsigned long long peek(const double* p) {
@@ -964,76 +1096,6 @@ __device__ __forceinline__ double await_lds(const double* p, int* stall) {
     u = *w;
   }
   return bits_double(u);
-}
-
-// Synchronisation of one wavefront's lanes around its own LDS tile: a
-// wavefront-scope fence (orders the LDS accesses; the wavefront's LDS
-// operations execute in order) and a wave barrier.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// v of the next lane (up) or of the previous one (down); the lane at the
-// wavefront's edge gets its `edge`.
-#ifndef FL_WAVE_SHIFT
-__device__ __forceinline__ double shift_lanes(double edge, double v, int from) {
-  __shared__ double fl_shift_tile[16][64];
-  const int lane = (int)(threadIdx.x & 63u);
-  double* t = fl_shift_tile[threadIdx.x >> 6];
-  t[lane] = v;
-  wave_sync();
-  const int src = lane + from;
-  const double r = src >= 0 && src < 64 ? t[src] : edge;
-  wave_sync();
-  return r;
-}
-__device__ __forceinline__ double from_next(double edge, double v) { return shift_lanes(edge, v, 1); }
-__device__ __forceinline__ double from_prev(double edge, double v) { return shift_lanes(edge, v, -1); }
-#else
-__device__ __forceinline__ double from_next(double edge, double v) {  // DPP wave_shl:1
-  const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x130, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x130, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double from_prev(double edge, double v) {  // DPP wave_shr:1
-  const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), 0x138, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), 0x138, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-#endif
-__device__ __forceinline__ double of_lane(double v, uint32_t lane) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), (int)lane);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), (int)lane);
-  return __hiloint2double(hi, lo);
-}
-
-// Sums over lanes 0..lane.
-#ifndef FL_WAVE_SHIFT
-__device__ __forceinline__ double prefix_lanes(double v) {
-  for (int off = 1; off < 64; off <<= 1) v = v + shift_lanes(0.0, v, -off);
-  return v;
-}
-#else
-template <int ctrl, int rows>
-__device__ __forceinline__ double plus_dpp(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, rows, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, rows, 0xf, false);
-  return v + __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double prefix_lanes(double v) {
-  v = plus_dpp<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8 within rows of 16 lanes
-  v = plus_dpp<0x112, 0xf>(v);
-  v = plus_dpp<0x114, 0xf>(v);
-  v = plus_dpp<0x118, 0xf>(v);
-  v = plus_dpp<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-  v = plus_dpp<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-  return v;
-}
-#endif
-__device__ __forceinline__ bool same_bits(double a, double b) {
-  return __double_as_longlong(a) == __double_as_longlong(b);
 }
 
 // A value that every lane of the wavefront holds, for scalar registers.
@@ -1884,19 +1946,12 @@ __global__ void k_tau_scatter(uint32_t bs, const uint32_t* __restrict__ guard, u
   // latency), then the second level (outlet flag, positions, the outlet's
   // elevation and uplift) together
   const bool in = v < n;
-  const bool on = in && act[v];
-  const double hv = in ? h[v] : 0.0;
-  unsigned long long rv = 0ull, cv = 0ull;
-  uint32_t rb = 0u, re = 0u, g = 0u;  // the row, for the change marks
-  double uv = 0.0;
-  if (on) {
-    rv = rt[v];
-    cv = cp[v];
-    rb = rp[v];
-    re = rp[v + 1];
-    uv = U[v];
-    g = tid ? tid[v] : 0u;
-  }
+  const uint32_t vv = in ? v : n - 1;
+  const bool on = act[vv] != 0 && in;
+  const double hv = h[vv], uv = U[vv];
+  const unsigned long long rv = rt[vv], cv = cp[vv];
+  const uint32_t rb = rp[vv], re = rp[vv + 1];  // the row, for the change marks
+  const uint32_t g = tid ? tid[vv] : 0u;
   if (*guard != 0) return;  // pointer jumping has not converged: the iteration is redone
   bool changed = false;
   if (in && !on) {
@@ -1905,7 +1960,7 @@ __global__ void k_tau_scatter(uint32_t bs, const uint32_t* __restrict__ guard, u
     h2[v] = hv;
   } else if (on) {
     const uint32_t o = pair_ptr(rv);
-    const uint8_t outlet = is_outlet[o];
+    const uint8_t outlet = is_outlet ? is_outlet[o] : 1;
     // (a site of a lake basin reads these for nothing; its values were
     // written by k_chain_perm)
     const uint32_t P = head_base[pair_ptr(cv)] + pair_cnt(cv);
@@ -2068,6 +2123,23 @@ __global__ void k_clear_iter(uint32_t bs, uint32_t nb, uint32_t* __restrict__ ct
   }
 }
 
+// A pipelined iteration's end: its control block and the terrains' changed
+// flags to their pinned host slots, and both cleared for the next iteration's
+// (one launch for two copies and two fills).
+__global__ void k_report(uint32_t bs, uint32_t count, uint32_t* __restrict__ ctrl, uint32_t* __restrict__ host_ctrl,
+                         uint32_t G, uint32_t* __restrict__ tchanged, uint32_t* __restrict__ host_tchanged) {
+  const uint32_t i = gid(bs);
+  if (i >= count) return;
+  if (i < FL_CTRL_WORDS) {
+    host_ctrl[i] = ctrl[i];
+    ctrl[i] = 0;
+  }
+  if (tchanged && i < G) {
+    host_tchanged[i] = tchanged[i];
+    tchanged[i] = 0;
+  }
+}
+
 // --------------------------------------------------------- launchers -----
 
 namespace {
@@ -2189,23 +2261,32 @@ void fl_launch_chain_jump(hipStream_t s, const fl_dev_terrain& t, const fl_dev_w
   FL_LAUNCH(k_chain_jump, t.n, s, t.n, (unsigned long long*)w.cp, (unsigned long long*)w.rt, fset, prev, w.act);
 }
 
-void fl_launch_chain_count(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w) {
+void fl_launch_chain_count(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool lakes) {
   uint32_t per = FL_BUCKET_BLOCK * FL_BUCKET_PER_THREAD;
   FL_LAUNCH_GRID(k_bucket_count, dim3((t.n + per - 1) / per), dim3(FL_BUCKET_BLOCK), t.n, s, w.guard, t.n, w.hc,
-                 (const unsigned long long*)w.cp, (const unsigned long long*)w.rt, t.is_outlet, w.bcnt, w.bnodes, w.counters + FL_CNT_MAXLD,
+                 (const unsigned long long*)w.cp, (const unsigned long long*)w.rt, lakes ? t.is_outlet : (const uint8_t*)nullptr, w.bcnt, w.bnodes, w.counters + FL_CNT_MAXLD,
                  w.long_min, w.act);
 }
 
-void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w) {
-  FL_LAUNCH_GRID(k_bucket_scan, dim3(1), dim3(FL_SCAN_BLOCK), 0, s, t.n, w.long_min, w.ctrl, w.bcnt, w.bnodes, w.boff,
-                 w.bnoff, w.ucum);
+void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool lakes, bool scan) {
+  const uint8_t* outlets = lakes ? t.is_outlet : (const uint8_t*)nullptr;
   uint32_t per = FL_BUCKET_BLOCK * FL_BUCKET_PER_THREAD;
-  FL_LAUNCH_GRID(k_bucket_place, dim3((t.n + per - 1) / per), dim3(FL_BUCKET_BLOCK), t.n, s, w.guard, t.n, w.hc,
-                 (const unsigned long long*)w.cp, (const unsigned long long*)w.rt, t.is_outlet, w.boff, w.bnoff,
-                 w.bcur, w.bncur, w.cmeta, w.pdest, w.head_base, w.long_min, w.act);
+  const dim3 grid((t.n + per - 1) / per), block(FL_BUCKET_BLOCK);
+  const fl_bucket_out bo{w.boff, w.bnoff, w.ucum, w.ctrl};
+  if (scan) {
+    FL_LAUNCH_GRID(k_bucket_place<true>, grid, block, t.n, s, w.guard, t.n, w.hc, (const unsigned long long*)w.cp,
+                   (const unsigned long long*)w.rt, outlets, w.bcnt, w.bnodes, bo, w.bcur, w.bncur, w.cmeta, w.pdest,
+                   w.head_base, w.long_min, w.act);
+  } else {
+    FL_LAUNCH_GRID(k_bucket_scan, dim3(1), dim3(FL_SCAN_BLOCK), 0, s, t.n, w.long_min, w.ctrl, w.bcnt, w.bnodes,
+                   w.boff, w.bnoff, w.ucum);
+    FL_LAUNCH_GRID(k_bucket_place<false>, grid, block, t.n, s, w.guard, t.n, w.hc, (const unsigned long long*)w.cp,
+                   (const unsigned long long*)w.rt, outlets, w.bcnt, w.bnodes, bo, w.bcur, w.bncur, w.cmeta, w.pdest,
+                   w.head_base, w.long_min, w.act);
+  }
   fl_perm_out o{w.perm, w.pcnt, w.pdest, w.parea, w.pK, w.pdn, w.up, w.tanp, w.hop, w.ppos, w.pro};
-  FL_LAUNCH(k_chain_perm, t.n, s, w.guard, t.n, (const unsigned long long*)w.cp, (const unsigned long long*)w.rt,
-            w.next, t.is_outlet, w.head_base, o, t.area, t.erod, w.dnext, t.uplift, t.tan_ms,
+  FL_LAUNCH(k_chain_perm, t.n, s, w.guard, t.n, (unsigned long long*)w.cp, (unsigned long long*)w.rt,
+            w.next, outlets, w.head_base, o, t.area, t.erod, w.dnext, t.uplift, t.tan_ms,
             t.any_max_slope ? 1 : 0, w.A, w.tau, w.h, w.h2, w.counters + FL_CNT_MAXLD, w.bcnt, w.bnodes, w.bcur,
             w.bncur, t.row_ptr, t.col, (const unsigned long long*)w.cmask, w.hc, w.act, w.root);
 }
@@ -2258,16 +2339,22 @@ void fl_launch_tau_tail(hipStream_t s, const fl_dev_work& w, uint32_t lsplit, ui
                    tau_args(w));
 }
 
-void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool clamp,
+void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool clamp, bool lakes,
                            const uint32_t* tid, const uint8_t* active, uint32_t* tchanged) {
   FL_LAUNCH(k_tau_scatter, t.n, s, w.guard, t.n, (const unsigned long long*)w.cp, (const unsigned long long*)w.rt,
-            t.is_outlet, w.head_base, w.taup, w.hnp, t.uplift, w.h, w.h2, w.tau, w.flags, clamp ? 1 : 0, tid, w.act,
+            lakes ? t.is_outlet : (const uint8_t*)nullptr, w.head_base, w.taup, w.hnp, t.uplift, w.h, w.h2, w.tau, w.flags, clamp ? 1 : 0, tid, w.act,
             tchanged, w.chg, w.dirty, t.row_ptr, t.col);
 }
 
 void fl_launch_clear_iter(hipStream_t s, const fl_dev_work& w, uint32_t nb) {
   uint32_t cnt = nb > FL_CTRL_WORDS ? nb : FL_CTRL_WORDS;
   FL_LAUNCH(k_clear_iter, cnt, s, nb, w.ctrl, w.bcnt, w.bnodes, w.bcur, w.bncur);
+}
+
+void fl_launch_report(hipStream_t s, const fl_dev_work& w, uint32_t* host_ctrl, uint32_t G, uint32_t* tchanged,
+                      uint32_t* host_tchanged) {
+  const uint32_t cnt = tchanged && G > FL_CTRL_WORDS ? G : FL_CTRL_WORDS;
+  FL_LAUNCH(k_report, cnt, s, cnt, w.ctrl, host_ctrl, G, tchanged, host_tchanged);
 }
 
 // (launched in parts: the kernel counts items in 32 bits)
