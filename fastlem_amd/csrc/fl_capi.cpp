@@ -123,6 +123,10 @@ struct fl_terrain {
   uint8_t* chgb[3] = {nullptr, nullptr, nullptr};  // per-site "elevation changed" of that iteration
   bool prev_valid = false;
   bool after_lake = true;  // the last iteration joined lakes (its tree is not raw receivers)
+  // the last confirmed iteration had lakes: the pipelined ones join lakes, too
+  // (a lake can last: one that no outlet reaches, a site whose drainage area
+  // gives no response time)
+  bool lakes = false;
   // w.A holds no drainage area of a tree like the next one (a solve's
   // start, new terrains in the union, the iteration after lake joins, whose
   // drainage changes wholesale where lakes were): the next iteration runs
@@ -620,18 +624,7 @@ int32_t ensure_visit_order(fl_ctx* c, fl_terrain* T) {
 // Chain-end labels of the receiver forest by pointer jumping (the subroot of
 // find_roots_with_lakes, stream_tree.rs:139-173) into w.sub.
 int32_t label_chain_ends(fl_ctx* c, fl_terrain* T) {
-  hipStream_t s = c->stream;
-  fl_launch_sub_init(s, T->t, T->w);
-  bool flip = false;
-  for (uint32_t round = 0;; round++) {
-    fl_launch_fill_u32(s, (uint32_t*)T->w.flags + FL_FLAG_JUMP, 1, 0);
-    fl_launch_sub_jump(s, T->t, T->w, flip);
-    flip = !flip;
-    FLCHK(read_ctrl(c, T));
-    if (!host_flag(c, FL_FLAG_JUMP)) break;
-    if (round > 64) return set_err(FL_ERR_HIP, "chain-end labelling did not converge");
-  }
-  if (flip) std::swap(T->w.sub, T->w.sub2);
+  fl_launch_sub_labels(c->stream, T->t, T->w);
   return FL_OK;
 }
 
@@ -639,7 +632,7 @@ int32_t label_chain_ends(fl_ctx* c, fl_terrain* T) {
 int32_t join_lakes(fl_ctx* c, fl_terrain* T) {
   FLCHK(label_chain_ends(c, T));
   FLCHK(ensure_visit_order(c, T));
-  fl_launch_lake_join(c->stream, T->t, T->w);
+  fl_launch_lake_join(c->stream, T->t, T->w, false);
   return FL_OK;
 }
 
@@ -832,7 +825,10 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
   }
   *changed = host_flag(c, FL_FLAG_CHANGED) != 0;
   std::swap(w.h, w.h2);
-  if (*had_lake) T->hint_stale = true;
+  // (the lakes of one iteration after another are few, and drainage has
+  // settled around them)
+  if (*had_lake && !T->lakes) T->hint_stale = true;
+  T->lakes = *had_lake;
   return FL_OK;
 }
 
@@ -840,30 +836,36 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
 // wavefronts), enqueued on the context's stream or recorded by a capture.
 // rec_* receive the profiler records of the launches (when profiling).
 void enqueue_fast_body(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool full, bool keep, bool scan,
-                       size_t* rec_da, size_t* rec_tau) {
+                       bool lakes, size_t* rec_da, size_t* rec_tau) {
   hipStream_t s = c->stream;
   fl_dev_work& w = T->w;
   bool clamp = T->t.any_max_slope;
   fl_launch_receivers(s, T->t, w, keep, !full);
+  if (lakes) {
+    fl_launch_sub_labels(s, T->t, w);
+    fl_launch_lake_join(s, T->t, w, true);
+    if (!full) fl_launch_dirty(s, T->t, w);
+  }
   fl_launch_children(s, T->t, w, full, T->d_tid, T->d_active);
   for (uint32_t r = 0; r < J; r++) fl_launch_chain_jump(s, T->t, w, r);
-  w.guard = (uint32_t*)w.flags + FL_FLAG_JUMP;
-  fl_launch_chain_count(s, T->t, w, false);
-  fl_launch_chain_layout(s, T->t, w, false, scan);
+  w.guard = (uint32_t*)w.flags + FL_FLAG_DEEP;
+  fl_launch_chain_count(s, T->t, w, lakes);
+  fl_launch_chain_layout(s, T->t, w, lakes, scan);
   if (c->prof && rec_da) *rec_da = c->prof->pending.size();
   fl_launch_da_fold(s, T->t, w, FL_NONE_ROUND, W, 0, clamp);
   if (c->prof && rec_tau) *rec_tau = c->prof->pending.size();
   fl_launch_tau_fold(s, w, FL_NONE_ROUND, W, 0, clamp);
-  fl_launch_tau_scatter(s, T->t, w, clamp, false, T->d_tid, T->d_active, T->d_tchanged);
+  fl_launch_tau_scatter(s, T->t, w, clamp, lakes, T->d_tid, T->d_active, T->d_tchanged);
 }
 
 // The pipelined iteration for J and the current buffer parity as a
 // graph, captured on first use.  False when capture is not possible (the
 // caller launches directly).
-bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool full, bool keep, bool scan) {
+bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool full, bool keep, bool scan,
+                       bool lakes) {
   if (T->graphs_failed) return false;
   int p = T->w.h == T->hb[0] ? 0 : (T->w.h == T->hb[1] ? 1 : 2);
-  const int mode = (full ? 1 : 0) | (keep ? 2 : 0) | (scan ? 4 : 0);
+  const int mode = (full ? 1 : 0) | (keep ? 2 : 0) | (scan ? 4 : 0) | (lakes ? 8 : 0);
   // (a captured launch size serves until the units differ by more than half)
   if (!T->gexec[p] || T->gJ[p] != J || W > T->gW[p] + T->gW[p] / 2 || T->gW[p] > W + W / 2 || T->gF[p] != mode ||
       T->gB[p] != fl_site_block || T->gL[p] != T->w.long_min) {
@@ -876,7 +878,7 @@ bool launch_fast_graph(fl_ctx* c, fl_terrain* T, uint32_t J, uint32_t W, bool fu
       T->graphs_failed = true;
       return false;
     }
-    enqueue_fast_body(c, T, J, W, full, keep, scan, nullptr, nullptr);
+    enqueue_fast_body(c, T, J, W, full, keep, scan, lakes, nullptr, nullptr);
     hipError_t e = hipStreamEndCapture(c->stream, &graph);
     if (e == hipSuccess) e = hipGraphInstantiate(&T->gexec[p], graph, nullptr, nullptr, 0);
     if (graph) hipGraphDestroy(graph);
@@ -901,6 +903,7 @@ struct Flight {
   int slot = 0;
   bool full = false;  // every basin recomputed (no previous tree)
   bool keep = false;  // receivers kept where the neighbourhood did not change
+  bool lakes = false;  // joins lakes
   uint32_t J = 0;
   std::vector<uint8_t> mask;  // terrains iterating in it
   size_t rec_da = SIZE_MAX, rec_tau = SIZE_MAX;
@@ -910,7 +913,8 @@ struct Flight {
 // Three things are taken from the last confirmed iteration instead of being
 // read back in between: the number of pointer-jumping rounds (pairs that need
 // more hop on where they are read; a round after a quiet one returns at once),
-// a decomposition of few enough rounds, and the absence of lakes.  The sweeps' launch size follows its sweep units (any size is
+// a decomposition of few enough rounds, and the absence of lakes (after an
+// iteration with lakes they are joined, found or not).  The sweeps' launch size follows its sweep units (any size is
 // correct).  Its control block and changed flags go to the host slot f.slot
 // and an event marks its end.
 int32_t enqueue_fast(fl_ctx* c, fl_terrain* T, Flight& f) {
@@ -931,8 +935,8 @@ int32_t enqueue_fast(fl_ctx* c, fl_terrain* T, Flight& f) {
     fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, T->t.n + 2));
     if (T->d_tchanged) fl_launch_fill_u32(s, T->d_tchanged, T->nterr, 0);
   }
-  bool graphed = !c->prof && c->graphs && launch_fast_graph(c, T, f.J, W, f.full, f.keep, scan);
-  if (!graphed) enqueue_fast_body(c, T, f.J, W, f.full, f.keep, scan, &f.rec_da, &f.rec_tau);
+  bool graphed = !c->prof && c->graphs && launch_fast_graph(c, T, f.J, W, f.full, f.keep, scan, f.lakes);
+  if (!graphed) enqueue_fast_body(c, T, f.J, W, f.full, f.keep, scan, f.lakes, &f.rec_da, &f.rec_tau);
   fl_launch_report(s, w, c->host_slot[f.slot], T->nterr, T->d_tchanged, T->h_tslot[f.slot]);
   T->ctrl_clean = true;
   HIPCHK(hipEventRecord(c->slot_ev[f.slot], s));
@@ -941,18 +945,19 @@ int32_t enqueue_fast(fl_ctx* c, fl_terrain* T, Flight& f) {
 
 // Wait for flight f and check what it assumed.  *valid is false when any
 // assumption failed: the decomposition was too deep (the kernels after it then
-// did nothing), a lake was found, or a sweep's wait ended without its value.
+// did nothing), a lake was found and not joined, or a sweep's wait ended without
+// its value.
 // (The form of minimal speculation takes a decomposition that one jump round
 // did not settle for a failed one, too.)  Its input hb[f.in] is untouched either way.  *changed: the changed flag; per-terrain
 // flags are in T->h_tslot[f.slot].
-int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool* changed) {
+int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool* changed, bool* lake_found) {
   HIPCHK(hipEventSynchronize(c->slot_ev[f.slot]));
   T->stat_syncs++;
   const uint32_t* hc = c->host_slot[f.slot];
   uint32_t n = T->t.n;
   bool lake = hc[FL_FLAG_LAKE] != 0;
   bool converged = hc[FL_CTRL_JUMPS + f.J - 1] == 0;
-  bool deep = hc[FL_FLAG_JUMP] != 0;
+  bool deep = hc[FL_FLAG_DEEP] != 0;
   uint32_t nb = 2 * (hc[FL_NUM_FLAGS + FL_CNT_MAXLD] + 1);
   *valid = false;
   *changed = false;
@@ -968,8 +973,9 @@ int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool
     T->stalled = T->reset_words = true;
     return FL_OK;
   }
-  if (lake) return FL_OK;
+  if (lake && !f.lakes) return FL_OK;
   *valid = true;
+  *lake_found = T->lakes = lake;
   T->prev_nb = nb;
   T->last_rounds = nb / 2;
   // the next iterations would speculate as many rounds: they wait for a
@@ -1003,6 +1009,7 @@ int32_t reset_state(fl_ctx* c, fl_terrain* T) {
   uint32_t n = T->t.n;
   T->prev_valid = false;
   T->after_lake = true;
+  T->lakes = false;
   T->hint_stale = true;
   HIPCHK(hipMemcpyAsync(T->w.h, T->t.init_h, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
   HIPCHK(hipMemcpyAsync(T->w.A, T->t.area, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
@@ -1214,7 +1221,7 @@ int32_t layout_device(fl_terrain* P, uint32_t n, uint32_t nnz, uint32_t count, b
   if (clamp)
     for (double** p : {&w.hnp, &w.up, &w.tanp, &w.hop}) FLCHK(dev_alloc(P, p, n));
   if (clamp) FLCHK(dev_alloc(P, &w.pro, n));
-  for (uint32_t** p : {&w.sub, &w.sub2, &w.hc, &w.pcnt, &w.pdest, &w.ppos, &w.head_base, &w.perm})
+  for (uint32_t** p : {&w.sub, &w.hc, &w.pcnt, &w.pdest, &w.ppos, &w.head_base, &w.perm})
     FLCHK(dev_alloc(P, p, n));
   FLCHK(dev_alloc(P, &w.cover, n));
   FLCHK(dev_alloc(P, &w.cmeta, n));
@@ -1873,7 +1880,8 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
         f.full = !cur->prev_valid || c->recompute_all;
         f.keep = !f.full && !cur->after_lake;
         cur->prev_valid = true;
-        cur->after_lake = false;  // a flight that finds lakes is redone synchronously
+        // a flight that finds lakes and does not join them is redone synchronously
+        cur->after_lake = f.lakes = cur->lakes && cur->have_order;
         FLCHK(enqueue_fast(c, cur, f));
         for (uint32_t g = 0; g < cur->nterr; g++) enq[g] += mask[g];
         q.push_back(std::move(f));
@@ -1881,8 +1889,8 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
       if (q.empty()) break;  // cannot happen while a terrain is active
       Flight f = std::move(q.front());
       q.pop_front();
-      bool valid = false, changed = false;
-      FLCHK(finish_fast(c, cur, f, &valid, &changed));
+      bool valid = false, changed = false, lake = false;
+      FLCHK(finish_fast(c, cur, f, &valid, &changed, &lake));
       const uint32_t* tflags = cur->d_tchanged ? cur->h_tslot[f.slot] : nullptr;
       if (!valid) {
         // the flights after it started from a wrong input: let them land,
@@ -1892,14 +1900,13 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
           for (uint32_t g = 0; g < cur->nterr; g++) enq[g] -= x.mask[g];
         q.clear();
         T->stat_redone++;
-        bool lake = false;
         FLCHK(upload_mask(f.mask));
         set_slots(cur, f.in);
         FLCHK(one_iteration(c, cur, f.full, f.keep, &changed, &lake));
         cur->after_lake = lake;
-        T->stat_lake_iterations += lake ? 1 : 0;
         tflags = cur->d_tchanged ? cur->h_tchanged : nullptr;
       }
+      T->stat_lake_iterations += lake ? 1 : 0;
       confirm(f.mask, tflags, changed);
       T->stat_recomputed += all_positions(cur->last_boff);
       note_rounds(T, cur->last_rounds, it);
@@ -2236,7 +2243,8 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
       f.full = !cur->prev_valid || c->recompute_all;
       f.keep = !f.full && !cur->after_lake;
       cur->prev_valid = true;
-      cur->after_lake = false;  // a flight that finds lakes is redone synchronously
+      // a flight that finds lakes and does not join them is redone synchronously
+      cur->after_lake = f.lakes = cur->lakes && cur->have_order;
       FLCHK(enqueue_fast(c, cur, f));
       for (uint32_t g = 0; g < cur->nterr; g++) L->enq[g] += mask[g];
       L->q.push_back(std::move(f));
@@ -2244,8 +2252,8 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
     if (L->q.empty()) return FL_OK;
     Flight f = std::move(L->q.front());
     L->q.pop_front();
-    bool valid = false, changed = false;
-    FLCHK(finish_fast(c, cur, f, &valid, &changed));
+    bool valid = false, changed = false, lake = false;
+    FLCHK(finish_fast(c, cur, f, &valid, &changed, &lake));
     const uint32_t* tflags = cur->h_tslot[f.slot];
     if (!valid) {
       // the flights after it started from a wrong input: let them land, then
@@ -2255,7 +2263,6 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
         for (uint32_t g = 0; g < cur->nterr; g++) L->enq[g] -= x.mask[g];
       L->q.clear();
       cur->stat_redone++;
-      bool lake = false;
       FLCHK(lane_upload_mask(L, f.mask));
       set_slots(cur, f.in);
       FLCHK(one_iteration(c, cur, f.full, f.keep, &changed, &lake));
@@ -2481,7 +2488,7 @@ extern "C" int32_t fl_stage_stream_tree(fl_ctx* c, fl_terrain* T, const double* 
   FLCHK(label_chain_ends(c, T));
   if (lake) {
     FLCHK(ensure_visit_order(c, T));
-    fl_launch_lake_join(c->stream, T->t, T->w);
+    fl_launch_lake_join(c->stream, T->t, T->w, false);
   }
   FLCHK(download_idx_old(c, T, next_out, T->w.next));
   FLCHK(download_idx_old(c, T, subroot_out, T->w.sub));

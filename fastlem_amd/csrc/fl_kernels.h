@@ -33,10 +33,10 @@ struct fl_profiler {
 extern thread_local fl_profiler* fl_current_profiler;
 
 // Control block read back once per phase: [flags | counters | boff head | bnoff head].
-// FL_FLAG_JUMP: chain-end labels moved; in a pipelined iteration: its
-// decomposition is deeper than its placement takes (fl_dev_work::guard)
+// FL_FLAG_DEEP: a pipelined iteration's decomposition is deeper than its
+// placement takes (fl_dev_work::guard)
 // FL_FLAG_STALL: a sweep's wait ended without its value
-enum { FL_FLAG_LAKE = 0, FL_FLAG_JUMP = 1, FL_FLAG_STALL = 2, FL_FLAG_CHANGED = 3, FL_NUM_FLAGS = 4 };
+enum { FL_FLAG_LAKE = 0, FL_FLAG_DEEP = 1, FL_FLAG_STALL = 2, FL_FLAG_CHANGED = 3, FL_NUM_FLAGS = 4 };
 enum {
   FL_CNT_MAXLD = 0,
   FL_CNT_CHAINS = 1,
@@ -102,7 +102,6 @@ struct fl_dev_work {
   uint32_t* next = nullptr; // [n]
   // lakes
   uint32_t* sub = nullptr;
-  uint32_t* sub2 = nullptr;
   uint64_t* lake_key = nullptr;
   // decomposition
   uint64_t* cmask = nullptr;  // [n] child slots of each site
@@ -168,9 +167,10 @@ extern thread_local uint32_t fl_site_block;
 // cleared by the previous iteration's k_tau_scatter).
 void fl_launch_receivers(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool keep_unchanged,
                          bool mark);
-void fl_launch_sub_init(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w);
-void fl_launch_sub_jump(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool flip);
-void fl_launch_lake_join(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w);
+// Chain ends of the receivers into w.sub, the lakes' keys emptied.
+void fl_launch_sub_labels(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w);
+// Joins the lakes (after fl_launch_sub_labels); few: few sites lie in one.
+void fl_launch_lake_join(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool few);
 // Marks the dirty basins from the final receivers after a lake join (the
 // receivers marked those of their own changes; k_tau_scatter clears the
 // marks for the next iteration).

@@ -280,11 +280,6 @@ __global__ void k_receivers(uint32_t bs, uint32_t n, const uint32_t* __restrict_
 
 // ------------------------------------------------------------ lake join ---
 
-__global__ void k_copy_u32(uint32_t bs, uint32_t n, const uint32_t* __restrict__ src, uint32_t* __restrict__ dst) {
-  uint32_t i = gid(bs);
-  if (i < n) dst[i] = src[i];
-}
-
 __global__ void k_fill_u64(uint32_t bs, uint32_t n, uint64_t* __restrict__ dst, uint64_t v) {
   uint32_t i = gid(bs);
   if (i < n) dst[i] = v;
@@ -295,15 +290,39 @@ __global__ void k_fill_u32(uint32_t bs, uint32_t n, uint32_t* __restrict__ dst, 
   if (i < n) dst[i] = v;
 }
 
-// One pointer-jumping round: out[i] = in[in[i]]; raises *flag if anything moved.
-__global__ void k_sub_jump(uint32_t bs, uint32_t n, const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                           int* __restrict__ flag) {
+// Chain ends of the receiver forest by pointer jumping: four receivers ahead,
+// then rounds in place of three hops (the reach quadruples; a pointer read while
+// its owner rewrites it is an older or a newer one of the same path), then the
+// rest of the way, which is short after enough rounds for the usual path.
+// Nothing is read back in between, so lakes cost no synchronisation (ten of them
+// when every round was checked).  The last kernel empties the lakes' keys.
+__global__ void k_sub_start(uint32_t bs, uint32_t n, const uint32_t* __restrict__ next, uint32_t* __restrict__ sub) {
+  uint32_t i = gid(bs);
+  if (i < n) sub[i] = next[next[next[next[i]]]];
+}
+
+__global__ void k_sub_jump(uint32_t bs, uint32_t n, uint32_t* sub) {
   uint32_t i = gid(bs);
   if (i >= n) return;
-  uint32_t s = in[i];
-  uint32_t ss = in[s];
-  out[i] = ss;
-  if (ss != s) *flag = 1;
+  const uint32_t a = __atomic_load_n(sub + i, __ATOMIC_RELAXED);
+  const uint32_t b = __atomic_load_n(sub + a, __ATOMIC_RELAXED);
+  if (b == a) return;
+  const uint32_t c = __atomic_load_n(sub + b, __ATOMIC_RELAXED);
+  __atomic_store_n(sub + i, __atomic_load_n(sub + c, __ATOMIC_RELAXED), __ATOMIC_RELAXED);
+}
+
+__global__ void k_sub_settle(uint32_t bs, uint32_t n, uint32_t* sub, unsigned long long* __restrict__ key) {
+  uint32_t i = gid(bs);
+  if (i >= n) return;
+  key[i] = ~0ull;
+  const uint32_t a = __atomic_load_n(sub + i, __ATOMIC_RELAXED);
+  uint32_t s = a;
+  for (;;) {
+    const uint32_t t = __atomic_load_n(sub + s, __ATOMIC_RELAXED);
+    if (t == s) break;
+    s = t;
+  }
+  if (s != a) __atomic_store_n(sub + i, s, __ATOMIC_RELAXED);
 }
 
 // For every reached site i and every neighbour j lying in a different
@@ -326,6 +345,28 @@ __global__ void k_lake_keys(uint32_t bs, uint32_t n, const uint32_t* __restrict_
       unsigned long long kv = ((unsigned long long)r << 32) | (unsigned long long)(k - b);
       atomicMin(key + s, kv);
     }
+  }
+}
+
+// The same keys offered from the lakes' side: each site j of a lake looks its
+// neighbours' slots for it up in their rows (rows are symmetric and without
+// duplicates).  For the later iterations, whose lakes are a few sites
+// (k_lake_keys takes 81 us at a million sites for any number of them).
+__global__ void k_lake_offers(uint32_t bs, uint32_t n, const uint32_t* __restrict__ rp,
+                              const uint32_t* __restrict__ col, const uint32_t* __restrict__ rank,
+                              const uint32_t* __restrict__ sub, const uint8_t* __restrict__ is_outlet,
+                              unsigned long long* __restrict__ key) {
+  uint32_t j = gid(bs);
+  if (j >= n) return;
+  const uint32_t s = sub[j];
+  if (is_outlet[s]) return;
+  for (uint32_t k = rp[j]; k < rp[j + 1]; ++k) {
+    const uint32_t i = col[k], r = rank[i];
+    if (r == FL_NONE || sub[i] == s) continue;
+    const uint32_t b = rp[i], e = rp[i + 1];
+    uint32_t x = b;
+    while (x < e && col[x] != j) ++x;
+    if (x < e) atomicMin(key + s, ((unsigned long long)r << 32) | (unsigned long long)(x - b));
   }
 }
 
@@ -2226,19 +2267,22 @@ void fl_launch_receivers(hipStream_t s, const fl_dev_terrain& t, const fl_dev_wo
             mark ? w.dirty : (uint8_t*)nullptr, w.chg);
 }
 
-void fl_launch_sub_init(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w) {
-  FL_LAUNCH(k_copy_u32, t.n, s, t.n, w.next, w.sub);
+void fl_launch_sub_labels(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w) {
+  // rounds until a path of four times sqrt(n) sites is walked
+  uint32_t rounds = 0;
+  for (uint64_t reach = 4; reach * reach < 16ull * t.n; reach *= 4) rounds++;
+  FL_LAUNCH(k_sub_start, t.n, s, t.n, w.next, w.sub);
+  for (uint32_t r = 0; r < rounds; r++) FL_LAUNCH(k_sub_jump, t.n, s, t.n, w.sub);
+  FL_LAUNCH(k_sub_settle, t.n, s, t.n, w.sub, (unsigned long long*)w.lake_key);
 }
 
-void fl_launch_sub_jump(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool flip) {
-  const uint32_t* in = flip ? w.sub2 : w.sub;
-  uint32_t* out = flip ? w.sub : w.sub2;
-  FL_LAUNCH(k_sub_jump, t.n, s, t.n, in, out, w.flags + FL_FLAG_JUMP);
-}
-
-void fl_launch_lake_join(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w) {
-  FL_LAUNCH(k_fill_u64, t.n, s, t.n, w.lake_key, ~0ull);
-  FL_LAUNCH(k_lake_keys, t.n, s, t.n, t.row_ptr, t.col, t.rank, w.sub, t.is_outlet, (unsigned long long*)w.lake_key);
+void fl_launch_lake_join(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool few) {
+  if (few)
+    FL_LAUNCH(k_lake_offers, t.n, s, t.n, t.row_ptr, t.col, t.rank, w.sub, t.is_outlet,
+              (unsigned long long*)w.lake_key);
+  else
+    FL_LAUNCH(k_lake_keys, t.n, s, t.n, t.row_ptr, t.col, t.rank, w.sub, t.is_outlet,
+              (unsigned long long*)w.lake_key);
   FL_LAUNCH(k_lake_flip, t.n, s, t.n, t.row_ptr, t.col, t.len, t.order, (const unsigned long long*)w.lake_key,
             t.is_outlet, w.next, w.dnext);
 }
