@@ -543,7 +543,7 @@ int32_t ensure_visit_order(fl_ctx* c, fl_terrain* T) {
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - p0).count();
     return (int)FL_OK;
   });
-  std::future<int> exact_phase = std::async(std::launch::async, [&]() {
+  std::future<int> exact_phase = std::async(n_exact ? std::launch::async : std::launch::deferred, [&]() {
     if (!n_exact) return (int)FL_OK;
     std::vector<int> rcs(G, FL_OK);
     host_each(
@@ -565,24 +565,14 @@ int32_t ensure_visit_order(fl_ctx* c, fl_terrain* T) {
   int rc_dev = FL_OK;
   if (n_fast) {
     auto p1 = std::chrono::steady_clock::now();
-    std::vector<uint32_t> init(n), base(G);
-    host_parallel(n, 1 << 18, [&](uint64_t a, uint64_t b) {
-      for (uint64_t v = a; v < b; v++) init[v] = (uint32_t)v;
-    });
+    std::vector<uint32_t> labels(G), base(G);
     for (uint32_t g = 0; g < G; g++) {
-      const uint32_t s0 = T->site_off[g], s1 = T->site_off[g + 1];
-      base[g] = s0 + (T->outlet_off[g + 1] - T->outlet_off[g]);
-      if (how[g] == 0) {
-        for (uint32_t q = T->outlet_off[g]; q < T->outlet_off[g + 1]; q++)
-          init[T->h_outlets[q]] = T->h_outlets[T->outlet_off[g]];
-      } else {
-        for (uint32_t v = s0; v < s1; v++) init[v] = s0;
-      }
+      base[g] = T->site_off[g] + (T->outlet_off[g + 1] - T->outlet_off[g]);
+      labels[g] = how[g] == 0 ? T->h_outlets[T->outlet_off[g]] : T->site_off[g] | 0x80000000u;
     }
     fl_visit_stats vs;
-    rc_dev = fl_device_ranks(s, n, T->t.row_ptr, T->t.col, T->t.len, T->t.is_outlet, T->d_tid, init, base,
+    rc_dev = fl_device_ranks(s, n, T->t.row_ptr, T->t.col, T->t.len, T->t.is_outlet, T->d_tid, labels, base,
                              T->t.rank, &vs, &err, &T->arena);
-    // the forest part includes the set-up of its labels on the host
     T->stat_order_parts[1] =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - p1).count() - vs.ranks_ms;
     T->stat_order_parts[2] = vs.ranks_ms;

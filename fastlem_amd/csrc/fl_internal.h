@@ -97,14 +97,15 @@ struct fl_visit_stats {
   double ranks_ms = 0.0;
 };
 // Prim ranks of the traversal after its outlet phase, from the minimum
-// spanning forest of the graph with the sites of each init_comp component
-// (host, n labels: each terrain's outlets share one outlet's label) merged:
+// spanning forest of the graph with the sites of one label merged (labels, one
+// per terrain: the label of its outlets, one of them, or with the top bit set of
+// all of its sites; any other site is its own):
 // every site reached from an outlet through a forest edge gets
 // rank[v] = d_base[tid[v]] + its position in Prim order.  Other entries of
 // `rank` are not written.  Lengths must be positive and pairwise distinct
 // within every component that holds an outlet.
 int fl_device_ranks(hipStream_t s, uint32_t n, const uint32_t* rp, const uint32_t* col, const double* len,
-                    const uint8_t* is_outlet, const uint32_t* tid, const std::vector<uint32_t>& init_comp,
+                    const uint8_t* is_outlet, const uint32_t* tid, const std::vector<uint32_t>& labels,
                     const std::vector<uint32_t>& base, uint32_t* rank, fl_visit_stats* st, std::string* err,
                     fl_arena* arena);
 // dst[idx[q]] = val[q] for the `count` host pairs.

@@ -24,10 +24,10 @@
 // ancestor of v with a heavier parent edge (S, of infinite weight, if none).
 // So the order is the preorder of the tree of q with each site's children
 // taken in increasing weight.  Steps:
-//   1. rooting: an Euler tour of the forest (arcs sorted by source, the
-//      successor of arc u->v the arc after v->u in v's list), cut where it
-//      returns to S, ranked by pointer jumping; of the two arcs of an edge
-//      the earlier one points away from S;
+//   1. rooting: an Euler tour of the forest (arcs in lists by source, in any
+//      order, the successor of arc u->v the arc after v->u in v's list), cut
+//      where it returns to S, ranked by pointer jumping; of the two arcs of an
+//      edge the earlier one points away from S;
 //   2. q by pointer jumping: while w(q(v)) < w(v), q(v) <- q(q(v)) (every
 //      site skipped is lighter than q(v), hence lighter than v);
 //   3. the children of each q-tree site in increasing weight: the forest's
@@ -35,6 +35,10 @@
 //      them;
 //   4. preorder: an Euler tour of the q-tree ranked by pointer jumping,
 //      counting the down steps from the tour's start.
+// What bounds it is the number of short launches and of read-backs: pointers
+// jump three hops a round, a fixed number of rounds for the usual (or, in a list
+// ranking, for any) path, the next kernel hops the rest of the way, and only the
+// forest's rounds are counted on the host, from where they usually end.
 // The outlet phase (host, fl_outlet_pop_order) ranks the outlets; terrains
 // whose lengths repeat or are not positive are ranked by the exact heap
 // simulation on the host (fl_lake_visit_order).
@@ -52,6 +56,8 @@
 #define FL_NONE 0xffffffffu
 
 namespace {
+
+constexpr uint32_t kMaxFlags = 256;
 
 // Workgroup b runs on XCD b % 8; each XCD takes one contiguous eighth of the
 // index range (a bijection of [0, gridDim.x)), so neighbouring sites share an L2.
@@ -130,11 +136,21 @@ __global__ void k_len_check(uint32_t n, const uint32_t* __restrict__ rp, const u
 
 // ------------------------------------------------------------- Boruvka ----
 
-__global__ void k_bv_init(uint32_t n, const uint32_t* __restrict__ init_comp, uint32_t* __restrict__ comp,
-                          unsigned long long* __restrict__ cbest) {
+// The labels that the forest starts from: a terrain's outlets share one (meta:
+// the ranks before its first other site, then the label of its outlets, the top
+// bit set when the whole terrain has it).
+#define FL_WHOLE 0x80000000u
+__global__ void k_bv_init(uint32_t n, uint32_t G, const uint32_t* __restrict__ meta, const uint32_t* __restrict__ tid,
+                          const uint8_t* __restrict__ is_outlet, uint32_t* __restrict__ icomp,
+                          uint32_t* __restrict__ comp, unsigned long long* __restrict__ cbest,
+                          uint32_t* __restrict__ flags) {
   uint32_t v = gid();
+  if (v < kMaxFlags) flags[v] = 0;
   if (v >= n) return;
-  comp[v] = init_comp[v];
+  const uint32_t l = meta[G + (tid ? tid[v] : 0u)];
+  const uint32_t c = (l & FL_WHOLE) || is_outlet[v] ? l & ~FL_WHOLE : v;
+  icomp[v] = c;
+  comp[v] = c;
   cbest[v] = ~0ull;
 }
 
@@ -201,7 +217,8 @@ __global__ void k_bv_hook(uint32_t n, const uint32_t* __restrict__ col, const ui
                           const unsigned long long* __restrict__ cbest, const uint32_t* __restrict__ cedge,
                           const uint32_t* __restrict__ csrc, uint32_t* __restrict__ parent,
                           uint32_t* __restrict__ msf_a, uint32_t* __restrict__ msf_b,
-                          unsigned long long* __restrict__ msf_w, uint32_t* __restrict__ count) {
+                          unsigned long long* __restrict__ msf_w, uint32_t* __restrict__ msf_i,
+                          uint32_t* __restrict__ count, uint32_t* __restrict__ hooked) {
   uint32_t c = gid();
   bool hook = false;
   uint32_t e = 0, t = 0;
@@ -222,58 +239,60 @@ __global__ void k_bv_hook(uint32_t n, const uint32_t* __restrict__ col, const ui
   if (m == 0) return;
   const uint32_t lane = threadIdx.x & 63u, leader = (uint32_t)__builtin_ctzll(m);
   uint32_t base = 0;
-  if (lane == leader) base = atomicAdd(count, (uint32_t)__builtin_popcountll(m));
+  if (lane == leader) {
+    base = atomicAdd(count, (uint32_t)__builtin_popcountll(m));
+    *hooked = 1;
+  }
   base = __builtin_amdgcn_readlane(base, leader);
   if (hook) {
     const uint32_t slot = base + (uint32_t)__builtin_popcountll(m & ((1ull << lane) - 1ull));
     msf_a[slot] = csrc[c];
     msf_b[slot] = col[e];
     msf_w[slot] = w;
+    msf_i[slot] = slot;
   }
 }
 
-// One in-place doubling round on the hook pointers; a round after one that
-// moved nothing returns at once.  A pointer read while its owner rewrites it
-// is its old or its new value (aligned 32-bit accesses are single-copy
-// atomic), both ancestors on the same hook path.
-__global__ void k_bv_jump(uint32_t n, uint32_t* parent, uint32_t* __restrict__ flag_set,
-                          const uint32_t* __restrict__ prev_flag) {
-  if (prev_flag && *prev_flag == 0) return;
+// One in-place round of three hops on the hook pointers.  A pointer read while
+// its owner rewrites it is its old or its new value (aligned 32-bit accesses are
+// single-copy atomic), both ancestors on the same hook path.
+__global__ void k_bv_jump(uint32_t n, uint32_t* parent) {
   uint32_t c = gid();
-  bool moved = false;
-  if (c < n) {
-    uint32_t p = __atomic_load_n(parent + c, __ATOMIC_RELAXED);
-    uint32_t pp = __atomic_load_n(parent + p, __ATOMIC_RELAXED);
-    if (pp != p) {
-      __atomic_store_n(parent + c, pp, __ATOMIC_RELAXED);
-      moved = true;
-    }
-  }
-  if (__any(moved) && (threadIdx.x & 63u) == 0) *flag_set = 1;
+  if (c >= n) return;
+  const uint32_t p = __atomic_load_n(parent + c, __ATOMIC_RELAXED);
+  const uint32_t p2 = __atomic_load_n(parent + p, __ATOMIC_RELAXED);
+  if (p2 == p) return;
+  const uint32_t p3 = __atomic_load_n(parent + p2, __ATOMIC_RELAXED);
+  __atomic_store_n(parent + c, __atomic_load_n(parent + p3, __ATOMIC_RELAXED), __ATOMIC_RELAXED);
 }
 
+// The components' new labels, the rest of the way along the hooks.
 __global__ void k_bv_relabel(uint32_t n, const uint32_t* __restrict__ parent, uint32_t* __restrict__ comp,
                              unsigned long long* __restrict__ cbest) {
   uint32_t v = gid();
   if (v >= n) return;
-  comp[v] = parent[comp[v]];
+  uint32_t c = parent[comp[v]];
+  for (;;) {
+    const uint32_t p = parent[c];
+    if (p == c) break;
+    c = p;
+  }
+  comp[v] = c;
   cbest[v] = ~0ull;
 }
 
-__global__ void k_iota(uint32_t m, uint32_t* __restrict__ out) {
-  uint32_t i = gid();
-  if (i < m) out[i] = i;
-}
-
-__global__ void k_gather_pairs(uint32_t m, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ a,
-                               const uint32_t* __restrict__ b, uint32_t* __restrict__ a2, uint32_t* __restrict__ b2) {
-  uint32_t i = gid();
-  if (i >= m) return;
-  a2[i] = a[idx[i]];
-  b2[i] = b[idx[i]];
-}
-
 // ------------------------------------------------- ranks from the forest ----
+
+// Cleared lists; S (every outlet label) is heavier than any edge.
+__global__ void k_rank_init(uint32_t n, uint8_t* __restrict__ reached, uint32_t* __restrict__ head,
+                            uint32_t* __restrict__ wt, uint32_t* __restrict__ fch) {
+  uint32_t v = gid();
+  if (v >= n) return;
+  reached[v] = 0;
+  head[v] = FL_NONE;
+  wt[v] = FL_NONE;
+  fch[v] = FL_NONE;
+}
 
 // Components holding an outlet are reached by the traversal.
 __global__ void k_mark_reached(uint32_t n, const uint8_t* __restrict__ is_outlet, const uint32_t* __restrict__ comp,
@@ -282,56 +301,62 @@ __global__ void k_mark_reached(uint32_t n, const uint8_t* __restrict__ is_outlet
   if (v < n && is_outlet[v]) reached[comp[v]] = 1;
 }
 
-// The two arcs of forest edge j (in length order) keyed by their source's
-// label (an outlet's label is its terrain's S); edges of unreached
-// components get the key FL_NONE and sort last.
-__global__ void k_arcs(uint32_t m, const uint32_t* __restrict__ a2, const uint32_t* __restrict__ b2,
+// The two arcs 2 j, 2 j + 1 of forest edge j (those of reached components)
+// linked into the lists of their sources' labels (an outlet's label is its
+// terrain's S).  S may have a hundred thousand arcs: a wavefront's arcs from one
+// S are linked to each other and join its list with one exchange.
+__global__ void k_arcs(uint32_t m, const uint32_t* __restrict__ ma, const uint32_t* __restrict__ mb,
                        const uint32_t* __restrict__ icomp, const uint32_t* __restrict__ comp,
-                       const uint8_t* __restrict__ reached, uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
-  uint32_t j = gid();
-  if (j >= m) return;
-  const uint32_t a = a2[j], b = b2[j];
-  const bool ok = reached[comp[a]] != 0;
-  key[2 * j] = ok ? icomp[a] : FL_NONE;
-  key[2 * j + 1] = ok ? icomp[b] : FL_NONE;
-  val[2 * j] = 2 * j;
-  val[2 * j + 1] = 2 * j + 1;
-}
-
-// Position of every arc in source order, and the first position of every
-// source's list.
-__global__ void k_arc_pos(uint32_t M, const uint32_t* __restrict__ skey, const uint32_t* __restrict__ sarc,
-                          uint32_t* __restrict__ pos, uint32_t* __restrict__ start) {
-  uint32_t p = gid();
-  if (p >= M) return;
-  pos[sarc[p]] = p;
-  const uint32_t u = skey[p];
-  if (u != FL_NONE && (p == 0 || skey[p - 1] != u)) start[u] = p;
-}
-
-// Euler-tour successor of the arc at position p (u->v): the arc after v->u
-// in v's list, cyclically; the tour is cut where it would start S's list
-// again.  Element p = (successor position or FL_NONE, 1).
-__global__ void k_arc_tour(uint32_t M, const uint32_t* __restrict__ skey, const uint32_t* __restrict__ sarc,
-                           const uint32_t* __restrict__ pos, const uint32_t* __restrict__ start,
-                           const uint8_t* __restrict__ is_outlet, unsigned long long* __restrict__ tour) {
-  uint32_t p = gid();
-  if (p >= M) return;
-  if (skey[p] == FL_NONE) {
-    tour[p] = pr(FL_NONE, 1u);
-    return;
+                       const uint8_t* __restrict__ reached, const uint8_t* __restrict__ is_outlet,
+                       uint32_t* __restrict__ head, uint32_t* __restrict__ anext) {
+  const uint32_t a = gid(), j = a >> 1, lane = threadIdx.x & 63u;
+  uint32_t src = FL_NONE;
+  bool many = false;
+  if (j < m && reached[comp[ma[j]]]) {
+    src = icomp[(a & 1u) ? mb[j] : ma[j]];
+    many = is_outlet[src] != 0;
   }
-  const uint32_t t = pos[sarc[p] ^ 1u];
-  const uint32_t v = skey[t];
-  const bool last = !(t + 1 < M && skey[t + 1] == v);
-  uint32_t nx = last ? start[v] : t + 1;
-  if (last && is_outlet[v]) nx = FL_NONE;  // back at S after its last arc
-  tour[p] = pr(nx, 1u);
+  if (src != FL_NONE && !many) anext[a] = atomicExch(head + src, a);
+  unsigned long long left = __ballot(many);
+  while (left) {
+    const uint32_t first = (uint32_t)__builtin_ctzll(left);
+    const uint32_t S = (uint32_t)__builtin_amdgcn_readlane((int)src, (int)first);
+    const unsigned long long same = __ballot(many && src == S);
+    const uint32_t last = 63u - (uint32_t)__builtin_clzll(same);
+    // each lane's arc points to the next lane's, the last one's to the list
+    if (many && src == S) {
+      const unsigned long long after = same & ~(~0ull >> (63u - lane));
+      if (lane != last) anext[a] = a - lane + (uint32_t)__builtin_ctzll(after);
+    }
+    if (lane == last) anext[a] = atomicExch(head + S, a - lane + first);
+    left &= ~same;
+  }
 }
 
-// One in-place doubling round of a list ranking over elements [0, M) (or the
-// elements of the children list, see k_qtour_jump): (p, c) <- (p', c + c') with
-// (p', c') the pair of p; FL_NONE ends a list.  Pairs read while their owner
+// Euler-tour successor of arc a (u->v): the arc after v->u in v's list,
+// cyclically; the tour is cut where it would start S's list again.  Element a =
+// (successor or FL_NONE, 1).
+__global__ void k_arc_tour(uint32_t m, const uint32_t* __restrict__ ma, const uint32_t* __restrict__ mb,
+                           const uint32_t* __restrict__ icomp, const uint32_t* __restrict__ comp,
+                           const uint8_t* __restrict__ reached, const uint32_t* __restrict__ head,
+                           const uint32_t* __restrict__ anext, const uint8_t* __restrict__ is_outlet,
+                           unsigned long long* __restrict__ tour) {
+  const uint32_t a = gid(), j = a >> 1;
+  if (j >= m) return;
+  uint32_t nx = FL_NONE;
+  if (reached[comp[ma[j]]]) {
+    nx = anext[a ^ 1u];
+    if (nx == FL_NONE) {
+      const uint32_t v = icomp[(a & 1u) ? ma[j] : mb[j]];
+      if (!is_outlet[v]) nx = head[v];  // (else back at S after its last arc)
+    }
+  }
+  tour[a] = pr(nx, 1u);
+}
+
+// One in-place round of a list ranking over elements [0, M) (or the elements of
+// the children list, see k_qtour_jump): (p, c) <- (p', c + c') with (p', c') the
+// pair of p, three times over (the reach quadruples); FL_NONE ends a list.  Pairs read while their owner
 // rewrites them are old or new values of the same list, both valid (aligned
 // 64-bit accesses are single-copy atomic).
 __global__ void k_list_jump(uint32_t M, unsigned long long* list, uint32_t* __restrict__ flag_set,
@@ -343,15 +368,13 @@ __global__ void k_list_jump(uint32_t M, unsigned long long* list, uint32_t* __re
     unsigned long long x = __atomic_load_n(list + p, __ATOMIC_RELAXED);
     uint32_t nx = pr_ptr(x);
     if (nx != FL_NONE) {
-      // two hops: (p'', c + c' + c''), the reach triples per round
-      unsigned long long y = __atomic_load_n(list + nx, __ATOMIC_RELAXED);
-      const uint32_t ny = pr_ptr(y);
-      if (ny != FL_NONE) {
-        unsigned long long z = __atomic_load_n(list + ny, __ATOMIC_RELAXED);
-        __atomic_store_n(list + p, pr(pr_ptr(z), pr_cnt(x) + pr_cnt(y) + pr_cnt(z)), __ATOMIC_RELAXED);
-      } else {
-        __atomic_store_n(list + p, pr(FL_NONE, pr_cnt(x) + pr_cnt(y)), __ATOMIC_RELAXED);
+      uint32_t cnt = pr_cnt(x);
+      for (int hop = 0; hop < 3 && nx != FL_NONE; ++hop) {
+        const unsigned long long y = __atomic_load_n(list + nx, __ATOMIC_RELAXED);
+        cnt += pr_cnt(y);
+        nx = pr_ptr(y);
       }
+      __atomic_store_n(list + p, pr(nx, cnt), __ATOMIC_RELAXED);
       moved = true;
     }
   }
@@ -415,68 +438,77 @@ __global__ void k_st_size(uint32_t n, const uint32_t* __restrict__ next, const u
   size[v] = (double)((a - b + 1u) / 2u);
 }
 
-// Parent and weight of every forest site: of an edge's two arcs the one
-// earlier in the tour (more arcs after it) points away from S.  The weight
-// is the edge's position in length order; S weighs FL_NONE (infinite).
-__global__ void k_edge_dir(uint32_t m, const uint32_t* __restrict__ a2, const uint32_t* __restrict__ b2,
-                           const uint32_t* __restrict__ icomp, const uint32_t* __restrict__ key,
-                           const uint32_t* __restrict__ pos, const unsigned long long* __restrict__ tour,
-                           uint32_t* __restrict__ child, uint32_t* __restrict__ par, uint32_t* __restrict__ wt) {
+// Parent and weight of every forest site, edges in length order (edge j of it
+// is slot idx[j]): of an edge's two arcs the one earlier in the tour (more arcs
+// after it) points away from S.  The weight is the edge's position in length
+// order; S weighs FL_NONE (infinite).  q starts as the parent.
+__global__ void k_edge_dir(uint32_t m, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ ma,
+                           const uint32_t* __restrict__ mb, const uint32_t* __restrict__ icomp,
+                           const uint32_t* __restrict__ comp, const uint8_t* __restrict__ reached,
+                           const unsigned long long* __restrict__ tour, uint32_t* __restrict__ child,
+                           uint32_t* __restrict__ q, uint32_t* __restrict__ wt) {
   uint32_t j = gid();
   if (j >= m) return;
-  if (key[2 * j] == FL_NONE) {
+  const uint32_t e = idx[j], a = ma[e], b = mb[e];
+  if (!reached[comp[a]]) {
     child[j] = FL_NONE;
     return;
   }
-  const uint32_t da = pr_cnt(tour[pos[2 * j]]), db = pr_cnt(tour[pos[2 * j + 1]]);
-  const uint32_t c = da > db ? b2[j] : a2[j];
-  const uint32_t p = da > db ? icomp[a2[j]] : icomp[b2[j]];
+  const uint32_t da = pr_cnt(tour[2ull * e]), db = pr_cnt(tour[2ull * e + 1]);
+  const uint32_t c = da > db ? b : a;
   child[j] = c;
-  par[c] = p;
+  q[c] = da > db ? icomp[a] : icomp[b];
   wt[c] = j;
 }
 
-// q(c) <- q(q(c)) while q(c) is lighter than c, in place (a value read while
-// being rewritten is an older or newer pointer of the same site, both valid).
-__global__ void k_q_jump(uint32_t m, const uint32_t* __restrict__ child, const uint32_t* __restrict__ wt,
-                         uint32_t* q, uint32_t* __restrict__ flag_set, const uint32_t* __restrict__ prev_flag) {
+// q(c) <- q(q(c)) while q(c) is lighter than c, up to three steps a round, in
+// place (a value read while being rewritten is an older or newer pointer of the
+// same site, both valid).
+__global__ void k_q_jump(uint32_t m, const uint32_t* __restrict__ child, const uint32_t* __restrict__ wt, uint32_t* q,
+                         uint32_t* __restrict__ flag_set, const uint32_t* __restrict__ prev_flag) {
   if (prev_flag && *prev_flag == 0) return;
   uint32_t j = gid();
   bool moved = false;
   if (j < m) {
     const uint32_t c = child[j];
     if (c != FL_NONE) {
-      const uint32_t qc = __atomic_load_n(q + c, __ATOMIC_RELAXED);
-      if (wt[qc] < j) {
-        // up to two steps a round: past qc, and past its q when that is
-        // lighter too
-        const uint32_t q2 = __atomic_load_n(q + qc, __ATOMIC_RELAXED);
-        const uint32_t q3 = wt[q2] < j ? __atomic_load_n(q + q2, __ATOMIC_RELAXED) : q2;
-        __atomic_store_n(q + c, q3, __ATOMIC_RELAXED);
+      uint32_t qc = __atomic_load_n(q + c, __ATOMIC_RELAXED);
+      for (int step = 0; step < 3 && wt[qc] < j; ++step) {
+        qc = __atomic_load_n(q + qc, __ATOMIC_RELAXED);
         moved = true;
       }
+      if (moved) __atomic_store_n(q + c, qc, __ATOMIC_RELAXED);
     }
   }
   if (__any(moved) && (threadIdx.x & 63u) == 0) *flag_set = 1;
 }
 
-// The q-tree's children, keyed by their q, in increasing weight (edge order).
-__global__ void k_q_keys(uint32_t m, const uint32_t* __restrict__ child, const uint32_t* __restrict__ q,
-                         uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
+// The q-tree's children, keyed by their q (`none` for unreached ones), in
+// increasing weight (edge order); q the rest of the way.
+__global__ void k_q_keys(uint32_t m, uint32_t none, const uint32_t* __restrict__ child,
+                         const uint32_t* __restrict__ wt, uint32_t* q, uint32_t* __restrict__ key,
+                         uint32_t* __restrict__ val) {
   uint32_t j = gid();
   if (j >= m) return;
   const uint32_t c = child[j];
-  key[j] = c == FL_NONE ? FL_NONE : q[c];
+  uint32_t qc = none;
+  if (c != FL_NONE) {
+    const uint32_t q0 = __atomic_load_n(q + c, __ATOMIC_RELAXED);
+    qc = q0;
+    while (wt[qc] < j) qc = __atomic_load_n(q + qc, __ATOMIC_RELAXED);
+    if (qc != q0) __atomic_store_n(q + c, qc, __ATOMIC_RELAXED);
+  }
+  key[j] = qc;
   val[j] = c;
 }
 
 // First child of every q-tree site and next sibling of every child.
-__global__ void k_q_links(uint32_t m, const uint32_t* __restrict__ qs, const uint32_t* __restrict__ cs,
+__global__ void k_q_links(uint32_t m, uint32_t none, const uint32_t* __restrict__ qs, const uint32_t* __restrict__ cs,
                           uint32_t* __restrict__ fch, uint32_t* __restrict__ nsib) {
   uint32_t p = gid();
   if (p >= m) return;
   const uint32_t u = qs[p];
-  if (u == FL_NONE) return;
+  if (u == none) return;
   const uint32_t c = cs[p];
   if (p == 0 || qs[p - 1] != u) fch[u] = c;
   nsib[c] = (p + 1 < m && qs[p + 1] == u) ? cs[p + 1] : FL_NONE;
@@ -492,7 +524,7 @@ __global__ void k_q_tour(uint32_t m, uint32_t n, const uint32_t* __restrict__ qs
                          const uint32_t* __restrict__ nsib, const uint8_t* __restrict__ is_outlet,
                          unsigned long long* __restrict__ qt) {
   uint32_t p = gid();
-  if (p < m && qs[p] != FL_NONE) {
+  if (p < m && qs[p] != n) {
     const uint32_t c = cs[p];
     const uint32_t f = fch[c];
     const uint32_t s1 = f != FL_NONE ? 2 * f : 2 * c + 1;  // after entering c
@@ -510,26 +542,24 @@ __global__ void k_q_tour(uint32_t m, uint32_t n, const uint32_t* __restrict__ qs
 
 // As k_list_jump over the tour elements of the children (element 2c + b of
 // child cs[p / 2], b = p & 1).
-__global__ void k_qtour_jump(uint32_t M, const uint32_t* __restrict__ qs, const uint32_t* __restrict__ cs,
+__global__ void k_qtour_jump(uint32_t M, uint32_t none, const uint32_t* __restrict__ qs, const uint32_t* __restrict__ cs,
                              unsigned long long* qt, uint32_t* __restrict__ flag_set,
                              const uint32_t* __restrict__ prev_flag) {
   if (prev_flag && *prev_flag == 0) return;
   uint32_t p = gid();
   bool moved = false;
-  if (p < M && qs[p >> 1] != FL_NONE) {
+  if (p < M && qs[p >> 1] != none) {
     const uint32_t e = 2 * cs[p >> 1] + (p & 1u);
     unsigned long long x = __atomic_load_n(qt + e, __ATOMIC_RELAXED);
     uint32_t nx = pr_ptr(x);
     if (nx != FL_NONE) {
-      // two hops, as k_list_jump
-      unsigned long long y = __atomic_load_n(qt + nx, __ATOMIC_RELAXED);
-      const uint32_t ny = pr_ptr(y);
-      if (ny != FL_NONE) {
-        unsigned long long z = __atomic_load_n(qt + ny, __ATOMIC_RELAXED);
-        __atomic_store_n(qt + e, pr(pr_ptr(z), pr_cnt(x) + pr_cnt(y) + pr_cnt(z)), __ATOMIC_RELAXED);
-      } else {
-        __atomic_store_n(qt + e, pr(FL_NONE, pr_cnt(x) + pr_cnt(y)), __ATOMIC_RELAXED);
+      uint32_t cnt = pr_cnt(x);
+      for (int hop = 0; hop < 3 && nx != FL_NONE; ++hop) {
+        const unsigned long long y = __atomic_load_n(qt + nx, __ATOMIC_RELAXED);
+        cnt += pr_cnt(y);
+        nx = pr_ptr(y);
       }
+      __atomic_store_n(qt + e, pr(nx, cnt), __ATOMIC_RELAXED);
       moved = true;
     }
   }
@@ -538,11 +568,11 @@ __global__ void k_qtour_jump(uint32_t M, const uint32_t* __restrict__ qs, const 
 
 // rank(c) = its terrain's first non-outlet rank + its preorder position
 // (down steps from the tour's start up to c's, minus one).
-__global__ void k_q_rank(uint32_t m, const uint32_t* __restrict__ qs, const uint32_t* __restrict__ cs,
+__global__ void k_q_rank(uint32_t m, uint32_t none, const uint32_t* __restrict__ qs, const uint32_t* __restrict__ cs,
                          const unsigned long long* __restrict__ qt, const uint32_t* __restrict__ tid,
                          const uint32_t* __restrict__ base, uint32_t* __restrict__ rank) {
   uint32_t p = gid();
-  if (p >= m || qs[p] == FL_NONE) return;
+  if (p >= m || qs[p] == none) return;
   const uint32_t c = cs[p];
   rank[c] = base[tid ? tid[c] : 0u] + pr_cnt(qt[2 * c]) - 1u;
 }
@@ -595,47 +625,46 @@ uint64_t len_tables(uint32_t G, const uint32_t* entry_off, std::vector<uint32_t>
   return total;
 }
 
-// Rounds of pointer jumping per host check.
-constexpr uint32_t kJumpBatch = 8;
-constexpr uint32_t kMaxFlags = 256;
+// One word per round: "hooked" of the forest's, "moved" of the three rankings'.
+constexpr uint32_t kMaxRounds = 64;
 
 // The forest and rank buffers of fl_device_ranks (n sites): allocated from
 // `buf`, also in a COUNT arena for sizing.
 struct RankBufs {
-  uint32_t *comp, *parent, *vbest, *cedge, *csrc, *ma, *mb, *icomp, *idx, *idx2, *a2, *b2, *flags;
+  uint32_t *comp, *parent, *vbest, *cedge, *csrc, *ma, *mb, *icomp, *idx, *idx2, *flags;
   unsigned long long *cbest, *mw, *mw2;
   uint8_t* reached;
-  uint32_t *key, *val, *skey, *sarc, *pos, *start;
+  uint32_t *head, *anext;
   unsigned long long* tour;
-  uint32_t *child, *par, *wt, *q, *qk, *qv, *qs, *cs, *fch, *nsib;
+  uint32_t *child, *wt, *q, *qk, *qv, *qs, *cs, *fch, *nsib;
   unsigned long long* qt;
   void *tmp1, *tmp2;
   size_t tmp1_bytes = 0, tmp2_bytes = 0;
 };
 
+// Bits of the sort keys of n sites and n itself.
+int key_bits(uint32_t n) { return 32 - __builtin_clz(n | 1u); }
+
 hipError_t rank_bufs(DevBuf& buf, uint32_t n, RankBufs& r) {
   hipError_t e;
   const uint64_t N4 = (uint64_t)n * 4, N8 = (uint64_t)n * 8;
   for (uint32_t** p : {&r.comp, &r.parent, &r.vbest, &r.cedge, &r.csrc, &r.ma, &r.mb, &r.icomp, &r.idx, &r.idx2,
-                       &r.a2, &r.b2, &r.start, &r.child, &r.par, &r.wt, &r.q, &r.qk, &r.qv, &r.qs, &r.cs, &r.fch,
-                       &r.nsib})
+                       &r.head, &r.child, &r.wt, &r.q, &r.qk, &r.qv, &r.qs, &r.cs, &r.fch, &r.nsib})
     if ((e = buf.alloc((void**)p, N4)) != hipSuccess) return e;
-  for (uint32_t** p : {&r.key, &r.val, &r.skey, &r.sarc, &r.pos})
-    if ((e = buf.alloc((void**)p, 2 * N4)) != hipSuccess) return e;
+  if ((e = buf.alloc((void**)&r.anext, 2 * N4)) != hipSuccess) return e;
   for (unsigned long long** p : {&r.cbest, &r.mw, &r.mw2})
     if ((e = buf.alloc((void**)p, N8)) != hipSuccess) return e;
   for (unsigned long long** p : {&r.tour, &r.qt})
     if ((e = buf.alloc((void**)p, 2 * N8)) != hipSuccess) return e;
   if ((e = buf.alloc((void**)&r.reached, (uint64_t)n + 16)) != hipSuccess) return e;
-  if ((e = buf.alloc((void**)&r.flags, kMaxFlags * 4)) != hipSuccess) return e;
-  // radix sort scratch: edges by length (64-bit keys), arcs by source and
-  // children by q (32-bit keys, up to 2n items)
+  if ((e = buf.alloc((void**)&r.flags, (kMaxFlags + 1) * 4)) != hipSuccess) return e;
+  // radix sort scratch: edges by length (64-bit keys) and children by q
   const int items = n > 0 ? (int)n : 1;
   if ((e = hipcub::DeviceRadixSort::SortPairs(nullptr, r.tmp1_bytes, r.mw, r.mw2, r.idx, r.idx2, items, 0, 64,
                                               buf.s)) != hipSuccess)
     return e;
-  if ((e = hipcub::DeviceRadixSort::SortPairs(nullptr, r.tmp2_bytes, r.key, r.skey, r.val, r.sarc, 2 * items, 0,
-                                              32, buf.s)) != hipSuccess)
+  if ((e = hipcub::DeviceRadixSort::SortPairs(nullptr, r.tmp2_bytes, r.qk, r.qs, r.qv, r.cs, items, 0, key_bits(n),
+                                              buf.s)) != hipSuccess)
     return e;
   if ((e = buf.alloc(&r.tmp1, r.tmp1_bytes)) != hipSuccess) return e;
   if ((e = buf.alloc(&r.tmp2, r.tmp2_bytes)) != hipSuccess) return e;
@@ -651,30 +680,17 @@ uint64_t rank_scratch_bytes(uint32_t n, uint64_t G) {
     RankBufs r;
     rank_bufs(buf, n, r);
     void* p;
-    buf.alloc(&p, 4 * G);
+    buf.alloc(&p, 8 * G);
   }
   return a.peak;
 }
 
-// Pointer-jumping rounds launched `batch` at a time, each flagging movement
-// in its own word of r.flags (cleared beforehand); returns after the first
-// batch whose last round moved nothing, or an error past kMaxFlags rounds.
-template <class Launch>
-int jump_to_fixpoint(hipStream_t s, uint32_t* d_flags, uint32_t nflags, uint32_t first_batch, Launch launch,
-                     std::string* err, const char* what) {
-  uint32_t h[kMaxFlags];
-  uint32_t round = 0, target = first_batch;
-  for (;;) {
-    if (target > nflags) {
-      *err = std::string(what) + " did not converge";
-      return FL_ERR_HIP;
-    }
-    for (; round < target; round++) launch(d_flags + round, round ? d_flags + round - 1 : nullptr);
-    HIPTRY(hipMemcpyAsync(h, d_flags, round * 4, hipMemcpyDeviceToHost, s));
-    HIPTRY(hipStreamSynchronize(s));
-    if (h[round - 1] == 0) return FL_OK;
-    target = round + kJumpBatch;
-  }
+// Rounds of three hops after which every pointer of a list of L elements has
+// reached its end.
+uint32_t list_rounds(uint64_t L) {
+  uint32_t rounds = 1;
+  for (uint64_t reach = 4; reach < L; reach *= 4) rounds++;
+  return rounds;
 }
 
 }  // namespace
@@ -698,7 +714,7 @@ uint64_t fl_msf_scratch_bytes(uint32_t n, uint32_t nnz) {
     RankBufs r;
     rank_bufs(buf, n, r);
     void* p;
-    buf.alloc(&p, 4ull * (n + 1));  // terrain bases
+    buf.alloc(&p, 8ull * (n + 1));  // terrain bases and labels
   }
   uint64_t ranks = a.peak, scatter = fl_round256(8ull * (n + 1));
   uint64_t peak = check > ranks ? check : ranks;
@@ -733,50 +749,55 @@ int fl_device_len_check(hipStream_t s, uint32_t n, const uint32_t* rp, const uin
 }
 
 int fl_device_ranks(hipStream_t s, uint32_t n, const uint32_t* rp, const uint32_t* col, const double* len,
-                    const uint8_t* is_outlet, const uint32_t* tid, const std::vector<uint32_t>& init_comp,
+                    const uint8_t* is_outlet, const uint32_t* tid, const std::vector<uint32_t>& labels,
                     const std::vector<uint32_t>& base, uint32_t* rank, fl_visit_stats* st, std::string* err,
                     fl_arena* arena) {
   if (n == 0) return FL_OK;
   auto t0 = std::chrono::steady_clock::now();
   DevBuf buf(s, arena);
-  HIPTRY(buf.reserve(rank_scratch_bytes(n, base.size())));
+  const uint32_t G = (uint32_t)base.size();
+  HIPTRY(buf.reserve(rank_scratch_bytes(n, G)));
   RankBufs r;
   HIPTRY(rank_bufs(buf, n, r));
-  uint32_t* d_base = nullptr;
-  HIPTRY(buf.alloc((void**)&d_base, base.size() * 4));
+  uint32_t* d_meta = nullptr;
+  HIPTRY(buf.alloc((void**)&d_meta, 8ull * G));
+  std::vector<uint32_t> meta(base);
+  meta.insert(meta.end(), labels.begin(), labels.end());
   const dim3 B(256), Gn = grid_for(n);
-  HIPTRY(hipMemcpyAsync(d_base, base.data(), base.size() * 4, hipMemcpyHostToDevice, s));
-  HIPTRY(hipMemcpyAsync(r.icomp, init_comp.data(), (size_t)n * 4, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_fill32, dim3(1), B, 0, s, kMaxFlags, r.flags, 0u);
-  hipLaunchKernelGGL(k_bv_init, Gn, B, 0, s, n, r.icomp, r.comp, r.cbest);
-  // Boruvka: one host check per round
-  uint32_t m = 0, h_count = 0;
-  for (uint32_t round = 0;; ++round) {
-    if (round > 64) {
+  HIPTRY(hipMemcpyAsync(d_meta, meta.data(), meta.size() * 4, hipMemcpyHostToDevice, s));
+  // flags: the edge count, "hooked" of every forest round, "moved" of the
+  // rankings' rounds
+  uint32_t* hooked = r.flags + 1;
+  hipLaunchKernelGGL(k_bv_init, grid_for(n > kMaxFlags ? n : kMaxFlags), B, 0, s, n, G, d_meta, tid, is_outlet,
+                     r.icomp, r.comp, r.cbest, r.flags);
+  // Boruvka: a forest takes at least a third of log2(n) rounds as a rule (a
+  // round after the last one hooks nothing); each round past them is looked at
+  uint32_t lg = 1;
+  while (lg < 31 && (1u << lg) < n) lg++;
+  uint32_t m = 0, target = lg / 3 + 2;
+  for (uint32_t round = 0;;) {
+    if (target > kMaxRounds) {
       *err = "minimum spanning forest did not converge";
       return FL_ERR_HIP;
     }
-    hipLaunchKernelGGL(k_fill32, dim3(1), B, 0, s, kMaxFlags - 1, r.flags + 1, 0u);
-    hipLaunchKernelGGL(k_bv_best, Gn, B, 0, s, n, rp, col, len, r.comp, r.cbest, r.vbest);
-    hipLaunchKernelGGL(k_bv_pick, Gn, B, 0, s, n, len, r.comp, r.cbest, r.vbest, r.cedge, r.csrc);
-    hipLaunchKernelGGL(k_bv_hook, Gn, B, 0, s, n, col, r.comp, r.cbest, r.cedge, r.csrc, r.parent, r.ma, r.mb, r.mw,
-                       r.flags);
-    int rc = jump_to_fixpoint(
-        s, r.flags + 1, kMaxFlags - 1, 4,
-        [&](uint32_t* fset, const uint32_t* prev) {
-          hipLaunchKernelGGL(k_bv_jump, Gn, B, 0, s, n, r.parent, fset, prev);
-        },
-        err, "forest hooking");
-    if (rc != FL_OK) return rc;
-    hipLaunchKernelGGL(k_bv_relabel, Gn, B, 0, s, n, r.parent, r.comp, r.cbest);
-    HIPTRY(hipMemcpyAsync(&h_count, r.flags, 4, hipMemcpyDeviceToHost, s));
+    for (; round < target; round++) {
+      hipLaunchKernelGGL(k_bv_best, Gn, B, 0, s, n, rp, col, len, r.comp, r.cbest, r.vbest);
+      hipLaunchKernelGGL(k_bv_pick, Gn, B, 0, s, n, len, r.comp, r.cbest, r.vbest, r.cedge, r.csrc);
+      hipLaunchKernelGGL(k_bv_hook, Gn, B, 0, s, n, col, r.comp, r.cbest, r.cedge, r.csrc, r.parent, r.ma, r.mb, r.mw,
+                         r.idx, r.flags, hooked + round);
+      for (int k = 0; k < 2; k++) hipLaunchKernelGGL(k_bv_jump, Gn, B, 0, s, n, r.parent);
+      hipLaunchKernelGGL(k_bv_relabel, Gn, B, 0, s, n, r.parent, r.comp, r.cbest);
+    }
+    uint32_t h[kMaxRounds + 1];
+    HIPTRY(hipMemcpyAsync(h, r.flags, (round + 1) * 4, hipMemcpyDeviceToHost, s));
     HIPTRY(hipStreamSynchronize(s));
-    if (h_count == m) break;  // no component hooked this round
-    m = h_count;
+    m = h[0];
     if (m >= n) {
       *err = "forest edge count out of range";
       return FL_ERR_HIP;
     }
+    if (h[round] == 0) break;  // no component hooked in the last round
+    target = round + 1;
   }
   auto t1 = std::chrono::steady_clock::now();
   if (st) {
@@ -786,60 +807,36 @@ int fl_device_ranks(hipStream_t s, uint32_t n, const uint32_t* rp, const uint32_
   if (m == 0) return FL_OK;
   const dim3 Gm = grid_for(m), G2m = grid_for(2ull * m);
   // edges by length
-  hipLaunchKernelGGL(k_iota, Gm, B, 0, s, m, r.idx);
   HIPTRY(hipcub::DeviceRadixSort::SortPairs(r.tmp1, r.tmp1_bytes, r.mw, r.mw2, r.idx, r.idx2, (int)m, 0, 64, s));
-  hipLaunchKernelGGL(k_gather_pairs, Gm, B, 0, s, m, r.idx2, r.ma, r.mb, r.a2, r.b2);
   // 1. rooting at S
-  hipLaunchKernelGGL(k_fill32, grid_for((n + 3) / 4), B, 0, s, (n + 3) / 4, (uint32_t*)r.reached, 0u);
+  uint32_t* moved = hooked + kMaxRounds;
+  hipLaunchKernelGGL(k_rank_init, Gn, B, 0, s, n, r.reached, r.head, r.wt, r.fch);
   hipLaunchKernelGGL(k_mark_reached, Gn, B, 0, s, n, is_outlet, r.comp, r.reached);
-  hipLaunchKernelGGL(k_arcs, Gm, B, 0, s, m, r.a2, r.b2, r.icomp, r.comp, r.reached, r.key, r.val);
-  HIPTRY(hipcub::DeviceRadixSort::SortPairs(r.tmp2, r.tmp2_bytes, r.key, r.skey, r.val, r.sarc, (int)(2 * m), 0, 32,
-                                            s));
-  hipLaunchKernelGGL(k_arc_pos, G2m, B, 0, s, 2 * m, r.skey, r.sarc, r.pos, r.start);
-  hipLaunchKernelGGL(k_arc_tour, G2m, B, 0, s, 2 * m, r.skey, r.sarc, r.pos, r.start, is_outlet, r.tour);
-  // a list of L elements is ranked after ceil(log3 L) rounds (each round at
-  // least triples every pointer's reach); one more proves it
-  uint32_t lg = 1;
-  for (uint64_t reach = 3; reach < 2ull * m; reach *= 3) lg++;
-  hipLaunchKernelGGL(k_fill32, dim3(1), B, 0, s, kMaxFlags, r.flags, 0u);
-  int rc = jump_to_fixpoint(
-      s, r.flags, kMaxFlags, lg + 1,
-      [&](uint32_t* fset, const uint32_t* prev) {
-        hipLaunchKernelGGL(k_list_jump, G2m, B, 0, s, 2 * m, r.tour, fset, prev);
-      },
-      err, "forest tour ranking");
-  if (rc != FL_OK) return rc;
-  // S (every outlet label) is heavier than any edge
-  hipLaunchKernelGGL(k_fill32, Gn, B, 0, s, n, r.wt, FL_NONE);
-  hipLaunchKernelGGL(k_edge_dir, Gm, B, 0, s, m, r.a2, r.b2, r.icomp, r.key, r.pos, r.tour, r.child, r.par, r.wt);
-  HIPTRY(hipMemcpyAsync(r.q, r.par, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
+  hipLaunchKernelGGL(k_arcs, G2m, B, 0, s, m, r.ma, r.mb, r.icomp, r.comp, r.reached, is_outlet, r.head, r.anext);
+  hipLaunchKernelGGL(k_arc_tour, G2m, B, 0, s, m, r.ma, r.mb, r.icomp, r.comp, r.reached, r.head, r.anext, is_outlet,
+                     r.tour);
+  const uint32_t rounds = list_rounds(2ull * m);
+  static_assert(1 + kMaxRounds + 3 * 32 <= kMaxFlags, "a word for every round");
+  for (uint32_t k = 0; k < rounds; k++)
+    hipLaunchKernelGGL(k_list_jump, G2m, B, 0, s, 2 * m, r.tour, moved + k, k ? moved + k - 1 : nullptr);
+  hipLaunchKernelGGL(k_edge_dir, Gm, B, 0, s, m, r.idx2, r.ma, r.mb, r.icomp, r.comp, r.reached, r.tour, r.child, r.q,
+                     r.wt);
   // 2. q: the nearest heavier ancestor
-  hipLaunchKernelGGL(k_fill32, dim3(1), B, 0, s, kMaxFlags, r.flags, 0u);
-  rc = jump_to_fixpoint(
-      s, r.flags, kMaxFlags, kJumpBatch,
-      [&](uint32_t* fset, const uint32_t* prev) {
-        hipLaunchKernelGGL(k_q_jump, Gm, B, 0, s, m, r.child, r.wt, r.q, fset, prev);
-      },
-      err, "heavier-ancestor jumping");
-  if (rc != FL_OK) return rc;
+  moved += 32;
+  for (uint32_t k = 0; k < lg / 2; k++)
+    hipLaunchKernelGGL(k_q_jump, Gm, B, 0, s, m, r.child, r.wt, r.q, moved + k, k ? moved + k - 1 : nullptr);
   // 3. children in increasing weight under each q
-  hipLaunchKernelGGL(k_q_keys, Gm, B, 0, s, m, r.child, r.q, r.qk, r.qv);
-  HIPTRY(hipcub::DeviceRadixSort::SortPairs(r.tmp2, r.tmp2_bytes, r.qk, r.qs, r.qv, r.cs, (int)m, 0, 32, s));
-  hipLaunchKernelGGL(k_fill32, Gn, B, 0, s, n, r.fch, FL_NONE);
-  hipLaunchKernelGGL(k_q_links, Gm, B, 0, s, m, r.qs, r.cs, r.fch, r.nsib);
+  hipLaunchKernelGGL(k_q_keys, Gm, B, 0, s, m, n, r.child, r.wt, r.q, r.qk, r.qv);
+  HIPTRY(hipcub::DeviceRadixSort::SortPairs(r.tmp2, r.tmp2_bytes, r.qk, r.qs, r.qv, r.cs, (int)m, 0, key_bits(n), s));
+  hipLaunchKernelGGL(k_q_links, Gm, B, 0, s, m, n, r.qs, r.cs, r.fch, r.nsib);
   // 4. preorder: the q-tree's tour ranked from its start (qt is indexed by
   // 2 * site + {0, 1}: 2n entries)
   hipLaunchKernelGGL(k_q_tour, grid_for(m > n ? m : n), B, 0, s, m, n, r.qs, r.cs, r.q, r.fch, r.nsib, is_outlet,
                      r.qt);
-  hipLaunchKernelGGL(k_fill32, dim3(1), B, 0, s, kMaxFlags, r.flags, 0u);
-  rc = jump_to_fixpoint(
-      s, r.flags, kMaxFlags, lg + 1,
-      [&](uint32_t* fset, const uint32_t* prev) {
-        hipLaunchKernelGGL(k_qtour_jump, G2m, B, 0, s, 2 * m, r.qs, r.cs, r.qt, fset, prev);
-      },
-      err, "preorder ranking");
-  if (rc != FL_OK) return rc;
-  hipLaunchKernelGGL(k_q_rank, Gm, B, 0, s, m, r.qs, r.cs, r.qt, tid, d_base, rank);
+  moved += 32;
+  for (uint32_t k = 0; k < rounds; k++)
+    hipLaunchKernelGGL(k_qtour_jump, G2m, B, 0, s, 2 * m, n, r.qs, r.cs, r.qt, moved + k, k ? moved + k - 1 : nullptr);
+  hipLaunchKernelGGL(k_q_rank, Gm, B, 0, s, m, n, r.qs, r.cs, r.qt, tid, d_meta, rank);
   // the scratch is released (or rewound) on return: nothing may still read it
   HIPTRY(hipStreamSynchronize(s));
   if (st) st->ranks_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t1).count();
@@ -893,12 +890,10 @@ int fl_device_subtree_sizes(hipStream_t s, uint32_t n, const uint32_t* next, con
   hipLaunchKernelGGL(k_fill32, dim3(1), B, 0, s, kMaxFlags, flags, 0u);
   hipLaunchKernelGGL(k_st_link, Gn, B, 0, s, n, next, tid, t_active, head, sib);
   hipLaunchKernelGGL(k_st_tour, Gn, B, 0, s, n, next, tid, t_active, head, sib, tour);
-  // a list of L arcs is ranked after ceil(log3 L) rounds (each round at
-  // least triples every pointer's reach), rounds after a quiet one return
-  // at once; nothing is read back: the sizes are a hint, the stream goes on
-  uint32_t lg = 1;
-  for (uint64_t reach = 3; reach < 2ull * n; reach *= 3) lg++;
-  for (uint32_t r = 0; r < lg && r < kMaxFlags; r++)
+  // rounds after a quiet one return at once; nothing is read back: the sizes
+  // are a hint, the stream goes on
+  const uint32_t rounds = list_rounds(2ull * n);
+  for (uint32_t r = 0; r < rounds; r++)
     hipLaunchKernelGGL(k_list_jump, G2, B, 0, s, 2u * n, tour, flags + r, r ? flags + r - 1 : nullptr);
   hipLaunchKernelGGL(k_st_size, Gn, B, 0, s, n, next, tid, t_active, tour, size);
   HIPTRY(hipGetLastError());
