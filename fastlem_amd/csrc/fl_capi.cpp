@@ -99,11 +99,13 @@ struct fl_terrain {
   uint32_t prev_nb = 0;      // bucket entries the previous decomposition used (cleared next)
   uint32_t jump_rounds = 4;  // pointer-jumping rounds of the previous iteration
   uint32_t last_rounds = 0;  // sweep rounds of the previous iteration
+  uint64_t last_active = 0;  // sites it recomputed: chain positions and leaves
   std::vector<uint32_t> last_boff;  // its bucket offsets (boff[nb+1], bnoff[nb+1]): launch-size estimates
   uint32_t tail_units = FL_TAIL_WAVES;  // synchronous iterations: rounds of at most this many units go to the tail launches
-  // a sweep's wait ended without its value (FL_FLAG_STALL): the hand-over
-  // words are reset, and the terrain's later iterations run every round
-  // behind barriers
+  // stalled: a sweep's wait ended without its value (FL_FLAG_STALL), and the
+  // terrain's later iterations run every round behind barriers; reset_words: the
+  // hand-over words may hold values (after a stall, or a decomposition that no
+  // sweep followed)
   bool stalled = false, reset_words = false;
   // the device's control block, bucket entries and changed flags are zero (the
   // last thing enqueued that used them was a pipelined iteration)
@@ -634,6 +636,8 @@ int32_t decompose(fl_ctx* c, fl_terrain* T, bool full, bool joined) {
   hipStream_t s = c->stream;
   fl_dev_work& w = T->w;
   uint32_t n = T->t.n;
+  if (T->reset_words) fl_launch_reset_words(s, T->t, w);
+  T->reset_words = true;  // k_chain_perm fills some, the drainage-area sweep empties them
   if (!full && joined) fl_launch_dirty(s, T->t, w);
   fl_launch_children(s, T->t, w, full, T->d_tid, T->d_active);
   uint32_t round = 0;
@@ -674,6 +678,7 @@ int32_t decompose(fl_ctx* c, fl_terrain* T, bool full, bool joined) {
   }
   T->last_boff = c->host_boff;
   T->last_rounds = nb / 2;
+  T->last_active = (uint64_t)host_counter(c, FL_CNT_POSITIONS) + host_counter(c, FL_CNT_LEAVES);
   return FL_OK;
 }
 
@@ -706,8 +711,7 @@ uint32_t tail_start(const std::vector<uint32_t>& off, uint32_t rounds, uint32_t 
   return rounds - l >= 2 ? l : rounds;
 }
 
-// Chain positions of all rounds: the sites of the basins an iteration
-// recomputed (0 when the offsets were not read back).
+// Chain positions of all rounds (0 when the offsets were not read back).
 uint64_t all_positions(const std::vector<uint32_t>& off) {
   if (off.size() < 2) return 0;
   return off.back();
@@ -746,10 +750,6 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
   fl_dev_work& w = T->w;
   uint32_t n = T->t.n;
   const bool hint_stale = T->hint_stale;
-  if (T->reset_words) {
-    fl_launch_reset_words(s, T->t, w);
-    T->reset_words = false;
-  }
   fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, n + 2));
   fl_launch_receivers(s, T->t, w, keep, !full);
   if (T->hint_stale) {
@@ -799,6 +799,7 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
   const RoundSize flow = rounds_size(off, 0, split, lm), tail = rounds_size(off, split, rounds, lm);
   if (split < rounds) fl_launch_da_tail(s, T->t, w, split, tail.positions, clamp);
   if (split > 0) fl_launch_da_fold(s, T->t, w, split, flow.units, flow.positions, clamp);
+  T->reset_words = false;
   if (split > 0) fl_launch_tau_fold(s, w, split, flow.units, flow.positions, clamp);
   if (split < rounds) fl_launch_tau_tail(s, w, split, tail.positions, clamp);
   if (T->d_tchanged) fl_launch_fill_u32(s, T->d_tchanged, T->nterr, 0);
@@ -968,6 +969,7 @@ int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool
   *lake_found = T->lakes = lake;
   T->prev_nb = nb;
   T->last_rounds = nb / 2;
+  T->last_active = (uint64_t)hc[FL_NUM_FLAGS + FL_CNT_POSITIONS] + hc[FL_NUM_FLAGS + FL_CNT_LEAVES];
   // the next iterations would speculate as many rounds: they wait for a
   // synchronous one with subtree sizes (the flights already enqueued land)
   if (deep_rounds(c, T->last_rounds, n)) {
@@ -1211,7 +1213,7 @@ int32_t layout_device(fl_terrain* P, uint32_t n, uint32_t nnz, uint32_t count, b
   if (clamp)
     for (double** p : {&w.hnp, &w.up, &w.tanp, &w.hop}) FLCHK(dev_alloc(P, p, n));
   if (clamp) FLCHK(dev_alloc(P, &w.pro, n));
-  for (uint32_t** p : {&w.sub, &w.hc, &w.pcnt, &w.pdest, &w.ppos, &w.head_base, &w.perm})
+  for (uint32_t** p : {&w.sub, &w.hc, &w.pcnt, &w.pdest, &w.ppos, &w.spos, &w.head_base, &w.perm})
     FLCHK(dev_alloc(P, p, n));
   FLCHK(dev_alloc(P, &w.cover, n));
   FLCHK(dev_alloc(P, &w.cmeta, n));
@@ -1846,7 +1848,7 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
       T->stat_lake_iterations += lake ? 1 : 0;
       for (uint32_t g = 0; g < cur->nterr; g++) enq[g] += mask[g];
       confirm(mask, cur->d_tchanged ? cur->h_tchanged : nullptr, changed);
-      T->stat_recomputed += all_positions(cur->last_boff);
+      T->stat_recomputed += cur->last_active;
       note_rounds(T, cur->last_rounds, it);
       hin = (hin + 1) % 3;
       it++;
@@ -1898,7 +1900,7 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
       }
       T->stat_lake_iterations += lake ? 1 : 0;
       confirm(f.mask, tflags, changed);
-      T->stat_recomputed += all_positions(cur->last_boff);
+      T->stat_recomputed += cur->last_active;
       note_rounds(T, cur->last_rounds, it);
       hin = (f.in + 1) % 3;
       it++;

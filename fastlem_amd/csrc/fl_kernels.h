@@ -43,6 +43,7 @@ enum {
   FL_CNT_POSITIONS = 2,
   FL_CNT_TICKET_DA = 3,  // units taken from the sweeps
   FL_CNT_TICKET_TAU = 4,
+  FL_CNT_LEAVES = 5,  // active sites on no chain
   FL_NUM_COUNTERS = 6
 };
 // Entries of a bucket array past its n: a light edge has a heavy sibling, so
@@ -101,7 +102,7 @@ struct fl_dev_work {
   double* dnext = nullptr;  // [n] distance to the receiver
   uint32_t* next = nullptr; // [n]
   // lakes
-  uint32_t* sub = nullptr;
+  uint32_t* sub = nullptr;    // chain ends; from the decomposition on its workgroups' leaf counts
   uint64_t* lake_key = nullptr;
   // decomposition
   uint64_t* cmask = nullptr;  // [n] child slots of each site
@@ -119,6 +120,7 @@ struct fl_dev_work {
   double* cover = nullptr;    // [n] hand-over words past the lists, at the children's bases, and between a chain's tiles
   uint32_t* pdest = nullptr;  // [n]
   uint32_t* ppos = nullptr;   // [n]
+  uint32_t* spos = nullptr;   // [n] by site: its position, a leaf's receiver's
 
   // pointer jumping, two (pointer, count) pairs per site, pointer in the low
   // word: cp = (chain ancestor, distance to it), rt = (tree ancestor, light
@@ -149,7 +151,7 @@ struct fl_dev_work {
   const uint32_t* root_prev = nullptr;  // [n] its basin (root) of every site
   uint32_t* root = nullptr;             // [n] this iteration's, for the next one
   uint8_t* dirty = nullptr;             // [n] by root: basin to recompute
-  uint8_t* act = nullptr;               // [n] site recomputed in this iteration
+  uint8_t* act = nullptr;               // [n] kind of a site recomputed in this iteration, 0: not
   // [n] the previous iteration changed the elevation of the site or of a
   // neighbour (zeroed by k_receivers, marked by k_tau_scatter)
   const uint8_t* chg_prev = nullptr;

@@ -49,6 +49,7 @@
 #define FL_LIST_OVERFLOW 0x10000u   // pcnt flag: more light children than listed
 #define FL_ROW 8                    // graph row entries loaded together
 static_assert(FL_ROW <= FL_LIST, "a row loaded at once fits its position's list");
+#define FL_SENT 0x7ff45eed0badf00dull  // a hand-over word without its value (see the sweeps)
 #define FL_TAIL 0x20000u            // pcnt flag: the position is its chain's tail
 #define FL_HEAD 0x40000u            // ... its chain's head
 #define FL_DEST_OVER 0xfffffffeu    // pdest: the receiver reads the chain's word in cover, not a slot
@@ -92,6 +93,15 @@ __device__ __forceinline__ uint32_t pair_ptr(unsigned long long p) { return (uin
 __device__ __forceinline__ uint32_t pair_cnt(unsigned long long p) { return (uint32_t)(p >> 32) & ~FL_FIN; }
 __device__ __forceinline__ bool pair_fin(unsigned long long p) { return (p >> 63) != 0; }
 
+// Kinds of an active site (act).  A leaf has no children: its drainage area is
+// its own area, and its response time and elevation follow from its receiver's
+// alone, so it is on no chain (two of three sites are leaves): chains, sweeps
+// and pointer jumping have the other sites only.  At a chain's tail every child
+// is a leaf.
+#define FL_ACTIVE 1u
+#define FL_LEAF 2u
+#define FL_CHAIN_END 4u
+
 // Is slot s of row k (starting at b) a child of k?
 __device__ __forceinline__ bool is_child(unsigned long long m, uint32_t deg, uint32_t s, uint32_t b,
                                          const uint32_t* __restrict__ col, const uint32_t* __restrict__ next,
@@ -119,6 +129,12 @@ __device__ __forceinline__ double first_len(const uint32_t* __restrict__ rp, con
 
 __device__ __forceinline__ double bits_double(unsigned long long u) {
   return __hiloint2double((int)(uint32_t)(u >> 32), (int)(uint32_t)u);
+}
+
+// v, quieted if it is the word that stands for no value.
+__device__ __forceinline__ double no_word(double v) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  return u == FL_SENT ? bits_double(u | (1ull << 51)) : v;
 }
 
 // Synchronisation of one wavefront's lanes around its own LDS tile: a
@@ -351,7 +367,7 @@ __global__ void k_lake_keys(uint32_t bs, uint32_t n, const uint32_t* __restrict_
 // The same keys offered from the lakes' side: each site j of a lake looks its
 // neighbours' slots for it up in their rows (rows are symmetric and without
 // duplicates).  For the later iterations, whose lakes are a few sites
-// (k_lake_keys takes 81 us at a million sites for any number of them).
+// (3.4 us at a million sites, where k_lake_keys takes 51 to 81).
 __global__ void k_lake_offers(uint32_t bs, uint32_t n, const uint32_t* __restrict__ rp,
                               const uint32_t* __restrict__ col, const uint32_t* __restrict__ rank,
                               const uint32_t* __restrict__ sub, const uint8_t* __restrict__ is_outlet,
@@ -516,14 +532,26 @@ __global__ void k_children(uint32_t bs, uint32_t n, const uint32_t* __restrict__
 // pair is still unmarked after it: a round without the flag proves
 // convergence in the round that completes it, and the rounds launched after
 // it return at once.
+//
+// The first round also tells the kinds of the sites (hc: heavy children, all
+// made by k_children); leaves take part in none.
 __global__ void k_chain_jump(uint32_t bs, uint32_t n, unsigned long long* cp, unsigned long long* rt,
                              uint32_t* __restrict__ flag_set, const uint32_t* __restrict__ prev_flag,
-                             const uint8_t* __restrict__ act) {
+                             uint8_t* __restrict__ act, const uint32_t* __restrict__ hc) {
   uint32_t v = gid(bs);
   // the site's own pairs are read together with the previous round's flag
   // (an inactive site's pairs are stale and unused: no active site points
   // at one, as a dirty basin holds its sites' whole paths)
-  const bool on = v < n && act[v] != 0;
+  bool on = v < n && (act[v] & (FL_ACTIVE | FL_LEAF)) == FL_ACTIVE;
+  if (!prev_flag && on) {
+    const uint32_t hk = hc[v];
+    if (hk == FL_NONE) {
+      act[v] = FL_ACTIVE | FL_LEAF;
+      on = false;
+    } else if (hc[hk] == FL_NONE) {
+      act[v] = FL_ACTIVE | FL_CHAIN_END;
+    }
+  }
   unsigned long long c = 0, r = 0;
   if (on) {
     c = __atomic_load_n(cp + v, __ATOMIC_RELAXED);
@@ -597,34 +625,32 @@ __device__ __forceinline__ uint32_t bucket_weight(uint32_t len, uint32_t long_mi
 #define FL_BUCKET_PER_THREAD 2
 
 // The chain tails among a thread's FL_BUCKET_PER_THREAD sites of the
-// workgroup's range starting at `base`, with their pairs: activity and heavy
-// child of every site loaded first (clamped in range, all together), the
-// pairs of the tails second, the outlet flag of their roots third (without
-// lakes every root is an outlet: is_outlet is null and this load, 0.7 us in
-// each kernel of the decomposition, is left out).
+// workgroup's range starting at `base`, with their pairs: the kind of every site
+// loaded first (clamped in range, all together), the pairs of the tails second,
+// the outlet flag of their roots third (without lakes every root is an outlet:
+// is_outlet is null and this load, 0.7 us in each kernel of the decomposition, is
+// left out).
 struct fl_tail {
   unsigned long long r, c;
-  bool t;
+  bool t, leaf;
 };
-__device__ __forceinline__ void load_tails(uint32_t base, uint32_t n, const uint32_t* __restrict__ hc,
-                                           const unsigned long long* __restrict__ cp,
+__device__ __forceinline__ void load_tails(uint32_t base, uint32_t n, const unsigned long long* __restrict__ cp,
                                            const unsigned long long* __restrict__ rt,
                                            const uint8_t* __restrict__ is_outlet, const uint8_t* __restrict__ act,
                                            fl_tail (&q)[FL_BUCKET_PER_THREAD]) {
   uint8_t a[FL_BUCKET_PER_THREAD];
-  uint32_t h[FL_BUCKET_PER_THREAD];
 #pragma unroll
   for (uint32_t j = 0; j < FL_BUCKET_PER_THREAD; ++j) {
-    const uint32_t v = base + j * FL_BUCKET_BLOCK + threadIdx.x, vv = v < n ? v : n - 1;
-    a[j] = act[vv];
-    h[j] = hc[vv];
+    const uint32_t v = base + j * FL_BUCKET_BLOCK + threadIdx.x;
+    a[j] = act[v < n ? v : n - 1];
   }
 #pragma unroll
   for (uint32_t j = 0; j < FL_BUCKET_PER_THREAD; ++j) {
     const uint32_t v = base + j * FL_BUCKET_BLOCK + threadIdx.x;
-    q[j].t = v < n && a[j] && h[j] == FL_NONE;
+    q[j].t = v < n && (a[j] & FL_CHAIN_END);
     q[j].r = q[j].t ? rt[v] : 0ull;
     q[j].c = q[j].t ? cp[v] : 0ull;
+    q[j].leaf = v < n && (a[j] & FL_LEAF);
   }
 #pragma unroll
   for (uint32_t j = 0; j < FL_BUCKET_PER_THREAD; ++j)
@@ -637,26 +663,34 @@ __device__ __forceinline__ void load_tails(uint32_t base, uint32_t n, const uint
 
 // Light-depth histogram of the chains (buckets' counts and total length), aggregated
 // per workgroup in LDS before one global atomic per (workgroup, bucket).
-// Each chain is counted by its tail (the member without a heavy child),
-// which knows the chain's length (its position + 1) and light depth.
+// Each chain is counted by its tail, which knows the chain's length (its
+// position + 1) and light depth; leaves_of: each workgroup's leaves (for the
+// statistics; summed with the offsets, as one more atomic a workgroup on one word
+// took 4 us at a million sites).
 __global__ void __launch_bounds__(FL_BUCKET_BLOCK)
-k_bucket_count(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* __restrict__ hc, const unsigned long long* __restrict__ cp,
+k_bucket_count(const uint32_t* __restrict__ guard, uint32_t n, const unsigned long long* __restrict__ cp,
                const unsigned long long* __restrict__ rt, const uint8_t* __restrict__ is_outlet,
-               uint32_t* __restrict__ bcnt, uint32_t* __restrict__ bnodes, uint32_t* __restrict__ maxld,
+               uint32_t* __restrict__ bcnt, uint32_t* __restrict__ bnodes, uint32_t* __restrict__ counters,
+               uint32_t* __restrict__ leaves_of,
                uint32_t long_min, const uint8_t* __restrict__ act) {
   const uint32_t base = xcd_block() * (FL_BUCKET_BLOCK * FL_BUCKET_PER_THREAD);
   fl_tail q[FL_BUCKET_PER_THREAD];
-  load_tails(base, n, hc, cp, rt, is_outlet, act, q);  // in flight while the guard is read
+  load_tails(base, n, cp, rt, is_outlet, act, q);  // in flight while the guard is read
   if (*guard) return;  // pointer jumping has not converged: the iteration is redone
   __shared__ uint32_t s_c[FL_LDS_BUCKETS], s_n[FL_LDS_BUCKETS];
-  __shared__ uint32_t s_max;
+  __shared__ uint32_t s_max, s_leaves;
   for (uint32_t t = threadIdx.x; t < FL_LDS_BUCKETS; t += FL_BUCKET_BLOCK) {
     s_c[t] = 0;
     s_n[t] = 0;
   }
-  if (threadIdx.x == 0) s_max = 0;
+  if (threadIdx.x == 0) {
+    s_max = 0;
+    s_leaves = 0;
+  }
   __syncthreads();
   for (uint32_t j = 0; j < FL_BUCKET_PER_THREAD; ++j) {
+    const unsigned long long leaves = __ballot(q[j].leaf);
+    if ((threadIdx.x & 63u) == 0 && leaves) atomicAdd(&s_leaves, (uint32_t)__builtin_popcountll(leaves));
     if (q[j].t) {
       uint32_t lw = pair_cnt(q[j].r), len = pair_cnt(q[j].c) + 1, l = 2u * lw + (len >= long_min ? 1u : 0u);
       const uint32_t wt = bucket_weight(len, long_min);
@@ -677,7 +711,10 @@ k_bucket_count(const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* _
       atomicAdd(bnodes + t, s_n[t]);
     }
   }
-  if (threadIdx.x == 0) atomicMax(maxld, s_max);
+  if (threadIdx.x == 0) {
+    atomicMax(counters + FL_CNT_MAXLD, s_max);
+    leaves_of[blockIdx.x] = s_leaves;
+  }
 }
 
 // Exclusive scans of the bucket histograms over the light depths actually
@@ -689,7 +726,8 @@ __global__ void __launch_bounds__(FL_SCAN_BLOCK)
 k_bucket_scan(uint32_t n, uint32_t long_min, uint32_t* __restrict__ ctrl,
                               const uint32_t* __restrict__ bcnt, const uint32_t* __restrict__ bnodes,
                               uint32_t* __restrict__ boff, uint32_t* __restrict__ bnoff,
-                              uint32_t* __restrict__ ucum) {
+                              uint32_t* __restrict__ ucum, uint32_t groups, const uint32_t* __restrict__ leaves_of) {
+  __shared__ uint32_t s_leaves;
   __shared__ uint32_t s_a[FL_SCAN_BLOCK], s_b[FL_SCAN_BLOCK];
   __shared__ uint32_t s_u[FL_SCAN_BLOCK];
   __shared__ uint32_t carry_a, carry_b, carry_u;
@@ -703,7 +741,10 @@ k_bucket_scan(uint32_t n, uint32_t long_min, uint32_t* __restrict__ ctrl,
     carry_a = 0;
     carry_b = 0;
     carry_u = 0;
+    s_leaves = 0;
   }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < groups; i += FL_SCAN_BLOCK) atomicAdd(&s_leaves, leaves_of[i]);
   __syncthreads();
   for (uint32_t base = 0; base < nb; base += FL_SCAN_BLOCK) {
     uint32_t i = base + threadIdx.x;
@@ -751,6 +792,7 @@ k_bucket_scan(uint32_t n, uint32_t long_min, uint32_t* __restrict__ ctrl,
       head_c[nb] = carry_a;
       head_n[nb] = carry_b;
     }
+    counters[FL_CNT_LEAVES] = s_leaves;
     counters[FL_CNT_CHAINS] = carry_a;
     counters[FL_CNT_POSITIONS] = carry_b;
   }
@@ -781,10 +823,11 @@ __device__ __forceinline__ void place_chain(uint32_t q, uint32_t pos, uint32_t l
 // decomposition with more rounds raises the guard (the iteration is redone).
 struct fl_bucket_out {
   uint32_t *boff, *bnoff, *ucum, *ctrl;
+  const uint32_t* leaves_of;
 };
 template <bool scan>
 __global__ void __launch_bounds__(FL_BUCKET_BLOCK)
-k_bucket_place(uint32_t* __restrict__ guard, uint32_t n, const uint32_t* __restrict__ hc, const unsigned long long* __restrict__ cp,
+k_bucket_place(uint32_t* __restrict__ guard, uint32_t n, const unsigned long long* __restrict__ cp,
                const unsigned long long* __restrict__ rt, const uint8_t* __restrict__ is_outlet,
                const uint32_t* __restrict__ bcnt, const uint32_t* __restrict__ bnodes,
                fl_bucket_out o, uint32_t* __restrict__ bcur, uint32_t* __restrict__ bncur,
@@ -794,13 +837,23 @@ k_bucket_place(uint32_t* __restrict__ guard, uint32_t n, const uint32_t* __restr
   fl_tail tl[FL_BUCKET_PER_THREAD];
   __shared__ uint32_t s_c[FL_LDS_BUCKETS], s_n[FL_LDS_BUCKETS], s_bc[FL_LDS_BUCKETS], s_bn[FL_LDS_BUCKETS];
   __shared__ uint32_t s_boff[FL_LDS_BUCKETS], s_bnoff[FL_LDS_BUCKETS];
+  __shared__ uint32_t s_leaves;
   static_assert(FL_LDS_BUCKETS == 128 && FL_LDS_BUCKETS == 2 * FL_SCAN_ROUNDS, "one wavefront scans the rounds");
   const uint32_t maxld = o.ctrl[FL_NUM_FLAGS + FL_CNT_MAXLD];
-  load_tails(base, n, hc, cp, rt, is_outlet, act, tl);  // in flight while the guard is read
+  load_tails(base, n, cp, rt, is_outlet, act, tl);  // in flight while the guard is read
   if (*guard) return;  // the iteration is redone
   if (scan && maxld >= FL_LDS_BUCKETS / 2) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *guard = 1;
     return;
+  }
+  if (scan && blockIdx.x == 0) {
+    // the leaves, by the other wavefronts
+    if (threadIdx.x == 0) s_leaves = 0;
+    __syncthreads();
+    uint32_t sum = 0;
+    for (uint32_t i = threadIdx.x - 64u; threadIdx.x >= 64 && i < gridDim.x; i += FL_BUCKET_BLOCK - 64)
+      sum += o.leaves_of[i];
+    if (sum) atomicAdd(&s_leaves, sum);
   }
   if (scan && threadIdx.x < 64) {
     const uint32_t l = threadIdx.x;  // its round
@@ -830,6 +883,10 @@ k_bucket_place(uint32_t* __restrict__ guard, uint32_t n, const uint32_t* __restr
         o.bnoff[2 * l + 2] = head_n[2 * l + 2] = counters[FL_CNT_POSITIONS] = m;
       }
     }
+  }
+  if (scan && blockIdx.x == 0) {
+    __syncthreads();
+    if (threadIdx.x == 0) o.ctrl[FL_NUM_FLAGS + FL_CNT_LEAVES] = s_leaves;
   }
   auto c_off = [&](uint32_t l) { return scan ? s_boff[l] : o.boff[l]; };
   auto n_off = [&](uint32_t l) { return scan ? s_bnoff[l] : o.bnoff[l]; };
@@ -874,15 +931,16 @@ k_bucket_place(uint32_t* __restrict__ guard, uint32_t n, const uint32_t* __restr
   }
 }
 
-// Scatter sites to their chain-major positions with the inputs the sweeps
-// read there: the drainage-area fold's list counts, area, erodibility and
-// receiver distance (with max slopes also uplift, tan(max slope), old
-// elevation and the basin outlet's position), and for each listed light child
-// the slot its chain's head fills with its drainage area (pdest at the child
-// chain's base).  A chain's base gets the position of the head's receiver
-// (FL_NONE for an outlet).  Sites outside every basin keep their elevation,
-// drainage area = own area and response time 0 (generator.rs:144-145), as the
-// reference leaves them.
+// Scatter the chains' sites to their chain-major positions with the inputs the
+// sweeps read there: the drainage-area fold's list counts, area, erodibility and
+// receiver distance (with max slopes also uplift, tan(max slope), old elevation
+// and the basin outlet's position), for each listed light child that is a leaf
+// its drainage area, which is its own area, and for each other one the slot its
+// chain's head fills with it (pdest at the child chain's base).  A chain's base
+// gets the position of the head's receiver (FL_NONE for an outlet).  spos: a
+// chain site's position, a leaf's receiver's.  Sites outside every basin keep
+// their elevation, drainage area = own area and response time 0
+// (generator.rs:144-145), as the reference leaves them.
 struct fl_perm_out {
   uint32_t* perm;
   uint32_t* pcnt;
@@ -895,6 +953,8 @@ struct fl_perm_out {
   double* hop;
   uint32_t* ppos;
   uint32_t* pro;
+  double* cval;
+  uint32_t* spos;
 };
 
 __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, uint32_t n, unsigned long long* cp,
@@ -914,13 +974,27 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
   uint32_t v = gid(bs);
   // the site's own words are read together with the guard (one load
   // latency; a site of a lake basin reads some it does not use)
-  // (an inactive site's too: one load latency less for the active ones)
-  const uint32_t mld = *maxld, redo = *guard, vv = v < n ? v : n - 1;
-  const bool on = act[vv] != 0 && v < n;
-  unsigned long long rv = rt[vv], cv = cp[vv];
-  const unsigned long long m = cmask[vv];
-  const uint32_t b = rp[vv], e = rp[vv + 1], hk = hc[vv], p = next[vv];
-  const double Kv = K[vv], dv = dnext[vv], av = area[vv];
+  const uint32_t mld = *maxld, redo = *guard;
+  const uint32_t kind = v < n ? act[v] : 0u;
+  const bool chain = kind != 0 && !(kind & FL_LEAF);
+  unsigned long long rv = 0ull, cv = 0ull, m = 0ull;
+  uint32_t b = 0u, e = 0u, hk = FL_NONE, p = 0u;
+  double Kv = 0.0, dv = 0.0, av = 0.0;
+  if (kind) {
+    p = next[v];
+    av = area[v];
+  }
+  if (chain) {
+    rv = rt[v];
+    cv = cp[v];
+    b = rp[v];
+    e = rp[v + 1];
+    m = cmask[v];
+    hk = hc[v];
+    Kv = K[v];
+    dv = dnext[v];
+  }
+  if (kind & FL_CHAIN_END) hk = FL_NONE;  // a leaf: one more of the list
   // the bucket histograms are used up (count, scan, place): clear the
   // entries this decomposition touched for the next one
   const uint32_t nb = 2u * (mld + 1u);
@@ -930,12 +1004,27 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
     bcur[i] = 0;
     bncur[i] = 0;
   }
-  if (redo || !on) return;
+  if (redo || !kind) return;
+  if (!chain) {
+    // a leaf: the rest of its words come from its receiver's thread, which has
+    // them at hand (a branch of its own, with two more loads one after the
+    // other, made every wavefront wait for both: 1M sites 20.8 us, now PERM_NOW)
+    A[v] = av;
+    if (p == v) {
+      root[v] = v;
+      o.spos[v] = FL_NONE;
+      if (is_outlet && !is_outlet[v]) {
+        tau[v] = 0.0;
+        h2[v] = h[v];
+      }
+    }
+    return;
+  }
   if (!pair_fin(rv) || !pair_fin(cv)) {
     rv = settle(rv, rt);
     cv = settle(cv, cp);
-    // for the heads below it, k_tau_scatter (nothing else reads v's pair from
-    // here on but as one to hop over, which either value serves)
+    // (others read v's pair from here on only as one to hop over, which
+    // either value serves)
     __atomic_store_n(rt + v, rv | (1ull << 63), __ATOMIC_RELAXED);
     __atomic_store_n(cp + v, cv | (1ull << 63), __ATOMIC_RELAXED);
   }
@@ -947,7 +1036,7 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
   const uint8_t outlet = is_outlet ? is_outlet[r] : 1;
   const uint32_t base = head_base[hd];
   const bool head = hd == v;
-  const unsigned long long cpp = head ? settle(cp[p], cp) : 0ull;
+  unsigned long long cpp = head ? cp[p] : 0ull;
   const uint32_t hbr = clamp ? head_base[r] : 0u;
   uint32_t cc[FL_ROW];
   const bool short_row = deg <= FL_ROW;
@@ -959,9 +1048,17 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
     A[v] = av;
     tau[v] = 0.0;
     h2[v] = h[v];
+    for (uint32_t s = 0; s < deg; ++s) {
+      const uint32_t ch = col[b + s];
+      if (!is_child(m, deg, s, b, col, next, v) || hc[ch] != FL_NONE) continue;
+      root[ch] = r;
+      tau[ch] = 0.0;
+      h2[ch] = h[ch];
+    }
     return;
   }
   const uint32_t P = base + pair_cnt(cv);
+  o.spos[v] = P;
   o.perm[P] = v;
   o.pK[P] = Kv;
   o.pdn[P] = dv;
@@ -973,20 +1070,26 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
   }
   // the light children in fold order (descending slot): those before the
   // heavy child get their receiver's slots 0, 1, ..., those after it the slots
-  // FL_LIST - 1, FL_LIST - 2, ... for their chains' heads to fill; with more
-  // than FL_LIST the overflow bit is set (the fold walks the row) and all of
-  // their heads hand over at their own bases
+  // FL_LIST - 1, FL_LIST - 2, ...; with more than FL_LIST the overflow bit is
+  // set (the fold walks the row) and all of their heads hand over at their own
+  // bases
   {
     uint32_t npre = 0, npost = 0;
     bool after = false;
     if (short_row) {
       // the children's bases loaded together (a row of at most FL_ROW
       // entries, no more than a list holds: the child mask covers it)
-      uint32_t hb[FL_ROW];
+      uint32_t hb[FL_ROW], hj[FL_ROW];
+      double aj[FL_ROW];
 #pragma unroll
       for (int j = 0; j < FL_ROW; ++j) {
-        hb[j] = 0u;
-        if (j < (int)deg && ((m >> j) & 1ull) && cc[j] != hk) hb[j] = head_base[cc[j]];
+        hb[j] = hj[j] = 0u;
+        aj[j] = 0.0;
+        if (j < (int)deg && ((m >> j) & 1ull) && cc[j] != hk) {
+          hj[j] = hc[cc[j]];
+          hb[j] = head_base[cc[j]];  // (of a leaf: unused)
+          aj[j] = area[cc[j]];
+        }
       }
 #pragma unroll
       for (int j = FL_ROW - 1; j >= 0; --j) {
@@ -995,7 +1098,14 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
           after = true;
           continue;
         }
-        o.pdest[hb[j]] = after ? FL_LIST - 1 - npost++ : npre++;
+        const uint32_t slot = after ? FL_LIST - 1 - npost++ : npre++;
+        if (hj[j] == FL_NONE) {
+          o.cval[(uint64_t)FL_LIST * P + slot] = no_word(aj[j]);
+          o.spos[cc[j]] = P;
+          root[cc[j]] = r;
+        } else {
+          o.pdest[hb[j]] = slot;
+        }
       }
       o.pcnt[P] = npre | (npost << 8) | (hk == FL_NONE ? FL_TAIL : 0u) | (head ? FL_HEAD : 0u);
     } else {
@@ -1010,7 +1120,13 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
           continue;
         }
         const uint32_t slot = over ? FL_DEST_OVER : (after ? FL_LIST - 1 - npost : npre);
-        o.pdest[head_base[ch]] = slot;
+        if (hc[ch] != FL_NONE) {
+          o.pdest[head_base[ch]] = slot;
+        } else {
+          if (!over) o.cval[(uint64_t)FL_LIST * P + slot] = no_word(area[ch]);
+          o.spos[ch] = P;
+          root[ch] = r;
+        }
         if (after) ++npost;
         else ++npre;
       }
@@ -1019,7 +1135,10 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
     }
     o.parea[P] = av;
   }
-  if (head) o.ppos[P] = (p == v) ? FL_NONE : head_base[pair_ptr(cpp)] + pair_cnt(cpp);
+  if (head) {
+    cpp = settle(cpp, cp);
+    o.ppos[P] = (p == v) ? FL_NONE : head_base[pair_ptr(cpp)] + pair_cnt(cpp);
+  }
 }
 
 // --------------------------------------------------------------- sweeps ---
@@ -1059,7 +1178,6 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
 // last FL_SPIN_MAX polls, the wavefront raises FL_FLAG_STALL and goes on, every
 // other wait sees the flag and ends, and the host redoes the iteration in one
 // workgroup with barriers between the rounds (k_da_tail, k_tau_tail).
-#define FL_SENT 0x7ff45eed0badf00dull
 #define FL_SPIN_MAX (1u << 20)
 #define FL_NEG0 (-0.0)
 
@@ -1415,14 +1533,14 @@ __device__ __forceinline__ void da_give_back(const fl_da_args& g, uint32_t P, ui
 }
 
 // A position with more light children than listed (rare) walks its row; their
-// chains' words are in cover.
+// chains' words are in cover (a leaf's drainage area is its own).
 __device__ __forceinline__ bool da_over_ready(const fl_da_args& g, uint32_t k) {
   const uint32_t b = g.rp[k], deg = g.rp[k + 1] - b, hk = g.hc[k];
   const unsigned long long m = g.cmask[k];
   for (uint32_t s = deg; s-- > 0;) {
     if (!is_child(m, deg, s, b, g.col, g.next, k)) continue;
     const uint32_t c = g.col[b + s];
-    if (c != hk && peek(g.cover + g.head_base[c]) == FL_SENT) return false;
+    if (c != hk && g.hc[c] != FL_NONE && peek(g.cover + g.head_base[c]) == FL_SENT) return false;
   }
   return true;
 }
@@ -1433,6 +1551,10 @@ __device__ __forceinline__ double da_over_fold(const fl_da_args& g, uint32_t k, 
   for (uint32_t s = deg; s-- > 0;) {
     if (!is_child(m, deg, s, b, g.col, g.next, k)) continue;
     const uint32_t c = g.col[b + s];
+    if (g.hc[c] == FL_NONE) {
+      acc = acc + g.area[c];
+      continue;
+    }
     if (c == hk) {
       acc = acc + r;
       continue;
@@ -1963,16 +2085,23 @@ k_tau_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, fl_flow f, fl_ta
 // Back to site order: response time, new elevation (computed here when no
 // site has a max slope: h_i' = h_o' + U_i * max(rt_i - rt_o, 0) with
 // h_o' = h_o + U_o * max(0, 0), generator.rs:178-180) and the changed flag
-// (generator.rs:201).  One thread per site, which finds its chain position
-// from its converged chain pair (head, position): the site-ordered accesses
-// are coalesced, the position-ordered ones are gathers.  Sites outside every
-// basin were settled by k_chain_perm.  In a batch (tid != null) a terrain
-// that stopped iterating keeps its elevations and each terrain has its own
-// flag.
-__global__ void k_tau_scatter(uint32_t bs, const uint32_t* __restrict__ guard, uint32_t n, const unsigned long long* __restrict__ cp,
-                              const unsigned long long* __restrict__ rt, const uint8_t* __restrict__ is_outlet,
-                              const uint32_t* __restrict__ head_base, const double* __restrict__ taup,
-                              const double* __restrict__ hnp, const double* __restrict__ U,
+// (generator.rs:201).  One thread per site: the site-ordered accesses are
+// coalesced, the position-ordered ones (spos, root: k_chain_perm) are gathers.
+// A leaf takes its one step from its receiver's values here: rt_i = rt_next + x_i,
+// x_i = 1.0 / (K_i * a_i^0.5) * d_i (generator.rs:162-173), and the max-slope
+// limit against the receiver's new elevation.  Sites outside every basin were
+// settled by k_chain_perm.  In a batch (tid != null) a terrain that stopped
+// iterating keeps its elevations and each terrain has its own flag.
+struct fl_leaf_in {
+  const double* area;
+  const double* K;
+  const double* dnext;
+  const double* tan_ms;
+};
+__global__ void k_tau_scatter(uint32_t bs, const uint32_t* __restrict__ guard, uint32_t n, const uint32_t* __restrict__ spos,
+                              const uint32_t* __restrict__ root, const uint8_t* __restrict__ is_outlet,
+                              const double* __restrict__ taup,
+                              const double* __restrict__ hnp, const double* __restrict__ U, fl_leaf_in lf,
                               const double* __restrict__ h, double* __restrict__ h2, double* __restrict__ tau,
                               int* __restrict__ flags, int clamp, const uint32_t* __restrict__ tid,
                               const uint8_t* __restrict__ act, uint32_t* __restrict__ tchanged,
@@ -1987,35 +2116,53 @@ __global__ void k_tau_scatter(uint32_t bs, const uint32_t* __restrict__ guard, u
   // latency), then the second level (outlet flag, positions, the outlet's
   // elevation and uplift) together
   const bool in = v < n;
-  const uint32_t vv = in ? v : n - 1;
-  const bool on = act[vv] != 0 && in;
-  const double hv = h[vv], uv = U[vv];
-  const unsigned long long rv = rt[vv], cv = cp[vv];
-  const uint32_t rb = rp[vv], re = rp[vv + 1];  // the row, for the change marks
-  const uint32_t g = tid ? tid[vv] : 0u;
-  if (*guard != 0) return;  // pointer jumping has not converged: the iteration is redone
+  const uint32_t kind = in ? act[v] : 0u;
+  const double hv = in ? h[v] : 0.0;
+  uint32_t o = 0u, P = FL_NONE, rb = 0u, re = 0u, g = 0u;  // (the row, for the change marks)
+  double uv = 0.0, K = 0.0, a = 0.0, d = 1.0, tm = 0.0;
+  if (kind) {
+    o = root[v];
+    P = spos[v];
+    rb = rp[v];
+    re = rp[v + 1];
+    uv = U[v];
+    g = tid ? tid[v] : 0u;
+  }
+  const bool leaf = (kind & FL_LEAF) != 0;
+  if (leaf) {
+    K = lf.K[v];
+    a = lf.area[v];
+    d = lf.dnext[v];
+    if (clamp) tm = lf.tan_ms[v];
+  }
+  if (*guard != 0) return;  // the iteration is redone
   bool changed = false;
-  if (in && !on) {
+  if (in && !kind) {
     // a site of a basin that keeps its tree (or of a terrain that stopped)
     // keeps its elevation
     h2[v] = hv;
-  } else if (on) {
-    const uint32_t o = pair_ptr(rv);
+  } else if (kind) {
     const uint8_t outlet = is_outlet ? is_outlet[o] : 1;
     // (a site of a lake basin reads these for nothing; its values were
     // written by k_chain_perm)
-    const uint32_t P = head_base[pair_ptr(cv)] + pair_cnt(cv);
-    const uint32_t Po = clamp ? 0u : head_base[o];
+    const bool alone = leaf && o == v;  // an outlet that nothing drains to
+    const uint32_t Po = alone || (clamp && !leaf) || !outlet ? 0u : spos[o];
     const double h_o = clamp ? 0.0 : h[o], u_o = clamp ? 0.0 : U[o];
     if (outlet) {
-      const double tk = taup[P];
-      double nh;
-      if (clamp) {
-        nh = hnp[P];
+      double tk = alone ? 0.0 : taup[P], nh;
+      const double hp = clamp && !alone ? hnp[P] : 0.0;
+      if (leaf) tk = tk + 1.0 / (K * rust_pow_half(a)) * d;
+      if (clamp && !leaf) {
+        nh = hp;
       } else {
-        const double to = taup[Po];
-        const double ho = h_o + u_o * rust_max(to - to, 0.0);
+        const double to = alone ? tk : taup[Po];
+        const double ho = clamp ? (alone ? hv + uv * rust_max(to - to, 0.0) : hnp[Po])
+                                : h_o + u_o * rust_max(to - to, 0.0);
         nh = (v == o) ? ho : ho + uv * rust_max(tk - to, 0.0);
+        if (clamp) {
+          const double below = alone ? hv : hp;  // (an outlet: its own old elevation)
+          if ((nh - below) / d > tm) nh = below + tm * d;
+        }
       }
       tau[v] = tk;
       h2[v] = nh;
@@ -2302,33 +2449,33 @@ void fl_launch_chain_jump(hipStream_t s, const fl_dev_terrain& t, const fl_dev_w
   uint32_t r = round < FL_MAX_JUMP_ROUNDS ? round : FL_MAX_JUMP_ROUNDS - 1;
   uint32_t* fset = w.ctrl + FL_CTRL_JUMPS + r;
   const uint32_t* prev = r > 0 ? w.ctrl + FL_CTRL_JUMPS + r - 1 : nullptr;
-  FL_LAUNCH(k_chain_jump, t.n, s, t.n, (unsigned long long*)w.cp, (unsigned long long*)w.rt, fset, prev, w.act);
+  FL_LAUNCH(k_chain_jump, t.n, s, t.n, (unsigned long long*)w.cp, (unsigned long long*)w.rt, fset, prev, w.act, w.hc);
 }
 
 void fl_launch_chain_count(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool lakes) {
   uint32_t per = FL_BUCKET_BLOCK * FL_BUCKET_PER_THREAD;
-  FL_LAUNCH_GRID(k_bucket_count, dim3((t.n + per - 1) / per), dim3(FL_BUCKET_BLOCK), t.n, s, w.guard, t.n, w.hc,
-                 (const unsigned long long*)w.cp, (const unsigned long long*)w.rt, lakes ? t.is_outlet : (const uint8_t*)nullptr, w.bcnt, w.bnodes, w.counters + FL_CNT_MAXLD,
-                 w.long_min, w.act);
+  FL_LAUNCH_GRID(k_bucket_count, dim3((t.n + per - 1) / per), dim3(FL_BUCKET_BLOCK), t.n, s, w.guard, t.n,
+                 (const unsigned long long*)w.cp, (const unsigned long long*)w.rt,
+                 lakes ? t.is_outlet : (const uint8_t*)nullptr, w.bcnt, w.bnodes, w.counters, w.sub, w.long_min, w.act);
 }
 
 void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool lakes, bool scan) {
   const uint8_t* outlets = lakes ? t.is_outlet : (const uint8_t*)nullptr;
   uint32_t per = FL_BUCKET_BLOCK * FL_BUCKET_PER_THREAD;
   const dim3 grid((t.n + per - 1) / per), block(FL_BUCKET_BLOCK);
-  const fl_bucket_out bo{w.boff, w.bnoff, w.ucum, w.ctrl};
+  const fl_bucket_out bo{w.boff, w.bnoff, w.ucum, w.ctrl, w.sub};
   if (scan) {
-    FL_LAUNCH_GRID(k_bucket_place<true>, grid, block, t.n, s, w.guard, t.n, w.hc, (const unsigned long long*)w.cp,
+    FL_LAUNCH_GRID(k_bucket_place<true>, grid, block, t.n, s, w.guard, t.n, (const unsigned long long*)w.cp,
                    (const unsigned long long*)w.rt, outlets, w.bcnt, w.bnodes, bo, w.bcur, w.bncur, w.cmeta, w.pdest,
                    w.head_base, w.long_min, w.act);
   } else {
     FL_LAUNCH_GRID(k_bucket_scan, dim3(1), dim3(FL_SCAN_BLOCK), 0, s, t.n, w.long_min, w.ctrl, w.bcnt, w.bnodes,
-                   w.boff, w.bnoff, w.ucum);
-    FL_LAUNCH_GRID(k_bucket_place<false>, grid, block, t.n, s, w.guard, t.n, w.hc, (const unsigned long long*)w.cp,
+                   w.boff, w.bnoff, w.ucum, grid.x, w.sub);
+    FL_LAUNCH_GRID(k_bucket_place<false>, grid, block, t.n, s, w.guard, t.n, (const unsigned long long*)w.cp,
                    (const unsigned long long*)w.rt, outlets, w.bcnt, w.bnodes, bo, w.bcur, w.bncur, w.cmeta, w.pdest,
                    w.head_base, w.long_min, w.act);
   }
-  fl_perm_out o{w.perm, w.pcnt, w.pdest, w.parea, w.pK, w.pdn, w.up, w.tanp, w.hop, w.ppos, w.pro};
+  fl_perm_out o{w.perm, w.pcnt, w.pdest, w.parea, w.pK, w.pdn, w.up, w.tanp, w.hop, w.ppos, w.pro, w.cval, w.spos};
   FL_LAUNCH(k_chain_perm, t.n, s, w.guard, t.n, (unsigned long long*)w.cp, (unsigned long long*)w.rt,
             w.next, outlets, w.head_base, o, t.area, t.erod, w.dnext, t.uplift, t.tan_ms,
             t.any_max_slope ? 1 : 0, w.A, w.tau, w.h, w.h2, w.counters + FL_CNT_MAXLD, w.bcnt, w.bnodes, w.bcur,
@@ -2385,9 +2532,10 @@ void fl_launch_tau_tail(hipStream_t s, const fl_dev_work& w, uint32_t lsplit, ui
 
 void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool clamp, bool lakes,
                            const uint32_t* tid, const uint8_t* active, uint32_t* tchanged) {
-  FL_LAUNCH(k_tau_scatter, t.n, s, w.guard, t.n, (const unsigned long long*)w.cp, (const unsigned long long*)w.rt,
-            lakes ? t.is_outlet : (const uint8_t*)nullptr, w.head_base, w.taup, w.hnp, t.uplift, w.h, w.h2, w.tau, w.flags, clamp ? 1 : 0, tid, w.act,
-            tchanged, w.chg, w.dirty, t.row_ptr, t.col);
+  const fl_leaf_in lf{t.area, t.erod, w.dnext, t.tan_ms};
+  FL_LAUNCH(k_tau_scatter, t.n, s, w.guard, t.n, w.spos, w.root, lakes ? t.is_outlet : (const uint8_t*)nullptr, w.taup,
+            w.hnp, t.uplift, lf, w.h, w.h2, w.tau, w.flags, clamp ? 1 : 0, tid, w.act, tchanged, w.chg, w.dirty,
+            t.row_ptr, t.col);
 }
 
 void fl_launch_clear_iter(hipStream_t s, const fl_dev_work& w, uint32_t nb) {
