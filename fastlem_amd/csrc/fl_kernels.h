@@ -131,7 +131,7 @@ struct fl_dev_work {
            *bncur = nullptr;                                  // [n + FL_BUCKET_PAD] light-depth buckets
   uint32_t* ucum = nullptr;                                  // [n + FL_BUCKET_PAD] sweep units before each round
   uint2* cmeta = nullptr;                                    // [n] long chains' tiles: (base position, length or end)
-  uint32_t* head_base = nullptr;                             // [n] at a chain head: its base position
+  uint32_t* head_base = nullptr;                             // [n] at a chain head: its base position, at a leaf: none
   uint32_t* perm = nullptr;                                  // [n] chain-major site order
   uint32_t* ctrl = nullptr;                                  // [FL_CTRL_WORDS]
   // the kernels after the decomposition do nothing unless it is zero

@@ -537,7 +537,8 @@ __global__ void k_children(uint32_t bs, uint32_t n, const uint32_t* __restrict__
 // made by k_children); leaves take part in none.
 __global__ void k_chain_jump(uint32_t bs, uint32_t n, unsigned long long* cp, unsigned long long* rt,
                              uint32_t* __restrict__ flag_set, const uint32_t* __restrict__ prev_flag,
-                             uint8_t* __restrict__ act, const uint32_t* __restrict__ hc) {
+                             uint8_t* __restrict__ act, const uint32_t* __restrict__ hc,
+                             uint32_t* __restrict__ head_base) {
   uint32_t v = gid(bs);
   // the site's own pairs are read together with the previous round's flag
   // (an inactive site's pairs are stale and unused: no active site points
@@ -547,6 +548,7 @@ __global__ void k_chain_jump(uint32_t bs, uint32_t n, unsigned long long* cp, un
     const uint32_t hk = hc[v];
     if (hk == FL_NONE) {
       act[v] = FL_ACTIVE | FL_LEAF;
+      head_base[v] = FL_NONE;  // no chain's head
       on = false;
     } else if (hc[hk] == FL_NONE) {
       act[v] = FL_ACTIVE | FL_CHAIN_END;
@@ -1079,15 +1081,14 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
     if (short_row) {
       // the children's bases loaded together (a row of at most FL_ROW
       // entries, no more than a list holds: the child mask covers it)
-      uint32_t hb[FL_ROW], hj[FL_ROW];
+      uint32_t hb[FL_ROW];
       double aj[FL_ROW];
 #pragma unroll
       for (int j = 0; j < FL_ROW; ++j) {
-        hb[j] = hj[j] = 0u;
+        hb[j] = 0u;
         aj[j] = 0.0;
         if (j < (int)deg && ((m >> j) & 1ull) && cc[j] != hk) {
-          hj[j] = hc[cc[j]];
-          hb[j] = head_base[cc[j]];  // (of a leaf: unused)
+          hb[j] = head_base[cc[j]];  // FL_NONE: a leaf
           aj[j] = area[cc[j]];
         }
       }
@@ -1099,7 +1100,7 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
           continue;
         }
         const uint32_t slot = after ? FL_LIST - 1 - npost++ : npre++;
-        if (hj[j] == FL_NONE) {
+        if (hb[j] == FL_NONE) {
           o.cval[(uint64_t)FL_LIST * P + slot] = no_word(aj[j]);
           o.spos[cc[j]] = P;
           root[cc[j]] = r;
@@ -1120,8 +1121,9 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
           continue;
         }
         const uint32_t slot = over ? FL_DEST_OVER : (after ? FL_LIST - 1 - npost : npre);
-        if (hc[ch] != FL_NONE) {
-          o.pdest[head_base[ch]] = slot;
+        const uint32_t hb = head_base[ch];
+        if (hb != FL_NONE) {
+          o.pdest[hb] = slot;
         } else {
           if (!over) o.cval[(uint64_t)FL_LIST * P + slot] = no_word(area[ch]);
           o.spos[ch] = P;
@@ -2449,7 +2451,8 @@ void fl_launch_chain_jump(hipStream_t s, const fl_dev_terrain& t, const fl_dev_w
   uint32_t r = round < FL_MAX_JUMP_ROUNDS ? round : FL_MAX_JUMP_ROUNDS - 1;
   uint32_t* fset = w.ctrl + FL_CTRL_JUMPS + r;
   const uint32_t* prev = r > 0 ? w.ctrl + FL_CTRL_JUMPS + r - 1 : nullptr;
-  FL_LAUNCH(k_chain_jump, t.n, s, t.n, (unsigned long long*)w.cp, (unsigned long long*)w.rt, fset, prev, w.act, w.hc);
+  FL_LAUNCH(k_chain_jump, t.n, s, t.n, (unsigned long long*)w.cp, (unsigned long long*)w.rt, fset, prev, w.act, w.hc,
+            w.head_base);
 }
 
 void fl_launch_chain_count(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool lakes) {
