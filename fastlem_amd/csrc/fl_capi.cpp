@@ -1106,6 +1106,8 @@ int32_t fl_ctx_stream(fl_ctx* c, hipStream_t* stream, int* device) {
   return FL_OK;
 }
 
+hipMemPool_t fl_ctx_pool(fl_ctx* c) { return c->pool; }
+
 extern "C" int32_t fl_ctx_destroy(fl_ctx* c) {
   if (!c) return FL_OK;
   hipSetDevice(c->device);

@@ -12,6 +12,8 @@ void fl_internal_set_error(const char* msg);
 
 // The context's stream and device (for the library's other parts).
 int32_t fl_ctx_stream(fl_ctx* c, hipStream_t* stream, int* device);
+// The memory pool of the context's device (a context that fl_ctx_stream accepts).
+hipMemPool_t fl_ctx_pool(fl_ctx* ctx);
 
 #include <mutex>
 #include <string>
