@@ -86,6 +86,7 @@ __device__ __forceinline__ uint32_t gid(uint32_t bs) { return xcd_block() * bs +
 // known to be a fixed point (a chain head, a root).  Counts stay below 2^31
 // (they count sites).
 #define FL_FIN 0x80000000u
+#define FL_HOPS 7  // of a jumping round
 __device__ __forceinline__ unsigned long long pair(uint32_t ptr, uint32_t cnt) {
   return ((unsigned long long)cnt << 32) | ptr;
 }
@@ -514,24 +515,25 @@ __global__ void k_children(uint32_t bs, uint32_t n, const uint32_t* __restrict__
 }
 
 // One jumping round on both pointer systems, in place:
-// (a, d) <- (a''', d + d' + d'' + d''') with (a', d') the pair of a,
-// (a'', d'') that of a' and (a''', d''') that of a'' (three hops: the reach
-// quadruples per round).  A pair read while its
-// owner rewrites it is either its old or its new value (aligned 64-bit
-// accesses are single-copy atomic), and both are (ancestor, count) pairs of
-// the same path, so rounds may mix them.  After convergence
+// (a, d) <- (a', d + d') with (a', d') the pair of a, FL_HOPS times (the reach
+// grows by a factor of FL_HOPS + 1).  A pair read while its owner rewrites it is
+// either its old or its new value (aligned 64-bit accesses are single-copy
+// atomic), and both are (ancestor, count) pairs of the same path, so rounds may
+// mix them.  After convergence
 // cp[v] = (chain head, position in chain), rt[v] = (root of v's tree, light
 // edges between v and the root = light depth of v's chain).
 //
+// Seven hops: a launch is 2 us and its gap before the first load, a hop less
+// than 0.7 us for those not at the end, fewer each time.  A solve takes with 3, 5,
+// 7, 11, 15 hops: 1M sites 28.4, 28.2, 27.7, 28.0, 28.2 ms; 10k 2.52, 2.45, 2.41,
+// 2.43, 2.40; strip 39.5, 38.7, 38.5, 39.1, 38.8.
+//
 // Fixed points (a head's cp, a root's rt: pairs (x, 0) of x itself) carry
-// FL_FIN, and so does a pair that reaches one: a site finding its pointer at
-// a fixed point marks its pair, and a hop inherits the mark of the pair it
-// copies (the pair of a'' is marked when a''' is a fixed point).  A marked
-// pair never changes and its site loads nothing more.  A round flags, in its
-// own control word (zeroed at the start of the iteration), whether some
-// pair is still unmarked after it: a round without the flag proves
-// convergence in the round that completes it, and the rounds launched after
-// it return at once.
+// FL_FIN, and so does a pair that reaches one.  A marked pair never changes and
+// its site loads nothing more.  A round flags, in its own control word (zeroed at
+// the start of the iteration), whether some pair is still unmarked after it: a
+// round without the flag proves convergence in the round that completes it, and
+// the rounds launched after it return at once.
 //
 // The first round also tells the kinds of the sites (hc: heavy children, all
 // made by k_children); leaves take part in none.
@@ -563,36 +565,27 @@ __global__ void k_chain_jump(uint32_t bs, uint32_t n, unsigned long long* cp, un
   if (prev_flag && *prev_flag == 0) return;
   bool open = false;
   if (on) {
+    // FL_HOPS hops on both; a pair at a fixed point's is (x, 0) of x itself and
+    // marks the pair that reaches it
     const bool oc = !pair_fin(c), orr = !pair_fin(r);
-    const uint32_t a = pair_ptr(c), b = pair_ptr(r);
-    const unsigned long long ca = oc ? __atomic_load_n(cp + a, __ATOMIC_RELAXED) : 0ull;
-    const unsigned long long rb = orr ? __atomic_load_n(rt + b, __ATOMIC_RELAXED) : 0ull;
-    // at a fixed point already (a is a head, b a root): mark; else hop
-    const bool fc = oc && pair_ptr(ca) == a, fr = orr && pair_ptr(rb) == b;
-    const bool mc = oc && !fc, mr = orr && !fr;
-    const unsigned long long ca2 = mc ? __atomic_load_n(cp + pair_ptr(ca), __ATOMIC_RELAXED) : 0ull;
-    const unsigned long long rb2 = mr ? __atomic_load_n(rt + pair_ptr(rb), __ATOMIC_RELAXED) : 0ull;
-    // a third hop (a fixed point's pair is (x, 0) of x itself: hops past one
-    // stay there and add nothing)
-    const unsigned long long ca3 = mc ? __atomic_load_n(cp + pair_ptr(ca2), __ATOMIC_RELAXED) : 0ull;
-    const unsigned long long rb3 = mr ? __atomic_load_n(rt + pair_ptr(rb2), __ATOMIC_RELAXED) : 0ull;
-    if (fc) __atomic_store_n(cp + v, c | (1ull << 63), __ATOMIC_RELAXED);
-    if (fr) __atomic_store_n(rt + v, r | (1ull << 63), __ATOMIC_RELAXED);
-    if (mc) {
-      const bool f = pair_fin(ca3);
-      __atomic_store_n(
-          cp + v,
-          pair(pair_ptr(ca3), (pair_cnt(c) + pair_cnt(ca) + pair_cnt(ca2) + pair_cnt(ca3)) | (f ? FL_FIN : 0u)),
-          __ATOMIC_RELAXED);
-      open = open || !f;
+    uint32_t dc = pair_cnt(c), dr = pair_cnt(r);
+#pragma unroll
+    for (int hop = 0; hop < FL_HOPS; ++hop) {
+      const bool mc = !pair_fin(c), mr = !pair_fin(r);
+      const unsigned long long nc = mc ? __atomic_load_n(cp + pair_ptr(c), __ATOMIC_RELAXED) : c;
+      const unsigned long long nr = mr ? __atomic_load_n(rt + pair_ptr(r), __ATOMIC_RELAXED) : r;
+      if (mc) dc += pair_cnt(nc);
+      if (mr) dr += pair_cnt(nr);
+      c = nc;
+      r = nr;
     }
-    if (mr) {
-      const bool f = pair_fin(rb3);
-      __atomic_store_n(
-          rt + v,
-          pair(pair_ptr(rb3), (pair_cnt(r) + pair_cnt(rb) + pair_cnt(rb2) + pair_cnt(rb3)) | (f ? FL_FIN : 0u)),
-          __ATOMIC_RELAXED);
-      open = open || !f;
+    if (oc) {
+      __atomic_store_n(cp + v, pair(pair_ptr(c), dc | (pair_fin(c) ? FL_FIN : 0u)), __ATOMIC_RELAXED);
+      open = open || !pair_fin(c);
+    }
+    if (orr) {
+      __atomic_store_n(rt + v, pair(pair_ptr(r), dr | (pair_fin(r) ? FL_FIN : 0u)), __ATOMIC_RELAXED);
+      open = open || !pair_fin(r);
     }
   }
   if (__any(open) && (threadIdx.x & 63u) == 0) *flag_set = 1;
