@@ -1287,13 +1287,8 @@ int32_t alloc_device(fl_ctx* c, fl_terrain* P, uint32_t n, uint32_t nnz, uint32_
   }
   hipStream_t s = c->stream;
   // basin roots are site indices at all times (dirty-basin marks index by them)
-  for (int k = 0; k < 3; k++) fl_launch_fill_u32(s, P->rtb[k], n, 0);
+  fl_launch_init_arrays(s, P->t, w, P->rtb);
   P->prev_valid = false;
-  fl_launch_fill_u32(s, w.bcnt, (uint64_t)n + FL_BUCKET_PAD, 0);
-  fl_launch_fill_u32(s, w.bnodes, (uint64_t)n + FL_BUCKET_PAD, 0);
-  fl_launch_fill_u32(s, w.bcur, (uint64_t)n + FL_BUCKET_PAD, 0);
-  fl_launch_fill_u32(s, w.bncur, (uint64_t)n + FL_BUCKET_PAD, 0);
-  fl_launch_reset_words(s, P->t, w);
   P->prev_nb = 0;
   return FL_OK;
 }

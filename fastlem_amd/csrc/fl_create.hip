@@ -171,24 +171,30 @@ __global__ void k_hook(fl_raw_union R, uint32_t* __restrict__ p) {
   p[i] = best;
 }
 
-// One round of pointer jumping in place (every pointer leads to a smaller
-// hash, so the pointers form a forest and each read is an ancestor, old or
-// new).  Skipped once the previous round moved nothing.
-__global__ void k_hook_jump(uint32_t n, uint32_t* __restrict__ p, uint32_t* __restrict__ moved,
-                            const uint32_t* __restrict__ prev) {
-  if (prev && *prev == 0) return;
+// A round of three hops in place (every pointer leads to a smaller hash, so
+// the pointers form a forest and each read is an ancestor, old or new), then the
+// rest of the way, and f[i]: i is a root.  (Rounds checked on the host were six
+// launches and a read-back more, 40 us.)
+__global__ void k_hook_jump(uint32_t n, uint32_t* p) {
   uint32_t i = gid();
   if (i >= n) return;
-  const uint32_t a = p[i], b = p[a];
-  if (a != b) {
-    p[i] = b;
-    *moved = 1;
-  }
+  const uint32_t a = __atomic_load_n(p + i, __ATOMIC_RELAXED), b = __atomic_load_n(p + a, __ATOMIC_RELAXED);
+  if (a == b) return;
+  const uint32_t c = __atomic_load_n(p + b, __ATOMIC_RELAXED);
+  __atomic_store_n(p + i, __atomic_load_n(p + c, __ATOMIC_RELAXED), __ATOMIC_RELAXED);
 }
-
-__global__ void k_root_flags(uint32_t n, const uint32_t* __restrict__ p, uint32_t* __restrict__ f) {
+__global__ void k_hook_roots(uint32_t n, uint32_t* p, uint32_t* __restrict__ f) {
   uint32_t i = gid();
-  if (i < n) f[i] = p[i] == i ? 1u : 0u;
+  if (i >= n) return;
+  const uint32_t a = __atomic_load_n(p + i, __ATOMIC_RELAXED);
+  uint32_t r = a;
+  for (;;) {
+    const uint32_t q = __atomic_load_n(p + r, __ATOMIC_RELAXED);
+    if (q == r) break;
+    r = q;
+  }
+  if (r != a) __atomic_store_n(p + i, r, __ATOMIC_RELAXED);
+  f[i] = r == i ? 1u : 0u;
 }
 
 // cid[i] = number of the cluster root p[i] (roots numbered in label order),
@@ -312,11 +318,10 @@ __global__ void k_mark_u8(uint32_t count, const uint32_t* __restrict__ idx, uint
 
 using Scratch = fl_scratch;
 
-constexpr uint32_t kMaxFlags = 64;
 
 // Buffers of the locality order for n sites and nnz entries (C <= n clusters).
 struct LocBufs {
-  uint32_t *p, *y, *cid, *val, *skey, *ssite, *cstart, *cnt, *cptr, *corder, *noff, *flags, *nbrs;
+  uint32_t *p, *y, *cid, *val, *skey, *ssite, *cstart, *cnt, *cptr, *corder, *noff, *nbrs;
   void *tmp_scan, *tmp_sort, *tmp_scan2;
   size_t scan_bytes = 0, sort_bytes = 0, scan2_bytes = 0;
 };
@@ -328,7 +333,6 @@ hipError_t loc_bufs(Scratch& S, uint32_t n, uint32_t nnz, LocBufs& b) {
   if ((e = S.alloc(&b.cstart, (uint64_t)n + 1)) != hipSuccess) return e;
   if ((e = S.alloc(&b.cnt, (uint64_t)n + 1)) != hipSuccess) return e;
   if ((e = S.alloc(&b.cptr, (uint64_t)n + 1)) != hipSuccess) return e;
-  if ((e = S.alloc(&b.flags, kMaxFlags)) != hipSuccess) return e;
   if ((e = S.alloc(&b.nbrs, nnz)) != hipSuccess) return e;
   const int items = n > 0 ? (int)n : 1;
   if ((e = hipcub::DeviceScan::InclusiveSum(nullptr, b.scan_bytes, b.val, b.y, items, S.s)) != hipSuccess) return e;
@@ -461,22 +465,9 @@ int fl_device_locality(hipStream_t s, const fl_raw_union& R, uint32_t* old_of_ne
   const dim3 B(256), Gn = grid_for(n);
   // 1. hooks and their roots
   hipLaunchKernelGGL(k_hook, Gn, B, 0, s, R, b.p);
-  hipLaunchKernelGGL(k_fill32, dim3(1), B, 0, s, (uint64_t)kMaxFlags, b.flags, 0u);
-  uint32_t h_flags[kMaxFlags];
-  uint32_t rounds = 0;
-  for (uint32_t target = 4;; target += 4) {
-    if (target > kMaxFlags) {
-      *err = "locality clustering did not converge";
-      return FL_ERR_HIP;
-    }
-    for (; rounds < target; rounds++)
-      hipLaunchKernelGGL(k_hook_jump, Gn, B, 0, s, n, b.p, b.flags + rounds, rounds ? b.flags + rounds - 1 : nullptr);
-    HIPTRY(hipMemcpyAsync(h_flags, b.flags, rounds * 4, hipMemcpyDeviceToHost, s));
-    HIPTRY(hipStreamSynchronize(s));
-    if (h_flags[rounds - 1] == 0) break;
-  }
+  hipLaunchKernelGGL(k_hook_jump, Gn, B, 0, s, n, b.p);
+  hipLaunchKernelGGL(k_hook_roots, Gn, B, 0, s, n, b.p, b.val);
   // 2. clusters numbered and grouped
-  hipLaunchKernelGGL(k_root_flags, Gn, B, 0, s, n, b.p, b.val);
   HIPTRY(hipcub::DeviceScan::InclusiveSum(b.tmp_scan, b.scan_bytes, b.val, b.y, (int)n, s));
   hipLaunchKernelGGL(k_cid, Gn, B, 0, s, n, b.p, b.y, b.cid, b.val);
   uint32_t C = 0;

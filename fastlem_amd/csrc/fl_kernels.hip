@@ -1002,8 +1002,8 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
   if (redo || !kind) return;
   if (!chain) {
     // a leaf: the rest of its words come from its receiver's thread, which has
-    // them at hand (a branch of its own, with two more loads one after the
-    // other, made every wavefront wait for both: 1M sites 20.8 us, now PERM_NOW)
+    // them at hand (20.7 us at a million sites; 16.7 with all sites on chains,
+    // which cost the sweeps and the placement 10 us more)
     A[v] = av;
     if (p == v) {
       root[v] = v;
@@ -2292,6 +2292,22 @@ k_basin_order(uint32_t outlet, uint32_t cap, const uint32_t* __restrict__ rp, co
   if (tid == 0) *len_out = s_tail;
 }
 
+// The arrays of new terrains that are read before they are written: hand-over
+// words without values, bucket entries and basin roots zero.  One launch for 16.
+struct fl_new_arrays {
+  uint32_t* zero[7];  // three of n, four of n + FL_BUCKET_PAD
+  unsigned long long *cval, *cover;
+};
+__global__ void k_init_arrays(uint32_t bs, uint32_t n, fl_new_arrays w) {
+  const uint32_t i = gid(bs);
+#pragma unroll
+  for (int k = 0; k < 7; ++k)
+    if (i < (k < 3 ? n : n + FL_BUCKET_PAD)) w.zero[k][i] = 0;
+  if (i >= n) return;
+  w.cover[i] = FL_SENT;
+  for (uint32_t k = 0; k < FL_LIST; ++k) w.cval[(uint64_t)k * n + i] = FL_SENT;
+}
+
 // Zero the control block and the first `nb` bucket entries.
 __global__ void k_clear_iter(uint32_t bs, uint32_t nb, uint32_t* __restrict__ ctrl, uint32_t* __restrict__ bcnt,
                              uint32_t* __restrict__ bnodes, uint32_t* __restrict__ bcur,
@@ -2543,6 +2559,13 @@ void fl_launch_report(hipStream_t s, const fl_dev_work& w, uint32_t* host_ctrl, 
                       uint32_t* host_tchanged) {
   const uint32_t cnt = tchanged && G > FL_CTRL_WORDS ? G : FL_CTRL_WORDS;
   FL_LAUNCH(k_report, cnt, s, cnt, w.ctrl, host_ctrl, G, tchanged, host_tchanged);
+}
+
+void fl_launch_init_arrays(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t* const roots[3]) {
+  const fl_new_arrays a{{roots[0], roots[1], roots[2], w.bcnt, w.bnodes, w.bcur, w.bncur},
+                        (unsigned long long*)w.cval,
+                        (unsigned long long*)w.cover};
+  FL_LAUNCH(k_init_arrays, t.n + FL_BUCKET_PAD, s, t.n, a);
 }
 
 // (launched in parts: the kernel counts items in 32 bits)
