@@ -4,7 +4,9 @@
 // max_sites and terrain kind match a solve gives its tuning.  A tuning
 // shapes launches only: every row gives the same results.
 //
-// Written by fastlem_amd/autotune.py on 2026-12-03 (one MI355X).
+// Workgroup sizes of the per-site kernels: smaller ones spread a small terrain
+// over more compute units (fewer wavefronts of a workgroup wait for its slowest
+// row); at hundreds of thousands of sites the sizes differ by under one percent.
 #pragma once
 
 #include <stdint.h>
@@ -16,10 +18,10 @@ struct fl_tuning_row {
 };
 
 static const fl_tuning_row fl_tuning_table[] = {
-    {32768ull, 0, 128, 16, 32, 1, 65536u},  // terrain 16384 sites: 2.41 -> 2.35 ms
-    {131072ull, 0, 256, 16, 32, 1, 65536u},  // terrain 65536 sites: 5.46 -> 5.46 ms
-    {524288ull, 0, 256, 16, 32, 1, 65536u},  // terrain 262144 sites: 18.23 -> 18.23 ms
-    {UINT64_MAX, 0, 256, 16, 16, 1, 65536u},  // terrain 1048576 sites: 48.06 -> 48.06 ms
-    {1317794ull, 1, 128, 16, 16, 1, 65536u},  // batch of 32 terrains, 1000..65536 sites (540264 in all): 33.04 -> 32.47 ms
-    {UINT64_MAX, 1, 256, 16, 16, 1, 65536u},  // batch of 64 terrains, 1000..262144 sites (3214323 in all): 216.62 -> 216.62 ms
+    {32768ull, 0, 64, 16, 32, 1, 65536u},  // two terrains of 10k sites: 256 4.94, 128 4.74, 64 4.68 ms
+    {131072ull, 0, 64, 16, 32, 1, 65536u},  // two of 80k: 256 8.12, 128 7.90, 64 7.85 ms
+    {524288ull, 0, 128, 16, 32, 1, 65536u},  // two of 400k: 256 29.94, 128 29.72, 64 29.91, 512 30.78 ms
+    {UINT64_MAX, 0, 128, 16, 16, 1, 65536u},  // two of 1M: 256 59.45, 128 59.03, 64 59.24, 512 60.85 ms
+    {1317794ull, 1, 128, 16, 16, 1, 65536u},  // two batches of 48 terrains, 1000..32768: 256 16.82, 128 16.74 ms
+    {UINT64_MAX, 1, 256, 16, 16, 1, 65536u},  // batch of 64 terrains, 1000..262144 sites
 };
