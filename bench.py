@@ -64,11 +64,13 @@ def kernel_bytes_per_unit(name: str, n: int, nnz: int, clamp: bool, active: floa
         # row_ptr 4 + next 4 + previous area 8, writes cmask 8 + hc 4 and the two chain
         # pointers 16 (written by the parent); col 4 per entry; others copy their root 8
         "k_children": 6 + a * (44 + 4 * deg) + (1 - a) * 8,
-        # act 1; active: the two pairs read 16 + written 16
+        # act 1; active (every site counted, leaves among them): the two pairs read 16 +
+        # written 16
         "k_chain_jump": 1 + a * 32,
-        # act 1; active: hc 4 (the tails' extra reads are not counted)
-        "k_bucket_count": 1 + a * 4,
-        "k_bucket_place": 1 + a * 4,
+        # act 1 (the tails' extra reads are not counted)
+        "k_bucket_count": 1,
+        "k_bucket_place<true>": 1,
+        "k_bucket_place<false>": 1,
         # rt 8 + is_outlet 1 + cp 8 + head_base 4 + row_ptr 4 + cmask 8 + hc 4 + area 8 + col 4
         # + K 8 + dnext 8, writes perm 4 + count 4 + area 8 + K 8 + dnext 8 + root 4 (+ U, tan,
         # h read and four chain-major copies written with max slopes)
@@ -289,9 +291,10 @@ def profiled_roofline(L, ctx, t, n, nnz, clamp):
     st = t.last_stats()
     active = min(1.0, st["recomputed_sites"] / (float(n) * max(st["iterations"], 1))) if n else 1.0
     names = ["k_receivers", "k_children", "k_chain_jump", "k_bucket_count",
-             "k_bucket_scan", "k_bucket_place", "k_chain_perm", "k_da_fold", "k_tau_fold<false>",
+             "k_bucket_scan", "k_bucket_place<true>", "k_bucket_place<false>", "k_chain_perm", "k_da_fold", "k_tau_fold<false>",
              "k_tau_fold<true>", "k_da_tail", "k_tau_tail<false>", "k_tau_tail<true>", "k_tau_scatter",
-             "k_clear_iter", "k_sub_jump", "k_lake_keys", "k_lake_flip", "k_fill_u32", "k_fill_u64", "k_copy_u32"]
+             "k_clear_iter", "k_report", "k_sub_start", "k_sub_jump", "k_sub_settle", "k_lake_keys", "k_lake_offers",
+             "k_lake_flip", "k_init_arrays", "k_fill_u32", "k_fill_u64"]
     prof = {}
     for nm in names:
         cnt = ctypes.c_uint64()
