@@ -214,7 +214,8 @@ void fl_launch_clear_iter(hipStream_t s, const fl_dev_work& w, uint32_t nb);
 // The work arrays of new terrains (basin roots, bucket entries, hand-over words).
 void fl_launch_init_arrays(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t* const roots[3]);
 // The control block to host_ctrl and, with tchanged, its G words to
-// host_tchanged (pinned host memory); both zeroed on the device.
+// host_tchanged (pinned host memory); both zeroed on the device, FL_FLAG_DEEP
+// apart.
 void fl_launch_report(hipStream_t s, const fl_dev_work& w, uint32_t* host_ctrl, uint32_t G, uint32_t* tchanged,
                       uint32_t* host_tchanged);
 // Back to site order, one thread per site.

@@ -2324,14 +2324,16 @@ __global__ void k_clear_iter(uint32_t bs, uint32_t nb, uint32_t* __restrict__ ct
 
 // A pipelined iteration's end: its control block and the terrains' changed
 // flags to their pinned host slots, and both cleared for the next iteration's
-// (one launch for two copies and two fills).
+// (one launch for two copies and two fills).  The guard of a too deep
+// decomposition stays up: it left its tree half made, and an iteration already
+// enqueued behind it must not follow that (the redo's k_clear_iter takes it down).
 __global__ void k_report(uint32_t bs, uint32_t count, uint32_t* __restrict__ ctrl, uint32_t* __restrict__ host_ctrl,
                          uint32_t G, uint32_t* __restrict__ tchanged, uint32_t* __restrict__ host_tchanged) {
   const uint32_t i = gid(bs);
   if (i >= count) return;
   if (i < FL_CTRL_WORDS) {
     host_ctrl[i] = ctrl[i];
-    ctrl[i] = 0;
+    if (i != FL_FLAG_DEEP) ctrl[i] = 0;
   }
   if (tchanged && i < G) {
     host_tchanged[i] = tchanged[i];
