@@ -593,8 +593,10 @@ __global__ void k_chain_jump(uint32_t bs, uint32_t n, unsigned long long* cp, un
 
 // v's pair p at its fixed point.  Most are after as many rounds as the
 // previous iteration's tree took; the others of a tree that needs more hop on
-// here (bounded by the path), so that no round is launched only to prove that
-// all are.
+// here, so that no round is launched only to prove that all are.  Bounded by the
+// path, which holds for a whole tree only: never called before the guard is seen
+// to be down (the pairs of an iteration behind a too deep decomposition are those
+// of two trees, and may lead in a circle).
 __device__ __forceinline__ unsigned long long settle(unsigned long long p, const unsigned long long* pairs) {
   while (!pair_fin(p)) {
     const unsigned long long q = __atomic_load_n(pairs + pair_ptr(p), __ATOMIC_RELAXED);
@@ -620,19 +622,17 @@ __device__ __forceinline__ uint32_t bucket_weight(uint32_t len, uint32_t long_mi
 #define FL_BUCKET_PER_THREAD 2
 
 // The chain tails among a thread's FL_BUCKET_PER_THREAD sites of the
-// workgroup's range starting at `base`, with their pairs: the kind of every site
-// loaded first (clamped in range, all together), the pairs of the tails second,
-// the outlet flag of their roots third (without lakes every root is an outlet:
-// is_outlet is null and this load, 0.7 us in each kernel of the decomposition, is
-// left out).
+// workgroup's range starting at `base`, with their pairs as they are: the kind of
+// every site loaded first (clamped in range, all together), the pairs of the tails
+// second.  Nothing is followed here: these loads are in flight while the guard is
+// read, and settle_tails comes after it.
 struct fl_tail {
   unsigned long long r, c;
   bool t, leaf;
 };
 __device__ __forceinline__ void load_tails(uint32_t base, uint32_t n, const unsigned long long* __restrict__ cp,
                                            const unsigned long long* __restrict__ rt,
-                                           const uint8_t* __restrict__ is_outlet, const uint8_t* __restrict__ act,
-                                           fl_tail (&q)[FL_BUCKET_PER_THREAD]) {
+                                           const uint8_t* __restrict__ act, fl_tail (&q)[FL_BUCKET_PER_THREAD]) {
   uint8_t a[FL_BUCKET_PER_THREAD];
 #pragma unroll
   for (uint32_t j = 0; j < FL_BUCKET_PER_THREAD; ++j) {
@@ -647,6 +647,14 @@ __device__ __forceinline__ void load_tails(uint32_t base, uint32_t n, const unsi
     q[j].c = q[j].t ? cp[v] : 0ull;
     q[j].leaf = v < n && (a[j] & FL_LEAF);
   }
+}
+// The tails' pairs at their fixed points, and the outlet flag of their roots
+// (without lakes every root is an outlet: is_outlet is null and this load, 0.7 us
+// in each kernel of the decomposition, is left out).
+__device__ __forceinline__ void settle_tails(const unsigned long long* __restrict__ cp,
+                                             const unsigned long long* __restrict__ rt,
+                                             const uint8_t* __restrict__ is_outlet,
+                                             fl_tail (&q)[FL_BUCKET_PER_THREAD]) {
 #pragma unroll
   for (uint32_t j = 0; j < FL_BUCKET_PER_THREAD; ++j)
     if (q[j].t) {
@@ -670,8 +678,9 @@ k_bucket_count(const uint32_t* __restrict__ guard, uint32_t n, const unsigned lo
                uint32_t long_min, const uint8_t* __restrict__ act) {
   const uint32_t base = xcd_block() * (FL_BUCKET_BLOCK * FL_BUCKET_PER_THREAD);
   fl_tail q[FL_BUCKET_PER_THREAD];
-  load_tails(base, n, cp, rt, is_outlet, act, q);  // in flight while the guard is read
-  if (*guard) return;  // pointer jumping has not converged: the iteration is redone
+  load_tails(base, n, cp, rt, act, q);  // in flight while the guard is read
+  if (*guard) return;  // the iteration is redone
+  settle_tails(cp, rt, is_outlet, q);
   __shared__ uint32_t s_c[FL_LDS_BUCKETS], s_n[FL_LDS_BUCKETS];
   __shared__ uint32_t s_max, s_leaves;
   for (uint32_t t = threadIdx.x; t < FL_LDS_BUCKETS; t += FL_BUCKET_BLOCK) {
@@ -835,8 +844,9 @@ k_bucket_place(uint32_t* __restrict__ guard, uint32_t n, const unsigned long lon
   __shared__ uint32_t s_leaves;
   static_assert(FL_LDS_BUCKETS == 128 && FL_LDS_BUCKETS == 2 * FL_SCAN_ROUNDS, "one wavefront scans the rounds");
   const uint32_t maxld = o.ctrl[FL_NUM_FLAGS + FL_CNT_MAXLD];
-  load_tails(base, n, cp, rt, is_outlet, act, tl);  // in flight while the guard is read
+  load_tails(base, n, cp, rt, act, tl);  // in flight while the guard is read
   if (*guard) return;  // the iteration is redone
+  settle_tails(cp, rt, is_outlet, tl);
   if (scan && maxld >= FL_LDS_BUCKETS / 2) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *guard = 1;
     return;
