@@ -1171,19 +1171,26 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
 // FL_SENT by the one unit that reads them, response times and elevations by
 // the drainage-area sweep before.
 //
-// A workgroup takes FL_FOLD_WAVES units at a time: those of its own number when
-// the launch has a wavefront for every unit, else from one counter (17 ns a
-// workgroup one after the other on one word: 22 us for the 10 500 units of a
-// million sites).
+// A workgroup takes FL_FOLD_WAVES units at a time from one counter, once it
+// runs; with a wavefront for every unit, which the launch usually has, the
+// workgroups that are enough take once and the others none.  That is 17 ns a
+// workgroup one after the other on one word.  Units by the workgroups' own
+// numbers would save them (solve of 1M sites 28.1 -> 27.4 ms, 400k 14.1 -> 13.9,
+// strip 38.5 -> 38.3), but a wavefront would then wait for workgroups that do not
+// run yet: with two streams sweeping, each can fill the XCD that the other's next
+// workgroup is to start on.  Two or four units a wavefront of one taking: 1M sites
+// 32 and 41 ms (the second waits for the first).
 //
-// Waits end.  Units are in the order of the counter, and workgroups start in
-// the order of their numbers on each XCD, so every unit a wavefront waits for was
-// taken by a wavefront that runs or runs next: the lowest unit not finished waits
-// for nothing.  Should a wait still
-// last FL_SPIN_MAX polls, the wavefront raises FL_FLAG_STALL and goes on, every
-// other wait sees the flag and ends, and the host redoes the iteration in one
-// workgroup with barriers between the rounds (k_da_tail, k_tau_tail).
+// Waits end.  Units are in the order of the counter, so every unit a wavefront
+// waits for was taken before its own, by a wavefront that runs, in whatever order
+// and beside whatever else the workgroups start: the lowest unit not finished
+// waits for nothing.  Should a wait still last FL_SPIN_MAX polls (a second: the
+// whole queue taken off the GPU), the wavefront raises FL_FLAG_STALL and goes on,
+// every other wait sees the flag and ends, and the host redoes the iteration in
+// one workgroup with barriers between the rounds (k_da_tail, k_tau_tail).
+#ifndef FL_SPIN_MAX
 #define FL_SPIN_MAX (1u << 20)
+#endif
 #define FL_NEG0 (-0.0)
 
 // The rounds of a decomposition and the counters its units are taken from.
@@ -1761,12 +1768,13 @@ k_da_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_da_arg
   const uint32_t rounds = deepest < cap ? deepest + 1 : cap;
   const uint32_t total = f.ucum[rounds];
   fl_rounds R = load_rounds(f, 0, rounds, lane);
-  const bool own = (uint64_t)gridDim.x * FL_FOLD_WAVES >= total;
+  const bool once = (uint64_t)gridDim.x * FL_FOLD_WAVES >= total;
+  if (once && (uint64_t)blockIdx.x * FL_FOLD_WAVES >= total) return;  // the others are enough
   __shared__ uint32_t s_ticket;
   __shared__ double s_carry[FL_FOLD_WAVES];  // from each wavefront's tile to the next one's
   for (;;) {
     __syncthreads();
-    if (threadIdx.x == 0) s_ticket = own ? blockIdx.x * FL_FOLD_WAVES : atomicAdd(f.ticket_da, (uint32_t)FL_FOLD_WAVES);
+    if (threadIdx.x == 0) s_ticket = atomicAdd(f.ticket_da, (uint32_t)FL_FOLD_WAVES);
     if (threadIdx.x < FL_FOLD_WAVES) s_carry[threadIdx.x] = bits_double(FL_SENT);
     __syncthreads();
     const uint32_t t = s_ticket;
@@ -1775,7 +1783,7 @@ k_da_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_da_arg
       const fl_unit un = find_unit(f, R, rounds, total - 1 - (t + wave), true, lane);
       da_unit(g, un, 65u - f.long_min, lane, s_carry, wave);
     }
-    if (own) return;
+    if (once) return;
   }
 }
 
@@ -2054,11 +2062,12 @@ k_tau_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_tau_a
   const uint32_t rounds = deepest < cap ? deepest + 1 : cap;
   const uint32_t total = f.ucum[rounds];
   fl_rounds R = load_rounds(f, 0, rounds, lane);
-  const bool own = (uint64_t)gridDim.x * FL_FOLD_WAVES >= total;
+  const bool once = (uint64_t)gridDim.x * FL_FOLD_WAVES >= total;
+  if (once && (uint64_t)blockIdx.x * FL_FOLD_WAVES >= total) return;  // the others are enough
   __shared__ uint32_t s_ticket;
   for (;;) {
     __syncthreads();
-    if (threadIdx.x == 0) s_ticket = own ? blockIdx.x * FL_FOLD_WAVES : atomicAdd(f.ticket_tau, (uint32_t)FL_FOLD_WAVES);
+    if (threadIdx.x == 0) s_ticket = atomicAdd(f.ticket_tau, (uint32_t)FL_FOLD_WAVES);
     __syncthreads();
     const uint32_t t = s_ticket;
     if (t >= total) return;
@@ -2066,7 +2075,7 @@ k_tau_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_tau_a
       const fl_unit un = find_unit(f, R, rounds, t + wave, false, lane);
       tau_unit<clamp>(g, un, 65u - f.long_min, lane);
     }
-    if (own) return;
+    if (once) return;
   }
 }
 

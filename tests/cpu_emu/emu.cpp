@@ -1,5 +1,6 @@
 // CPU emulation runtime for the HIP subset in include/hip/hip_runtime.h
-// (test infrastructure).  Workgroups run one after another; the threads of
+// (test infrastructure).  Workgroups run one after another (FLEMU_LAST_FIRST:
+// the last one first); the threads of
 // a workgroup are fibers on private stacks, switched with _setjmp/_longjmp
 // and scheduled round-robin until each reaches a barrier, a wavefront
 // operation or its end.  Launches from several host threads are serialised.
@@ -227,7 +228,12 @@ void run_launch(dim3 grid, dim3 block, const std::function<void()>& body) {
   g_body = &body;
   g_bdim = block;
   g_gdim = grid;
-  for (uint32_t b = 0; b < grid.x; b++) {
+  for (uint32_t k = 0; k < grid.x; k++) {
+#ifdef FLEMU_LAST_FIRST
+    const uint32_t b = grid.x - 1 - k;
+#else
+    const uint32_t b = k;
+#endif
     g_block = dim3(b, 0, 0);
     run_block(block.x);
   }
