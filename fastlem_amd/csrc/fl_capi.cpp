@@ -102,11 +102,13 @@ struct fl_terrain {
   uint64_t last_active = 0;  // sites it recomputed: chain positions and leaves
   std::vector<uint32_t> last_boff;  // its bucket offsets (boff[nb+1], bnoff[nb+1]): launch-size estimates
   uint32_t tail_units = FL_TAIL_WAVES;  // synchronous iterations: rounds of at most this many units go to the tail launches
-  // stalled: a sweep's wait ended without its value (FL_FLAG_STALL), and the
-  // terrain's later iterations run every round behind barriers; reset_words: the
-  // hand-over words may hold values (after a stall, or a decomposition that no
-  // sweep followed)
-  bool stalled = false, reset_words = false;
+  // After a sweep's wait that ended without its value (FL_FLAG_STALL; it took a
+  // second) barrier_its iterations run every round behind barriers: the redone one
+  // after a solve's first such wait, twice as many after each further one.
+  // reset_words: the hand-over words may hold values (after such a wait, or a
+  // decomposition that no sweep followed)
+  uint32_t barrier_its = 0, barrier_next = 1;
+  bool reset_words = false;
   // the device's control block, bucket entries and changed flags are zero (the
   // last thing enqueued that used them was a pipelined iteration)
   bool ctrl_clean = false;
@@ -738,6 +740,13 @@ bool deep_rounds(const fl_ctx* c, uint32_t rounds, uint32_t n) {
   return rounds > 2 * lg + 8;
 }
 
+// A wait of T's sweeps ended without its value.
+void wait_ended(fl_terrain* T) {
+  T->reset_words = true;
+  T->barrier_its = T->barrier_next;
+  T->barrier_next = std::min<uint32_t>(2 * T->barrier_next, 1u << 20);
+}
+
 // One outer iteration (generator.rs:141-209), synchronous form: the host
 // confirms pointer-jumping convergence and reads the bucket offsets before
 // the sweeps.  The decomposition is built speculatively before the lake test
@@ -749,7 +758,7 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
   hipStream_t s = c->stream;
   fl_dev_work& w = T->w;
   uint32_t n = T->t.n;
-  const bool hint_stale = T->hint_stale;
+  const bool hint_stale = T->hint_stale, barriers = T->barrier_its > 0;
   fl_launch_clear_iter(s, w, std::min<uint32_t>(T->prev_nb + 1, n + 2));
   fl_launch_receivers(s, T->t, w, keep, !full);
   if (T->hint_stale) {
@@ -792,10 +801,10 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
   bool clamp = T->t.any_max_slope;
   uint32_t rounds = nb / 2;
   // the deep rounds, which hold few units, behind barriers in one workgroup
-  // (every round of a terrain whose waits have ended without their values),
+  // (every round of an iteration whose waits have ended without their values),
   // the others in one launch
   const uint32_t lm = w.long_min;
-  const uint32_t split = T->stalled ? 0 : tail_start(off, rounds, lm, T->tail_units);
+  const uint32_t split = barriers ? 0 : tail_start(off, rounds, lm, T->tail_units);
   const RoundSize flow = rounds_size(off, 0, split, lm), tail = rounds_size(off, split, rounds, lm);
   if (split < rounds) fl_launch_da_tail(s, T->t, w, split, tail.positions, clamp);
   if (split > 0) fl_launch_da_fold(s, T->t, w, split, flow.units, flow.positions, clamp);
@@ -809,11 +818,12 @@ int32_t one_iteration(fl_ctx* c, fl_terrain* T, bool full, bool keep, bool* chan
   FLCHK(read_ctrl(c, T));
   if (host_flag(c, FL_FLAG_STALL)) {
     // its input is untouched: once more, without waits
-    if (T->stalled) return set_err(FL_ERR_HIP, "a sweep did not finish");
-    T->stalled = T->reset_words = true;
+    if (barriers) return set_err(FL_ERR_HIP, "a sweep did not finish");
+    wait_ended(T);
     T->hint_stale = hint_stale;
     return one_iteration(c, T, full, keep, changed, had_lake);
   }
+  if (barriers) T->barrier_its--;
   *changed = host_flag(c, FL_FLAG_CHANGED) != 0;
   std::swap(w.h, w.h2);
   // (the lakes of one iteration after another are few, and drainage has
@@ -961,7 +971,7 @@ int32_t finish_fast(fl_ctx* c, fl_terrain* T, const Flight& f, bool* valid, bool
       break;
     }
   if (hc[FL_FLAG_STALL]) {
-    T->stalled = T->reset_words = true;
+    wait_ended(T);
     return FL_OK;
   }
   if (lake && !f.lakes) return FL_OK;
@@ -1003,6 +1013,8 @@ int32_t reset_state(fl_ctx* c, fl_terrain* T) {
   T->after_lake = true;
   T->lakes = false;
   T->hint_stale = true;
+  T->barrier_its = 0;
+  T->barrier_next = 1;
   HIPCHK(hipMemcpyAsync(T->w.h, T->t.init_h, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
   HIPCHK(hipMemcpyAsync(T->w.A, T->t.area, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
   return FL_OK;
@@ -1832,7 +1844,7 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
     // the first iteration, those whose heavy-child hint is stale (after lake
     // joins: a deep decomposition there would also make a poor speculation
     // for the iterations after it) and the unpipelined form
-    if (it == 0 || ((cur->hint_stale || cur->stalled) && q.empty()) || !c->pipelined) {
+    if (it == 0 || ((cur->hint_stale || cur->barrier_its) && q.empty()) || !c->pipelined) {
       bool changed = false, lake = false;
       std::vector<uint8_t> mask(cur->t_active);
       FLCHK(upload_mask(mask));
@@ -1852,7 +1864,7 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
     } else {
       // keep two iterations in flight: the host enqueues the next one while
       // the device runs the current one
-      while (!drain && !cur->hint_stale && !cur->stalled && q.size() < 2) {
+      while (!drain && !cur->hint_stale && !cur->barrier_its && q.size() < 2) {
         std::vector<uint8_t> mask(cur->nterr);
         bool any = false;
         for (uint32_t g = 0; g < cur->nterr; g++) {
@@ -2197,7 +2209,7 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
     }
   };
   const double* result = nullptr;  // the buffer holding the confirmed iteration's elevations
-  if (L->sync_next || ((cur->hint_stale || cur->stalled) && L->q.empty()) || !c->pipelined) {
+  if (L->sync_next || ((cur->hint_stale || cur->barrier_its) && L->q.empty()) || !c->pipelined) {
     std::vector<uint8_t> mask(cur->t_active);
     FLCHK(lane_upload_mask(L, mask));
     set_slots(cur, L->hin);
@@ -2215,7 +2227,7 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
   } else {
     // a drain for a join whose terrains went to another lane: go on
     if (L->drain && L->q.empty() && !L->compact_wanted) L->drain = false;
-    while (!L->drain && !cur->hint_stale && !cur->stalled && L->q.size() < 2) {
+    while (!L->drain && !cur->hint_stale && !cur->barrier_its && L->q.size() < 2) {
       std::vector<uint8_t> mask(cur->nterr);
       bool any = false;
       for (uint32_t g = 0; g < cur->nterr; g++) {

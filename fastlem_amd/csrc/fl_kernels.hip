@@ -1188,8 +1188,9 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
 // whole queue taken off the GPU), the wavefront raises FL_FLAG_STALL and goes on,
 // every other wait sees the flag and ends, and the host redoes the iteration in
 // one workgroup with barriers between the rounds (k_da_tail, k_tau_tail).
-#ifndef FL_SPIN_MAX
 #define FL_SPIN_MAX (1u << 20)
+#ifndef FL_SPIN_FOLD
+#define FL_SPIN_FOLD FL_SPIN_MAX  // of the sweeps in one launch (k_da_fold, k_tau_fold)
 #endif
 #define FL_NEG0 (-0.0)
 
@@ -1229,23 +1230,28 @@ __device__ __forceinline__ void publish(double* p, double v) {
   poke(p, u);
 }
 
+// The flag of ended waits, and the polls after which a wait raises it.
+struct fl_patience {
+  int* stall;
+  uint32_t polls;
+};
 // One more poll of a wait: false when the wait is to end without its value.
-__device__ __forceinline__ bool wait_more(uint32_t& spins, int* stall) {
+__device__ __forceinline__ bool wait_more(uint32_t& spins, const fl_patience& w) {
   ++spins;
 #ifdef FL_WAVE_SHIFT
   __builtin_amdgcn_s_sleep(1);
 #endif
-  if ((spins & 255u) != 0) return true;
-  if (spins >= FL_SPIN_MAX) __atomic_store_n(stall, 1, __ATOMIC_RELAXED);
-  return __atomic_load_n(stall, __ATOMIC_RELAXED) == 0;
+  if ((spins & 255u) != 0 && spins < w.polls) return true;
+  if (spins >= w.polls) __atomic_store_n(w.stall, 1, __ATOMIC_RELAXED);
+  return __atomic_load_n(w.stall, __ATOMIC_RELAXED) == 0;
 }
 
 // The word at p where `need`, waited for by the whole wavefront.
-__device__ __forceinline__ double await(const double* p, bool need, double otherwise, int* stall) {
+__device__ __forceinline__ double await(const double* p, bool need, double otherwise, const fl_patience& w) {
   unsigned long long u = need ? peek(p) : 0ull;
   uint32_t spins = 0;
   while (__any(need && u == FL_SENT)) {
-    if (!wait_more(spins, stall)) break;
+    if (!wait_more(spins, w)) break;
     if (need && u == FL_SENT) u = peek(p);
   }
   return need ? bits_double(u) : otherwise;
@@ -1258,12 +1264,12 @@ __device__ __forceinline__ void publish_lds(double* p, double v) {
   if (u == FL_SENT) u |= 1ull << 51;
   *reinterpret_cast<volatile unsigned long long*>(p) = u;
 }
-__device__ __forceinline__ double await_lds(const double* p, int* stall) {
+__device__ __forceinline__ double await_lds(const double* p, const fl_patience& patience) {
   const volatile unsigned long long* w = reinterpret_cast<const volatile unsigned long long*>(p);
   unsigned long long u = *w;
   uint32_t spins = 0;
   while (__any(u == FL_SENT)) {
-    if (!wait_more(spins, stall)) break;
+    if (!wait_more(spins, patience)) break;
     u = *w;
   }
   return bits_double(u);
@@ -1506,7 +1512,7 @@ struct fl_da_args {
   const uint32_t* head_base;
   const double* area;
   double* A;
-  int* stall;
+  fl_patience wait;
 };
 
 __device__ __forceinline__ fl_da_pos da_load(const fl_da_args& g, uint32_t P) {
@@ -1634,7 +1640,7 @@ __device__ __forceinline__ void da_tile_walk(const fl_da_args& g, const fl_da_po
 #pragma unroll
     for (int b = 0; b < B; ++b)
       wait = wait || (mine[b] && (cn[b] & FL_LIST_OVERFLOW) && !da_over_ready(g, t[b].k));
-    if (!__any(wait) || !wait_more(spins, g.stall)) break;
+    if (!__any(wait) || !wait_more(spins, g.wait)) break;
   }
   double v = carry;
   for (uint32_t i = 0; i < 64; ++i) {
@@ -1686,7 +1692,7 @@ __device__ __forceinline__ void da_unit(const fl_da_args& g, const fl_unit& un, 
     fl_da_words w = da_words(g, t.P, cn[0], t.own);
     uint32_t spins = 0;
     while (__any(da_missing(w))) {
-      if (!wait_more(spins, g.stall)) break;
+      if (!wait_more(spins, g.wait)) break;
       da_again(g, t.P, w);
     }
     const double pre[1] = {da_pre(cn[0], at[0].area, w, t.own)};
@@ -1725,7 +1731,7 @@ __device__ __forceinline__ void da_unit(const fl_da_args& g, const fl_unit& un, 
   for (int b = 0; b < 2; ++b) w[b] = da_words(g, P[b], cn[b], mine[b]);
   uint32_t spins = 0;
   while (__any(da_missing(w[0]) || da_missing(w[1]))) {
-    if (!wait_more(spins, g.stall)) break;
+    if (!wait_more(spins, g.wait)) break;
     da_again(g, P[0], w[0]);
     da_again(g, P[1], w[1]);
   }
@@ -1734,10 +1740,10 @@ __device__ __forceinline__ void da_unit(const fl_da_args& g, const fl_unit& un, 
   double carry = FL_NEG0;
   if (!first) {
     if (s_carry && wave > 0) {
-      carry = await_lds(s_carry + wave - 1, g.stall);
+      carry = await_lds(s_carry + wave - 1, g.wait);
     } else {
       double* word = g.cover + base + end - 1;
-      carry = await(word, true, 0.0, g.stall);
+      carry = await(word, true, 0.0, g.wait);
       if (lane == 0) *reinterpret_cast<unsigned long long*>(word) = FL_SENT;
     }
   }
@@ -1822,7 +1828,7 @@ struct fl_tau_args {
   const double* dp;
   const double* hop;
   double* hnp;
-  int* stall;
+  fl_patience wait;
 };
 
 // Response times of a tile, each from the position before it (a chain's head
@@ -1936,14 +1942,14 @@ __device__ __forceinline__ void tau_unit(const fl_tau_args& g, const fl_unit& un
       ho = g.hop[P];
       ro = g.pro[P];
     }
-    const double tp = await(g.taup + pp, head && !outlet, 0.0, g.stall);
+    const double tp = await(g.taup + pp, head && !outlet, 0.0, g.wait);
     const uint32_t steps = run_steps(__ballot(t.own && !head));
     const double tau[1] = {tau_short_fold(x, head, tp, steps)};
     if (t.own) publish(g.taup + P, tau[0]);
     if (clamp) {
       const bool deep = un.l > 0;
-      double to = await(g.taup + ro, deep && t.own, 0.0, g.stall);
-      double h0 = await(g.hnp + ro, deep && t.own, 0.0, g.stall);
+      double to = await(g.taup + ro, deep && t.own, 0.0, g.wait);
+      double h0 = await(g.hnp + ro, deep && t.own, 0.0, g.wait);
       if (!deep) {
         // the chains of the outlets: an outlet's elevation is
         // h_o + U_o * max(0, 0), limited against its own old elevation
@@ -1961,7 +1967,7 @@ __device__ __forceinline__ void tau_unit(const fl_tau_args& g, const fl_unit& un
         }
       }
       const double z = outlet ? h0 : h0 + u * rust_max(tau[0] - to, 0.0);
-      const double hp = await(g.hnp + pp, head && !outlet, 0.0, g.stall);
+      const double hp = await(g.hnp + pp, head && !outlet, 0.0, g.wait);
       const fl_clamp_pos q[1] = {{z, tm, d, outlet || !t.own}};
       double h[1];
       clamp_tile_fold<1, true>(q, head, hp, steps, h);
@@ -2035,11 +2041,11 @@ __device__ __forceinline__ void tau_unit(const fl_tau_args& g, const fl_unit& un
   load(tile, q1);
   uint32_t ro = 0;
   if (clamp) ro = g.pro[base];
-  tau_c = await(g.taup + pp, !outlet, 0.0, g.stall);
+  tau_c = await(g.taup + pp, !outlet, 0.0, g.wait);
   if (clamp) {
-    to = await(g.taup + ro, !outlet, 0.0, g.stall);
-    h0 = await(g.hnp + ro, !outlet, 0.0, g.stall);
-    h_c = await(g.hnp + pp, !outlet, 0.0, g.stall);
+    to = await(g.taup + ro, !outlet, 0.0, g.wait);
+    h0 = await(g.hnp + ro, !outlet, 0.0, g.wait);
+    h_c = await(g.hnp + pp, !outlet, 0.0, g.wait);
   }
   for (uint32_t t0 = 0;;) {
     fold(t0, q0);
@@ -2520,14 +2526,14 @@ fl_flow flow(const fl_dev_work& w) {
   return fl_flow{w.counters + FL_CNT_MAXLD,       w.ucum, w.boff, w.bnoff, w.counters + FL_CNT_TICKET_DA,
                  w.counters + FL_CNT_TICKET_TAU, w.long_min};
 }
-fl_da_args da_args(const fl_dev_terrain& t, const fl_dev_work& w, bool clamp) {
+fl_da_args da_args(const fl_dev_terrain& t, const fl_dev_work& w, bool clamp, uint32_t polls) {
   return fl_da_args{w.perm, w.pcnt,  w.cval, w.cover, w.parea, w.pK, w.pdn, w.pdest, w.ppos, w.cmeta, w.xp, w.taup,
                     clamp ? w.hnp : nullptr, t.row_ptr, t.col, w.next, (const unsigned long long*)w.cmask, w.hc,
-                    w.head_base, t.area, w.A, w.flags + FL_FLAG_STALL};
+                    w.head_base, t.area, w.A, {w.flags + FL_FLAG_STALL, polls}};
 }
-fl_tau_args tau_args(const fl_dev_work& w) {
+fl_tau_args tau_args(const fl_dev_work& w, uint32_t polls) {
   return fl_tau_args{w.pcnt, w.ppos, w.cmeta, w.xp, w.taup, w.pro, w.up, w.tanp, w.pdn, w.hop, w.hnp,
-                     w.flags + FL_FLAG_STALL};
+                     {w.flags + FL_FLAG_STALL, polls}};
 }
 dim3 fold_grid(uint32_t waves) { return dim3((std::max<uint32_t>(waves, 1) + FL_FOLD_WAVES - 1) / FL_FOLD_WAVES); }
 }  // namespace
@@ -2535,32 +2541,32 @@ dim3 fold_grid(uint32_t waves) { return dim3((std::max<uint32_t>(waves, 1) + FL_
 void fl_launch_da_fold(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t cap, uint32_t waves,
                        uint64_t positions, bool clamp) {
   FL_LAUNCH_GRID(k_da_fold, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w),
-                 da_args(t, w, clamp));
+                 da_args(t, w, clamp, FL_SPIN_FOLD));
 }
 
 void fl_launch_da_tail(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t lsplit,
                        uint64_t positions, bool clamp) {
   FL_LAUNCH_GRID(k_da_tail, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w),
-                 da_args(t, w, clamp));
+                 da_args(t, w, clamp, FL_SPIN_MAX));
 }
 
 void fl_launch_tau_fold(hipStream_t s, const fl_dev_work& w, uint32_t cap, uint32_t waves, uint64_t positions,
                         bool clamp) {
   if (clamp)
     FL_LAUNCH_GRID(k_tau_fold<true>, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w),
-                   tau_args(w));
+                   tau_args(w, FL_SPIN_FOLD));
   else
     FL_LAUNCH_GRID(k_tau_fold<false>, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w),
-                   tau_args(w));
+                   tau_args(w, FL_SPIN_FOLD));
 }
 
 void fl_launch_tau_tail(hipStream_t s, const fl_dev_work& w, uint32_t lsplit, uint64_t positions, bool clamp) {
   if (clamp)
     FL_LAUNCH_GRID(k_tau_tail<true>, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w),
-                   tau_args(w));
+                   tau_args(w, FL_SPIN_MAX));
   else
     FL_LAUNCH_GRID(k_tau_tail<false>, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w),
-                   tau_args(w));
+                   tau_args(w, FL_SPIN_MAX));
 }
 
 void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool clamp, bool lakes,

@@ -43,5 +43,5 @@ def test_last_workgroup_first(case):
 
     ts = CASES[case]()
     _check(solve(emu.lib()), ts)
-    _check(solve(variants.lib("last_first", FLEMU_LAST_FIRST=1, FL_SPIN_MAX=512)), ts)
+    _check(solve(variants.lib("last_first", FLEMU_LAST_FIRST=1, FL_SPIN_FOLD=512)), ts)
     assert syncs[0] == syncs[1]
