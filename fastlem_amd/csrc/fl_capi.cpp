@@ -1007,6 +1007,17 @@ void note_rounds(fl_terrain* T, uint32_t rounds, uint32_t it) {
   T->stat_rounds_max = std::max(T->stat_rounds_max, rounds);
 }
 
+// The flights of q land; their results are not used (the one before them is
+// redone, or was the solve's last).  A wait of theirs that ended without its value
+// left hand-over words all the same.
+int32_t drop_flights(fl_ctx* c, fl_terrain* T, std::deque<Flight>& q) {
+  HIPCHK(hipStreamSynchronize(c->stream));
+  for (const Flight& f : q)
+    if (c->host_slot[f.slot][FL_FLAG_STALL]) T->reset_words = true;
+  q.clear();
+  return FL_OK;
+}
+
 int32_t reset_state(fl_ctx* c, fl_terrain* T) {
   uint32_t n = T->t.n;
   T->prev_valid = false;
@@ -1896,10 +1907,9 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
       if (!valid) {
         // the flights after it started from a wrong input: let them land,
         // then redo this iteration synchronously on its own input and mask
-        HIPCHK(hipStreamSynchronize(s));
         for (const Flight& x : q)
           for (uint32_t g = 0; g < cur->nterr; g++) enq[g] -= x.mask[g];
-        q.clear();
+        FLCHK(drop_flights(c, cur, q));
         T->stat_redone++;
         FLCHK(upload_mask(f.mask));
         set_slots(cur, f.in);
@@ -1938,8 +1948,8 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
     }
   }
   // iterations still in flight after the last one that counted recompute a
-  // fixed point (or masked terrains): wait for them, their results are unused
-  HIPCHK(hipStreamSynchronize(s));
+  // fixed point (or masked terrains)
+  FLCHK(drop_flights(c, cur, q));
   set_slots(cur, hin);
   if (cur != T) {
     for (uint32_t g = 0; g < cur->nterr; g++) {
@@ -2259,10 +2269,9 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
     if (!valid) {
       // the flights after it started from a wrong input: let them land, then
       // redo this iteration synchronously on its own input and mask
-      HIPCHK(hipStreamSynchronize(s));
       for (const Flight& x : L->q)
         for (uint32_t g = 0; g < cur->nterr; g++) L->enq[g] -= x.mask[g];
-      L->q.clear();
+      FLCHK(drop_flights(c, cur, L->q));
       cur->stat_redone++;
       FLCHK(lane_upload_mask(L, f.mask));
       set_slots(cur, f.in);

@@ -2540,33 +2540,33 @@ dim3 fold_grid(uint32_t waves) { return dim3((std::max<uint32_t>(waves, 1) + FL_
 
 void fl_launch_da_fold(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t cap, uint32_t waves,
                        uint64_t positions, bool clamp) {
-  FL_LAUNCH_GRID(k_da_fold, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w),
-                 da_args(t, w, clamp, FL_SPIN_FOLD));
+  const fl_da_args a = da_args(t, w, clamp, FL_SPIN_FOLD);
+  FL_LAUNCH_GRID(k_da_fold, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w), a);
 }
 
 void fl_launch_da_tail(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, uint32_t lsplit,
                        uint64_t positions, bool clamp) {
-  FL_LAUNCH_GRID(k_da_tail, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w),
-                 da_args(t, w, clamp, FL_SPIN_MAX));
+  const fl_da_args a = da_args(t, w, clamp, FL_SPIN_MAX);
+  FL_LAUNCH_GRID(k_da_tail, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w), a);
 }
 
 void fl_launch_tau_fold(hipStream_t s, const fl_dev_work& w, uint32_t cap, uint32_t waves, uint64_t positions,
                         bool clamp) {
+  const fl_tau_args a = tau_args(w, FL_SPIN_FOLD);
   if (clamp)
     FL_LAUNCH_GRID(k_tau_fold<true>, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w),
-                   tau_args(w, FL_SPIN_FOLD));
+                   a);
   else
     FL_LAUNCH_GRID(k_tau_fold<false>, fold_grid(waves), dim3(64 * FL_FOLD_WAVES), positions, s, w.guard, cap, flow(w),
-                   tau_args(w, FL_SPIN_FOLD));
+                   a);
 }
 
 void fl_launch_tau_tail(hipStream_t s, const fl_dev_work& w, uint32_t lsplit, uint64_t positions, bool clamp) {
+  const fl_tau_args a = tau_args(w, FL_SPIN_MAX);
   if (clamp)
-    FL_LAUNCH_GRID(k_tau_tail<true>, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w),
-                   tau_args(w, FL_SPIN_MAX));
+    FL_LAUNCH_GRID(k_tau_tail<true>, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w), a);
   else
-    FL_LAUNCH_GRID(k_tau_tail<false>, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w),
-                   tau_args(w, FL_SPIN_MAX));
+    FL_LAUNCH_GRID(k_tau_tail<false>, dim3(1), dim3(64 * FL_TAIL_WAVES), positions, s, w.guard, lsplit, flow(w), a);
 }
 
 void fl_launch_tau_scatter(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool clamp, bool lakes,

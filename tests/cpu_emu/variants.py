@@ -14,19 +14,24 @@ from . import build as _build
 _libs = {}
 
 
-def lib(name: str, **macros):
-    """The library built with ``macros``, as build/libfastlem_emu_<name>.so."""
+def lib(name: str, source: str = "", header: str = "", **macros):
+    """The library built with ``macros``, as build/libfastlem_emu_<name>.so;
+    ``source`` (a file of this folder) compiled in, ``header`` included in every
+    file."""
     if name not in _libs:
         out = os.path.join(os.path.dirname(_build.lib_path()), f"libfastlem_emu_{name}.so")
         os.makedirs(os.path.dirname(out), exist_ok=True)
         srcs = [os.path.join(_build.CSRC, s) for s in _build.SOURCES] + [os.path.join(_build.HERE, "emu.cpp")]
         headers = [os.path.join(_build.CSRC, h) for h in os.listdir(_build.CSRC) if h.endswith(".h")]
+        srcs += [os.path.join(_build.HERE, source)] if source else []
+        headers += [os.path.join(_build.HERE, header)] if header else []
         headers += [os.path.join(_build.HERE, "include", "hip", "hip_runtime.h"), os.path.abspath(__file__)]
         if not os.path.exists(out) or os.path.getmtime(out) < max(map(os.path.getmtime, srcs + headers)):
             cmd = ["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-pthread", "-ffp-contract=off", "-fno-fast-math",
                    "-U_FORTIFY_SOURCE", "-D_FORTIFY_SOURCE=0", "-fno-omit-frame-pointer", "-w",
                    "-I", os.path.join(_build.HERE, "include"), "-I", os.path.join(_build.ROOT, "include")]
             cmd += [f"-D{k}={v}" for k, v in macros.items()]
+            cmd += ["-include", os.path.join(_build.HERE, header)] if header else []
             for s in srcs:
                 cmd += ["-x", "c++", s, "-x", "none"] if s.endswith(".hip") else [s]
             subprocess.run(cmd + ["-o", out + ".tmp"], check=True)
