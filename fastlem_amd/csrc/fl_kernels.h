@@ -190,7 +190,9 @@ void fl_launch_chain_count(hipStream_t s, const fl_dev_terrain& t, const fl_dev_
 // Bucket offsets (scan), chain placement and the chain-major permutation.
 // scan: the placement makes the offsets itself; a decomposition of more than
 // FL_SCAN_ROUNDS rounds raises the guard instead.
-enum { FL_SCAN_ROUNDS = 64 };
+#ifndef FL_SCAN_ROUNDS
+#define FL_SCAN_ROUNDS 64
+#endif
 void fl_launch_chain_layout(hipStream_t s, const fl_dev_terrain& t, const fl_dev_work& w, bool lakes, bool scan);
 // The sweeps.  Rounds 0..min(deepest, cap - 1) in one launch of about `waves`
 // wavefronts (any number is correct; the sweep units of the rounds are best);

@@ -842,12 +842,12 @@ k_bucket_place(uint32_t* __restrict__ guard, uint32_t n, const unsigned long lon
   __shared__ uint32_t s_c[FL_LDS_BUCKETS], s_n[FL_LDS_BUCKETS], s_bc[FL_LDS_BUCKETS], s_bn[FL_LDS_BUCKETS];
   __shared__ uint32_t s_boff[FL_LDS_BUCKETS], s_bnoff[FL_LDS_BUCKETS];
   __shared__ uint32_t s_leaves;
-  static_assert(FL_LDS_BUCKETS == 128 && FL_LDS_BUCKETS == 2 * FL_SCAN_ROUNDS, "one wavefront scans the rounds");
+  static_assert(FL_LDS_BUCKETS == 128 && FL_LDS_BUCKETS >= 2 * FL_SCAN_ROUNDS, "one wavefront scans the rounds");
   const uint32_t maxld = o.ctrl[FL_NUM_FLAGS + FL_CNT_MAXLD];
   load_tails(base, n, cp, rt, act, tl);  // in flight while the guard is read
   if (*guard) return;  // the iteration is redone
   settle_tails(cp, rt, is_outlet, tl);
-  if (scan && maxld >= FL_LDS_BUCKETS / 2) {
+  if (scan && maxld >= FL_SCAN_ROUNDS) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *guard = 1;
     return;
   }
