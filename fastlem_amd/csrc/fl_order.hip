@@ -36,9 +36,10 @@
 //   4. preorder: an Euler tour of the q-tree ranked by pointer jumping,
 //      counting the down steps from the tour's start.
 // What bounds it is the number of short launches and of read-backs: pointers
-// jump three hops a round, a fixed number of rounds for the usual (or, in a list
-// ranking, for any) path, the next kernel hops the rest of the way, and only the
-// forest's rounds are counted on the host, from where they usually end.
+// jump three hops a round (the forest's hooks up to fifteen), a fixed number of
+// rounds for the usual (or, in a list ranking, for any) path, the next kernel hops
+// the rest of the way, and only the forest's rounds are counted on the host, from
+// where they usually end.
 // The outlet phase (host, fl_outlet_pop_order) ranks the outlets; terrains
 // whose lengths repeat or are not positive are ranked by the exact heap
 // simulation on the host (fl_lake_visit_order).
@@ -269,29 +270,45 @@ __global__ void __launch_bounds__(1024) k_bv_hook(uint32_t n, const uint32_t* __
   }
 }
 
-// One in-place round of three hops on the hook pointers.  A pointer read while
-// its owner rewrites it is its old or its new value (aligned 32-bit accesses are
-// single-copy atomic), both ancestors on the same hook path.
+// One in-place round of up to fifteen hops on the hook pointers.  A pointer read
+// while its owner rewrites it is its old or its new value (aligned 32-bit accesses
+// are single-copy atomic), both ancestors on the same hook path.
 __global__ void k_bv_jump(uint32_t n, uint32_t* parent) {
   uint32_t c = gid();
   if (c >= n) return;
   const uint32_t p = __atomic_load_n(parent + c, __ATOMIC_RELAXED);
-  const uint32_t p2 = __atomic_load_n(parent + p, __ATOMIC_RELAXED);
-  if (p2 == p) return;
-  const uint32_t p3 = __atomic_load_n(parent + p2, __ATOMIC_RELAXED);
-  __atomic_store_n(parent + c, __atomic_load_n(parent + p3, __ATOMIC_RELAXED), __ATOMIC_RELAXED);
+  uint32_t r = p;
+  for (int hop = 0; hop < 15; ++hop) {
+    const uint32_t q = __atomic_load_n(parent + r, __ATOMIC_RELAXED);
+    if (q == r) break;
+    r = q;
+  }
+  if (r != p) __atomic_store_n(parent + c, r, __ATOMIC_RELAXED);
 }
 
-// The components' new labels, the rest of the way along the hooks.
-__global__ void k_bv_relabel(uint32_t n, const uint32_t* __restrict__ parent, uint32_t* __restrict__ comp,
+// The components' new labels, the rest of the way along the hooks.  Two rounds
+// reach 256 hooks, which is enough for any usual component; a longer walk halves
+// the path behind it (every other hook made to lead two further), or a line of
+// sites whose lengths only grow, one path of n hooks, would take n / 256 steps a
+// site.  Forest of a line of a million sites with growing, falling and shuffled
+// lengths: 0.84, 1.24 and 0.73 ms (two rounds of three hops and a plain walk: 50, 50
+// and 0.75).
+__global__ void k_bv_relabel(uint32_t n, uint32_t* parent, uint32_t* __restrict__ comp,
                              unsigned long long* __restrict__ cbest) {
   uint32_t v = gid();
   if (v >= n) return;
   uint32_t c = parent[comp[v]];
-  for (;;) {
-    const uint32_t p = parent[c];
-    if (p == c) break;
-    c = p;
+  if (parent[c] != c) {
+    for (;;) {
+      const uint32_t p = __atomic_load_n(parent + c, __ATOMIC_RELAXED);
+      const uint32_t q = __atomic_load_n(parent + p, __ATOMIC_RELAXED);
+      if (p == q) {
+        c = p;
+        break;
+      }
+      __atomic_store_n(parent + c, q, __ATOMIC_RELAXED);
+      c = q;
+    }
   }
   comp[v] = c;
   cbest[v] = ~0ull;
