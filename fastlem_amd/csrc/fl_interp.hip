@@ -346,6 +346,9 @@ extern "C" int32_t fl_interp_create(fl_ctx* ctx, uint64_t n, const double* xs, c
   return FL_OK;
 }
 
+// A query's buffers up to this size stay with the library's pool.
+constexpr uint64_t kKeptBytes = 64ull << 20;
+
 extern "C" int32_t fl_interp_query(fl_ctx* ctx, fl_interp* P, const double* values, uint64_t m, const double* qx,
                                    const double* qy, double* out, uint8_t* found) {
   if (!ctx || !P || (P->dev.n && !values) || (m && (!qx || !qy || !out || !found)))
@@ -358,10 +361,14 @@ extern "C" int32_t fl_interp_query(fl_ctx* ctx, fl_interp* P, const double* valu
   if (rc != FL_OK) return rc;
   IHIP(hipSetDevice(device));
   // one block of the library's pool, which keeps its memory: five of the default
-  // pool's, given back to the driver after every call, took 80 us of a call of 240
-  const uint64_t n = P->dev.n;
+  // pool's, given back to the driver after every call, took 80 us of a call of 240.
+  // A large block is the default pool's again (25 bytes a point: a hundred million
+  // points would leave 2.5 GB held until the last context goes); its 80 us are then
+  // a small part of a call of some milliseconds.
+  const uint64_t n = P->dev.n, bytes = (n + 3 * m + 1) * 8 + m;
   double* block = nullptr;
-  IHIP(hipMallocFromPoolAsync((void**)&block, (n + 3 * m + 1) * 8 + m, fl_ctx_pool(ctx), s));
+  if (bytes <= kKeptBytes) IHIP(hipMallocFromPoolAsync((void**)&block, bytes, fl_ctx_pool(ctx), s));
+  else IHIP(hipMallocAsync((void**)&block, bytes, s));
   double *dval = block, *dq = dval + n, *dout = dq + 2 * m;
   uint32_t* dstatus = (uint32_t*)(dout + m);
   uint8_t* dfound = (uint8_t*)(dout + m + 1);

@@ -1,0 +1,28 @@
+"""A query's device memory goes back: after a query of many points the card has as
+much free memory as before it, up to the block that the library keeps for the next
+one, while the context and the interpolator live on."""
+import numpy as np
+import pytest
+
+
+@pytest.mark.gpu
+def test_large_query_gives_its_memory_back():
+    import torch
+
+    from fastlem_amd.surface import TerrainInterpolator2D
+
+    rng = np.random.default_rng(3)
+    n, m = 2000, 8_000_000
+    interp, z = TerrainInterpolator2D(rng.uniform(0.0, 10.0, n), rng.uniform(0.0, 10.0, n)), rng.uniform(0.0, 1.0, n)
+
+    def query(k):
+        v, ok = interp.interpolate_many(z, rng.uniform(0.0, 10.0, k), rng.uniform(0.0, 10.0, k))
+        assert np.isfinite(v[ok]).all() and ok.mean() > 0.9
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    query(1000)  # (the kernel and the first block)
+    before = query(1000)
+    after = query(m)  # 25 bytes a point: 200 MB
+    interp.close()
+    assert before - after <= 64 << 20, (before, after)
