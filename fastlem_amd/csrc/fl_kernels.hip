@@ -1113,27 +1113,52 @@ __global__ void k_chain_perm(uint32_t bs, const uint32_t* __restrict__ guard, ui
       }
       o.pcnt[P] = npre | (npost << 8) | (hk == FL_NONE ? FL_TAIL : 0u) | (head ? FL_HEAD : 0u);
     } else {
-      uint32_t light = 0;
-      for (uint32_t s = deg; s-- > 0;) light += is_child(m, deg, s, b, col, next, v) && col[b + s] != hk ? 1u : 0u;
+      // in fold order, FL_ROW entries loaded together: a hub's row is one thread's
+      // (20 000 entries 14.6 ms one by one, 5.3 so), and a row of nine or more, which
+      // one site in sixty has, is the last of its wavefront to end (solve of 10k
+      // random sites 2.36 -> 2.22 ms)
+      uint32_t light = (uint32_t)__builtin_popcountll(m);
+      if (deg > 64) {
+        light = 0;
+        for (uint32_t s = 0; s < deg; s += FL_ROW) {
+          uint32_t nx[FL_ROW];
+#pragma unroll
+          for (int j = 0; j < FL_ROW; ++j) nx[j] = next[col[b + min(s + j, deg - 1)]];
+#pragma unroll
+          for (int j = 0; j < FL_ROW; ++j) light += s + j < deg && nx[j] == v ? 1u : 0u;
+        }
+      }
+      if (hk != FL_NONE) --light;
       const bool over = light > FL_LIST;
-      for (uint32_t s = deg; s-- > 0;) {
-        if (!is_child(m, deg, s, b, col, next, v)) continue;
-        uint32_t ch = col[b + s];
-        if (ch == hk) {
-          after = true;
-          continue;
+      for (uint32_t top = deg; top > 0; top -= min(top, (uint32_t)FL_ROW)) {
+        uint32_t ch[FL_ROW], nx[FL_ROW], hb[FL_ROW];
+        double aj[FL_ROW];
+#pragma unroll
+        for (int j = 0; j < FL_ROW; ++j) ch[j] = col[b + (top > (uint32_t)j ? top - 1 - j : 0u)];
+#pragma unroll
+        for (int j = 0; j < FL_ROW; ++j) {
+          nx[j] = next[ch[j]];
+          hb[j] = head_base[ch[j]];
+          aj[j] = area[ch[j]];
         }
-        const uint32_t slot = over ? FL_DEST_OVER : (after ? FL_LIST - 1 - npost : npre);
-        const uint32_t hb = head_base[ch];
-        if (hb != FL_NONE) {
-          o.pdest[hb] = slot;
-        } else {
-          if (!over) o.cval[(uint64_t)FL_LIST * P + slot] = no_word(area[ch]);
-          o.spos[ch] = P;
-          root[ch] = r;
+#pragma unroll
+        for (int j = 0; j < FL_ROW; ++j) {
+          if ((uint32_t)j >= top || nx[j] != v) continue;
+          if (ch[j] == hk) {
+            after = true;
+            continue;
+          }
+          const uint32_t slot = over ? FL_DEST_OVER : (after ? FL_LIST - 1 - npost : npre);
+          if (hb[j] != FL_NONE) {
+            o.pdest[hb[j]] = slot;
+          } else {
+            if (!over) o.cval[(uint64_t)FL_LIST * P + slot] = no_word(aj[j]);
+            o.spos[ch[j]] = P;
+            root[ch[j]] = r;
+          }
+          if (after) ++npost;
+          else ++npre;
         }
-        if (after) ++npost;
-        else ++npre;
       }
       o.pcnt[P] = (over ? FL_LIST_OVERFLOW : (npre | (npost << 8))) | (hk == FL_NONE ? FL_TAIL : 0u) |
                   (head ? FL_HEAD : 0u);
@@ -1550,36 +1575,30 @@ __device__ __forceinline__ void da_give_back(const fl_da_args& g, uint32_t P, ui
     if (mine && da_slot(cn, i)) w[i] = FL_SENT;
 }
 
-// A position with more light children than listed (rare) walks its row; their
-// chains' words are in cover (a leaf's drainage area is its own).
-__device__ __forceinline__ bool da_over_ready(const fl_da_args& g, uint32_t k) {
-  const uint32_t b = g.rp[k], deg = g.rp[k + 1] - b, hk = g.hc[k];
-  const unsigned long long m = g.cmask[k];
-  for (uint32_t s = deg; s-- > 0;) {
-    if (!is_child(m, deg, s, b, g.col, g.next, k)) continue;
-    const uint32_t c = g.col[b + s];
-    if (c != hk && g.hc[c] != FL_NONE && peek(g.cover + g.head_base[c]) == FL_SENT) return false;
-  }
-  return true;
-}
-__device__ __forceinline__ double da_over_fold(const fl_da_args& g, uint32_t k, double r) {
-  const uint32_t b = g.rp[k], deg = g.rp[k + 1] - b, hk = g.hc[k];
-  const unsigned long long m = g.cmask[k];
-  double acc = g.area[k];
-  for (uint32_t s = deg; s-- > 0;) {
-    if (!is_child(m, deg, s, b, g.col, g.next, k)) continue;
-    const uint32_t c = g.col[b + s];
-    if (g.hc[c] == FL_NONE) {
-      acc = acc + g.area[c];
-      continue;
+// A position with more light children than listed (rare): the wavefront walks its
+// row together, 64 entries at a time in fold order, one a lane.  Their chains' words
+// are in cover (a leaf's drainage area is its own), r is the heavy child's value.
+// k, its area a, its row and r are the same in every lane.  Bound by the latency of
+// three dependent loads per 64 entries; one lane on its own had them per entry: the
+// sweep of a hub with 20 000 leaves 15.3 -> 1.2 ms, solve of 30 000 sites in a chain
+// with nine leaves each 110 -> 39 ms.
+__device__ __forceinline__ double da_over_fold(const fl_da_args& g, uint32_t k, double a, uint32_t b, uint32_t deg,
+                                               uint32_t hk, double r, uint32_t lane) {
+  double acc = a;
+  for (uint32_t top = deg; top > 0; top -= min(top, 64u)) {
+    const bool in = lane < top;
+    const uint32_t c = g.col[b + (in ? top - 1 - lane : 0u)];
+    const bool kid = in && g.next[c] == k, leaf = g.hc[c] == FL_NONE, light = kid && !leaf && c != hk;
+    const double area = g.area[c];
+    double* w = g.cover + (light ? g.head_base[c] : 0u);
+    const double x = await(w, light, area, g.wait);
+    if (light) *reinterpret_cast<unsigned long long*>(w) = FL_SENT;
+    unsigned long long kids = __ballot(kid);
+    const unsigned long long heavy = __ballot(kid && !leaf && c == hk);
+    for (; kids; kids &= kids - 1) {
+      const uint32_t i = (uint32_t)__builtin_ctzll(kids);
+      acc = acc + (((heavy >> i) & 1ull) ? r : of_lane(x, i));
     }
-    if (c == hk) {
-      acc = acc + r;
-      continue;
-    }
-    double* w = g.cover + g.head_base[c];
-    acc = acc + bits_double(peek(w));
-    *reinterpret_cast<unsigned long long*>(w) = FL_SENT;
   }
   return acc;
 }
@@ -1634,26 +1653,30 @@ template <int B, bool up>
 __device__ __forceinline__ void da_tile_walk(const fl_da_args& g, const fl_da_pos (&t)[B], const uint32_t (&cn)[B],
                                              const bool (&mine)[B], const double (&pre)[B],
                                              const fl_da_words (&w)[B], bool tail, double carry, uint32_t lane, double (&r)[B]) {
-  uint32_t spins = 0;
-  for (;;) {
-    bool wait = false;
+  unsigned long long over[B];
+  uint32_t row[B], deg[B], hk[B];
 #pragma unroll
-    for (int b = 0; b < B; ++b)
-      wait = wait || (mine[b] && (cn[b] & FL_LIST_OVERFLOW) && !da_over_ready(g, t[b].k));
-    if (!__any(wait) || !wait_more(spins, g.wait)) break;
+  for (int b = 0; b < B; ++b) {
+    const bool o = mine[b] && (cn[b] & FL_LIST_OVERFLOW);
+    over[b] = __ballot(o);
+    row[b] = o ? g.rp[t[b].k] : 0u;
+    deg[b] = o ? g.rp[t[b].k + 1] - row[b] : 0u;
+    hk[b] = o ? g.hc[t[b].k] : 0u;
   }
+  const unsigned long long tails = __ballot(tail);
+  auto at = [](uint32_t v, uint32_t e) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)e); };
   double v = carry;
   for (uint32_t i = 0; i < 64; ++i) {
     const uint32_t e = up ? i : 63 - i;
-    if (lane == e) {
-      double x = tail ? FL_NEG0 : v;
+    if ((tails >> e) & 1ull) v = FL_NEG0;
 #pragma unroll
-      for (int b = 0; b < B; ++b)
-        r[b] = x = mine[b] && (cn[b] & FL_LIST_OVERFLOW) ? da_over_fold(g, t[b].k, x)
-                   : da_step<FL_LIST>(pre[b], w[b], x);
-      v = x;
+    for (int b = 0; b < B; ++b) {
+      if ((over[b] >> e) & 1ull)
+        v = da_over_fold(g, at(t[b].k, e), of_lane(t[b].area, e), at(row[b], e), at(deg[b], e), at(hk[b], e), v, lane);
+      else
+        v = of_lane(da_step<FL_LIST>(pre[b], w[b], v), e);
+      if (lane == e) r[b] = v;
     }
-    v = of_lane(v, e);
   }
 }
 
