@@ -44,16 +44,22 @@ def log(msg: str) -> None:
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
 
 
-def kernel_bytes_per_unit(name: str, n: int, nnz: int, clamp: bool, active: float = 1.0) -> float:
+def kernel_bytes_per_unit(name: str, n: int, nnz: int, clamp: bool, active: float = 1.0, chain: float = 1.0) -> float:
     """Algorithmic (compulsory) bytes per work item of one kernel: every array
     it must touch, read or written once; gathers that re-read an array are not
     counted.  Units are sites for the per-site kernels and chain positions
-    (sites inside basins, in chain-major order) for the sweeps; the profiler
-    accumulates the units of every launch.  deg = nnz / n adjacency entries.
-    `active`: the fraction of the sites whose basins are recomputed (the
-    per-site kernels of the decomposition read one flag for the others)."""
+    (the recomputed sites that are no leaves, in chain-major order) for the
+    sweeps; the profiler accumulates the units of every launch.  deg = nnz / n
+    adjacency entries.  `active`: the fraction of the sites whose basins are
+    recomputed (the per-site kernels of the decomposition read one flag for the
+    others); `chain`: the fraction at chain positions, the rest of the active ones
+    being leaves."""
     deg = nnz / max(n, 1)
-    a = active
+    a, c = active, min(chain, active)
+    leaf = a - c
+    # light children listed per position, in words of 8: the leaves, and the heads
+    # of chains (not counted)
+    listed = leaf / c if c else 0.0
     table = {
         # every site: is_outlet 1 + its neighbourhood flag 1 + the previous receiver and
         # distance 12, writes next 4 + dnext 8 + this iteration's flag 1; sites near a
@@ -64,32 +70,36 @@ def kernel_bytes_per_unit(name: str, n: int, nnz: int, clamp: bool, active: floa
         # row_ptr 4 + next 4 + previous area 8, writes cmask 8 + hc 4 and the two chain
         # pointers 16 (written by the parent); col 4 per entry; others copy their root 8
         "k_children": 6 + a * (44 + 4 * deg) + (1 - a) * 8,
-        # act 1; active (every site counted, leaves among them): the two pairs read 16 +
-        # written 16
-        "k_chain_jump": 1 + a * 32,
+        # act 1; chain positions: the two pairs read 16 + written 16 (the first round's
+        # words that tell the kinds are not counted)
+        "k_chain_jump": 1 + c * 32,
         # act 1 (the tails' extra reads are not counted)
         "k_bucket_count": 1,
         "k_bucket_place<true>": 1,
         "k_bucket_place<false>": 1,
-        # rt 8 + is_outlet 1 + cp 8 + head_base 4 + row_ptr 4 + cmask 8 + hc 4 + area 8 + col 4
-        # + K 8 + dnext 8, writes perm 4 + count 4 + area 8 + K 8 + dnext 8 + root 4 (+ U, tan,
-        # h read and four chain-major copies written with max slopes)
-        "k_chain_perm": 1 + a * (157 if clamp else 101),
-        # perm 4 + count 4 + area 8 + K 8 + dnext 8 + a listed child's A 8 (chain-major), writes
-        # A 8 + x 8
-        "k_da_fold": 56,
+        # act 1; active: next 4 + area 8, head_base 4, writes root 4 + spos 4; chain
+        # positions: rt 8 + cp 8 + row_ptr 4 + cmask 8 + hc 4 + K 8 + dnext 8 + col 4 per
+        # entry, writes perm 4 + count 4 + area 8 + K 8 + dnext 8 (+ U, tan, h read, their
+        # copies and the outlet's position 4 written with max slopes); leaves: writes A 8
+        # and the receiver's listed word 8
+        "k_chain_perm": 1 + a * 24 + c * (80 + 4 * deg + (52 if clamp else 0)) + leaf * 16,
+        # perm 4 + count 4 + area 8 + K 8 + dnext 8, each listed child's word 8 read and 8
+        # given back, writes A 8 + x 8 + the response time's empty word 8 (+ the elevation's)
+        "k_da_fold": 56 + 16 * listed + (8 if clamp else 0),
         # x 8, writes tau 8 (+ U, tan, d read and h written)
         "k_tau_fold<false>": 16,
         "k_tau_fold<true>": 48,
-        # the deep rounds of both sweeps, one launch each: as their round kernels
-        "k_da_tail": 56,
+        # rounds of both sweeps behind barriers: as their one-launch kernels
+        "k_da_tail": 56 + 16 * listed + (8 if clamp else 0),
         "k_tau_tail<false>": 16,
         "k_tau_tail<true>": 48,
-        # every site: act 1, clears a basin mark 1; active: rt 8 + cp 8 + head_base 4 +
-        # tau 8 + h 8 + U 8 (or the chain-major h 8), writes tau 8 + h 8 (the roots' values
-        # are shared), and a changed site (taken as every active one) row_ptr 8, col 4 per
-        # entry and its neighbourhood's flags 1 + 1 per entry; others copy h 16
-        "k_tau_scatter": 2 + a * (69 + 5 * deg) + (1 - a) * 16,
+        # every site: act 1, clears a basin mark 1; active: root 4 + spos 4 + h 8 + U 8,
+        # writes tau 8 + h 8 (the roots' and receivers' values are shared), and a changed
+        # site (taken as every active one) row_ptr 4, col 4 per entry and its neighbourhood's
+        # flags 1 + 1 per entry; chain positions: tau 8 (+ h 8 with max slopes); leaves: K 8 +
+        # area 8 + dnext 8 (+ tan 8); others copy h 16
+        "k_tau_scatter": 2 + a * (45 + 5 * deg) + c * (16 if clamp else 8) + leaf * (32 if clamp else 24)
+        + (1 - a) * 16,
     }
     return float(table.get(name, 0.0))
 
@@ -305,20 +315,23 @@ def profiled_roofline(L, ctx, t, n, nnz, clamp):
             prof[nm] = (cnt.value, ms.value, units.value)
     L.fl_ctx_set_profiling(ctx, 0)
     total_kernel_ms = sum(v[1] for v in prof.values())
+    positions = sum(prof[k][2] for k in ("k_da_fold", "k_da_tail") if k in prof)
+    chain = min(active, positions / (float(n) * max(st["iterations"], 1))) if n else 1.0
     for nm, (cnt, ms, units) in sorted(prof.items(), key=lambda kv: -kv[1][1]):
-        bpu = kernel_bytes_per_unit(nm, n, nnz, clamp, active)
+        bpu = kernel_bytes_per_unit(nm, n, nnz, clamp, active, chain)
         gbs = bpu * units / (ms / 1e3) / 1e9 if bpu and ms else 0.0
         log(f"  {nm:16s} launches={cnt:7d} total={ms:9.3f} ms avg={ms / cnt * 1e3:8.2f} us "
             f"units/launch={units / cnt:11.1f} {gbs:7.1f} GB/s")
     dom = max(prof.items(), key=lambda kv: kv[1][1])[0]
     dcnt, dms, dunits = prof[dom]
     avg_s = dms / dcnt / 1e3
-    bytes_per_launch = kernel_bytes_per_unit(dom, n, nnz, clamp, active) * dunits / dcnt
+    bytes_per_launch = kernel_bytes_per_unit(dom, n, nnz, clamp, active, chain) * dunits / dcnt
     achieved = bytes_per_launch / avg_s / 1e9 if bytes_per_launch else None
     roofline = {"bound": "hbm", "kernel": dom, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": (achieved / HBM_PEAK_GBS) if achieved else None, "traffic": None,
                 "algorithmic_bytes_per_launch": bytes_per_launch, "avg_launch_us": avg_s * 1e6,
-                "launches_per_solve": dcnt, "kernel_share": dms / total_kernel_ms if total_kernel_ms else None}
+                "launches_per_solve": dcnt, "recomputed_fraction": active, "chain_fraction": chain,
+                "kernel_share": dms / total_kernel_ms if total_kernel_ms else None}
     return roofline, total_kernel_ms
 
 
@@ -503,7 +516,7 @@ def main() -> int:
 
 
 TRAFFIC_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
-                               "k_da_fold_traffic_fbm1M.md")
+                               "traffic_fbm1M.md")
 
 
 def measured_traffic(kernel: str, algorithmic_bytes: float):

@@ -4,8 +4,8 @@ library's tuning table (fastlem_amd/csrc/fl_tuning_table.h).
 For every class -- single fBm terrains of 16,384 .. 1,048,576 sites, and
 batches of terrains with log-uniform site counts -- it builds the workload,
 uploads it, and calls the library's ``fl_autotune`` (coordinate descent over
-the per-site workgroup size, the short/long chain switch, the rounds merged
-into one launch per sweep, pipelining or graph replay and batch compaction,
+the per-site workgroup size, the short/long chain switch, the sweep rounds that
+synchronous iterations run behind barriers, pipelining or graph replay and batch compaction,
 each candidate timed over full solves and checked to give the same bits).
 Rows of the table cover the site counts between neighbouring classes.
 
@@ -13,7 +13,9 @@ Usage (on a GPU, from the repository root)::
 
     python -m fastlem_amd.autotune --out gpurun_out/fl_tuning_table.h
 
-then copy the file over fastlem_amd/csrc/fl_tuning_table.h and rebuild.
+then compare the file with fastlem_amd/csrc/fl_tuning_table.h: a value that gains
+a percent on a class's terrain here can lose on others of the class, so a row is
+taken over once other terrains of its sizes are not slower with it.
 """
 from __future__ import annotations
 
@@ -49,6 +51,12 @@ def header(rows: list[dict], source: str) -> str:
         "// and writes this file).  Rows are tried in order; the first whose",
         "// max_sites and terrain kind match a solve gives its tuning.  A tuning",
         "// shapes launches only: every row gives the same results.",
+        "//",
+        "// Workgroup sizes of the per-site kernels: smaller ones spread a small terrain",
+        "// over more compute units (fewer wavefronts of a workgroup wait for its slowest",
+        "// row); at hundreds of thousands of sites the sizes differ by under one percent.",
+        "// A row's two times: the table before it and its own tuning, another value of a",
+        "// parameter taken only where it is faster by more than one percent.",
         "//",
         f"// {source}",
         "#pragma once",

@@ -2611,7 +2611,7 @@ extern "C" int32_t fl_autotune(fl_ctx* c, fl_terrain* T, uint32_t repeats, fl_tu
   // coordinate descent, two passes; a candidate replaces the current one
   // only when it is faster by more than 1% (timing noise)
   const std::vector<uint32_t> chains = {6, 8, 12, 16, 24, 33}, tails = {0, 8, 16, 32, 64},
-                              blocks = {128, 256, 512, 1024}, pipes = {1, 3},
+                              blocks = {64, 128, 256, 512, 1024}, pipes = {1, 3},
                               compacts = {16384, 65536, 262144, 0xffffffffu};
   for (int pass = 0; pass < 2 && rc == FL_OK; pass++) {
     auto sweep = [&](uint32_t fl_tuning::*field, const std::vector<uint32_t>& values) {
