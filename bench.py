@@ -521,21 +521,18 @@ TRAFFIC_PROFILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "prof
 
 def measured_traffic(kernel: str, algorithmic_bytes: float):
     """HBM bytes per launch of ``kernel`` as recorded by the committed counter
-    summary (lines ``traffic_kernel:``, ``traffic_algorithmic_bytes:`` and
-    ``traffic_bytes_per_launch:``).  Used only when the summary was made for the
-    same kernel and the same work per launch (algorithmic bytes within 1%);
-    otherwise None."""
+    summary (a line ``traffic: <kernel> <algorithmic bytes> <bytes per launch>``).
+    Used only when the summary was made for the same kernel and the same work per
+    launch (algorithmic bytes within 1%); otherwise None."""
     try:
         with open(TRAFFIC_PROFILE) as f:
-            fields = dict(line.split(":", 1) for line in f if line.startswith("traffic_"))
-        if fields["traffic_kernel"].strip() != kernel:
-            return None
-        ref = float(fields["traffic_algorithmic_bytes"])
-        if abs(ref - algorithmic_bytes) > 0.01 * algorithmic_bytes:
-            return None
-        return float(fields["traffic_bytes_per_launch"])
-    except (OSError, KeyError, ValueError):
-        return None
+            rows = [line.split()[1:] for line in f if line.startswith("traffic:")]
+        for name, ref, measured in rows:
+            if name == kernel and abs(float(ref) - algorithmic_bytes) <= 0.01 * algorithmic_bytes:
+                return float(measured)
+    except (OSError, ValueError):
+        pass
+    return None
 
 
 def copy_calibration() -> int:
