@@ -9,7 +9,7 @@ import numpy as np
 
 from . import _native
 from ._native import TerrainDesc, check, ptr
-from .generator import UNBOUNDED, ParameterArrays, context, make_desc
+from .generator import UNBOUNDED, ParameterArrays, _Context, context, make_desc
 
 
 class DeviceTerrain:
@@ -39,6 +39,7 @@ class DeviceTerrain:
         h = ctypes.c_void_p()
         check(_native.lib().fl_terrain_create(self._ctx, ctypes.byref(desc), ctypes.byref(h)))
         self._h = h
+        _Context.hold(self)
         self.max_iteration = max_iteration
 
     @staticmethod
@@ -163,6 +164,7 @@ class DeviceBatch:
         h = ctypes.c_void_p()
         check(_native.lib().fl_batch_create(self._ctx, descs, len(terrains), ctypes.byref(h)))
         self._h = h
+        _Context.hold(self)
 
     @staticmethod
     def terrain_of(w, init_elevation=None, max_iteration: int = UNBOUNDED) -> dict:

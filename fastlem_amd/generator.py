@@ -11,6 +11,7 @@ from __future__ import annotations
 import atexit
 import ctypes
 import threading
+import weakref
 from typing import Optional, Sequence
 
 import numpy as np
@@ -56,12 +57,19 @@ class _Context:
     Calls on one context must not overlap (its stream and host slots are
     shared by everything the call enqueues), and ctypes releases the GIL
     during foreign calls, so every thread gets a context of its own; their
-    work overlaps on the device.  Contexts live until the interpreter exits.
+    work overlaps on the device.  Contexts live until the interpreter exits;
+    what is on one of them by then (``hold``) is closed before it goes.
     """
 
     _local = threading.local()
     _lock = threading.Lock()
     _all: list = []
+    _held: weakref.WeakSet = weakref.WeakSet()
+
+    @classmethod
+    def hold(cls, owner):
+        with cls._lock:
+            cls._held.add(owner)
 
     @classmethod
     def get(cls):
@@ -77,6 +85,8 @@ class _Context:
     @classmethod
     def _destroy_all(cls):
         with cls._lock:
+            for owner in list(cls._held):
+                owner.close()
             for h in cls._all:
                 _native.lib().fl_ctx_destroy(h)
             cls._all.clear()
