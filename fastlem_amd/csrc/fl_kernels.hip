@@ -97,8 +97,9 @@ __device__ __forceinline__ bool pair_fin(unsigned long long p) { return (p >> 63
 // Kinds of an active site (act).  A leaf has no children: its drainage area is
 // its own area, and its response time and elevation follow from its receiver's
 // alone, so it is on no chain (two of three sites are leaves): chains, sweeps
-// and pointer jumping have the other sites only.  At a chain's tail every child
-// is a leaf.
+// and pointer jumping have the other sites only.  A chain ends at a site whose
+// heavy child is a leaf, which is then one more of its listed children (the others,
+// chosen light by the previous areas, may head chains of their own).
 #define FL_ACTIVE 1u
 #define FL_LEAF 2u
 #define FL_CHAIN_END 4u
@@ -1793,7 +1794,7 @@ __global__ void __launch_bounds__(64 * FL_FOLD_WAVES)
 k_da_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_da_args g) {
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   const uint32_t deepest = *f.maxld;
-  if (*guard != 0) return;  // pointer jumping has not converged: the iteration is redone
+  if (*guard != 0) return;  // the iteration is redone
   const uint32_t rounds = deepest < cap ? deepest + 1 : cap;
   const uint32_t total = f.ucum[rounds];
   fl_rounds R = load_rounds(f, 0, rounds, lane);
@@ -1824,7 +1825,7 @@ k_da_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_da_arg
 __global__ void __launch_bounds__(64 * FL_TAIL_WAVES)
 k_da_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, fl_flow f, fl_da_args g) {
   const uint32_t top = *f.maxld;
-  if (*guard != 0 || top > 0xfffffffeu) return;  // pointer jumping has not converged: the iteration is redone
+  if (*guard != 0 || top > 0xfffffffeu) return;  // the iteration is redone
   const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
   for (uint32_t l = top + 1; l-- > lsplit;) {
     const uint32_t n = f.ucum[l + 1] - f.ucum[l];
@@ -2087,7 +2088,7 @@ __global__ void __launch_bounds__(64 * FL_FOLD_WAVES)
 k_tau_fold(const uint32_t* __restrict__ guard, uint32_t cap, fl_flow f, fl_tau_args g) {
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   const uint32_t deepest = *f.maxld;
-  if (*guard != 0) return;  // pointer jumping has not converged: the iteration is redone
+  if (*guard != 0) return;  // the iteration is redone
   const uint32_t rounds = deepest < cap ? deepest + 1 : cap;
   const uint32_t total = f.ucum[rounds];
   fl_rounds R = load_rounds(f, 0, rounds, lane);
@@ -2113,7 +2114,7 @@ template <bool clamp>
 __global__ void __launch_bounds__(64 * FL_TAIL_WAVES)
 k_tau_tail(const uint32_t* __restrict__ guard, uint32_t lsplit, fl_flow f, fl_tau_args g) {
   const uint32_t top = *f.maxld;
-  if (*guard != 0 || top > 0xfffffffeu) return;  // pointer jumping has not converged: the iteration is redone
+  if (*guard != 0 || top > 0xfffffffeu) return;  // the iteration is redone
   const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
   for (uint32_t l = lsplit; l <= top; ++l) {
     const uint32_t n = f.ucum[l + 1] - f.ucum[l];
