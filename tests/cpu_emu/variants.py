@@ -6,6 +6,7 @@ from __future__ import annotations
 import ctypes
 import os
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 
 from fastlem_amd import _native
 
@@ -27,14 +28,20 @@ def lib(name: str, source: str = "", header: str = "", **macros):
         headers += [os.path.join(_build.HERE, header)] if header else []
         headers += [os.path.join(_build.HERE, "include", "hip", "hip_runtime.h"), os.path.abspath(__file__)]
         if not os.path.exists(out) or os.path.getmtime(out) < max(map(os.path.getmtime, srcs + headers)):
-            cmd = ["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-pthread", "-ffp-contract=off", "-fno-fast-math",
-                   "-U_FORTIFY_SOURCE", "-D_FORTIFY_SOURCE=0", "-fno-omit-frame-pointer", "-w",
-                   "-I", os.path.join(_build.HERE, "include"), "-I", os.path.join(_build.ROOT, "include")]
-            cmd += [f"-D{k}={v}" for k, v in macros.items()]
-            cmd += ["-include", os.path.join(_build.HERE, header)] if header else []
-            for s in srcs:
-                cmd += ["-x", "c++", s, "-x", "none"] if s.endswith(".hip") else [s]
-            subprocess.run(cmd + ["-o", out + ".tmp"], check=True)
+            flags = ["-std=c++17", "-O1", "-fPIC", "-pthread", "-ffp-contract=off", "-fno-fast-math",
+                     "-U_FORTIFY_SOURCE", "-D_FORTIFY_SOURCE=0", "-fno-omit-frame-pointer", "-w",
+                     "-I", os.path.join(_build.HERE, "include"), "-I", os.path.join(_build.ROOT, "include")]
+            flags += [f"-D{k}={v}" for k, v in macros.items()]
+            flags += ["-include", os.path.join(_build.HERE, header)] if header else []
+            objects = [f"{out}.{os.path.basename(src)}.o" for src in srcs]
+
+            def compile_one(src, obj):
+                lang = ["-x", "c++"] if src.endswith(".hip") else []
+                subprocess.run(["g++"] + flags + lang + ["-c", src, "-o", obj], check=True)
+
+            with ThreadPoolExecutor(4) as pool:
+                list(pool.map(compile_one, srcs, objects))
+            subprocess.run(["g++", "-shared", "-pthread"] + objects + ["-o", out + ".tmp"], check=True)
             os.replace(out + ".tmp", out)
         _libs[name] = _native._declare(ctypes.CDLL(out))
     return _libs[name]

@@ -5,7 +5,6 @@ take two and three rounds (64 otherwise), with lakes that last, alone and in
 unions; bit for bit against the oracle."""
 import pytest
 
-from cpu_emu import emu, variants
 from test_cpu_emulation import _emu_solve
 from test_lasting_lakes import _terrain
 from test_sweeps import _check
@@ -16,6 +15,8 @@ CASES = [(30, 8, 6, 2, True, 42), (30, 8, 6, 2, True, 52), (25, 25, 8, 3, False,
 
 
 def _solve(rounds, ts, **kw):
+    from cpu_emu import emu, variants
+
     L = variants.lib(f"scan{rounds}", FL_SCAN_ROUNDS=rounds) if rounds else emu.lib()
     _check(lambda x: _emu_solve(L, x, **kw), ts)
     return _emu_solve.last_stats

@@ -7,7 +7,6 @@ import ctypes
 import numpy as np
 import pytest
 
-from cpu_emu import emu, variants
 from test_lasting_lakes import _terrain
 from test_sweeps import _reference
 
@@ -16,6 +15,8 @@ class _Polls:
     """The library with the number of sweep launches and those whose waits are short."""
 
     def __init__(self):
+        from cpu_emu import variants
+
         self.lib = variants.lib("polls", source="polls.cpp", header="polls.h", FL_SPIN_FOLD="flemu_polls()")
         self._at = lambda name: ctypes.c_uint32.in_dll(self.lib, name)
 
@@ -31,6 +32,7 @@ class _Polls:
 def test_after_the_last_iteration(nx, ny, seed):
     """Every basin recomputed in every iteration: the one in flight when the solve
     ends has the whole terrain's sweeps."""
+    from cpu_emu import emu
     from fastlem_amd import _native
     from fastlem_amd.device import batch_descs
 

@@ -9,7 +9,6 @@ import ctypes
 import numpy as np
 import pytest
 
-from cpu_emu import emu, variants
 from test_cpu_emulation import _emu_solve
 from test_lasting_lakes import _terrain as lakes
 from test_long_chains import _chain
@@ -18,6 +17,8 @@ from test_sweeps import _check, _reference
 
 
 def _ended():
+    from cpu_emu import variants
+
     return variants.lib("ended_waits", FL_SPIN_FOLD=1)
 
 
@@ -39,6 +40,7 @@ CASES = {
 
 @pytest.mark.parametrize("case", CASES)
 def test_solved_again(case):
+    from cpu_emu import emu
     from fastlem_amd import _native
 
     L, t = _ended(), CASES[case]()

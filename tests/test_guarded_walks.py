@@ -4,12 +4,12 @@ compiled against the HIP subset in cpu_emu)."""
 import os
 import subprocess
 
-from cpu_emu import build as emu_build
-
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 def test_no_walk_behind_the_guard(tmp_path):
+    from cpu_emu import build as emu_build
+
     exe = tmp_path / "guarded_walk"
     subprocess.run(["g++", "-std=c++17", "-O1", "-ffp-contract=off", "-fno-fast-math", "-U_FORTIFY_SOURCE",
                     "-D_FORTIFY_SOURCE=0", "-w", "-pthread", "-I", os.path.join(HERE, "cpu_emu", "include"),

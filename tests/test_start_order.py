@@ -5,7 +5,6 @@ host synchronisations as in the usual order (an ended wait takes more)."""
 import numpy as np
 import pytest
 
-from cpu_emu import emu, variants
 from test_cpu_emulation import _emu_solve
 from test_lasting_lakes import _terrain as lakes
 from test_long_chains import _chain
@@ -32,6 +31,8 @@ CASES = {
 
 @pytest.mark.parametrize("case", CASES)
 def test_last_workgroup_first(case):
+    from cpu_emu import emu, variants
+
     syncs = []
 
     def solve(L):
