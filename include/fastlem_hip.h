@@ -155,8 +155,8 @@ int32_t fl_ctx_set_rehint_rounds(fl_ctx *ctx, uint32_t rounds);
  * same bits); they shape the work:
  *   site_block        workgroup size of the per-site kernels (64..1024, a
  *                     multiple of 64);
- *   long_chain        chains of at least this many sites take a wavefront
- *                     each in the sweeps, shorter ones share tiles of 64
+ *   long_chain        chains of at least this many sites have wavefronts of
+ *                     their own in the sweeps, shorter ones share tiles of 64
  *                     positions (>= 1; more than 33 acts as 33);
  *   tail_units        iterations whose sizes the host reads first (a
  *                     solve's first ones): deep sweep rounds of at most
@@ -164,8 +164,8 @@ int32_t fl_ctx_set_rehint_rounds(fl_ctx *ctx, uint32_t rounds);
  *                     barrier between rounds;
  *   pipelining        0, 1 or 3 as fl_ctx_set_pipelining (3: HIP graphs);
  *   compact_min_idle  batches: as fl_ctx_set_batch_compaction.
- * Without fl_ctx_set_tuning a solve takes the library's table, chosen by
- * fl_autotune per workload class (site count, one terrain or a batch);
+ * Without fl_ctx_set_tuning a solve takes the library's table, a row per
+ * workload class (site count, one terrain or a batch);
  * fl_ctx_set_pipelining / fl_ctx_set_batch_compaction override those fields. */
 typedef struct fl_tuning {
   uint32_t site_block, long_chain, tail_units, pipelining, compact_min_idle;
