@@ -143,7 +143,9 @@ struct fl_terrain {
   // cutoff): another tuning captures afresh, so that it is the one timed
   uint32_t gB[3] = {0, 0, 0}, gL[3] = {0, 0, 0};
   uint32_t* h_tslot[2] = {nullptr, nullptr};  // pinned per-terrain changed flags of iterations in flight
-  uint8_t* h_mask = nullptr;                  // pinned staging of the active mask
+  // pinned staging of the active mask, one per flight slot: a flight's copy from it
+  // may run as late as the flight
+  uint8_t* h_mask[2] = {nullptr, nullptr};
   bool graphs_failed = false;
   bool have_order = false;
   // statistics of the last solve
@@ -1298,7 +1300,7 @@ int32_t alloc_device(fl_ctx* c, fl_terrain* P, uint32_t n, uint32_t nnz, uint32_
     if (count > c->pin_cap) {
       const uint32_t cap = std::max<uint32_t>({count, 2 * c->pin_cap, 1024});
       void* block = nullptr;
-      HIPCHK(hipHostMalloc(&block, (size_t)cap * 13, hipHostMallocDefault));
+      HIPCHK(hipHostMalloc(&block, (size_t)cap * 14, hipHostMallocDefault));
       c->pin_blocks.push_back(block);
       c->pin = (uint8_t*)block;
       c->pin_cap = cap;
@@ -1306,7 +1308,8 @@ int32_t alloc_device(fl_ctx* c, fl_terrain* P, uint32_t n, uint32_t nnz, uint32_
     P->h_tchanged = (uint32_t*)c->pin;
     P->h_tslot[0] = P->h_tchanged + c->pin_cap;
     P->h_tslot[1] = P->h_tslot[0] + c->pin_cap;
-    P->h_mask = (uint8_t*)(P->h_tslot[1] + c->pin_cap);
+    P->h_mask[0] = (uint8_t*)(P->h_tslot[1] + c->pin_cap);
+    P->h_mask[1] = P->h_mask[0] + c->pin_cap;
   }
   hipStream_t s = c->stream;
   // basin roots are site indices at all times (dirty-basin marks index by them)
@@ -1826,10 +1829,11 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
   std::vector<uint8_t> dev_mask(cur->t_active);  // the mask the device holds
   int next_slot = 0;
   bool drain = false;  // stop enqueueing: a compaction waits for the flights to land
-  auto upload_mask = [&](const std::vector<uint8_t>& m) -> int32_t {
+  // (slot: the flight's, or any when none is in flight)
+  auto upload_mask = [&](const std::vector<uint8_t>& m, int slot) -> int32_t {
     if (!cur->d_active || m == dev_mask) return FL_OK;
-    std::copy(m.begin(), m.end(), cur->h_mask);
-    HIPCHK(hipMemcpyAsync(cur->d_active, cur->h_mask, cur->nterr, hipMemcpyHostToDevice, s));
+    std::copy(m.begin(), m.end(), cur->h_mask[slot]);
+    HIPCHK(hipMemcpyAsync(cur->d_active, cur->h_mask[slot], cur->nterr, hipMemcpyHostToDevice, s));
     dev_mask = m;
     return FL_OK;
   };
@@ -1858,7 +1862,7 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
     if (it == 0 || ((cur->hint_stale || cur->barrier_its) && q.empty()) || !c->pipelined) {
       bool changed = false, lake = false;
       std::vector<uint8_t> mask(cur->t_active);
-      FLCHK(upload_mask(mask));
+      FLCHK(upload_mask(mask, 0));
       set_slots(cur, hin);
       const bool full = !cur->prev_valid || c->recompute_all;
       const bool keep = !full && !cur->after_lake;
@@ -1883,7 +1887,7 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
           any |= mask[g] != 0;
         }
         if (!any) break;
-        FLCHK(upload_mask(mask));
+        FLCHK(upload_mask(mask, next_slot));
         Flight f;
         f.in = q.empty() ? hin : (q.back().in + 1) % 3;
         f.slot = next_slot;
@@ -1911,7 +1915,7 @@ int32_t solve_union(fl_ctx* c, fl_terrain* T, const uint32_t* max_it) {
           for (uint32_t g = 0; g < cur->nterr; g++) enq[g] -= x.mask[g];
         FLCHK(drop_flights(c, cur, q));
         T->stat_redone++;
-        FLCHK(upload_mask(f.mask));
+        FLCHK(upload_mask(f.mask, 0));
         set_slots(cur, f.in);
         FLCHK(one_iteration(c, cur, f.full, f.keep, &changed, &lake));
         cur->after_lake = lake;
@@ -1998,11 +2002,12 @@ struct fl_lane {
 
 namespace {
 
-int32_t lane_upload_mask(fl_lane* L, const std::vector<uint8_t>& m) {
+// (slot: the flight's, or any when none is in flight)
+int32_t lane_upload_mask(fl_lane* L, const std::vector<uint8_t>& m, int slot) {
   fl_terrain* cur = L->cur;
   if (m == L->dev_mask) return FL_OK;
-  std::copy(m.begin(), m.end(), cur->h_mask);
-  HIPCHK(hipMemcpyAsync(cur->d_active, cur->h_mask, cur->nterr, hipMemcpyHostToDevice, L->c->stream));
+  std::copy(m.begin(), m.end(), cur->h_mask[slot]);
+  HIPCHK(hipMemcpyAsync(cur->d_active, cur->h_mask[slot], cur->nterr, hipMemcpyHostToDevice, L->c->stream));
   L->dev_mask = m;
   return FL_OK;
 }
@@ -2221,7 +2226,7 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
   const double* result = nullptr;  // the buffer holding the confirmed iteration's elevations
   if (L->sync_next || ((cur->hint_stale || cur->barrier_its) && L->q.empty()) || !c->pipelined) {
     std::vector<uint8_t> mask(cur->t_active);
-    FLCHK(lane_upload_mask(L, mask));
+    FLCHK(lane_upload_mask(L, mask, 0));
     set_slots(cur, L->hin);
     const bool full = !cur->prev_valid || c->recompute_all;
     const bool keep = !full && !cur->after_lake;
@@ -2245,7 +2250,7 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
         any |= mask[g] != 0;
       }
       if (!any) break;
-      FLCHK(lane_upload_mask(L, mask));
+      FLCHK(lane_upload_mask(L, mask, L->next_slot));
       Flight f;
       f.in = L->q.empty() ? L->hin : (L->q.back().in + 1) % 3;
       f.slot = L->next_slot;
@@ -2273,7 +2278,7 @@ int32_t fl_lane_step(fl_lane* L, std::vector<fl_lane_member>& stopped) {
         for (uint32_t g = 0; g < cur->nterr; g++) L->enq[g] -= x.mask[g];
       FLCHK(drop_flights(c, cur, L->q));
       cur->stat_redone++;
-      FLCHK(lane_upload_mask(L, f.mask));
+      FLCHK(lane_upload_mask(L, f.mask, 0));
       set_slots(cur, f.in);
       FLCHK(one_iteration(c, cur, f.full, f.keep, &changed, &lake));
       cur->after_lake = lake;

@@ -10,6 +10,7 @@
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
+#include <deque>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -208,10 +209,60 @@ thread_local std::vector<std::function<void()>>* g_capture = nullptr;
 
 void run_launch(dim3 grid, dim3 block, const std::function<void()>& body);
 
+// FLEMU_LATE: work enqueued on a stream runs at the last moment, when the host
+// waits for it (or frees memory, or copies to pageable memory); pinned host memory
+// is read and written then, pageable memory when the copy is enqueued.
+#ifdef FLEMU_LATE
+std::recursive_mutex g_late_mu;
+std::deque<std::function<void()>> g_late;
+uint64_t g_late_done = 0;
+std::vector<std::pair<const char*, size_t>> g_pinned;
+bool late() { return true; }
+void enqueue(std::function<void()> f) {
+  std::lock_guard<std::recursive_mutex> lk(g_late_mu);
+  g_late.push_back(std::move(f));
+}
+uint64_t enqueued() {
+  std::lock_guard<std::recursive_mutex> lk(g_late_mu);
+  return g_late_done + g_late.size();
+}
+void catch_up(uint64_t to) {
+  std::lock_guard<std::recursive_mutex> lk(g_late_mu);
+  while (!g_late.empty() && g_late_done < to) {
+    std::function<void()> f = std::move(g_late.front());
+    g_late.pop_front();
+    g_late_done++;
+    f();
+  }
+}
+bool pinned(const void* p) {
+  std::lock_guard<std::recursive_mutex> lk(g_late_mu);
+  for (auto& b : g_pinned)
+    if (p >= b.first && p < b.first + b.second) return true;
+  return false;
+}
+void pin(const void* p, size_t bytes) {
+  std::lock_guard<std::recursive_mutex> lk(g_late_mu);
+  g_pinned.push_back({(const char*)p, bytes});
+}
+#else
+bool late() { return false; }
+void enqueue(std::function<void()>) {}
+uint64_t enqueued() { return 0; }
+void catch_up(uint64_t) {}
+bool pinned(const void*) { return true; }
+void pin(const void*, size_t) {}
+#endif
+
 void launch(dim3 grid, dim3 block, const std::function<void()>& body) {
   if (g_capture) {
     std::function<void()> b = body;
     g_capture->push_back([grid, block, b]() { run_launch(grid, block, b); });
+    return;
+  }
+  if (late()) {
+    std::function<void()> b = body;
+    enqueue([grid, block, b]() { run_launch(grid, block, b); });
     return;
   }
   run_launch(grid, block, body);
@@ -280,6 +331,7 @@ struct ihipStream_t {
 };
 struct ihipEvent_t {
   std::chrono::steady_clock::time_point t;
+  uint64_t after = 0;  // (FLEMU_LATE) the work before it
 };
 
 namespace {
@@ -300,10 +352,15 @@ hipError_t hipMalloc(void** p, size_t bytes) {
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {
+  flemu::catch_up(~0ull);
   std::free(p);
   return hipSuccess;
 }
-hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) { return hipMalloc(p, bytes); }
+hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) flemu::pin(*p, bytes ? bytes : 1);
+  return e;
+}
 hipError_t hipHostFree(void* p) { return hipFree(p); }
 struct ihipGraph_t {
   std::vector<std::function<void()>> work;
@@ -312,11 +369,21 @@ struct ihipGraphExec_t {
   std::vector<std::function<void()>> work;
 };
 
-hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind, hipStream_t) {
+hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t) {
   if (flemu::g_capture) {
     flemu::g_capture->push_back([=]() {
       if (bytes) std::memmove(dst, src, bytes);
     });
+    return hipSuccess;
+  }
+  if (flemu::late() && bytes) {
+    if (kind == hipMemcpyHostToDevice && !flemu::pinned(src)) {
+      std::vector<char> staged((const char*)src, (const char*)src + bytes);
+      flemu::enqueue([=]() { std::memcpy(dst, staged.data(), bytes); });
+      return hipSuccess;
+    }
+    flemu::enqueue([=]() { std::memmove(dst, src, bytes); });
+    if (kind == hipMemcpyDeviceToHost && !flemu::pinned(dst)) flemu::catch_up(~0ull);
     return hipSuccess;
   }
   if (bytes) std::memmove(dst, src, bytes);
@@ -340,7 +407,10 @@ hipError_t hipGraphInstantiate(hipGraphExec_t* exec, hipGraph_t graph, hipGraphN
   return hipSuccess;
 }
 hipError_t hipGraphLaunch(hipGraphExec_t exec, hipStream_t) {
-  for (auto& f : exec->work) f();
+  for (auto& f : exec->work) {
+    if (flemu::late()) flemu::enqueue(f);
+    else f();
+  }
   return hipSuccess;
 }
 hipError_t hipGraphDestroy(hipGraph_t graph) {
@@ -352,10 +422,16 @@ hipError_t hipGraphExecDestroy(hipGraphExec_t exec) {
   return hipSuccess;
 }
 hipError_t hipMemcpy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
-  return hipMemcpyAsync(dst, src, bytes, kind, nullptr);
+  hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, nullptr);
+  flemu::catch_up(~0ull);
+  return e;
 }
 hipError_t hipMemsetAsync(void* dst, int value, size_t bytes, hipStream_t) {
   if (flemu::g_capture) return hipErrorInvalidValue;  // no memset nodes in captured work
+  if (flemu::late()) {
+    flemu::enqueue([=]() { std::memset(dst, value, bytes); });
+    return hipSuccess;
+  }
   if (bytes) std::memset(dst, value, bytes);
   return hipSuccess;
 }
@@ -364,11 +440,15 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t s) {
+  flemu::catch_up(~0ull);
   delete s;
   return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) {
+  flemu::catch_up(~0ull);
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() { return hipStreamSynchronize(nullptr); }
 hipError_t hipEventCreate(hipEvent_t* e) {
   *e = new ihipEvent_t();
   return hipSuccess;
@@ -380,9 +460,13 @@ hipError_t hipEventDestroy(hipEvent_t e) {
 }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
   e->t = std::chrono::steady_clock::now();
+  e->after = flemu::enqueued();
   return hipSuccess;
 }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  flemu::catch_up(e->after);
+  return hipSuccess;
+}
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
   *ms = std::chrono::duration<float, std::milli>(b->t - a->t).count();
   return hipSuccess;

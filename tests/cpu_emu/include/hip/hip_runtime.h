@@ -86,6 +86,7 @@ namespace flemu {
 extern dim3 g_block, g_bdim, g_gdim;
 extern dim3* g_tid;
 void launch(dim3 grid, dim3 block, const std::function<void()>& body);
+void catch_up(uint64_t to);  // (emu.cpp, FLEMU_LATE) runs the work enqueued so far
 void block_barrier();
 int wave_any(int pred);
 unsigned long long wave_ballot(int pred);

@@ -40,6 +40,7 @@ struct DeviceRadixSort {
       temp_bytes = 16;
       return hipSuccess;
     }
+    flemu::catch_up(~0ull);
     std::vector<int> idx(n);
     std::iota(idx.begin(), idx.end(), 0);
     std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) {
@@ -67,6 +68,7 @@ struct DeviceScan {
       temp_bytes = 16;
       return hipSuccess;
     }
+    flemu::catch_up(~0ull);
     T acc = T(0);
     for (int i = 0; i < n; i++) {
       acc = acc + in[i];
@@ -82,6 +84,7 @@ struct DeviceScan {
       temp_bytes = 16;
       return hipSuccess;
     }
+    flemu::catch_up(~0ull);
     T acc = T(0);
     for (int i = 0; i < n; i++) {
       const T v = in[i];
