@@ -33,7 +33,8 @@ def lib(name: str, source: str = "", header: str = "", **macros):
                      "-I", os.path.join(_build.HERE, "include"), "-I", os.path.join(_build.ROOT, "include")]
             flags += [f"-D{k}={v}" for k, v in macros.items()]
             flags += ["-include", os.path.join(_build.HERE, header)] if header else []
-            objects = [f"{out}.{os.path.basename(src)}.o" for src in srcs]
+            tmp = f"{out}.{os.getpid()}"  # (several processes may build it at a time)
+            objects = [f"{tmp}.{os.path.basename(src)}.o" for src in srcs]
 
             def compile_one(src, obj):
                 lang = ["-x", "c++"] if src.endswith(".hip") else []
@@ -41,7 +42,9 @@ def lib(name: str, source: str = "", header: str = "", **macros):
 
             with ThreadPoolExecutor(4) as pool:
                 list(pool.map(compile_one, srcs, objects))
-            subprocess.run(["g++", "-shared", "-pthread"] + objects + ["-o", out + ".tmp"], check=True)
-            os.replace(out + ".tmp", out)
+            subprocess.run(["g++", "-shared", "-pthread"] + objects + ["-o", tmp], check=True)
+            for obj in objects:
+                os.remove(obj)
+            os.replace(tmp, out)
         _libs[name] = _native._declare(ctypes.CDLL(out))
     return _libs[name]
